@@ -1,0 +1,473 @@
+"""Workloads whose speed is watched: what a user of this framework has it do, from one small
+matrix to a training step of the AlexNet shape at batch 256, through the public entry points.
+
+A case is a dict of plain values; its "kind" says which path it takes:
+
+  minibatches  a small network trained on a few host minibatches through the C++ host layer
+               (`hostapi.Net`): load, step, load, step, ..., then the probabilities and the
+               weights are read back
+  alexnet      the AlexNet-shaped network through the C ABI on device-resident tensors, as an
+               engine that links the library issues it: a training step (forward, backward,
+               SGD) or the forward pass alone, operator by operator or with the fused operators
+  sgemm        one matrix product
+  conv         one convolution layer: forward, data, filter and bias gradient
+  norm_pool    a normalisation and a pooling layer, forward and backward
+  matrix       the element-wise, broadcast, reduction, arg-max, soft-max and transpose operators
+               on one matrix
+
+Tensors are fp32, the only type of the operator path, column-major with dimension 0 fastest: a
+torch tensor of the reversed shape has the same bytes.
+"""
+import math
+
+import torch
+
+from minerva_amd import capi, configs, hostapi
+
+#: Layers of the AlexNet shape: (channels in, channels out, filter, pad, stride, pooled after).
+ALEXNET_CONVS = [(3, 96, 11, 0, 4, True), (96, 256, 5, 2, 1, True), (256, 384, 3, 1, 1, False),
+                 (384, 384, 3, 1, 1, False), (384, 256, 3, 1, 1, True)]
+ALEXNET_FCS = [(9216, 4096), (4096, 4096), (4096, 1000)]
+
+
+def listed():
+    return [
+        # The two MNIST networks of the reference's applications on their own batch: short
+        # operators, where launches, latency and the host layer count.
+        {"name": "mlp_b256", "kind": "minibatches", "net": "mlp", "batch": 256, "variant": 0, "steps": 4},
+        {"name": "cnn_b256", "kind": "minibatches", "net": "cnn", "batch": 256, "variant": 0, "steps": 4},
+        # The headline workload of the benchmark: one training step at batch 256.
+        {"name": "alexnet_train_b256", "kind": "alexnet", "batch": 256, "train": True, "fused": False},
+        # The same network on a smaller, uneven batch (what is left of a data set, or a share of
+        # a larger batch) with the fused operators.
+        {"name": "alexnet_train_fused_b50", "kind": "alexnet", "batch": 50, "train": True, "fused": True},
+        # Classification of single images, and of the ten views that a multi-view test scores.
+        {"name": "alexnet_forward_b1", "kind": "alexnet", "batch": 1, "train": False, "fused": True},
+        {"name": "alexnet_forward_b10", "kind": "alexnet", "batch": 10, "train": False, "fused": False},
+        # The matrix product: the benchmark's large square one, and an uneven one with a batch of
+        # 250 columns as an inner product over minibatches asks for it.
+        {"name": "sgemm_4096", "kind": "sgemm", "m": 4096, "n": 4096, "k": 4096},
+        {"name": "sgemm_1001x250x4099", "kind": "sgemm", "m": 1001, "n": 250, "k": 4099},
+        # A convolution layer of a deep network of 3 x 3 filters at a usual training batch.
+        {"name": "conv3x3_56_b32", "kind": "conv", "images": 32, "cin": 128, "cout": 256, "height": 56,
+         "width": 56, "filter": 3, "pad": 1, "stride": 1},
+        # norm1 and pool1 of the Caffe-style AlexNet at batch 256.
+        {"name": "norm_pool_55_b256", "kind": "norm_pool", "images": 256, "channels": 96, "height": 55,
+         "width": 55},
+        # The bandwidth-bound operators on the benchmark's 8192 x 8192 matrix and on a small,
+        # uneven one.
+        {"name": "matrix_8192", "kind": "matrix", "m": 8192, "n": 8192},
+        {"name": "matrix_1000x257", "kind": "matrix", "m": 1000, "n": 257},
+    ]
+
+
+def _between(rng, low, high):
+    """A whole number of [low, high], evenly spread over its logarithm."""
+    return min(high, max(low, int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))))
+
+
+def draw(rng):
+    kind = rng.choice(["minibatches", "alexnet", "alexnet", "sgemm", "sgemm", "conv", "conv", "norm_pool", "matrix"])
+    if kind == "minibatches":
+        net = rng.choice(["mlp", "cnn"])
+        return {"kind": kind, "net": net, "batch": _between(rng, 16, 512),
+                "variant": rng.randrange(2) if net == "cnn" else 0, "steps": rng.randrange(2, 6)}
+    if kind == "alexnet":
+        train = rng.random() < 0.5
+        return {"kind": kind, "batch": _between(rng, 8, 250) if train else _between(rng, 2, 250), "train": train,
+                "fused": rng.random() < 0.5}
+    if kind == "sgemm":
+        return {"kind": kind, "m": _between(rng, 16, 4096), "n": _between(rng, 16, 4096), "k": _between(rng, 32, 4096)}
+    if kind == "conv":
+        while True:
+            f = rng.choice([1, 3, 3, 5])
+            case = {"kind": kind, "images": _between(rng, 1, 128), "cin": 8 * _between(rng, 2, 48),
+                    "cout": 8 * _between(rng, 2, 48), "height": _between(rng, 7, 56), "width": _between(rng, 7, 56),
+                    "filter": f, "pad": rng.choice([0, f // 2]), "stride": rng.choice([1, 1, 1, 2])}
+            if 1e8 < _conv_flops(case) < 4e11:
+                return case
+    if kind == "norm_pool":
+        while True:
+            case = {"kind": kind, "images": _between(rng, 1, 256), "channels": _between(rng, 16, 384),
+                    "height": rng.randrange(7, 64), "width": rng.randrange(7, 64)}
+            if 1e5 < case["images"] * case["channels"] * case["height"] * case["width"] < 8e7:
+                return case
+    return {"kind": "matrix", "m": _between(rng, 64, 8192), "n": _between(rng, 64, 8192)}
+
+
+# ---------------------------------------------------------------- inputs
+
+
+class _State:
+    """A program's tensors and the calls of one pass over them, in order."""
+
+    def __init__(self, seed):
+        self.gen = torch.Generator(device="cuda")
+        self.gen.manual_seed(seed)
+        self.lib = capi.lib()
+        self.stream = torch.cuda.current_stream().cuda_stream
+        self.tensors, self.calls, self.out = [], [], {}
+        self.workspace, self.workspace_bytes = None, 0
+
+    def keep(self, t):
+        self.tensors.append(t)
+        return t
+
+    def normal(self, *shape, std=1.0, mean=0.0):
+        t = torch.empty(shape, dtype=torch.float32, device="cuda")
+        return self.keep(t.normal_(mean, std, generator=self.gen))
+
+    def empty(self, *shape):
+        return self.keep(torch.empty(shape, dtype=torch.float32, device="cuda"))
+
+    def call(self, name, *args):
+        """Adds mnv_<name>(args..., stream) to the pass; "ws" stands for the workspace pair."""
+        self.calls.append((name, args))
+
+    def needs(self, query, *args):
+        self.workspace_bytes = max(self.workspace_bytes, getattr(self.lib, "mnv_" + query + "_workspace_bytes")(*args))
+
+    def ready(self):
+        """One workspace for all operators of the pass, and the calls with plain pointers."""
+        self.workspace = torch.empty(max(self.workspace_bytes, 256), dtype=torch.uint8, device="cuda")
+        calls = []
+        for name, args in self.calls:
+            plain = []
+            for a in args:
+                if isinstance(a, torch.Tensor):
+                    plain.append(a.data_ptr())
+                elif a == "ws":
+                    plain += [self.workspace.data_ptr(), self.workspace.numel()]
+                else:
+                    plain.append(a)
+            calls.append((getattr(self.lib, "mnv_" + name), tuple(plain) + (self.stream,)))
+        self.calls = calls
+        return self
+
+    def run(self):
+        for fn, args in self.calls:
+            rc = fn(*args)
+            if rc:
+                capi.check(rc, fn.__name__)
+        return self.out
+
+
+def _conv_out(case):
+    f, p, s = case["filter"], case["pad"], case["stride"]
+    return (case["height"] + 2 * p - f) // s + 1, (case["width"] + 2 * p - f) // s + 1
+
+
+def _conv_flops(case):
+    ho, wo = _conv_out(case)
+    return 2.0 * case["images"] * case["cin"] * case["cout"] * ho * wo * case["filter"] ** 2
+
+
+def _conv_dims(n, cin, cout, h, w, pad, stride, f):
+    return (n, cin, cout, h, w, pad, pad, stride, stride, f, f)
+
+
+def _prepare_sgemm(case, seed):
+    s = _State(seed)
+    m, n, k = case["m"], case["n"], case["k"]
+    a, b, c = s.normal(k, m), s.normal(n, k), s.empty(n, m)
+    s.needs("sgemm_nn", m, n, k)
+    s.call("sgemm_nn", a, b, c, m, n, k, "ws")
+    s.out = {"c": c}
+    return s.ready()
+
+
+def _prepare_conv(case, seed):
+    s = _State(seed)
+    n, cin, cout, h, w, f = (case[v] for v in ("images", "cin", "cout", "height", "width", "filter"))
+    ho, wo = _conv_out(case)
+    dims = _conv_dims(n, cin, cout, h, w, case["pad"], case["stride"], f)
+    x = s.normal(n, cin, h, w).relu_()  # what a ReLU below hands on
+    filt, bias = s.normal(cout, cin, f, f, std=math.sqrt(2.0 / (cin * f * f))), s.normal(cout, std=0.1)
+    dy = s.normal(n, cout, ho, wo, std=1e-2)
+    y, dx, dw, db = s.empty(n, cout, ho, wo), s.empty(n, cin, h, w), s.empty(cout, cin, f, f), s.empty(cout)
+    for q in ("conv_fwd", "conv_bwd_data", "conv_bwd_filter"):
+        s.needs(q, *dims)
+    s.needs("conv_bwd_bias", n, cout)
+    s.call("conv_fwd", x, filt, bias, y, *dims, "ws")
+    s.call("conv_bwd_data", dy, filt, dx, *dims, "ws")
+    s.call("conv_bwd_filter", x, dy, dw, *dims, "ws")
+    s.call("conv_bwd_bias", dy, db, n, cout, ho, wo, "ws")
+    s.out = {"y": y, "dx": dx, "dw": dw, "db": db}
+    return s.ready()
+
+
+def _prepare_norm_pool(case, seed):
+    s = _State(seed)
+    n, c, h, w = (case[v] for v in ("images", "channels", "height", "width"))
+    hp, wp = (s.lib.mnv_pooled_size(v, 3, 2, 0) for v in (h, w))
+    lrn = (5, 1e-4, 0.75, n, c, h, w)
+    pool = (n, c, h, w, 2, 2, 3, 3, 0, 0)
+    x = s.normal(n, c, h, w, std=2.0).relu_()
+    scale, norm, dx = s.empty(n, c, h, w), s.empty(n, c, h, w), s.empty(n, c, h, w)
+    dnorm = s.normal(n, c, h, w, std=1e-2)
+    pooled, dpool = s.empty(n, c, hp, wp), s.empty(n, c, h, w)
+    dy = s.normal(n, c, hp, wp, std=1e-2)
+    # both layers on the same activations: a pooling layer above the normalisation would send a
+    # gradient elsewhere for the last bit of a normalised value
+    s.call("lrn_fwd", x, scale, norm, *lrn)
+    s.call("maxpool_fwd", x, pooled, *pool)
+    s.call("maxpool_bwd", x, pooled, dy, dpool, *pool)
+    s.call("lrn_bwd", x, norm, scale, dnorm, dx, *lrn)
+    s.out = {"scale": scale, "norm": norm, "pooled": pooled, "dpool": dpool, "dx": dx}
+    return s.ready()
+
+
+def _prepare_matrix(case, seed):
+    s = _State(seed)
+    m, n = case["m"], case["n"]
+    size = m * n
+    x, y = s.normal(n, m), s.normal(n, m)
+    row = s.normal(m)
+    e = lambda: s.empty(n, m)  # noqa: E731
+    o = {"sum": e(), "scaled": e(), "relu": e(), "relu_bwd": e(), "sigmoid": e(), "sigmoid_bwd": e(), "exp": e(),
+         "biased": e(), "softmax": e(), "softmax_bwd": e(), "transposed": s.empty(m, n), "colsum": s.empty(n),
+         "rowsum": s.empty(m), "argmax": s.empty(n)}
+    s.call("add", x, y, o["sum"], size)
+    s.call("const_mul", x, o["scaled"], 0.37, size)
+    s.call("relu_fwd", x, o["relu"], size)
+    s.call("relu_bwd", x, o["relu"], y, o["relu_bwd"], size)
+    s.call("sigmoid_fwd", x, o["sigmoid"], size)
+    s.call("sigmoid_bwd", x, o["sigmoid"], y, o["sigmoid_bwd"], size)
+    s.call("exp", x, o["exp"], size)
+    s.call("norm_add_row", x, row, o["biased"], m, n)
+    s.call("softmax_instance_fwd", x, o["softmax"], n, m, 1, 1)
+    s.call("softmax_instance_bwd", y, o["softmax"], o["softmax_bwd"], n, m, 1, 1)
+    s.call("transpose", x, o["transposed"], m, n)
+    s.call("reduce_sum_col", x, o["colsum"], m, n)
+    s.call("reduce_sum_row", x, o["rowsum"], m, n)
+    s.call("maxindex_col", x, o["argmax"], m, n)
+    s.out = o
+    return s.ready()
+
+
+def _prepare_alexnet(case, seed):
+    """The operator sequence of the host layer's AlexNet step.  Weights N(0, 0.01) and zero biases
+    as the applications start from, images N(0, 1), one-hot labels."""
+    s = _State(seed)
+    n, train, fused = case["batch"], case["train"], case["fused"]
+    x = s.normal(n, 3, 227, 227)
+    w = [s.normal(k, c, f, f, std=0.01) for c, k, f, _, _, _ in ALEXNET_CONVS]
+    w += [s.normal(i, o, std=0.01) for i, o in ALEXNET_FCS]
+    b = [s.keep(torch.zeros(k, device="cuda")) for _, k, _, _, _, _ in ALEXNET_CONVS]
+    b += [s.keep(torch.zeros(o, device="cuda")) for _, o in ALEXNET_FCS]
+
+    def relu(t):
+        y = s.empty(*t.shape)
+        s.call("relu_fwd", t, y, t.numel())
+        return y
+
+    # forward: convolutions (each with its dimensions and its input kept for the way back), then
+    # the inner products on {features, images} matrices
+    layers, act = [], x
+    for i, (c, k, f, p, st, pooled) in enumerate(ALEXNET_CONVS):
+        h = act.shape[-1]
+        ho = (h + 2 * p - f) // st + 1
+        dims, y = _conv_dims(n, c, k, h, h, p, st, f), s.empty(n, k, ho, ho)
+        s.needs("conv_fwd", *dims)
+        s.call("conv_fwd_relu" if fused else "conv_fwd", act, w[i], b[i], y, *dims, "ws")
+        layer = {"dims": dims, "in": act}
+        act = layer["act"] = y if fused else relu(y)
+        if pooled:
+            hp = s.lib.mnv_pooled_size(ho, 3, 2, 0)
+            layer["pool"] = (n, k, ho, ho, 2, 2, 3, 3, 0, 0)
+            act = layer["pooled"] = s.empty(n, k, hp, hp)
+            s.call("maxpool_fwd", layer["act"], act, *layer["pool"])
+        layers.append(layer)
+    flat, acts = act.view(n, -1), []
+    acts.append(flat)
+    for j, (i_, o_) in enumerate(ALEXNET_FCS):
+        y, last = s.empty(n, o_), j == 2
+        s.needs("sgemm_nn", o_, n, i_)
+        if fused:
+            s.call("sgemm_nn_bias", w[5 + j], acts[-1], b[5 + j], y, o_, n, i_, 0 if last else 1, "ws")
+        else:
+            t = s.empty(n, o_)
+            s.call("sgemm_nn", w[5 + j], acts[-1], t, o_, n, i_, "ws")
+            s.call("norm_add_row", t, b[5 + j], y, o_, n)
+            y = y if last else relu(y)
+        acts.append(y)
+    prob = s.empty(n, 1000)
+    s.call("softmax_instance_fwd", acts[3], prob, n, 1000, 1, 1)
+    s.out = {"scores": acts[3], "prob": prob}
+    if not train:
+        return s.ready()
+
+    label = s.keep(torch.zeros(n, 1000, device="cuda"))
+    label[torch.arange(n, device="cuda"), torch.randint(0, 1000, (n,), device="cuda", generator=s.gen)] = 1.0
+    gw, gb = [s.empty(*t.shape) for t in w], [s.empty(*t.shape) for t in b]
+
+    def relu_bwd(t, act):
+        y = s.empty(*t.shape)
+        s.call("relu_bwd", act, act, t, y, t.numel())
+        return y
+
+    # backward through the inner products
+    sens = s.empty(n, 1000)
+    s.call("sub", prob, label, sens, sens.numel())
+    for j in (2, 1, 0):
+        i_, o_ = ALEXNET_FCS[j]
+        s.needs("sgemm_nn", i_, n, o_)
+        s.needs("sgemm_nn", o_, i_, n)
+        below = s.empty(n, i_)
+        if fused:
+            s.call("sgemm_nt", sens, acts[j], gw[5 + j], o_, i_, n, "ws")
+            s.call("sgemm_tn", w[5 + j], sens, acts[j] if j else None, below, i_, n, o_, "ws")
+        else:
+            at, wt = s.empty(i_, n), s.empty(o_, i_)
+            s.call("transpose", acts[j], at, i_, n)
+            s.call("sgemm_nn", sens, at, gw[5 + j], o_, i_, n, "ws")
+            s.call("transpose", w[5 + j], wt, o_, i_)
+            s.call("sgemm_nn", wt, sens, below, i_, n, o_, "ws")
+        s.call("reduce_sum_row", sens, gb[5 + j], o_, n)
+        sens = below if fused or not j else relu_bwd(below, acts[j])
+    # backward through the convolutions
+    for i in (4, 3, 2, 1, 0):
+        layer = layers[i]
+        if "pool" in layer:
+            t = s.empty(*layer["act"].shape)
+            s.call("maxpool_bwd_relu" if fused else "maxpool_bwd", layer["act"], layer["pooled"], sens, t, *layer["pool"])
+            sens = t if fused else relu_bwd(t, layer["act"])
+        elif not fused:
+            sens = relu_bwd(sens, layer["act"])
+        dims = layer["dims"]
+        s.needs("conv_bwd_filter", *dims)
+        s.needs("conv_bwd_bias", n, dims[2])
+        s.call("conv_bwd_filter", layer["in"], sens, gw[i], *dims, "ws")
+        s.call("conv_bwd_bias", sens, gb[i], n, dims[2], layer["act"].shape[2], layer["act"].shape[3], "ws")
+        if i:
+            s.needs("conv_bwd_data", *dims)
+            t = s.empty(*layer["in"].shape)
+            if fused and "pool" not in layers[i - 1]:
+                s.call("conv_bwd_data_relu", sens, w[i], layer["in"], t, *dims, "ws")
+            else:
+                s.call("conv_bwd_data", sens, w[i], t, *dims, "ws")
+            sens = t
+    # plain SGD into the next step's parameters
+    for kind, params, grads in (("w", w, gw), ("b", b, gb)):
+        for i, (p, g) in enumerate(zip(params, grads)):
+            new = s.empty(*p.shape)
+            if fused:
+                s.call("sgd_update", p, g, 0.01 / n, new, p.numel())
+            else:
+                t = s.empty(*p.shape)
+                s.call("const_mul", g, t, 0.01 / n, p.numel())
+                s.call("sub", p, t, new, p.numel())
+            s.out["g_%s%d" % (kind, i)], s.out["%s%d" % (kind, i)] = g, new
+    return s.ready()
+
+
+class _Minibatches:
+    """A network of the host layer and the host minibatches it is trained on."""
+    runtime = None
+
+    def __init__(self, case, seed):
+        if _Minibatches.runtime is None:  # one device per program
+            _Minibatches.runtime = hostapi.Runtime(0, sync_each_op=False)
+        self.net = hostapi.Net(self.runtime, case["net"], case["batch"], case["variant"])
+        params, _, _ = configs.make_inputs(case["net"], 1, seed=seed)
+        for name, value in params.items():
+            self.net.set_param(name, value)
+        self.batches = [configs.make_inputs(case["net"], case["batch"], seed=seed + 7919 * (i + 1))[1:]
+                        for i in range(case["steps"])]
+        self.prob_floats = 10 * case["batch"]
+
+    def run(self):
+        for data, label in self.batches:
+            self.net.load_batch(data, label)
+            self.net.step(0.01)
+        out = {name: self.net.read(name, floats) for name, floats in self.net.params.items()}
+        out["prob"] = self.net.read("prob", self.prob_floats)
+        return out
+
+    def __del__(self):
+        self.net.close()
+
+
+_PREPARE = {"minibatches": _Minibatches, "alexnet": _prepare_alexnet, "sgemm": _prepare_sgemm, "conv": _prepare_conv,
+            "norm_pool": _prepare_norm_pool, "matrix": _prepare_matrix}
+
+
+def prepare(case, seed):
+    return _PREPARE[case["kind"]](case, seed)
+
+
+def run(state):
+    return state.run()
+
+
+# ---------------------------------------------------------------- what a pass cannot do without
+
+
+def _alexnet_work(case):
+    n, h = case["batch"], 227
+    flops, params = 0.0, 0
+    for i, (c, k, f, p, st, pooled) in enumerate(ALEXNET_CONVS):
+        ho = (h + 2 * p - f) // st + 1
+        passes = 1 if not case["train"] else 2 if i == 0 else 3  # the images need no gradient
+        flops += passes * 2.0 * n * c * k * ho * ho * f * f
+        params += k * c * f * f + k
+        h = (ho - 2) // 2 + 1 if pooled else ho
+    for i_, o_ in ALEXNET_FCS:
+        flops += (3 if case["train"] else 1) * 2.0 * n * i_ * o_
+        params += i_ * o_ + o_
+    values = params + n * (3 * 227 * 227 + 2000)
+    if case["train"]:  # labels, gradients and new parameters
+        values += n * 1000 + 2 * params
+    return {"bytes": 4.0 * values, "flops": flops}
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "alexnet":
+        return _alexnet_work(case)
+    if kind == "sgemm":
+        m, n, k = case["m"], case["n"], case["k"]
+        return {"bytes": 4.0 * (m * k + k * n + m * n), "flops": 2.0 * m * n * k}
+    if kind == "conv":
+        ho, wo = _conv_out(case)
+        x = case["images"] * case["cin"] * case["height"] * case["width"]
+        y, f = case["images"] * case["cout"] * ho * wo, case["cin"] * case["cout"] * case["filter"] ** 2
+        return {"bytes": 4.0 * (2 * x + 2 * y + 2 * f + 2 * case["cout"]), "flops": 3 * _conv_flops(case) + y}
+    if kind == "norm_pool":
+        planes, h, w = case["images"] * case["channels"], case["height"], case["width"]
+        x, y = planes * h * w, planes * (((h - 2) // 2) + 1) * (((w - 2) // 2) + 1)
+        # in: x, dnorm, dy; out: scale, norm, pooled, dpool, dx
+        return {"bytes": 4.0 * (6 * x + 2 * y), "flops": 40.0 * x}
+    if kind == "matrix":
+        m, n = case["m"], case["n"]
+        # in: two matrices and a vector; out: eleven matrices and three vectors
+        return {"bytes": 4.0 * (13 * m * n + 2 * m + 2 * n), "flops": 30.0 * m * n}
+    # minibatches: every batch read and the parameters of the last step written; three products
+    # per layer
+    batch, steps = case["batch"], case["steps"]
+    if case["net"] == "mlp":
+        per, params = 784 * 256 + 256 * 10, 784 * 256 + 256 * 11 + 10
+    else:
+        side = 12 if case["variant"] else 8
+        per, params = 24 * 24 * 16 * 25 + side * side * 32 * 16 * 25 + 5120, 416 + 12832 + 5130
+    return {"bytes": 4.0 * (steps * batch * 794 + 2 * params + 10 * batch), "flops": 6.0 * steps * batch * per}
+
+
+def tolerance(case):
+    """About four times what was measured between two correct ways of computing the same pass."""
+    kind = case["kind"]
+    if kind == "alexnet" and case["train"]:
+        # A pre-activation that rounds to the other side of 0, or two values of a pooling window
+        # that change places, opens or closes a gradient's way: 1 in 1e5 of them between the
+        # direct and the minimal-filtering convolutions, so that the lower layers' gradients are
+        # 0.5 - 0.7% apart and single entries up to 0.4 of their norm.
+        return {"rel": 0.025, "max": 0.95}
+    if kind == "alexnet":
+        return {"rel": 1e-5, "max": 5e-5}  # direct against minimal filtering: 2.7e-6 and 1.2e-5
+    if kind == "conv":
+        return {"rel": 2.5e-5, "max": 5e-4}  # direct against minimal filtering: 5.9e-6 and 1.3e-4
+    if kind == "sgemm":
+        return {"rel": 5e-6, "max": 5e-5}  # against float64: 1.1e-6 and 1.1e-5 at k = 4096
+    if kind == "minibatches":
+        return {"rel": 4e-6, "max": 1.2e-5}  # another order of summation: 9e-7 and 2.8e-6
+    return {"rel": 1e-6, "max": 5e-6}  # against float64: 2.2e-7 (a sum of 8192 values) and 9e-7
