@@ -297,7 +297,7 @@ def _prepare_alexnet(case, seed):
     if not train:
         return s.ready()
 
-    label = s.keep(torch.zeros(n, 1000, device="cuda"))
+    label = s.label = s.keep(torch.zeros(n, 1000, device="cuda"))
     label[torch.arange(n, device="cuda"), torch.randint(0, 1000, (n,), device="cuda", generator=s.gen)] = 1.0
     gw, gb = [s.empty(*t.shape) for t in w], [s.empty(*t.shape) for t in b]
 
@@ -471,3 +471,134 @@ def tolerance(case):
     if kind == "minibatches":
         return {"rel": 4e-6, "max": 1.2e-5}  # another order of summation: 9e-7 and 2.8e-6
     return {"rel": 1e-6, "max": 5e-6}  # against float64: 2.2e-7 (a sum of 8192 values) and 9e-7
+
+
+# ---------------------------------------------------------------- the same results in 64 bits
+
+
+def _conv64(x, w, b, pad, stride):
+    """True convolution (the filter is flipped), as one product per few images."""
+    k, f = w.shape[0], w.shape[-1]
+    ho, wo = ((v + 2 * pad - f) // stride + 1 for v in x.shape[-2:])
+    flat = w.flip(2, 3).reshape(k, -1)
+    each = max(1, int(2e8 // (flat.shape[1] * ho * wo)))
+    out = [torch.matmul(flat, torch.nn.functional.unfold(part, f, padding=pad, stride=stride)).view(-1, k, ho, wo)
+           for part in x.split(each)]
+    y = torch.cat(out)
+    return y if b is None else y + b.view(1, -1, 1, 1)
+
+
+def _inputs(case, seed):
+    """The tensors that prepare() makes for these inputs, in its order, in 64 bits where they are
+    computed with."""
+    return prepare(case, seed).tensors
+
+
+def _exact_sgemm(case, seed):
+    a, b = _inputs(case, seed)[:2]
+    return {"c": torch.matmul(b.double(), a.double())}
+
+
+def _exact_conv(case, seed):
+    x, filt, bias, dy = (t.double() for t in _inputs(case, seed)[:4])
+    f, p, st, h, w = case["filter"], case["pad"], case["stride"], case["height"], case["width"]
+    n, k, ho, wo = dy.shape
+    flat, c = filt.flip(2, 3).reshape(k, -1), filt.shape[1]
+    each = max(1, int(2e8 // (flat.shape[1] * ho * wo)))
+    dx, dw = [], torch.zeros_like(flat)
+    for xs, ds in zip(x.split(each), dy.split(each)):
+        ds = ds.reshape(ds.shape[0], k, -1)
+        dx.append(torch.nn.functional.fold(torch.matmul(flat.t().contiguous(), ds), (h, w), f, padding=p, stride=st))
+        cols = torch.nn.functional.unfold(xs, f, padding=p, stride=st)
+        dw += torch.matmul(ds, cols.transpose(1, 2).contiguous()).sum(0)
+    return {"y": _conv64(x, filt, bias, p, st), "dx": torch.cat(dx), "dw": dw.view(k, c, f, f).flip(2, 3),
+            "db": dy.sum((0, 2, 3))}
+
+
+def _exact_norm_pool(case, seed):
+    t = _inputs(case, seed)
+    x, dnorm, dy = t[0].double(), t[4].double(), t[7].double()
+    c, size, alpha, beta = case["channels"], 5, 1e-4, 0.75
+
+    def window(v):  # the sum over the channels c - 2 .. c + 2
+        total = torch.zeros_like(v)
+        for d in range(-2, 3):
+            lo, hi = max(0, -d), min(c, c - d)
+            total[:, lo:hi] += v[:, lo + d:hi + d]
+        return total
+
+    scale = 1 + window(x * x) * (alpha / size)
+    norm = x * scale ** -beta
+    dx = dnorm * scale ** -beta - 2 * alpha * beta / size * x * window(dnorm * norm / scale)
+    x.requires_grad_(True)
+    pooled = torch.nn.functional.max_pool2d(x, 3, 2, ceil_mode=True)  # the first of equal values, as in the layer
+    dpool, = torch.autograd.grad(pooled, x, dy)
+    return {"scale": scale, "norm": norm, "pooled": pooled.detach(), "dpool": dpool, "dx": dx}
+
+
+def _exact_matrix(case, seed):
+    x, y, row = (t.double() for t in _inputs(case, seed)[:3])
+    sig, soft = torch.sigmoid(x), torch.softmax(x, 1)
+    return {"sum": x + y, "scaled": x * 0.37, "relu": x.relu(), "relu_bwd": y * (x > 0), "sigmoid": sig,
+            "sigmoid_bwd": y * sig * (1 - sig), "exp": x.exp(), "biased": x + row, "softmax": soft,
+            "softmax_bwd": soft * (y - (y * soft).sum(1, keepdim=True)), "transposed": x.t().contiguous(),
+            "colsum": x.sum(1), "rowsum": x.sum(0), "argmax": x.argmax(1).double()}
+
+
+def _exact_alexnet(case, seed):
+    s = prepare(case, seed)
+    p = len(ALEXNET_CONVS) + len(ALEXNET_FCS)
+    act = s.tensors[0].double()
+    w, b = s.tensors[1:1 + p], s.tensors[1 + p:1 + 2 * p]
+    for i, (_, _, _, pad, st, pooled) in enumerate(ALEXNET_CONVS):
+        act = _conv64(act, w[i].double(), b[i].double(), pad, st).relu_()
+        if pooled:
+            act = torch.nn.functional.max_pool2d(act, 3, 2, ceil_mode=True)
+    act = act.flatten(1)
+    for j in range(3):
+        below, act = act, torch.matmul(act, w[5 + j].double()) + b[5 + j].double()
+        act = act if j == 2 else act.relu_()
+    prob = torch.softmax(act, 1)
+    out = {name: None for name in s.out}
+    out.update(scores=act, prob=prob)
+    if case["train"]:
+        # The last layer's parameters.  Further down a gradient's way opens or closes with the
+        # last bit of a value beside 0 or of two equal ones: 64 bits say nothing more there than
+        # tolerance() does.
+        sens = prob - s.label
+        g_w, g_b = torch.matmul(below.t().contiguous(), sens), sens.sum(0)
+        out.update(g_w7=g_w, g_b7=g_b, w7=w[7].double() - 0.01 / case["batch"] * g_w,
+                   b7=b[7].double() - 0.01 / case["batch"] * g_b)
+    return out
+
+
+def _exact_minibatches(case, seed):
+    net, n = case["net"], case["batch"]
+    raw = configs.make_inputs(net, 1, seed=seed)[0]
+    # Minerva extents (dimension 0 fastest): a tensor of the reversed shape has the same bytes
+    par = {k: torch.from_numpy(raw[k]).double().view(v[::-1]) for k, v in configs.param_shapes(net).items()}
+    pad, pool = (2, 3) if case["variant"] else (0, 2)
+    for i in range(case["steps"]):
+        data, label = (torch.from_numpy(v).double() for v in configs.make_inputs(net, n, seed=seed + 7919 * (i + 1))[1:])
+        label = label.view(n, 10)
+        for v in par.values():
+            v.requires_grad_(True)
+        if net == "mlp":
+            act = torch.matmul(data.view(n, 784), par["w0"]) + par["b0"]
+            score = torch.matmul(act.relu(), par["w1"]) + par["b1"]
+        else:
+            act = torch.nn.functional.max_pool2d(_conv64(data.view(n, 1, 28, 28), par["w0"], par["b0"], 0, 1).relu(), 2)
+            act = torch.nn.functional.max_pool2d(_conv64(act, par["w1"], par["b1"], pad, 1).relu(), pool)
+            score = torch.matmul(act.flatten(1), par["w2"]) + par["b2"]
+        loss = -(torch.log_softmax(score, 1) * label).sum()  # its gradient at the scores: prob - label
+        grads = torch.autograd.grad(loss, list(par.values()))
+        par = {k: (v - 0.01 / n * g).detach() for (k, v), g in zip(par.items(), grads)}
+    out = {k: v.reshape(-1).numpy() for k, v in par.items()}
+    out["prob"] = torch.softmax(score.detach(), 1).reshape(-1).numpy()
+    return out
+
+
+def exact(case, seed):
+    """What run() returns for these inputs, in 64 bits and without this repository's operators."""
+    return {"alexnet": _exact_alexnet, "minibatches": _exact_minibatches, "sgemm": _exact_sgemm, "conv": _exact_conv,
+            "norm_pool": _exact_norm_pool, "matrix": _exact_matrix}[case["kind"]](case, seed)
