@@ -468,6 +468,11 @@ def tolerance(case):
         return {"rel": 2.5e-5, "max": 5e-4}  # direct against minimal filtering: 5.9e-6 and 1.3e-4
     if kind == "sgemm":
         return {"rel": 5e-6, "max": 5e-5}  # against float64: 1.1e-6 and 1.1e-5 at k = 4096
+    if kind == "minibatches" and case["net"] == "cnn":
+        # As in the training step above: about one set of inputs in twenty has a pre-activation
+        # or a pooling window on the other side.  One that has is 1.2e-3 and 2.9e-3 from float64
+        # (the first layer's bias), the others 4e-7 and 2e-6.
+        return {"rel": 5e-3, "max": 1.2e-2}
     if kind == "minibatches":
         return {"rel": 4e-6, "max": 1.2e-5}  # another order of summation: 9e-7 and 2.8e-6
     return {"rel": 1e-6, "max": 5e-6}  # against float64: 2.2e-7 (a sum of 8192 values) and 9e-7
