@@ -649,7 +649,7 @@ struct ConvBwdFilterFast {
     const unsigned soff = ((unsigned)period * (unsigned)(g.K * g.HoWo) + (unsigned)s * 16u) * 4u;
     mnv_fetch_vec<1>(r.b, off, soff, v);
   }
-  __device__ void b_stash_fix(int s, int kl, float (&v)[4]) const {
+  __device__ void b_stash_fix(int, int s, int kl, float (&v)[4]) const {
     if (s * 16 + 16 > g.HoWo) {  // uniform
       const int first = s * 16 + kl;
 #pragma unroll

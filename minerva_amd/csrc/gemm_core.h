@@ -113,8 +113,8 @@ struct MnvFetchMap {
 //        loads element j (row tid / 16 + 16 j, k = kl) into v[j / 4][j % 4]; a_period is unused
 //   optional, for a right operand whose loads may fetch values that must read as 0 and that are
 //   cheaper to clear once they have arrived: static constexpr bool B_STASH_FIX = true;
-//   void b_stash_fix(int s, int kl, float (&v)[4]) const;   called on every vector of slab s of
-//        its period right before the vector is written to LDS
+//   void b_stash_fix(int period, int s, int kl, float (&v)[4]) const;   called on every vector of
+//        slab s of that period right before the vector is written to LDS
 //   optional, for an output whose m direction is contiguous in memory:
 //   static constexpr bool C_STORE4 = true;
 //   void c_store4(int m, int n, const float (&v)[4]) const;   the elements (m .. m + 3, n); m is a
@@ -395,10 +395,11 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
     for (int p = 0; p < T::BV; ++p)
       prob.b_period(bst[p], boff[p], n0 + MapB::x(tid, p), MapB::k(tid, p), period);
   };
-  int s_of_set[PF] = {};  // slab (inside its period) that each staging set holds
+  int s_of_set[PF] = {}, period_of_set[PF] = {};  // period and slab of it that each staging set holds
   auto fetch = [&](int period, int s, auto SET) {
     constexpr int set = decltype(SET)::value;
     s_of_set[set] = s;
+    period_of_set[set] = period;
     if constexpr (LK) {
       prob.a_load_lanek(res, ast[0], period, s, tid % 16, ra[set]);
     } else {
@@ -416,7 +417,7 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
     float* bb = Bs + buf * BTILE;
     if constexpr (MnvBStashFix<P>::value) {
 #pragma unroll
-      for (int p = 0; p < T::BV; ++p) prob.b_stash_fix(s_of_set[set], MapB::k(tid, p), rb[set][p]);
+      for (int p = 0; p < T::BV; ++p) prob.b_stash_fix(period_of_set[set], s_of_set[set], MapB::k(tid, p), rb[set][p]);
     }
     if constexpr (LK) {  // element j: row tid / 16 + 16 j, k = tid % 16
 #pragma unroll

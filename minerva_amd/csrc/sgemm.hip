@@ -23,10 +23,22 @@ namespace {
 // {n,k} (element (k,n) at n + k*ldb) -- which only swaps its fetch direction: a transposed A
 // is k-fast, a transposed B x-fast.  The values multiplied and the order they are added in
 // are those of the product of the explicitly transposed matrices.
-template <bool VEC, bool TA = false, bool TB = false>
+//
+// Every vector is one 16-byte load whatever the extents and the alignment: buffer loads want
+// 4-byte alignment only and check their range dword by dword.
+//  x-fast: a vector that reaches past the last row (column) brings values of the next one;
+//    they are summed into accumulators that are never stored.
+//  k-fast: a vector that reaches past K brings values that would be summed.  K4 (K % 4 == 0):
+//    there is none.  Otherwise B's vectors of the last, partial slab are cleared past K on
+//    their way to LDS (b_stash_fix: a uniform branch per slab; an infinity there times the
+//    other operand's 0 would not be 0), and a transposed A keeps four 4-byte loads.
+// Four 4-byte loads per vector, which odd extents took before, keep four times as many
+// load instructions in a slab: 1001 x 250 x 4099 41.0 -> 28.5 us, 4099 x 4099 x 1023
+// 292 -> 272, 10 x 256 x 256 9.4 -> 7.3; the same bits.
+template <bool K4, bool TA = false, bool TB = false>
 struct SgemmNN {
   static constexpr bool A_KFAST = TA, B_KFAST = !TB;
-  static constexpr int A_NOFF = VEC ? 1 : 4, B_NOFF = VEC ? 1 : 4;
+  static constexpr int A_NOFF = TA && !K4 ? 4 : 1, B_NOFF = 1;
   const float* __restrict__ A;
   const float* __restrict__ B;
   float* __restrict__ C;
@@ -70,7 +82,7 @@ struct SgemmNN {
     } else {
       const unsigned base = ((unsigned)k * (unsigned)lda + (unsigned)m) * 4u;
 #pragma unroll
-      for (int q = 0; q < A_NOFF; ++q) off[q] = ((m + q < M) & (k < K)) ? base + 4u * q : MNV_OOB;
+      for (int q = 0; q < A_NOFF; ++q) off[q] = ((m < M) & (k < K)) ? base + 4u * q : MNV_OOB;
     }
   }
   __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[A_NOFF], int, int s,
@@ -83,16 +95,24 @@ struct SgemmNN {
     if (TB) {
       const unsigned base = ((unsigned)k * (unsigned)ldb + (unsigned)n) * 4u;
 #pragma unroll
-      for (int q = 0; q < B_NOFF; ++q) off[q] = ((n + q < N) & (k < K)) ? base + 4u * q : MNV_OOB;
+      for (int q = 0; q < B_NOFF; ++q) off[q] = ((n < N) & (k < K)) ? base + 4u * q : MNV_OOB;
     } else {
       const unsigned base = ((unsigned)n * (unsigned)ldb + (unsigned)k) * 4u;
 #pragma unroll
-      for (int q = 0; q < B_NOFF; ++q) off[q] = ((n < N) & (k + q < K)) ? base + 4u * q : MNV_OOB;
+      for (int q = 0; q < B_NOFF; ++q) off[q] = ((n < N) & (k < K)) ? base + 4u * q : MNV_OOB;
     }
   }
   __device__ void b_load(const Res& r, const BState&, const unsigned (&off)[B_NOFF], int, int s,
                          int, float (&v)[4]) const {
     mnv_fetch_vec<B_NOFF>(r.b, off, (unsigned)s * (unsigned)bk * (TB ? (unsigned)ldb : 1u) * 4u, v);
+  }
+  static constexpr bool B_STASH_FIX = !K4 && !TB;
+  __device__ void b_stash_fix(int period, int, int kl, float (&v)[4]) const {
+    if (period == (K >= bk ? 1 : 0)) {  // the partial slab
+      const int rest = K % bk;
+#pragma unroll
+      for (int q = 1; q < 4; ++q) v[q] = kl + q < rest ? v[q] : 0.f;
+    }
   }
   size_t extra_lds_bytes() const { return 0; }
   void set_bk(int b) {
@@ -143,10 +163,10 @@ struct SgemmEpilogue {
   float sgd_scale = 0.f;
 };
 
-template <bool VEC, bool TA = false, bool TB = false>
-SgemmNN<VEC, TA, TB> make_sgemm(const float* a, const float* b, float* c, int m, int n, int k,
+template <bool K4, bool TA = false, bool TB = false>
+SgemmNN<K4, TA, TB> make_sgemm(const float* a, const float* b, float* c, int m, int n, int k,
                                 const SgemmEpilogue& e) {
-  SgemmNN<VEC, TA, TB> p;
+  SgemmNN<K4, TA, TB> p;
   p.A = a; p.B = b; p.C = c; p.M = m; p.N = n; p.K = k;
   p.bias = e.bias; p.gate = e.gate; p.relu = e.relu;
   p.lda = e.lda ? e.lda : (TA ? k : m); p.ldb = e.ldb ? e.ldb : (TB ? n : k); p.ldc = e.ldc ? e.ldc : m;
@@ -291,10 +311,8 @@ int scratch_address(float** out) {
 int sgemm_nn_impl(const float* a, const float* b, float* c, int m, int n, int k, void* workspace,
                   size_t workspace_bytes, hipStream_t s,
                   const SgemmEpilogue& e = SgemmEpilogue{nullptr, nullptr, 0}) {
-  bool vec = (m % 4 == 0) && (k % 4 == 0) && mnv_aligned16(a) && mnv_aligned16(b) &&
-             e.lda % 4 == 0 && e.ldb % 4 == 0;
   const SgemmPlan plan = plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
-  if (vec) return launch_plan(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
+  if (k % 4 == 0) return launch_plan(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
   return launch_plan(plan, make_sgemm<false>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
 }
 
@@ -303,13 +321,13 @@ int sgemm_nn_impl(const float* a, const float* b, float* c, int m, int n, int k,
 template <bool TA, bool TB>
 int sgemm_t_impl(const float* a, const float* b, float* c, int m, int n, int k, void* workspace,
                  size_t workspace_bytes, hipStream_t s, const SgemmEpilogue& e) {
-  const bool vec = mnv_aligned16(a) && mnv_aligned16(b) && (TA ? k % 4 == 0 : m % 4 == 0) &&
-                   (TB ? n % 4 == 0 : k % 4 == 0);
   SgemmPlan plan = plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
   // a B given transposed is fetched along n: measured on 4096^3, 0.987 ms on the 256 x 128
   // tile against 0.951 on 128 x 128 (the bits are the same on either)
   if (TB) plan.tall = false;
-  if (vec) return launch_plan(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
+  // with both operands x-fast no vector runs along k
+  if ((!TA && TB) || k % 4 == 0)
+    return launch_plan(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
   return launch_plan(plan, make_sgemm<false, TA, TB>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
 }
 

@@ -1,0 +1,50 @@
+"""Products and operators whose extents or addresses are off the 16-byte grid: the paths that
+fetch 16 bytes at a time there, at their edges."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_util import Gpu, normwise, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return Gpu()
+
+
+def _rand(n, seed):
+    return np.random.default_rng(seed).standard_normal(n).astype(np.float32)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 67, 1), (66, 33, 3), (129, 65, 18), (7, 130, 31), (131, 17, 46), (257, 66, 1027)])
+@pytest.mark.parametrize("form", ["nn", "tn", "nt"])
+def test_sgemm_vectors_past_an_edge_bring_nothing_in(gpu, m, n, k, form):
+    """A vector that reaches past a row or column end meets the next one's values: an infinity and
+    a NaN there reach their own row and column of the result only, and operands 4 bytes off the
+    16-byte grid give the bits of aligned ones.  Sums of k products against float64: k + 1
+    roundings of 2^-24 at most, relative to the sum of magnitudes."""
+    say("sgemm", form, m, n, k)
+    a, b = _rand(m * k, 1).reshape(k, m).T, _rand(k * n, 2).reshape(n, k).T  # A{m,k}, B{k,n}
+    a, b = a.copy(), b.copy()
+    a[0, :] = np.inf          # every vector that begins in row m - 1 ends in the next column's row 0
+    b[0, n - 1] = np.nan      # a vector past K of column n - 2 meets it
+    stored = {"nn": (a.T, b.T), "tn": (a, b.T), "nt": (a.T, b)}[form]
+    got = []
+    for shift in (0, 1):
+        dev = [gpu.up(np.concatenate([np.zeros(shift, np.float32), np.ascontiguousarray(v).reshape(-1)])) for v in stored]
+        dc = gpu.empty(m * n)
+        ws_bytes = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+        ws = gpu.empty(ws_bytes // 4 + 1)
+        args = [ctypes.c_void_p(ctypes.cast(d.p, ctypes.c_void_p).value + 4 * shift) for d in dev]
+        if form == "tn":
+            args.append(None)
+        gpu.call("mnv_sgemm_" + form, *args, dc.p, m, n, k, ws.p, ctypes.c_size_t(ws_bytes))
+        got.append(gpu.down(dc).reshape(n, m).T)
+    assert got[0].tobytes() == got[1].tobytes()
+    want = a[1:].astype(np.float64) @ b[:, :n - 1].astype(np.float64)
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(a[1:]).astype(np.float64) @ np.abs(b[:, :n - 1]))
+    assert np.all(np.abs(got[0][1:, :n - 1] - want) <= bound)
+    assert not np.isfinite(got[0][0]).any() and np.isnan(got[0][:, n - 1]).all()
