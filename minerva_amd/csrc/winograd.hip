@@ -388,26 +388,68 @@ __global__ __launch_bounds__(256) void mnv_wino_input_kernel(const float* __rest
   wino_store_v<AL, R>(d, V + (size_t)ci * g.Pp + p, (size_t)g.Cin * g.Pp);
 }
 
-// The same through LDS, for planes small enough that the planes of the images a workgroup's
-// 256 tiles belong to fit there: they are fetched whole, in runs of contiguous floats (a
-// plane of 13 x 13 is 676 contiguous bytes), where the kernel above gathers al^2 values per
-// thread at a stride of a few bytes between neighbouring tiles (F(2 x 2) on 384 channels of
-// 256 x 13 x 13: 107 -> 80 us).  One channel per workgroup: four (the tile arithmetic done once
-// for four) measured 84.7 against 79.6 us.
+// What of the planes the 256 tiles from p0 on read, in 16-byte chunks: chunk c of plane i of
+// the tiles' images (the first one's plane is 0) is number i chunks + c, chunks = ceil(HW / 4),
+// and the tiles need the numbers [lo, hi) -- of the first and the last image only the rows that
+// hold their tiles.  A tile row th needs the plane's rows from m th - pad on, `reach` of them.
+struct WinoSpan {
+  int lo, hi;
+};
+__host__ __device__ inline WinoSpan wino_span(int th0, int th1, int images, int m, int pad, int reach, int H, int W,
+                                              int chunks) {
+  const int y0 = m * th0 - pad > 0 ? m * th0 - pad : 0;
+  const int y1 = m * th1 - pad + reach < H ? m * th1 - pad + reach : H;
+  return WinoSpan{y0 * W / 4, (images - 1) * chunks + (y1 * W + 3) / 4};
+}
+
+// Fetches that span of the planes at `src` (img_floats from one image's plane to the next's;
+// `floats`: what lies from src to the tensor's end) into LDS, number lo first.  Four 16-byte
+// loads in flight per thread; a plane's last chunk may reach into the next plane (never read
+// from LDS) or past the tensor, where the buffer's range check answers 0.
+__device__ __forceinline__ void wino_stage(const float* src, size_t floats, int img_floats, WinoSpan span,
+                                           int chunks, const MnvFastDiv& d_chunks, float* lds) {
+  constexpr int U = 4;
+  const mnv_rsrc r = mnv_make_rsrc(src, floats < 0x1fffffff ? (unsigned)floats * 4u : 0x7ffffffcu);
+  mnv_f4* out = reinterpret_cast<mnv_f4*>(lds);
+  for (int i = span.lo + (int)threadIdx.x; i < span.hi; i += 256 * U) {
+    float v[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = i + 256 * u, pl = mnv_fastdiv(c, d_chunks);
+      mnv_buf_load4(r, c < span.hi ? ((unsigned)pl * (unsigned)img_floats + 4u * (unsigned)(c - pl * chunks)) * 4u : MNV_OOB,
+                    v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + 256 * u < span.hi) out[i + 256 * u - span.lo] = mnv_f4{v[u][0], v[u][1], v[u][2], v[u][3]};
+  }
+}
+
+// The same through LDS, for planes small enough that what a workgroup's 256 tiles read of them
+// fits there: it is fetched in runs of 16-byte chunks, where the kernel above gathers al^2
+// values per thread at a stride of a few bytes between neighbouring tiles (F(2 x 2) on 384
+// channels of 256 x 13 x 13: 107 -> 80 us).  One channel per workgroup: four (the tile
+// arithmetic done once for four) measured 84.7 against 79.6 us.  What bounds it is the trip to
+// memory before the first tile: with whole planes of every image touched, one float per
+// load, planes of 56 x 56 took ten trips for 37 KB, 1.8 times what the tiles read (4 x 4
+// tiles, 256 channels of 32 images: 148 -> 59 us, 5.7 TB/s).
 template <int AL, int R>
 __global__ __launch_bounds__(256) void mnv_wino_input_lds_kernel(const float* __restrict__ src,
                                                                  float* __restrict__ V, WinoGeom g,
-                                                                 MnvFastDiv d_HW) {
+                                                                 MnvFastDiv d_chunks) {
   extern __shared__ float planes[];
   const int p0 = blockIdx.x * 256, p = p0 + threadIdx.x;
   const int ci = blockIdx.y;
-  const int HW = g.Hs * g.Ws;
+  const int HW = g.Hs * g.Ws, T = g.TH * g.TW, chunks = (HW + 3) / 4;
   const int img0 = mnv_fastdiv(p0, g.d_T);
   const int last = p0 + 255 < g.P ? p0 + 255 : g.P - 1;
-  const int count = (last >= p0 ? mnv_fastdiv(last, g.d_T) - img0 + 1 : 0) * HW;
-  for (int i = threadIdx.x; i < count; i += 256) {
-    const int pl = mnv_fastdiv(i, d_HW);
-    planes[i] = src[((size_t)(img0 + pl) * g.Cin + ci) * HW + (i - pl * HW)];
+  WinoSpan span{0, 0};
+  if (last >= p0) {
+    const int img1 = mnv_fastdiv(last, g.d_T);
+    span = wino_span(mnv_fastdiv(p0 - img0 * T, g.d_TW), mnv_fastdiv(last - img1 * T, g.d_TW), img1 - img0 + 1,
+                     AL - R + 1, g.pad_h, AL, g.Hs, g.Ws, chunks);
+    const size_t at = ((size_t)img0 * g.Cin + ci) * HW;
+    wino_stage(src + at, (size_t)g.N * g.Cin * HW - at, g.Cin * HW, span, chunks, d_chunks, planes);
   }
   __syncthreads();
   if (p >= g.Pp) return;
@@ -418,10 +460,10 @@ __global__ __launch_bounds__(256) void mnv_wino_input_lds_kernel(const float* __
     for (int b = 0; b < AL; ++b) d[a][b] = 0.f;
   if (p < g.P) {
     const int img = mnv_fastdiv(p, g.d_T);
-    const int t = p - img * (g.TH * g.TW);
+    const int t = p - img * T;
     const int th = mnv_fastdiv(t, g.d_TW), tw = t - th * g.TW;
     const int y0 = (AL - R + 1) * th - g.pad_h, x0 = (AL - R + 1) * tw - g.pad_w;
-    const float* plane = planes + (img - img0) * HW;
+    const float* plane = planes + ((img - img0) * chunks - span.lo) * 4;
 #pragma unroll
     for (int a = 0; a < AL; ++a)
 #pragma unroll
@@ -633,23 +675,27 @@ __global__ __launch_bounds__(256) void mnv_wino_grad_kernel(const float* __restr
     for (int nu = 0; nu < AL; ++nu) out[(xi * AL + nu) * plane] = v[xi][nu];
 }
 
-// The same with the planes of top_diff fetched whole into LDS (see mnv_wino_input_lds_kernel).
+// The same with what the tiles read of top_diff's planes fetched into LDS (see
+// mnv_wino_input_lds_kernel; 256 channels of 32 x 56 x 56: 146 -> 60 us).
 template <int AL, int R>
 __global__ __launch_bounds__(256) void mnv_wino_grad_lds_kernel(const float* __restrict__ top_diff,
                                                                 float* __restrict__ Yt, WinoGeom g,
-                                                                MnvFastDiv d_HW) {
+                                                                MnvFastDiv d_chunks) {
   typedef WinoF<AL, R> F;
   constexpr int MO = AL - R + 1;
   extern __shared__ float planes[];
   const int p0 = blockIdx.x * 256, p = p0 + threadIdx.x;
   const int k = blockIdx.y;
-  const int HW = g.Hd * g.Wd;
+  const int HW = g.Hd * g.Wd, T = g.TH * g.TW, chunks = (HW + 3) / 4;
   const int img0 = mnv_fastdiv(p0, g.d_T);
   const int last = p0 + 255 < g.P ? p0 + 255 : g.P - 1;
-  const int count = (last >= p0 && k < g.Cout ? mnv_fastdiv(last, g.d_T) - img0 + 1 : 0) * HW;
-  for (int i = threadIdx.x; i < count; i += 256) {
-    const int pl = mnv_fastdiv(i, d_HW);
-    planes[i] = top_diff[((size_t)(img0 + pl) * g.Cout + k) * HW + (i - pl * HW)];
+  WinoSpan span{0, 0};
+  if (last >= p0 && k < g.Cout) {
+    const int img1 = mnv_fastdiv(last, g.d_T);
+    span = wino_span(mnv_fastdiv(p0 - img0 * T, g.d_TW), mnv_fastdiv(last - img1 * T, g.d_TW), img1 - img0 + 1, MO, 0,
+                     MO, g.Hd, g.Wd, chunks);
+    const size_t at = ((size_t)img0 * g.Cout + k) * HW;
+    wino_stage(top_diff + at, (size_t)g.N * g.Cout * HW - at, g.Cout * HW, span, chunks, d_chunks, planes);
   }
   __syncthreads();
   if (p >= g.Pp) return;
@@ -662,7 +708,7 @@ __global__ __launch_bounds__(256) void mnv_wino_grad_lds_kernel(const float* __r
     const int img = mnv_fastdiv(p, g.d_T);
     const int t = p - img * (g.TH * g.TW);
     const int th = mnv_fastdiv(t, g.d_TW), tw = t - th * g.TW;
-    const float* plane = planes + (img - img0) * HW;
+    const float* plane = planes + ((img - img0) * chunks - span.lo) * 4;
 #pragma unroll
     for (int a = 0; a < MO; ++a)
 #pragma unroll
@@ -858,15 +904,29 @@ int make_wino_geom(WinoGeom* g, int N, int Cin, int Cout, int Hs, int Ws, int pa
   return MNV_OK;
 }
 
+// LDS bytes for the largest span of a launch's workgroups (wino_span), or 0 where the planes are
+// too large for LDS (three workgroups per CU at least) or for 32-bit byte offsets.
+size_t span_lds_bytes(const WinoGeom& g, int channels, int H, int W, int m, int pad, int reach) {
+  const int T = g.TH * g.TW, chunks = (H * W + 3) / 4;
+  if ((255 / T + 2.0) * channels * H * W * 4.0 >= 2147483648.0 || (255 / T + 2.0) * chunks >= 2147483648.0) return 0;
+  int most = 0;
+  for (long long p0 = 0; p0 < g.P; p0 += 256) {
+    const int last = p0 + 255 < g.P ? (int)p0 + 255 : g.P - 1;
+    const int img0 = (int)p0 / T, img1 = last / T;
+    const WinoSpan span = wino_span(((int)p0 - img0 * T) / g.TW, (last - img1 * T) / g.TW, img1 - img0 + 1, m, pad,
+                                    reach, H, W, chunks);
+    if (span.hi - span.lo > most) most = span.hi - span.lo;
+  }
+  return most <= 48 * 1024 / 16 ? (size_t)most * 16 : 0;
+}
+
 // V of the group of images that `g` describes
 template <int AL, int R>
 int launch_input_transform(const float* src, float* V, const WinoGeom& g, hipStream_t s) {
-  const int T = g.TH * g.TW, HW = g.Hs * g.Ws;
-  // planes a workgroup's 256 consecutive tiles can touch
-  const size_t lds = (size_t)(255 / T + 2) * HW * sizeof(float);
-  if (lds <= 48 * 1024)
+  const size_t lds = span_lds_bytes(g, g.Cin, g.Hs, g.Ws, AL - R + 1, g.pad_h, AL);
+  if (lds)
     hipLaunchKernelGGL((mnv_wino_input_lds_kernel<AL, R>), dim3((g.Pp + 255) / 256, g.Cin), dim3(256), lds,
-                       s, src, V, g, mnv_fastdiv_make(HW));
+                       s, src, V, g, mnv_fastdiv_make((g.Hs * g.Ws + 3) / 4));
   else
     hipLaunchKernelGGL((mnv_wino_input_kernel<AL, R>), dim3((g.Pp + 255) / 256, g.Cin), dim3(256), 0, s, src,
                        V, g);
@@ -1015,10 +1075,10 @@ int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_d
     const int nn = N - n0 < images ? N - n0 : images;
     if (nn != g.N && (rc = make_wino_geom(&g, nn, C, K, g.Hs, g.Ws, g.pad_h, g.pad_w, AL, R))) return rc;
     if ((rc = launch_input_transform<AL, R>(bottom + n0 * per_bottom, V, g, s))) return rc;
-    const size_t lds = (size_t)(255 / (g.TH * g.TW) + 2) * g.Hd * g.Wd * sizeof(float);
-    if (lds <= 48 * 1024)
+    const size_t lds = span_lds_bytes(g, K, g.Hd, g.Wd, AL - R + 1, 0, AL - R + 1);
+    if (lds)
       hipLaunchKernelGGL((mnv_wino_grad_lds_kernel<AL, R>), dim3((g.Pp + 255) / 256, g.Coutp), dim3(256), lds, s,
-                         top_diff + n0 * per_top, Yt, g, mnv_fastdiv_make(g.Hd * g.Wd));
+                         top_diff + n0 * per_top, Yt, g, mnv_fastdiv_make((g.Hd * g.Wd + 3) / 4));
     else
       hipLaunchKernelGGL((mnv_wino_grad_kernel<AL, R>), dim3((g.Pp + 255) / 256, g.Coutp), dim3(256), 0, s,
                          top_diff + n0 * per_top, Yt, g);

@@ -5,7 +5,8 @@ import ctypes
 import numpy as np
 import pytest
 
-from gpu_util import Gpu, normwise, say
+import test_gpu_winograd as tw
+from gpu_util import Gpu, say
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +49,16 @@ def test_sgemm_vectors_past_an_edge_bring_nothing_in(gpu, m, n, k, form):
     bound = (k + 1) * 2.0 ** -24 * (np.abs(a[1:]).astype(np.float64) @ np.abs(b[:, :n - 1]))
     assert np.all(np.abs(got[0][1:, :n - 1] - want) <= bound)
     assert not np.isfinite(got[0][0]).any() and np.isnan(got[0][:, n - 1]).all()
+
+
+# N, C, K, H, W, pad: groups of 256 tiles that begin and end inside a plane, planes whose size is
+# no multiple of four (the last chunk of a plane reaches into the next one, or past the tensor),
+# one tile per plane (every group spans many whole planes)
+SPANS = [(2, 16, 32, 67, 61, 1), (1, 16, 16, 101, 99, 2), (3, 16, 32, 57, 55, 0), (70, 16, 16, 3, 5, 1)]
+
+
+@pytest.mark.parametrize("q", SPANS, ids=lambda q: "x".join(map(str, q)))
+@pytest.mark.parametrize("tile", [tw.F2, tw.F4, tw.F5], ids=["2x2", "4x4", "5x5"])
+def test_transforms_of_tiles_that_cross_planes(gpu, ora, q, tile):
+    """All three minimal-filtering passes against the oracle, with that path's own bounds."""
+    tw._passes_against_oracle(gpu, ora, q + (q[5],), tile, 3, tw.BOUND[tile])
