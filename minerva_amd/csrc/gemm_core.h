@@ -755,6 +755,17 @@ static int mnv_gemm_splitk_reduce_launch(const P& prob, const float* partial, in
   return MNV_LAUNCH_STATUS();
 }
 
+// Enough threads to cover the chip: one per element for a large output, up to 64 per element
+// (never more than half the ranges) for a small one.
+template <class P>
+static int mnv_gemm_reduce_launch(const P& prob, const float* part, int splits, hipStream_t s) {
+  const size_t mn = (size_t)prob.M * prob.N;
+  if (mn >= 65536 || splits < 8) return mnv_gemm_splitk_reduce_launch<P, 1>(prob, part, splits, s);
+  if (mn >= 16384 || splits < 32) return mnv_gemm_splitk_reduce_launch<P, 4>(prob, part, splits, s);
+  if (mn >= 4096 || splits < 128) return mnv_gemm_splitk_reduce_launch<P, 16>(prob, part, splits, s);
+  return mnv_gemm_splitk_reduce_launch<P, 64>(prob, part, splits, s);
+}
+
 // Adds the k ranges of the tail tiles (see mnv_gemm_kernel) in range order and hands every
 // element to the policy's store.  One thread per 16-byte group of the partial tiles (register
 // order, see mnv_partial_group_mn): four consecutive columns of one row.
@@ -984,14 +995,7 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
     return MNV_LAUNCH_STATUS();
   }
   if (splits > 1) {
-    // enough threads to cover the chip: one per element for a large output, up to 64 per
-    // element (never more than half the ranges) for a small one
-    const size_t mn = (size_t)prob.M * prob.N;
-    const float* part = reinterpret_cast<const float*>(workspace);
-    if (mn >= 65536 || splits < 8) rc = mnv_gemm_splitk_reduce_launch<P, 1>(prob, part, splits, s);
-    else if (mn >= 16384 || splits < 32) rc = mnv_gemm_splitk_reduce_launch<P, 4>(prob, part, splits, s);
-    else if (mn >= 4096 || splits < 128) rc = mnv_gemm_splitk_reduce_launch<P, 16>(prob, part, splits, s);
-    else rc = mnv_gemm_splitk_reduce_launch<P, 64>(prob, part, splits, s);
+    rc = mnv_gemm_reduce_launch(prob, reinterpret_cast<const float*>(workspace), splits, s);
   }
   return rc;
 }

@@ -154,6 +154,116 @@ struct SgemmNN {
   }
 };
 
+// Products with at most 12 columns (inner products over a few images): every value of A is
+// used that few times, so the product is bound by reading A once, while the smallest MFMA tile
+// of the core multiplies 64 columns.  Here a lane keeps its rows' sums for NC columns (N
+// rounded up to one of a few widths; the columns past N repeat the last one and are not stored)
+// and multiplies by B's values, which are the same for the whole wavefront and come through the
+// scalar cache.  x-fast A: four rows per lane, 1 KB of a column per load; transposed A: one row
+// per lane, four k per load.  A workgroup's four wavefronts take a quarter of its k range each,
+// and their sums are added through LDS, (w0 + w2) + (w1 + w3); the k ranges of the grid's y
+// dimension go through the workspace and the reduction kernel.  Either form adds the same
+// values in the same order.
+// Measured at 1 / 10 columns, with the reduction: 4096 x 9216 43.6 -> 26.4 us
+// and 42.7 -> 33.2 us, 1000 x 4096 at 1 column 11.1 -> 6.6 us.
+#define MNV_SKINNY_COLUMNS 12
+template <class P, int NC, bool TA, bool TB>
+__global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const float* __restrict__ B, int k_per_wave,
+                                                               float* __restrict__ partial) {
+  constexpr int RM = TA ? 1 : 4, U = NC <= 4 ? 16 : NC <= 8 ? 8 : 4;  // rows per lane, k per step
+  __shared__ float red[2 * MNV_WAVE * RM * NC];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
+  const int m = (blockIdx.x * MNV_WAVE + lane) * RM;
+  int k = ((int)blockIdx.y * 4 + wave) * k_per_wave;
+  const int k_end = k + k_per_wave < prob.K ? k + k_per_wave : prob.K;
+  typename P::Res res;
+  prob.make_res(res);
+  // B's element (k, j), its address the same in every lane
+  const int bk = TB ? prob.ldb : 1;
+  size_t col[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) col[j] = (size_t)(j < prob.N ? j : prob.N - 1) * (TB ? 1 : prob.ldb);
+  float acc[NC][RM];
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int q = 0; q < RM; ++q) acc[j][q] = 0.f;
+  // bytes from the wavefront's k to the lane's rows; the rest of the address is uniform
+  const unsigned off = m < prob.M ? (unsigned)m * (TA ? (unsigned)prob.lda : 1u) * 4u : MNV_OOB;
+  const unsigned ak = TA ? 4u : (unsigned)prob.lda * 4u;
+  for (; k + U <= k_end; k += U) {
+    float v[U][RM];
+    if constexpr (TA) {
+#pragma unroll
+      for (int u = 0; u < U; u += 4) {
+        float t[4];
+        const unsigned o[1] = {off};
+        mnv_fetch_vec<1>(res.a, o, (unsigned)(k + u) * ak, t);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[u + q][0] = t[q];
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float t[4];
+        const unsigned o[1] = {off};
+        mnv_fetch_vec<1>(res.a, o, (unsigned)(k + u) * ak, t);
+#pragma unroll
+        for (int q = 0; q < RM; ++q) v[u][q] = t[q];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) {
+        const float b = B[col[j] + (size_t)(k + u) * bk];
+#pragma unroll
+        for (int q = 0; q < RM; ++q) acc[j][q] = __builtin_fmaf(v[u][q], b, acc[j][q]);
+      }
+  }
+  for (; k < k_end; ++k) {
+    float v[RM];
+#pragma unroll
+    for (int q = 0; q < RM; ++q)
+      v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                           res.a, (int)(m + q < prob.M ? off + 4u * q : MNV_OOB), (int)((unsigned)k * ak), 0));
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      const float b = B[col[j] + (size_t)k * bk];
+#pragma unroll
+      for (int q = 0; q < RM; ++q) acc[j][q] = __builtin_fmaf(v[q], b, acc[j][q]);
+    }
+  }
+  auto put = [&](int region) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int q = 0; q < RM; ++q) red[((region * NC + j) * RM + q) * MNV_WAVE + lane] = acc[j][q];
+  };
+  auto add = [&](int region) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+      for (int q = 0; q < RM; ++q) acc[j][q] += red[((region * NC + j) * RM + q) * MNV_WAVE + lane];
+  };
+  if (wave >= 2) put(wave - 2);
+  __syncthreads();
+  if (wave < 2) add(wave);
+  __syncthreads();
+  if (wave == 1) put(0);
+  __syncthreads();
+  if (wave != 0) return;
+  add(0);
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+#pragma unroll
+    for (int q = 0; q < RM; ++q)
+      if (j < prob.N && m + q < prob.M) {
+        if (gridDim.y > 1) partial[((size_t)blockIdx.y * prob.N + j) * prob.M + m + q] = acc[j][q];
+        else prob.c_store(m + q, j, acc[j][q]);
+      }
+}
+
 struct SgemmEpilogue {
   const float* bias;
   const float* gate;
@@ -193,13 +303,44 @@ struct SgemmPlan {
   int splits;
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
+  int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel, with this many k per wavefront
 };
+
+// Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), at
+// least 16 k per wavefront.  The tiles stay for a small A, where the time is that of two launches
+// either way, and for more columns, where the multiplies, not A's bytes, take this kernel's time;
+// their own time does not change from 1 to 64 columns.  Before -> with this kernel, us:
+//   4 columns: 512 x 1 x 1024 6.6 -> 6.3, 1000 x 4 x 600 7.3 -> 7.3, 1000 x 1 x 4096 11.1 -> 6.6
+//   8 columns: 512 x 8 x 1024 6.9 -> 8.5, 1000 x 8 x 1000 7.8 -> 8.0, 256 x 8 x 4096 10.2 -> 8.6,
+//     4096 x 8 x 4096 24.7 -> 19.2
+//   12 columns: 1000 x 10 x 4096 12.3 -> 12.2, 4096 x 12 x 4096 24.4 -> 20.6, 9216 x 12 x 4096
+//     45.0 -> 33.4
+//   16 columns: 2000 x 16 x 2000 10.8 -> 16.9, 4096 x 16 x 4096 25.1 -> 25.4
+// They also stay where the workspace is too small for a quarter of the ranges, and below 256
+// rows (one block).
+bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
+  const long long least = n <= 4 ? 1LL << 19 : n <= 8 ? 1LL << 20 : 1LL << 24;  // elements of A
+  if (n > MNV_SKINNY_COLUMNS || m < 256 || k < 64 || (long long)m * k < least) return false;
+  const int blocks = (m + 255) / 256;
+  long long splits = 512 / blocks;
+  const size_t fit = ws_floats / ((size_t)m * n);
+  if (splits > k / 64) splits = k / 64;
+  if ((size_t)splits > fit) splits = (long long)fit;
+  if (splits < 1) splits = 1;
+  const int per = (int)((k + 4 * splits - 1) / (4 * splits) + 15) / 16 * 16;
+  const int ranges = (int)(((long long)k + 4LL * per - 1) / (4LL * per));
+  if ((long long)blocks * ranges < 128 && ranges < k / 64) return false;
+  *plan = SgemmPlan{false, ranges, 4};
+  plan->skinny = per;
+  return true;
+}
 
 SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   const int slabs = (k + 15) / 16;
   const size_t mn = (size_t)m * n;
   const double per_split = 8.0 * (double)mn / 6e6 / 1.2;
   SgemmPlan best{false, 1};
+  if (plan_skinny(m, n, k, ws_floats, &best)) return best;
   double best_cost = 0;
   for (int small = 0; small < 2; ++small) {
     const int bm = small ? 64 : 128;
@@ -266,6 +407,26 @@ SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   return best;
 }
 
+template <int NC, bool TA, bool TB, class P>
+int launch_skinny(const SgemmPlan& plan, const P& p, void* workspace, hipStream_t s) {
+  const int rows = TA ? MNV_WAVE : 4 * MNV_WAVE;
+  float* part = plan.splits > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
+  hipLaunchKernelGGL((mnv_sgemm_skinny_kernel<P, NC, TA, TB>), dim3((p.M + rows - 1) / rows, plan.splits), dim3(256), 0, s,
+                     p, p.B, plan.skinny, part);
+  const int rc = MNV_LAUNCH_STATUS();
+  if (rc || plan.splits == 1) return rc;
+  return mnv_gemm_reduce_launch(p, part, plan.splits, s);
+}
+
+template <bool K4, bool TA, bool TB>
+int launch_skinny_columns(const SgemmPlan& plan, const SgemmNN<K4, TA, TB>& p, void* workspace, hipStream_t s) {
+  if (p.N <= 1) return launch_skinny<1, TA, TB>(plan, p, workspace, s);
+  if (p.N <= 2) return launch_skinny<2, TA, TB>(plan, p, workspace, s);
+  if (p.N <= 4) return launch_skinny<4, TA, TB>(plan, p, workspace, s);
+  if (p.N <= 8) return launch_skinny<8, TA, TB>(plan, p, workspace, s);
+  return launch_skinny<MNV_SKINNY_COLUMNS, TA, TB>(plan, p, workspace, s);
+}
+
 // A launch without k ranges may use the workspace for the partial tiles of a cut tail.
 template <class P>
 int launch_plan(const SgemmPlan& plan, const P& p, void* workspace, size_t workspace_bytes,
@@ -312,6 +473,7 @@ int sgemm_nn_impl(const float* a, const float* b, float* c, int m, int n, int k,
                   size_t workspace_bytes, hipStream_t s,
                   const SgemmEpilogue& e = SgemmEpilogue{nullptr, nullptr, 0}) {
   const SgemmPlan plan = plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
+  if (plan.skinny) return launch_skinny_columns(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, s);
   if (k % 4 == 0) return launch_plan(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
   return launch_plan(plan, make_sgemm<false>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
 }
@@ -325,6 +487,7 @@ int sgemm_t_impl(const float* a, const float* b, float* c, int m, int n, int k, 
   // a B given transposed is fetched along n: measured on 4096^3, 0.987 ms on the 256 x 128
   // tile against 0.951 on 128 x 128 (the bits are the same on either)
   if (TB) plan.tall = false;
+  if (plan.skinny) return launch_skinny_columns(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, s);
   // with both operands x-fast no vector runs along k
   if ((!TA && TB) || k % 4 == 0)
     return launch_plan(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
@@ -377,9 +540,9 @@ int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_row
                       int* groups) {
   if (m <= 0 || n <= 0 || k <= 0 || !tile_rows || !k_ranges || !groups) return MNV_ERR_INVALID;
   const SgemmPlan plan = plan_sgemm(m, n, k, workspace_bytes / sizeof(float));
-  *tile_rows = plan.tall ? 256 : plan.small ? 64 : 128;
+  *tile_rows = plan.tall || plan.skinny ? 256 : plan.small ? 64 : 128;
   const int slabs = (k + 15) / 16, per = (slabs + plan.splits - 1) / plan.splits;
-  *k_ranges = (slabs + per - 1) / per;  // as the launch rounds it: ranges of equal length
+  *k_ranges = plan.skinny ? plan.splits : (slabs + per - 1) / per;  // as the launch rounds it: ranges of equal length
   *groups = plan.groups;
   return MNV_OK;
 }

@@ -62,3 +62,36 @@ SPANS = [(2, 16, 32, 67, 61, 1), (1, 16, 16, 101, 99, 2), (3, 16, 32, 57, 55, 0)
 def test_transforms_of_tiles_that_cross_planes(gpu, ora, q, tile):
     """All three minimal-filtering passes against the oracle, with that path's own bounds."""
     tw._passes_against_oracle(gpu, ora, q + (q[5],), tile, 3, tw.BOUND[tile])
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 8, 9, 12])
+@pytest.mark.parametrize("m,k", [(256, 4096), (257, 4098), (1003, 1047), (4099, 4101)])
+def test_sgemm_of_few_columns(gpu, m, n, k):
+    """Row blocks of 256 (64 for a transposed A), k ranges of four wavefronts, each width the
+    columns are rounded up to.  k + 1 roundings against float64; the transposed forms and a fused
+    bias have the bits of the plain product; so has a second call; a workspace for fewer k ranges and
+    none at all stay within the bound."""
+    say("sgemm, few columns", m, n, k)
+    a, b, bias = _rand(m * k, 3), _rand(k * n, 4), _rand(m, 5)
+    A, B = a.reshape(k, m).T, b.reshape(n, k).T
+    ws_bytes = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    ws, dc = gpu.empty(ws_bytes // 4 + 1), gpu.empty(m * n)
+    at, bt = gpu.up(np.ascontiguousarray(A).reshape(-1)), gpu.up(np.ascontiguousarray(B).reshape(-1))
+    da, db, dbias = gpu.up(a), gpu.up(b), gpu.up(bias)
+
+    def run(name, *args, nbytes=ws_bytes):
+        gpu.call("mnv_sgemm_" + name, *args, ws.p if nbytes else None, ctypes.c_size_t(nbytes))
+        return gpu.down(dc).copy()
+
+    got = run("nn", da.p, db.p, dc.p, m, n, k)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B))
+    assert np.all(np.abs(got.reshape(n, m).T - want) <= bound)
+    for other in (run("nn", da.p, db.p, dc.p, m, n, k), run("tn", at.p, db.p, None, dc.p, m, n, k),
+                  run("nt", da.p, bt.p, dc.p, m, n, k)):
+        assert other.tobytes() == got.tobytes()
+    assert run("nn_bias", da.p, db.p, dbias.p, dc.p, m, n, k, 1).tobytes() == \
+        np.maximum(got.reshape(n, m) + bias, np.float32(0)).reshape(-1).tobytes()
+    for nbytes in (ws_bytes // 3 // 4 * 4, 0):
+        few = run("nn", da.p, db.p, dc.p, m, n, k, nbytes=nbytes)
+        assert np.all(np.abs(few.reshape(n, m).T - want) <= bound)
