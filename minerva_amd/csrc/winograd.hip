@@ -520,11 +520,17 @@ __global__ __launch_bounds__(256) void mnv_wino_output_kernel(const float* __res
     }
 }
 
-// The same through LDS, for planes small enough that the output planes a workgroup's 256
-// tiles belong to fit there: a thread leaves its m x m outputs in LDS and the workgroup then
+__host__ __device__ inline WinoSpan wino_rows_span(int th0, int th1, int images, int m, int H, int W) {
+  return WinoSpan{m * th0 * W, (images - 1) * H * W + (m * (th1 + 1) < H ? m * (th1 + 1) : H) * W};
+}
+
+// The same through LDS, for planes small enough that the output rows of a workgroup's 256
+// tiles fit there (whole planes between its first and its last image): a thread leaves its m x m outputs in LDS and the workgroup then
 // stores every plane in runs of contiguous floats, where the kernel above stores m floats per
 // row and thread, neighbouring threads m floats apart (4 x 4 tiles on 384 channels of
 // 256 x 13 x 13: 95 us).  A pixel is stored by the workgroup that holds its tile.
+// Holding and walking every touched plane whole left 56 x 56 planes at four workgroups per CU
+// and 1.8 times the pixels (4 x 4 tiles, 256 channels of 32 images: 72 -> 57 us).
 template <int AL, int R>
 __global__ __launch_bounds__(256) void mnv_wino_output_lds_kernel(const float* __restrict__ Mx,
                                                                   const float* __restrict__ bias,
@@ -539,7 +545,10 @@ __global__ __launch_bounds__(256) void mnv_wino_output_lds_kernel(const float* _
   const int HW = g.Hd * g.Wd, T = g.TH * g.TW;
   const int img0 = mnv_fastdiv(p0, g.d_T);
   const int last = p0 + 255 < g.P ? p0 + 255 : g.P - 1;  // p0 < P: the grid covers P
-  const int count = (mnv_fastdiv(last, g.d_T) - img0 + 1) * HW;
+  const int img1 = mnv_fastdiv(last, g.d_T);
+  // floats of the images' planes, laid end to end, that the tiles' rows cover
+  const WinoSpan span = wino_rows_span(mnv_fastdiv(p0 - img0 * T, g.d_TW), mnv_fastdiv(last - img1 * T, g.d_TW),
+                                       img1 - img0 + 1, MO, g.Hd, g.Wd);
   if (p < g.P) {
     const size_t plane = (size_t)g.Coutp * g.Pp;
     const float* in = Mx + (size_t)co * g.Pp + p;
@@ -555,7 +564,7 @@ __global__ __launch_bounds__(256) void mnv_wino_output_lds_kernel(const float* _
     const int t = p - img * T;
     const int th = mnv_fastdiv(t, g.d_TW), tw = t - th * g.TW;
     const float b = bias ? bias[co] : 0.f;
-    float* out = planes + (img - img0) * HW;
+    float* out = planes + (img - img0) * HW - span.lo;
 #pragma unroll
     for (int a = 0; a < MO; ++a)
 #pragma unroll
@@ -570,14 +579,14 @@ __global__ __launch_bounds__(256) void mnv_wino_output_lds_kernel(const float* _
       }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < count; i += 256) {
+  for (int i = span.lo + (int)threadIdx.x; i < span.hi; i += 256) {
     const int pl = mnv_fastdiv(i, d_HW);
     const int r = i - pl * HW;
     const int yy = mnv_fastdiv(r, d_W), xx = r - yy * g.Wd;
     const int owner = (img0 + pl) * T + (yy / MO) * g.TW + xx / MO;
     if (owner >= p0 && owner <= last) {
       const size_t at = ((size_t)(img0 + pl) * g.Cout + co) * HW + r;
-      float v = planes[i];
+      float v = planes[i - span.lo];
       if (gate) v = gate[at] > 0.f ? v : 0.f;
       dst[at] = v;
     }
@@ -904,20 +913,38 @@ int make_wino_geom(WinoGeom* g, int N, int Cin, int Cout, int Hs, int Ws, int pa
   return MNV_OK;
 }
 
-// LDS bytes for the largest span of a launch's workgroups (wino_span), or 0 where the planes are
-// too large for LDS (three workgroups per CU at least) or for 32-bit byte offsets.
-size_t span_lds_bytes(const WinoGeom& g, int channels, int H, int W, int m, int pad, int reach) {
-  const int T = g.TH * g.TW, chunks = (H * W + 3) / 4;
-  if ((255 / T + 2.0) * channels * H * W * 4.0 >= 2147483648.0 || (255 / T + 2.0) * chunks >= 2147483648.0) return 0;
+// The largest span of a launch's workgroups: span(first tile row, last tile row, images).
+template <class Span>
+int most_of_spans(const WinoGeom& g, const Span& span) {
+  const int T = g.TH * g.TW;
   int most = 0;
   for (long long p0 = 0; p0 < g.P; p0 += 256) {
     const int last = p0 + 255 < g.P ? (int)p0 + 255 : g.P - 1;
     const int img0 = (int)p0 / T, img1 = last / T;
-    const WinoSpan span = wino_span(((int)p0 - img0 * T) / g.TW, (last - img1 * T) / g.TW, img1 - img0 + 1, m, pad,
-                                    reach, H, W, chunks);
-    if (span.hi - span.lo > most) most = span.hi - span.lo;
+    const WinoSpan s = span(((int)p0 - img0 * T) / g.TW, (last - img1 * T) / g.TW, img1 - img0 + 1);
+    if (s.hi - s.lo > most) most = s.hi - s.lo;
   }
+  return most;
+}
+
+// LDS bytes of the largest wino_span, or 0 where the planes are too large for LDS (three
+// workgroups per CU at least) or for 32-bit byte offsets.
+size_t span_lds_bytes(const WinoGeom& g, int channels, int H, int W, int m, int pad, int reach) {
+  const int T = g.TH * g.TW, chunks = (H * W + 3) / 4;
+  if ((255 / T + 2.0) * channels * H * W * 4.0 >= 2147483648.0) return 0;
+  const int most = most_of_spans(g, [&](int th0, int th1, int images) {
+    return wino_span(th0, th1, images, m, pad, reach, H, W, chunks);
+  });
   return most <= 48 * 1024 / 16 ? (size_t)most * 16 : 0;
+}
+
+// The same for the output rows; 0: too large for LDS.
+size_t rows_lds_bytes(const WinoGeom& g) {
+  if ((255 / (g.TH * g.TW) + 2.0) * g.Hd * g.Wd >= 2147483648.0) return 0;
+  const int most = most_of_spans(g, [&](int th0, int th1, int images) {
+    return wino_rows_span(th0, th1, images, g.m, g.Hd, g.Wd);
+  });
+  return most <= 48 * 1024 / 4 ? (size_t)most * 4 : 0;
 }
 
 // V of the group of images that `g` describes
@@ -1026,8 +1053,8 @@ int wino_conv(const WinoGeom& g0, const float* src, const float* filter, const f
     rc = mnv_gemm_launch<TileBig>(p, 1, nullptr, s);
     if (timed) profile_end(e0, e1, s, 0, 2.0 * AL * AL * Cout * Cin * g.P);
     if (rc) return rc;
-    const size_t lds = (size_t)(255 / (g.TH * g.TW) + 2) * g.Hd * g.Wd * sizeof(float);
-    if (lds <= 48 * 1024)
+    const size_t lds = rows_lds_bytes(g);
+    if (lds)
       hipLaunchKernelGGL((mnv_wino_output_lds_kernel<AL, R>), dim3((g.P + 255) / 256, Cout), dim3(256), lds, s,
                          Mx, bias, gate ? gate + n0 * per_dst : nullptr, dst + n0 * per_dst, g, relu,
                          mnv_fastdiv_make(g.Hd * g.Wd), mnv_fastdiv_make(g.Wd));
