@@ -66,6 +66,13 @@ __device__ __forceinline__ mnv_f4 mnv_ldx4(const mnv_f4* p) {
   if (NT) return __builtin_nontemporal_load(p);
   return *p;
 }
+// The same from an address of which only the 4-byte alignment is known.
+template <bool NT>
+__device__ __forceinline__ mnv_f4 mnv_ldx4u(const float* p) {
+  const mnv_f4u* q = reinterpret_cast<const mnv_f4u*>(p);
+  if (NT) return __builtin_nontemporal_load(q);
+  return *q;
+}
 #endif
 #define MNV_PAST_CACHE_BYTES ((size_t)256 << 20)
 

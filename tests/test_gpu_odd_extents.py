@@ -95,3 +95,66 @@ def test_sgemm_of_few_columns(gpu, m, n, k):
     for nbytes in (ws_bytes // 3 // 4 * 4, 0):
         few = run("nn", da.p, db.p, dc.p, m, n, k, nbytes=nbytes)
         assert np.all(np.abs(few.reshape(n, m).T - want) <= bound)
+
+
+# m, n, offset of the operands in floats: lines and columns that end in 1, 2 or 3 values, at every
+# alignment, around the widths that the kernels change at (64 and 128 columns of a tile, 2048, 4096
+# and 8192 values of a line)
+ODD = [(1, 1, 0), (3, 5, 1), (63, 65, 2), (65, 63, 3), (130, 127, 0), (128, 128, 1), (1001, 257, 0), (1027, 1021, 2),
+       (2049, 9, 0), (4093, 7, 3), (8191, 5, 1), (8192, 6, 2), (8197, 3, 0), (2047, 2051, 1)]
+
+
+@pytest.mark.parametrize("m,n,off", ODD)
+def test_matrix_operators_off_the_16_byte_grid(gpu, m, n, off):
+    """Results against numpy, and the floats before and behind them untouched.  Data movement,
+    single operations and maxima have no error.  A sum of L values: L roundings of 2^-24 relative
+    to the sum of magnitudes.  Soft-max: an exponential, a sum of L and a quotient, L + 8 roundings."""
+    say("matrix operators", m, n, off)
+    x, y, row, col = _rand(m * n, 6), _rand(m * n, 7), _rand(m, 8), _rand(n, 9)
+    lead = off + 4
+    at = lambda d: ctypes.c_void_p(ctypes.cast(d.p, ctypes.c_void_p).value + 4 * lead)  # noqa: E731
+    up = lambda v: gpu.up(np.concatenate([np.full(lead, 7, np.float32), v, np.full(5, 7, np.float32)]))  # noqa: E731
+    dx, dy_, drow, dcol = up(x), up(y), gpu.up(row), gpu.up(col)
+
+    def run(name, size, *args):
+        out = up(np.full(size, 3, np.float32))
+        gpu.call("mnv_" + name, *[at(out) if a == "out" else a for a in args])
+        whole = gpu.down(out)
+        assert np.all(whole[:lead] == 7) and np.all(whole[lead + size:] == 7), name
+        return whole[lead:lead + size].copy()
+
+    X, Y = x.reshape(n, m), y.reshape(n, m)  # X[column, row]
+    assert np.array_equal(run("transpose", m * n, at(dx), "out", m, n).reshape(m, n), X.T)
+    assert np.array_equal(run("norm_add_row", m * n, at(dx), drow.p, "out", m, n).reshape(n, m), X + row)
+    assert np.array_equal(run("norm_mul_col", m * n, at(dx), dcol.p, "out", m, n).reshape(n, m), X * col[:, None])
+    assert np.array_equal(run("reduce_max_col", n, at(dx), "out", m, n), X.max(1))
+    assert np.array_equal(run("reduce_max_row", m, at(dx), "out", m, n), X.max(0))
+    assert np.array_equal(run("maxindex_col", n, at(dx), "out", m, n), X.argmax(1))
+    assert np.array_equal(run("maxindex_row", m, at(dx), "out", m, n), X.argmax(0))
+    X64, Y64, u = X.astype(np.float64), Y.astype(np.float64), 2.0 ** -24
+    for name, axis, length in (("reduce_sum_col", 1, m), ("reduce_sum_row", 0, n)):
+        got = run(name, m * n // length, at(dx), "out", m, n)
+        assert np.all(np.abs(got - X64.sum(axis)) <= length * u * np.abs(X64).sum(axis))
+    e = np.exp(X64 - X64.max(1, keepdims=True))
+    p = e / e.sum(1, keepdims=True)
+    got = run("softmax_instance_fwd", m * n, at(dx), "out", n, m, 1, 1).reshape(n, m)
+    # the hardware exponential's argument -- up to 10 here -- is rounded once, 10 u more
+    assert np.all(np.abs(got - p) <= (m + 18) * u * p)
+    dot = (X64 * Y64).sum(1, keepdims=True)
+    got = run("softmax_instance_bwd", m * n, at(dy_), at(dx), "out", n, m, 1, 1).reshape(n, m)
+    bound = np.abs(X64) * ((m + 2) * u * np.abs(X64 * Y64).sum(1, keepdims=True) + 3 * u * np.abs(Y64 - dot))
+    assert np.all(np.abs(got - X64 * (Y64 - dot)) <= bound)
+
+
+@pytest.mark.parametrize("N,K,H,W", [(256, 16, 3, 5), (300, 7, 2, 2), (37, 65, 9, 7), (5, 3, 1, 1)])
+def test_bias_gradient_of_many_image_groups(gpu, N, K, H, W):
+    """One to more than 64 group sums per channel, channels off the four of a workgroup: a sum of
+    L values against float64, L roundings of 2^-24 relative to the sum of magnitudes."""
+    say("bias gradient", N, K, H, W)
+    dy = _rand(N * K * H * W, 10)
+    nbytes = gpu.L.mnv_conv_bwd_bias_workspace_bytes(N, K)
+    ws, db, ddy = gpu.empty(nbytes // 4 + 1), gpu.empty(K), gpu.up(dy)
+    gpu.call("mnv_conv_bwd_bias", ddy.p, db.p, N, K, H, W, ws.p, ctypes.c_size_t(nbytes))
+    t = dy.reshape(N, K, H * W).astype(np.float64)
+    bound = N * H * W * 2.0 ** -24 * np.abs(t).sum((0, 2))
+    assert np.all(np.abs(gpu.down(db) - t.sum((0, 2))) <= bound)
