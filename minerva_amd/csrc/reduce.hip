@@ -82,6 +82,8 @@ struct EmitIndex {
 // ---------------------------------------------------------------------------
 // Along dimension 0: each of the n columns is m contiguous floats.
 // GROUP threads (one wavefront, or the whole 256-thread workgroup) share a column.
+// VEC4: every column starts on the 16-byte grid.  (Columns that do not were read 4 bytes at a
+// time before, one load in flight: sums of 8191 x 8193 53 -> 38 us.)
 // ---------------------------------------------------------------------------
 #define MNV_RC_THREADS 256
 
@@ -112,7 +114,20 @@ __global__ __launch_bounds__(MNV_RC_THREADS) void mnv_reduce_col_kernel(
         acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
       }
     } else {
-      for (int i = t; i < m; i += GROUP) acc.push(col[i], i);
+      // the same loads at the address the column has, then its last 1 to 3 values
+      const int m4 = m >> 2;
+      int i = t;
+      for (; i + GROUP < m4; i += 2 * GROUP) {
+        mnv_f4 a = mnv_ldx4u<NT>(col + 4 * (size_t)i), b = mnv_ldx4u<NT>(col + 4 * (size_t)(i + GROUP));
+        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
+        int j = i + GROUP;
+        acc.push(b.x, 4 * j); acc.push(b.y, 4 * j + 1); acc.push(b.z, 4 * j + 2); acc.push(b.w, 4 * j + 3);
+      }
+      if (i < m4) {
+        mnv_f4 a = mnv_ldx4u<NT>(col + 4 * (size_t)i);
+        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
+      }
+      if (4 * m4 + t < m) acc.push(col[4 * m4 + t], 4 * m4 + t);
     }
 #pragma unroll
     for (int off = MNV_WAVE / 2; off > 0; off >>= 1) acc.merge(acc.shfl_down(off));
@@ -146,6 +161,9 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
     else if (vec4)
       hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, true, false>), dim3(grid),
                          dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
+    else if (big)
+      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, false, true>), dim3(grid),
+                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
     else
       hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, false, false>), dim3(grid),
                          dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
@@ -158,6 +176,9 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
     else if (vec4)
       hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, true, false>), dim3(grid),
                          dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
+    else if (big)
+      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, false, true>), dim3(grid),
+                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
     else
       hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, false, false>), dim3(grid),
                          dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
@@ -169,12 +190,16 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
 // Along dimension 1: out[r] = reduce_c in[r + c*m] (stride m between elements).
 // A workgroup owns RL*W consecutive rows (128 contiguous bytes per column) and
 // splits the columns over CG thread groups; partial results meet in LDS.
+// VEC4: m and the matrix on the 16-byte grid; otherwise the same loads at the addresses the
+// columns have, and the last 1 to 3 rows element by element.  (One row per thread, 4 bytes per
+// load, one load in flight before: sums of 8191 x 8193 140 -> 128 us, 65 x 4097
+// 27 -> 8.5; the 128-byte run of an unaligned column lies in two lines, both fetched whole.)
 // ---------------------------------------------------------------------------
 template <class Acc, class Emit, int RL, int CG, bool VEC4, bool NT>
 __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __restrict__ in,
                                                                 float* __restrict__ out, int m,
                                                                 int n) {
-  constexpr int W = VEC4 ? 4 : 1;
+  constexpr int W = 4;
   constexpr int ROWS = RL * W;
   __shared__ Acc part[CG][ROWS + 1];
   const int rl = threadIdx.x % RL;
@@ -184,7 +209,11 @@ __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __r
 #pragma unroll
   for (int q = 0; q < W; ++q) acc[q].init();
   if (r0 < m) {
-    if (VEC4) {
+    if (VEC4 || r0 + 3 < m) {
+      auto ld = [&](int c) {
+        const float* at = in + (size_t)c * m + r0;
+        return VEC4 ? mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(at)) : mnv_ldx4u<NT>(at);
+      };
       // several columns in flight per thread: with one workgroup per 32 rows there are few
       // wavefronts per SIMD, and the loads of a thread are what keeps HBM busy (measured:
       // four for the (value, index) pairs, 4.9 -> 6.0 TB/s; two for sums, where four lose 7%)
@@ -194,7 +223,7 @@ __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __r
         mnv_f4 v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          v[u] = mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(in + (size_t)(c + u * CG) * m + r0));
+          v[u] = ld(c + u * CG);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           acc[0].push(v[u].x, c + u * CG); acc[1 % W].push(v[u].y, c + u * CG);
@@ -202,11 +231,14 @@ __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __r
         }
       }
       for (; c < n; c += CG) {
-        mnv_f4 a = mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(in + (size_t)c * m + r0));
+        mnv_f4 a = ld(c);
         acc[0].push(a.x, c); acc[1 % W].push(a.y, c); acc[2 % W].push(a.z, c); acc[3 % W].push(a.w, c);
       }
     } else {
-      for (int c = cg; c < n; c += CG) acc[0].push(in[(size_t)c * m + r0], c);
+      for (int c = cg; c < n; c += CG)
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          if (r0 + q < m) acc[q].push(in[(size_t)c * m + r0 + q], c);
     }
   }
 #pragma unroll
@@ -234,22 +266,18 @@ int launch_reduce_row(const float* in, float* out, int m, int n, mnv_stream_t st
   if (m == 0) return MNV_OK;
   if (!in || !out || m < 0 || n <= 0) return MNV_ERR_INVALID;
   hipStream_t s = mnv_stream(stream);
-  bool vec4 = (m % 4 == 0) && mnv_aligned16(in);
-  if (vec4) {
-    constexpr int RL = 8, CG = 64;
-    unsigned grid = (unsigned)mnv_ceil_div((size_t)m, RL * 4);
-    if ((size_t)m * n * sizeof(float) >= MNV_PAST_CACHE_BYTES)
-      hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, true>), dim3(grid),
-                         dim3(RL * CG), 0, s, in, out, m, n);
-    else
-      hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, false>), dim3(grid),
-                         dim3(RL * CG), 0, s, in, out, m, n);
-  } else {
-    constexpr int RL = 32, CG = 16;
-    unsigned grid = (unsigned)mnv_ceil_div((size_t)m, RL);
-    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, false, false>), dim3(grid),
-                       dim3(RL * CG), 0, s, in, out, m, n);
-  }
+  const bool vec4 = (m % 4 == 0) && mnv_aligned16(in);
+  const bool big = (size_t)m * n * sizeof(float) >= MNV_PAST_CACHE_BYTES;
+  constexpr int RL = 8, CG = 64;
+  const dim3 grid((unsigned)mnv_ceil_div((size_t)m, RL * 4)), block(RL * CG);
+  if (vec4 && big)
+    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, true>), grid, block, 0, s, in, out, m, n);
+  else if (vec4)
+    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, false>), grid, block, 0, s, in, out, m, n);
+  else if (big)
+    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, false, true>), grid, block, 0, s, in, out, m, n);
+  else
+    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, false, false>), grid, block, 0, s, in, out, m, n);
   return MNV_LAUNCH_STATUS();
 }
 
@@ -260,7 +288,7 @@ int launch_reduce_row(const float* in, float* out, int m, int n, mnv_stream_t st
 // wavefronts take the group's images round-robin and read each run with 16-byte loads
 // from its first aligned address (at most three single floats on either side).  With
 // several groups per channel the group sums go to a scratch area and a second, tiny
-// kernel adds them in group order, so the result does not depend on scheduling.
+// kernel adds them in a fixed order, so the result does not depend on scheduling.
 // ---------------------------------------------------------------------------
 #define MNV_BIAS_THREADS 256
 
@@ -312,13 +340,17 @@ __global__ __launch_bounds__(MNV_BIAS_THREADS) void mnv_conv_bwd_bias_kernel(
   }
 }
 
+// One wavefront per channel: its group sums arrive in one or two loads.  (One thread per
+// channel walked them one trip to memory after the other: 128 groups, 16 channels of 256 images,
+// 6.4 -> 2.3 us.)
 __global__ __launch_bounds__(256) void mnv_conv_bwd_bias_finish_kernel(
     const float* __restrict__ partial, float* __restrict__ bias_diff, int K, int groups) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
+  const int k = blockIdx.x * (256 / MNV_WAVE) + threadIdx.x / MNV_WAVE, lane = threadIdx.x % MNV_WAVE;
   if (k >= K) return;
   float t = 0.f;
-  for (int g = 0; g < groups; ++g) t += partial[(size_t)k * groups + g];
-  bias_diff[k] = t;
+  for (int g = lane; g < groups; g += MNV_WAVE) t += partial[(size_t)k * groups + g];
+  t = mnv_wave_sum(t);
+  if (lane == 0) bias_diff[k] = t;
 }
 
 // Image groups per channel: enough workgroups to fill the chip, at least four images
@@ -386,7 +418,7 @@ int mnv_conv_bwd_bias(const float* top_diff, float* bias_diff, int num_images,
                        (int)hw, per);
   int rc = MNV_LAUNCH_STATUS();
   if (rc || groups == 1) return rc;
-  hipLaunchKernelGGL(mnv_conv_bwd_bias_finish_kernel, dim3((top_num_channels + 255) / 256),
+  hipLaunchKernelGGL(mnv_conv_bwd_bias_finish_kernel, dim3((top_num_channels + 3) / 4),
                      dim3(256), 0, s, reinterpret_cast<const float*>(workspace), bias_diff,
                      top_num_channels, groups);
   return MNV_LAUNCH_STATUS();
