@@ -61,31 +61,66 @@ __device__ __forceinline__ T* lane_pointer(T* p) {
 }
 
 // One line per GROUP threads of an NTH-thread workgroup (GROUP = one wavefront or the whole
-// workgroup); the line (len % 4 == 0, len <= GROUP*4*CACHE) is cached in registers.
+// workgroup); the line (len <= GROUP*4*CACHE) is cached in registers.
 // Stores are non-temporal; NT: so are the loads (inputs of 256 MB and more, which no cache
 // holds until the next operator).  Lines of up to 8192 values take 512 threads with four
 // vectors each rather than 256 with eight (more wavefronts, shorter per-thread chains): on
 // 8192 lines of 8192, operands cycled through four sets, 6.3 TB/s against 5.8 TB/s (a plain
 // copy of the same operands: 6.3 TB/s).
-template <int GROUP, int CACHE, int NTH, bool NT>
+// ODD: lines off the 16-byte grid, or of a length that is no multiple of four.  The same 16-byte
+// accesses at the addresses the lines have; the last 1 to 3 values of a line go element by
+// element, with -inf in the places past them, whose exponential is 0.  Exponentials and
+// quotients are the ones of the general kernel below, which made three passes over such lines,
+// 4 bytes per access (8193 lines of 8191: 314 -> 104 us; backward 233 -> 147).
+template <class LineVec>
+__device__ __forceinline__ void line_load(mnv_f4& v, const LineVec& whole, const float* p, int left, float fill) {
+  if (left >= 4) {
+    v = whole();
+  } else {
+    v.x = p[0];
+    v.y = left > 1 ? p[1] : fill;
+    v.z = left > 2 ? p[2] : fill;
+    v.w = fill;
+  }
+}
+__device__ __forceinline__ void line_store(float* p, int left, mnv_f4 o) {
+  if (left >= 4) {
+    *reinterpret_cast<mnv_f4u*>(p) = o;
+  } else {
+    p[0] = o.x;
+    if (left > 1) p[1] = o.y;
+    if (left > 2) p[2] = o.z;
+  }
+}
+
+template <int GROUP, int CACHE, int NTH, bool NT, bool ODD>
 __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     const float* __restrict__ in, float* __restrict__ out, int len, int lines) {
   __shared__ float lds[NTH / MNV_WAVE];
   constexpr int LPB = NTH / GROUP;
   const int t = threadIdx.x % GROUP;
-  const int len4 = len >> 2;
+  const int len4 = (len + 3) >> 2;
   // the trip count is block-uniform when GROUP spans the block (and the line index then a
   // scalar: the compiler cannot tell that threadIdx.x / GROUP is 0); with one wavefront per
   // line no barrier is used
   for (int line = blockIdx.x * LPB + (LPB > 1 ? threadIdx.x / GROUP : 0); line < lines; line += gridDim.x * LPB) {
-    const mnv_f4* x4 = lane_pointer(reinterpret_cast<const mnv_f4*>(in + (size_t)line * len) + t);
-    mnv_f4* y4 = lane_pointer(reinterpret_cast<mnv_f4*>(out + (size_t)line * len) + t);
+    const float* x = lane_pointer(in + (size_t)line * len + 4 * t);
+    float* y = lane_pointer(out + (size_t)line * len + 4 * t);
+    const mnv_f4* x4 = reinterpret_cast<const mnv_f4*>(x);
+    mnv_f4* y4 = reinterpret_cast<mnv_f4*>(y);
+    const int left = len - 4 * t;  // values from the thread's first vector on
     mnv_f4 v[CACHE];
     // all loads first, in a loop of their own: a use inside the same guarded block would
     // make each load wait for the one before it
 #pragma unroll
     for (int u = 0; u < CACHE; ++u)
-      if (t + u * GROUP < len4) v[u] = mnv_ldx4<NT>(x4 + u * GROUP);
+      if (t + u * GROUP < len4) {
+        if (ODD)
+          line_load(v[u], [&] { return mnv_ldx4u<NT>(x + 4 * u * GROUP); }, x + 4 * u * GROUP, left - 4 * u * GROUP,
+                    -INFINITY);
+        else
+          v[u] = mnv_ldx4<NT>(x4 + u * GROUP);
+      }
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < CACHE; ++u)
@@ -96,10 +131,10 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
         // exp through the hardware exp2: relative error ~1e-6 for the arguments <= 0 here
-        v[u].x = __expf(v[u].x - mx);
-        v[u].y = __expf(v[u].y - mx);
-        v[u].z = __expf(v[u].z - mx);
-        v[u].w = __expf(v[u].w - mx);
+        v[u].x = ODD ? expf(v[u].x - mx) : __expf(v[u].x - mx);
+        v[u].y = ODD ? expf(v[u].y - mx) : __expf(v[u].y - mx);
+        v[u].z = ODD ? expf(v[u].z - mx) : __expf(v[u].z - mx);
+        v[u].w = ODD ? expf(v[u].w - mx) : __expf(v[u].w - mx);
         s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
       }
     }
@@ -109,11 +144,12 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
         mnv_f4 o;
-        o.x = v[u].x * inv;
-        o.y = v[u].y * inv;
-        o.z = v[u].z * inv;
-        o.w = v[u].w * inv;
-        __builtin_nontemporal_store(o, y4 + u * GROUP);
+        o.x = ODD ? v[u].x / s : v[u].x * inv;
+        o.y = ODD ? v[u].y / s : v[u].y * inv;
+        o.z = ODD ? v[u].z / s : v[u].z * inv;
+        o.w = ODD ? v[u].w / s : v[u].w * inv;
+        if (ODD) line_store(y + 4 * u * GROUP, left - 4 * u * GROUP, o);
+        else __builtin_nontemporal_store(o, y4 + u * GROUP);
       }
     }
   }
@@ -146,24 +182,34 @@ __global__ __launch_bounds__(MNV_SM_THREADS) void mnv_softmax_fwd_generic_kernel
   }
 }
 
-template <int GROUP, int CACHE, int NTH>
+template <int GROUP, int CACHE, int NTH, bool ODD>
 __global__ __launch_bounds__(NTH) void mnv_softmax_bwd_cached_kernel(
     const float* __restrict__ dy, const float* __restrict__ y, float* __restrict__ dx, int len,
     int lines) {
   __shared__ float lds[NTH / MNV_WAVE];
   constexpr int LPB = NTH / GROUP;
   const int t = threadIdx.x % GROUP;
-  const int len4 = len >> 2;
+  const int len4 = (len + 3) >> 2;
   for (int line = blockIdx.x * LPB + (LPB > 1 ? threadIdx.x / GROUP : 0); line < lines; line += gridDim.x * LPB) {
-    const mnv_f4* d4 = lane_pointer(reinterpret_cast<const mnv_f4*>(dy + (size_t)line * len) + t);
-    const mnv_f4* t4 = lane_pointer(reinterpret_cast<const mnv_f4*>(y + (size_t)line * len) + t);
-    mnv_f4* o4 = lane_pointer(reinterpret_cast<mnv_f4*>(dx + (size_t)line * len) + t);
+    const float* dp = lane_pointer(dy + (size_t)line * len + 4 * t);
+    const float* tp = lane_pointer(y + (size_t)line * len + 4 * t);
+    float* op = lane_pointer(dx + (size_t)line * len + 4 * t);
+    const mnv_f4* d4 = reinterpret_cast<const mnv_f4*>(dp);
+    const mnv_f4* t4 = reinterpret_cast<const mnv_f4*>(tp);
+    mnv_f4* o4 = reinterpret_cast<mnv_f4*>(op);
+    const int left = len - 4 * t;
     mnv_f4 d[CACHE], p[CACHE];
 #pragma unroll
     for (int u = 0; u < CACHE; ++u) {  // loads only, so that none waits for another
       if (t + u * GROUP < len4) {
-        d[u] = d4[u * GROUP];
-        p[u] = __builtin_nontemporal_load(t4 + u * GROUP);
+        const int at = 4 * u * GROUP;
+        if (ODD) {  // zeros past the line's end: they add nothing to the sum
+          line_load(d[u], [&] { return mnv_ldx4u<false>(dp + at); }, dp + at, left - at, 0.f);
+          line_load(p[u], [&] { return mnv_ldx4u<true>(tp + at); }, tp + at, left - at, 0.f);
+        } else {
+          d[u] = d4[u * GROUP];
+          p[u] = __builtin_nontemporal_load(t4 + u * GROUP);
+        }
       }
     }
     float dot = 0.f;
@@ -180,7 +226,8 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_bwd_cached_kernel(
         o.y = p[u].y * (d[u].y - dot);
         o.z = p[u].z * (d[u].z - dot);
         o.w = p[u].w * (d[u].w - dot);
-        __builtin_nontemporal_store(o, o4 + u * GROUP);
+        if (ODD) line_store(op + 4 * u * GROUP, left - 4 * u * GROUP, o);
+        else __builtin_nontemporal_store(o, o4 + u * GROUP);
       }
     }
   }
@@ -345,56 +392,66 @@ unsigned line_grid(int lines, int lpb) {
   return (unsigned)(b < 65536 ? b : 65536);
 }
 
-// Contiguous lines of `len` floats (instance mode, or channel mode with H*W == 1).
+// Contiguous lines of `len` floats (instance mode, or channel mode with H*W == 1).  One wavefront
+// per line up to 2048 values; lines off the 16-byte grid, whose loads are guarded one by one, up to
+// 1024; up to 256 each lane has one vector and no guarded loads of more (256 lines of 10:
+// 4.3 us with eight; 1023 lines of 2047, one wavefront -> 256 threads: forward 7.9 -> 5.8 us, backward 8.4 -> 5.1).
 #define MNV_SM_WIDE 512      // threads per line for lines of more than 4096 values
 #define MNV_SM_WIDE_CACHE 4  // 16-byte vectors cached per thread in that configuration
 template <int GROUP, int CACHE, int NTH>
-void launch_fwd_cached(const float* in, float* out, int len, int lines, bool nt, hipStream_t s) {
+int launch_fwd_cached(const float* in, float* out, int len, int lines, bool vec, bool nt, hipStream_t s) {
   const dim3 grid(line_grid(lines, NTH / GROUP)), block(NTH);
-  if (nt)
-    hipLaunchKernelGGL((mnv_softmax_fwd_cached_kernel<GROUP, CACHE, NTH, true>), grid, block, 0, s, in,
-                       out, len, lines);
-  else
-    hipLaunchKernelGGL((mnv_softmax_fwd_cached_kernel<GROUP, CACHE, NTH, false>), grid, block, 0, s, in,
-                       out, len, lines);
+#define MNV_SM_LAUNCH(NT, ODD)                                                                             \
+  hipLaunchKernelGGL((mnv_softmax_fwd_cached_kernel<GROUP, CACHE, NTH, NT, ODD>), grid, block, 0, s, in, \
+                     out, len, lines)
+  if (vec) {
+    if (nt) MNV_SM_LAUNCH(true, false); else MNV_SM_LAUNCH(false, false);
+  } else {
+    if (nt) MNV_SM_LAUNCH(true, true); else MNV_SM_LAUNCH(false, true);
+  }
+#undef MNV_SM_LAUNCH
+  return MNV_LAUNCH_STATUS();
 }
 
 int softmax_lines_fwd(const float* in, float* out, int len, int lines, hipStream_t s) {
-  bool vec = (len % 4 == 0) && mnv_aligned16(in) && mnv_aligned16(out);
+  const bool vec = (len % 4 == 0) && mnv_aligned16(in) && mnv_aligned16(out);
   const bool big = (size_t)len * lines * sizeof(float) >= MNV_PAST_CACHE_BYTES;
-  if (vec && len <= MNV_WAVE * 4 * MNV_SM_CACHE)
-    launch_fwd_cached<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>(in, out, len, lines, big, s);
-  else if (vec && len <= MNV_SM_THREADS * 4 * MNV_SM_WIDE_CACHE)
-    launch_fwd_cached<MNV_SM_THREADS, MNV_SM_WIDE_CACHE, MNV_SM_THREADS>(in, out, len, lines, big, s);
-  else if (vec && len <= MNV_SM_WIDE * 4 * MNV_SM_WIDE_CACHE)
-    launch_fwd_cached<MNV_SM_WIDE, MNV_SM_WIDE_CACHE, MNV_SM_WIDE>(in, out, len, lines, big, s);
-  else if (len <= 1024)
-    hipLaunchKernelGGL((mnv_softmax_fwd_generic_kernel<MNV_WAVE>), dim3(line_grid(lines, 4)),
-                       dim3(MNV_SM_THREADS), 0, s, in, out, len, lines, 1, (size_t)len, (size_t)1);
+  if (len <= MNV_WAVE * 4) return launch_fwd_cached<MNV_WAVE, 1, MNV_SM_THREADS>(in, out, len, lines, vec, big, s);
+  if (len <= MNV_WAVE * 4 * MNV_SM_CACHE / (vec ? 1 : 2))
+    return launch_fwd_cached<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>(in, out, len, lines, vec, big, s);
+  if (len <= MNV_SM_THREADS * 4 * MNV_SM_WIDE_CACHE)
+    return launch_fwd_cached<MNV_SM_THREADS, MNV_SM_WIDE_CACHE, MNV_SM_THREADS>(in, out, len, lines, vec, big, s);
+  if (len <= MNV_SM_WIDE * 4 * MNV_SM_WIDE_CACHE)
+    return launch_fwd_cached<MNV_SM_WIDE, MNV_SM_WIDE_CACHE, MNV_SM_WIDE>(in, out, len, lines, vec, big, s);
+  hipLaunchKernelGGL((mnv_softmax_fwd_generic_kernel<MNV_SM_THREADS>), dim3(line_grid(lines, 1)),
+                     dim3(MNV_SM_THREADS), 0, s, in, out, len, lines, 1, (size_t)len, (size_t)1);
+  return MNV_LAUNCH_STATUS();
+}
+
+template <int GROUP, int CACHE, int NTH>
+int launch_bwd_cached(const float* dy, const float* y, float* dx, int len, int lines, bool vec, hipStream_t s) {
+  const dim3 grid(line_grid(lines, NTH / GROUP)), block(NTH);
+  if (vec)
+    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<GROUP, CACHE, NTH, false>), grid, block, 0, s, dy, y, dx,
+                       len, lines);
   else
-    hipLaunchKernelGGL((mnv_softmax_fwd_generic_kernel<MNV_SM_THREADS>), dim3(line_grid(lines, 1)),
-                       dim3(MNV_SM_THREADS), 0, s, in, out, len, lines, 1, (size_t)len, (size_t)1);
+    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<GROUP, CACHE, NTH, true>), grid, block, 0, s, dy, y, dx,
+                       len, lines);
   return MNV_LAUNCH_STATUS();
 }
 
 int softmax_lines_bwd(const float* dy, const float* y, float* dx, int len, int lines,
                       hipStream_t s) {
-  bool vec = (len % 4 == 0) && mnv_aligned16(dy) && mnv_aligned16(y) && mnv_aligned16(dx);
-  if (vec && len <= MNV_WAVE * 4 * MNV_SM_CACHE)
-    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>),
-                       dim3(line_grid(lines, 4)), dim3(MNV_SM_THREADS), 0, s, dy, y, dx, len, lines);
-  else if (vec && len <= MNV_SM_THREADS * 4 * MNV_SM_WIDE_CACHE)
-    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<MNV_SM_THREADS, MNV_SM_WIDE_CACHE, MNV_SM_THREADS>),
-                       dim3(line_grid(lines, 1)), dim3(MNV_SM_THREADS), 0, s, dy, y, dx, len, lines);
-  else if (vec && len <= MNV_SM_WIDE * 4 * MNV_SM_WIDE_CACHE)
-    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<MNV_SM_WIDE, MNV_SM_WIDE_CACHE, MNV_SM_WIDE>),
-                       dim3(line_grid(lines, 1)), dim3(MNV_SM_WIDE), 0, s, dy, y, dx, len, lines);
-  else if (len <= 1024)
-    hipLaunchKernelGGL((mnv_softmax_bwd_generic_kernel<MNV_WAVE>), dim3(line_grid(lines, 4)),
-                       dim3(MNV_SM_THREADS), 0, s, dy, y, dx, len, lines, 1, (size_t)len, (size_t)1);
-  else
-    hipLaunchKernelGGL((mnv_softmax_bwd_generic_kernel<MNV_SM_THREADS>), dim3(line_grid(lines, 1)),
-                       dim3(MNV_SM_THREADS), 0, s, dy, y, dx, len, lines, 1, (size_t)len, (size_t)1);
+  const bool vec = (len % 4 == 0) && mnv_aligned16(dy) && mnv_aligned16(y) && mnv_aligned16(dx);
+  if (len <= MNV_WAVE * 4) return launch_bwd_cached<MNV_WAVE, 1, MNV_SM_THREADS>(dy, y, dx, len, lines, vec, s);
+  if (len <= MNV_WAVE * 4 * MNV_SM_CACHE / (vec ? 1 : 2))
+    return launch_bwd_cached<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>(dy, y, dx, len, lines, vec, s);
+  if (len <= MNV_SM_THREADS * 4 * MNV_SM_WIDE_CACHE)
+    return launch_bwd_cached<MNV_SM_THREADS, MNV_SM_WIDE_CACHE, MNV_SM_THREADS>(dy, y, dx, len, lines, vec, s);
+  if (len <= MNV_SM_WIDE * 4 * MNV_SM_WIDE_CACHE)
+    return launch_bwd_cached<MNV_SM_WIDE, MNV_SM_WIDE_CACHE, MNV_SM_WIDE>(dy, y, dx, len, lines, vec, s);
+  hipLaunchKernelGGL((mnv_softmax_bwd_generic_kernel<MNV_SM_THREADS>), dim3(line_grid(lines, 1)),
+                     dim3(MNV_SM_THREADS), 0, s, dy, y, dx, len, lines, 1, (size_t)len, (size_t)1);
   return MNV_LAUNCH_STATUS();
 }
 
