@@ -156,21 +156,19 @@ struct SgemmNN {
 
 // Products with at most 12 columns (inner products over a few images): every value of A is
 // used that few times, so the product is bound by reading A once, while the smallest MFMA tile
-// of the core multiplies 64 columns.  Here a lane keeps its rows' sums for NC columns (N
+// of the core multiplies 64 columns.  Here a lane keeps its four rows' sums for NC columns (N
 // rounded up to one of a few widths; the columns past N repeat the last one and are not stored)
 // and multiplies by B's values, which are the same for the whole wavefront and come through the
-// scalar cache.  x-fast A: four rows per lane, 1 KB of a column per load; transposed A: one row
-// per lane, four k per load.  A workgroup's four wavefronts take a quarter of its k range each,
-// and their sums are added through LDS, (w0 + w2) + (w1 + w3); the k ranges of the grid's y
-// dimension go through the workspace and the reduction kernel.  Either form adds the same
-// values in the same order.
+// scalar cache.  A load is 1 KB of a column.  A workgroup's four wavefronts take a quarter of its k
+// range each, and their sums are added through LDS, (w0 + w2) + (w1 + w3); the k ranges of the
+// grid's y dimension go through the workspace and the reduction kernel.
 // Measured at 1 / 10 columns, with the reduction: 4096 x 9216 43.6 -> 26.4 us
 // and 42.7 -> 33.2 us, 1000 x 4096 at 1 column 11.1 -> 6.6 us.
 #define MNV_SKINNY_COLUMNS 12
-template <class P, int NC, bool TA, bool TB>
+template <class P, int NC, bool TB>
 __global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const float* __restrict__ B, int k_per_wave,
                                                                float* __restrict__ partial) {
-  constexpr int RM = TA ? 1 : 4, U = NC <= 4 ? 16 : NC <= 8 ? 8 : 4;  // rows per lane, k per step
+  constexpr int RM = 4, U = NC <= 4 ? 16 : NC <= 8 ? 8 : 4;  // rows per lane, k per step
   __shared__ float red[2 * MNV_WAVE * RM * NC];
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
   const int m = (blockIdx.x * MNV_WAVE + lane) * RM;
@@ -189,29 +187,11 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const flo
 #pragma unroll
     for (int q = 0; q < RM; ++q) acc[j][q] = 0.f;
   // bytes from the wavefront's k to the lane's rows; the rest of the address is uniform
-  const unsigned off = m < prob.M ? (unsigned)m * (TA ? (unsigned)prob.lda : 1u) * 4u : MNV_OOB;
-  const unsigned ak = TA ? 4u : (unsigned)prob.lda * 4u;
+  const unsigned off[1] = {m < prob.M ? (unsigned)m * 4u : MNV_OOB}, ak = (unsigned)prob.lda * 4u;
   for (; k + U <= k_end; k += U) {
     float v[U][RM];
-    if constexpr (TA) {
 #pragma unroll
-      for (int u = 0; u < U; u += 4) {
-        float t[4];
-        const unsigned o[1] = {off};
-        mnv_fetch_vec<1>(res.a, o, (unsigned)(k + u) * ak, t);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[u + q][0] = t[q];
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        float t[4];
-        const unsigned o[1] = {off};
-        mnv_fetch_vec<1>(res.a, o, (unsigned)(k + u) * ak, t);
-#pragma unroll
-        for (int q = 0; q < RM; ++q) v[u][q] = t[q];
-      }
-    }
+    for (int u = 0; u < U; ++u) mnv_fetch_vec<1>(res.a, off, (unsigned)(k + u) * ak, v[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -223,10 +203,7 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const flo
   }
   for (; k < k_end; ++k) {
     float v[RM];
-#pragma unroll
-    for (int q = 0; q < RM; ++q)
-      v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                           res.a, (int)(m + q < prob.M ? off + 4u * q : MNV_OOB), (int)((unsigned)k * ak), 0));
+    mnv_fetch_vec<1>(res.a, off, (unsigned)k * ak, v);
 #pragma unroll
     for (int j = 0; j < NC; ++j) {
       const float b = B[col[j] + (size_t)k * bk];
@@ -262,6 +239,109 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const flo
         if (gridDim.y > 1) partial[((size_t)blockIdx.y * prob.N + j) * prob.M + m + q] = acc[j][q];
         else prob.c_store(m + q, j, acc[j][q]);
       }
+}
+
+// The same with A given transposed: every value added in the order of the kernel above, so that
+// the bits are the same.  A row of A is contiguous along k, and a lane that walks its own row
+// reads 16 bytes of a line per load, 64 lines at once (4096 x 4096 at 4 / 12 columns 25.8 / 92.8 us,
+// where the tiles take 24.1 / 25.1; this kernel 16.7 / 18.0).  The workgroup's 64 rows and B's
+// columns come in runs of RUN k instead, through an LDS strip of the wavefront's own (a wavefront's
+// LDS accesses execute in order; the pitch spreads eight lanes' 16-byte reads over all banks), the
+// next run in flight under the multiplies.  A value of B would then meet one row per lane, too
+// few multiplies for a load from the scalar cache (24.7 / 55.5 us); the 16 x 16 x 1 and
+// 4 x 4 x 1 matrix instructions add one k to all 64 rows and 16 or 4 columns, one multiply-add per
+// element.  RUN: 128 bytes of a row, or 64 where a wavefront has no more than 16 k (half the
+// LDS, twice the workgroups on a CU: 8192 x 1 x 512 10.4 -> 8.0 us).  Neighbouring workgroups take
+// the k ranges of the same rows: with the row blocks first, a pitch that is a power of two keeps few memory
+// channels busy (9216 x 1 x 4096 50.6 -> 34.2 us).
+template <class P, int RUN, int COLS>
+__global__ __launch_bounds__(256) void mnv_sgemm_skinny_tn_kernel(P prob, int k_per_wave, int ranges,
+                                                                  float* __restrict__ partial) {
+  constexpr int REGS = COLS;                               // of a lane's 64 x COLS / 64 sums
+  typedef float Acc __attribute__((ext_vector_type(REGS)));
+  constexpr int PITCH = RUN + 4, LPL = RUN / 4, PER = MNV_WAVE / LPL;  // lanes per line, lines per load
+  constexpr int LINES = MNV_WAVE + (COLS > PER ? COLS : PER), VECS = LINES / PER, AV = MNV_WAVE / PER;  // A's rows, B's columns
+  __shared__ __align__(16) float strips[4 * LINES * PITCH];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
+  const int range = (int)blockIdx.x % ranges, m0 = (int)blockIdx.x / ranges * MNV_WAVE;
+  const int line = lane / LPL, k4 = lane % LPL * 4;
+  int k = (range * 4 + wave) * k_per_wave;
+  const int k_end = k + k_per_wave < prob.K ? k + k_per_wave : prob.K;
+  typename P::Res res;
+  prob.make_res(res);
+  float* const strip = strips + wave * LINES * PITCH;
+  // Rows past M and k past the last row's end lie past the tensor, where loads answer 0.  The
+  // columns past N repeat the last one and are not stored.
+  const unsigned pitch = (unsigned)prob.lda * 4u;
+  float v[VECS][4];
+  auto load = [&](int at) {
+    const bool on = at + k4 < k_end;
+#pragma unroll
+    for (int u = 0; u < VECS; ++u) {
+      const int j = (u - AV) * PER + line;
+      const unsigned row = u < AV ? (unsigned)(m0 + line) * pitch : (unsigned)(j < prob.N ? j : prob.N - 1) * (unsigned)prob.ldb * 4u;
+      const unsigned off[1] = {on ? row + (unsigned)k4 * 4u : MNV_OOB};
+      mnv_fetch_vec<1>(u < AV ? res.a : res.b, off, (u < AV ? (unsigned)(u * PER) * pitch : 0u) + (unsigned)at * 4u, v[u]);
+    }
+  };
+  Acc acc = 0.f;
+  if (k < k_end) load(k);
+  for (; k < k_end; k += RUN) {
+    const int count = k_end - k < RUN ? k_end - k : RUN;
+    if (count < RUN) {  // what lies past the range multiplies 0 by -0, which leaves every sum as it is
+#pragma unroll
+      for (int u = 0; u < VECS; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u][e] = k4 + e < count ? v[u][e] : u < AV ? 0.f : -0.f;
+    }
+#pragma unroll
+    for (int u = 0; u < VECS; ++u)
+      *reinterpret_cast<mnv_f4*>(strip + (u * PER + line) * PITCH + k4) = mnv_f4{v[u][0], v[u][1], v[u][2], v[u][3]};
+    __builtin_amdgcn_wave_barrier();
+    if (k + RUN < k_end) load(k + RUN);
+    auto multiply = [&](int kk) {
+      const mnv_f4 a = *reinterpret_cast<const mnv_f4*>(strip + lane * PITCH + kk);
+      const mnv_f4 b = *reinterpret_cast<const mnv_f4*>(strip + (MNV_WAVE + lane % COLS) * PITCH + kk);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (COLS == 16) acc = __builtin_amdgcn_mfma_f32_16x16x1f32(a[e], b[e], acc, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_f32_4x4x1f32(a[e], b[e], acc, 0, 0, 0);
+      }
+    };
+    if (count == RUN) {
+#pragma unroll
+      for (int kk = 0; kk < RUN; kk += 4) multiply(kk);
+    } else {
+      for (int kk = 0; kk < count; kk += 4) multiply(kk);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // Register q of lane l holds row q / 4 * 16 + l / 16 * 4 + q % 4 and column l % 16, or row l / 4 * 4 + q
+  // and column l % 4; it lies at q * 65 + l of a region, neighbouring rows of a column in different banks.
+  float* const red = strips;
+  constexpr int REGION = REGS * 65;
+  __syncthreads();  // the strips become the wavefronts' sums
+  if (wave >= 2) {
+#pragma unroll
+    for (int q = 0; q < REGS; ++q) red[(wave - 2) * REGION + q * 65 + lane] = acc[q];
+  }
+  __syncthreads();
+  if (wave < 2) {
+#pragma unroll
+    for (int q = 0; q < REGS; ++q) {
+      float* at = red + wave * REGION + q * 65 + lane;
+      *at = acc[q] + *at;
+    }
+  }
+  __syncthreads();
+  const int r = lane, m = m0 + r;
+  if (m >= prob.M) return;
+  for (int j = wave; j < prob.N; j += 4) {
+    const float* at = red + (COLS == 16 ? (r / 16 * 4 + r % 4) * 65 + r % 16 / 4 * 16 : r % 4 * 65 + r / 4 * 4) + j;
+    const float x = at[0] + at[REGION];
+    if (ranges > 1) partial[((size_t)range * prob.N + j) * prob.M + m] = x;
+    else prob.c_store(m, j, x);
+  }
 }
 
 struct SgemmEpilogue {
@@ -407,24 +487,38 @@ SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   return best;
 }
 
-template <int NC, bool TA, bool TB, class P>
-int launch_skinny(const SgemmPlan& plan, const P& p, void* workspace, hipStream_t s) {
-  const int rows = TA ? MNV_WAVE : 4 * MNV_WAVE;
-  float* part = plan.splits > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
-  hipLaunchKernelGGL((mnv_sgemm_skinny_kernel<P, NC, TA, TB>), dim3((p.M + rows - 1) / rows, plan.splits), dim3(256), 0, s,
-                     p, p.B, plan.skinny, part);
-  const int rc = MNV_LAUNCH_STATUS();
-  if (rc || plan.splits == 1) return rc;
-  return mnv_gemm_reduce_launch(p, part, plan.splits, s);
+template <int NC, bool TB, class P>
+void launch_skinny(const SgemmPlan& plan, const P& p, float* part, hipStream_t s) {
+  hipLaunchKernelGGL((mnv_sgemm_skinny_kernel<P, NC, TB>), dim3((p.M + 4 * MNV_WAVE - 1) / (4 * MNV_WAVE), plan.splits),
+                     dim3(256), 0, s, p, p.B, plan.skinny, part);
+}
+
+template <int RUN, int COLS, class P>
+void launch_skinny_tn(const SgemmPlan& plan, const P& p, float* part, hipStream_t s) {
+  hipLaunchKernelGGL((mnv_sgemm_skinny_tn_kernel<P, RUN, COLS>), dim3((p.M + MNV_WAVE - 1) / MNV_WAVE * plan.splits),
+                     dim3(256), 0, s, p, plan.skinny, plan.splits, part);
 }
 
 template <bool K4, bool TA, bool TB>
 int launch_skinny_columns(const SgemmPlan& plan, const SgemmNN<K4, TA, TB>& p, void* workspace, hipStream_t s) {
-  if (p.N <= 1) return launch_skinny<1, TA, TB>(plan, p, workspace, s);
-  if (p.N <= 2) return launch_skinny<2, TA, TB>(plan, p, workspace, s);
-  if (p.N <= 4) return launch_skinny<4, TA, TB>(plan, p, workspace, s);
-  if (p.N <= 8) return launch_skinny<8, TA, TB>(plan, p, workspace, s);
-  return launch_skinny<MNV_SKINNY_COLUMNS, TA, TB>(plan, p, workspace, s);
+  static_assert(!(TA && TB), "one operand transposed at most");
+  float* part = plan.splits > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
+  if constexpr (TA) {
+    if (p.N <= 4) {
+      if (plan.skinny <= 16) launch_skinny_tn<16, 4>(plan, p, part, s);
+      else launch_skinny_tn<32, 4>(plan, p, part, s);
+    } else {
+      if (plan.skinny <= 16) launch_skinny_tn<16, 16>(plan, p, part, s);
+      else launch_skinny_tn<32, 16>(plan, p, part, s);
+    }
+  } else if (p.N <= 1) launch_skinny<1, TB>(plan, p, part, s);
+  else if (p.N <= 2) launch_skinny<2, TB>(plan, p, part, s);
+  else if (p.N <= 4) launch_skinny<4, TB>(plan, p, part, s);
+  else if (p.N <= 8) launch_skinny<8, TB>(plan, p, part, s);
+  else launch_skinny<MNV_SKINNY_COLUMNS, TB>(plan, p, part, s);
+  const int rc = MNV_LAUNCH_STATUS();
+  if (rc || plan.splits == 1) return rc;
+  return mnv_gemm_reduce_launch(p, part, plan.splits, s);
 }
 
 // A launch without k ranges may use the workspace for the partial tiles of a cut tail.

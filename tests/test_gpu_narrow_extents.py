@@ -1,0 +1,88 @@
+"""Products and matrix operators with one narrow extent: the kernel that each of them takes at the
+sizes where the choice changes, and that none of them costs a multiple of the same work in a form
+that reads its operands alike.  Times are medians of calls of both forms in turn; the bounds
+leave a third and more to what the forms measured (both figures beside each bound)."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_util import Gpu, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return Gpu()
+
+
+def _rand(n, seed):
+    return np.random.default_rng(seed).standard_normal(n).astype(np.float32)
+
+
+def _ratio(gpu, slow, fast, iters=20):
+    """Median time of slow() over that of fast(), measured in turn."""
+    t = [[gpu.dev.time_ms(f, iters=iters, warmup=2) for f in (slow, fast)] for _ in range(9)]
+    a, b = (sorted(x)[4] for x in zip(*t))
+    say("  %.2f us against %.2f us" % (a * 1e3, b * 1e3))
+    return a / b
+
+
+def _plan(gpu, m, n, k, ws_bytes):
+    v = [ctypes.c_int() for _ in range(3)]
+    assert gpu.L.mnv_sgemm_nn_plan(m, n, k, ctypes.c_size_t(ws_bytes), *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+def _bits(gpu, form, a, b, m, n, k, ws_bytes, *more):
+    """The product through mnv_sgemm_<form>: a, b on the device as the form takes them."""
+    ws, dc = gpu.empty(ws_bytes // 4 + 1), gpu.empty(m * n)
+    gpu.call("mnv_sgemm_" + form, a.p, b.p, *more, dc.p, m, n, k, ws.p, ctypes.c_size_t(ws_bytes))
+    return gpu.down(dc)
+
+
+# 64 rows to a workgroup: one row, 63 and all of the last one's; k ranges that end in 1 to 4 values of
+# a vector, in the first half of a run of 32 and in the second; at most 16 k per wavefront and more
+@pytest.mark.parametrize("m,k,n", [(257, 16385, 1), (257, 16385, 5), (319, 16384, 4), (319, 16384, 8), (4160, 4110, 3),
+                                   (4160, 4110, 12), (4097, 8207, 1), (4097, 8207, 11)])
+def test_few_columns_of_a_transposed_operand_have_the_plain_forms_bits(gpu, m, k, n):
+    """Values over the whole exponent range (products that underflow and that overflow among them), an
+    infinity and a NaN in a row of A and in a column of B: the bits of mnv_sgemm_nn, and the other
+    rows and columns finite where all their products are."""
+    say("few columns, transposed", m, n, k)
+    ws_bytes = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    tile, _, groups = _plan(gpu, m, n, k, ws_bytes)
+    assert (tile, groups) == (256, 4), "the case must run the few-column kernels"
+    for wide in (False, True):
+        a, b = _rand(m * k, 20).reshape(k, m), _rand(n * k, 21).reshape(n, k)
+        if wide:
+            a[::7] *= np.float32(1e-30)
+            b[:, ::5] *= np.float32(1e-12)
+        else:
+            a[k - 1, m - 1], a[3, 7] = np.inf, np.nan
+            b[n - 1, 5] = -np.inf
+        da, dat = gpu.up(a.reshape(-1)), gpu.up(np.ascontiguousarray(a.T).reshape(-1))
+        db = gpu.up(b.reshape(-1))
+        want = _bits(gpu, "nn", da, db, m, n, k, ws_bytes)
+        assert _bits(gpu, "tn", dat, db, m, n, k, ws_bytes, None).tobytes() == want.tobytes()
+        if not wide:
+            C = want.reshape(n, m)
+            assert np.isfinite(np.delete(np.delete(C, n - 1, 0), (7, m - 1), 1)).all()
+            assert not np.isfinite(C[n - 1]).any() and not np.isfinite(C[:, (7, m - 1)]).any()
+        gate = _rand(m * n, 22)
+        dgate = gpu.up(gate)
+        got = _bits(gpu, "tn", dat, db, m, n, k, ws_bytes, dgate.p)
+        assert got.tobytes() == np.where(gate > 0, want, np.float32(0)).tobytes()
+
+
+@pytest.mark.parametrize("m,n,k", [(4096, 12, 4096), (9216, 2, 4096), (4096, 8, 9216)])
+def test_few_columns_of_a_transposed_operand_cost_what_the_plain_form_does(gpu, m, n, k):
+    """18.0 against 20.6 us, 35.3 / 26.5 and 33.2 / 30.4 (one lane per row of A: 92.8, 58.1 and 62.5)."""
+    say("few columns, transposed, time", m, n, k)
+    ws_bytes = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    a, b, c, ws = gpu.empty(m * k), gpu.empty(n * k), gpu.empty(m * n), gpu.empty(ws_bytes // 4 + 1)
+    for d, count in ((a, m * k), (b, n * k)):
+        gpu.call("mnv_randn", d.p, ctypes.c_size_t(count), ctypes.c_uint64(5), ctypes.c_float(0), ctypes.c_float(1))
+    tail = (c.p, m, n, k, ws.p, ctypes.c_size_t(ws_bytes), gpu.dev.stream)
+    assert _ratio(gpu, lambda: gpu.L.mnv_sgemm_tn(a.p, b.p, None, *tail), lambda: gpu.L.mnv_sgemm_nn(a.p, b.p, *tail)) < 1.8
