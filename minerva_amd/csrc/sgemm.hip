@@ -188,29 +188,31 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_kernel(P prob, const flo
     for (int q = 0; q < RM; ++q) acc[j][q] = 0.f;
   // bytes from the wavefront's k to the lane's rows; the rest of the address is uniform
   const unsigned off[1] = {m < prob.M ? (unsigned)m * 4u : MNV_OOB}, ak = (unsigned)prob.lda * 4u;
-  for (; k + U <= k_end; k += U) {
-    float v[U][RM];
+  auto step = [&](auto S, auto CUT) {
+    constexpr int steps = decltype(S)::value;
+    constexpr bool cut = decltype(CUT)::value;  // k + steps may pass k_end: 0 times -0 there, which leaves every sum as it is
+    float v[steps][RM];
 #pragma unroll
-    for (int u = 0; u < U; ++u) mnv_fetch_vec<1>(res.a, off, (unsigned)(k + u) * ak, v[u]);
+    for (int u = 0; u < steps; ++u) {
+      const unsigned o[1] = {cut && k + u >= k_end ? MNV_OOB : off[0]};
+      mnv_fetch_vec<1>(res.a, o, (unsigned)(k + u) * ak, v[u]);
+    }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < steps; ++u)
 #pragma unroll
       for (int j = 0; j < NC; ++j) {
-        const float b = B[col[j] + (size_t)(k + u) * bk];
+        const bool on = !cut || k + u < k_end;
+        const float x = B[col[j] + (size_t)(on ? k + u : k) * bk], b = on ? x : -0.f;
 #pragma unroll
         for (int q = 0; q < RM; ++q) acc[j][q] = __builtin_fmaf(v[u][q], b, acc[j][q]);
       }
-  }
-  for (; k < k_end; ++k) {
-    float v[RM];
-    mnv_fetch_vec<1>(res.a, off, (unsigned)k * ak, v);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      const float b = B[col[j] + (size_t)k * bk];
-#pragma unroll
-      for (int q = 0; q < RM; ++q) acc[j][q] = __builtin_fmaf(v[q], b, acc[j][q]);
-    }
-  }
+    k += steps;
+  };
+  typedef std::false_type Whole;
+  while (k + U <= k_end) step(std::integral_constant<int, U>{}, Whole{});
+  if (U > 8 && k + 8 <= k_end) step(std::integral_constant<int, 8>{}, Whole{});
+  if (U > 4 && k + 4 <= k_end) step(std::integral_constant<int, 4>{}, Whole{});
+  if (k < k_end) step(std::integral_constant<int, 4>{}, std::true_type{});
   auto put = [&](int region) {
 #pragma unroll
     for (int j = 0; j < NC; ++j)
@@ -386,8 +388,10 @@ struct SgemmPlan {
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel, with this many k per wavefront
 };
 
-// Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), at
-// least 16 k per wavefront.  The tiles stay for a small A, where the time is that of two launches
+// Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), with
+// at least 16 k per wavefront, beyond 65 ranges 32 (1024 x 1 x 8192 12.2 -> 9.4 us).  The ranges are
+// whole steps of 16 k: only the wavefront at the end of k meets the kernels' cut steps.
+// The tiles stay for a small A, where the time is that of two launches
 // either way, and for more columns, where the multiplies, not A's bytes, take this kernel's time;
 // their own time does not change from 1 to 64 columns.  Before -> with this kernel, us:
 //   4 columns: 512 x 1 x 1024 6.6 -> 6.3, 1000 x 4 x 600 7.3 -> 7.3, 1000 x 1 x 4096 11.1 -> 6.6
@@ -396,20 +400,27 @@ struct SgemmPlan {
 //   12 columns: 1000 x 10 x 4096 12.3 -> 12.2, 4096 x 12 x 4096 24.4 -> 20.6, 9216 x 12 x 4096
 //     45.0 -> 33.4
 //   16 columns: 2000 x 16 x 2000 10.8 -> 16.9, 4096 x 16 x 4096 25.1 -> 25.4
-// They also stay where the workspace is too small for a quarter of the ranges, and below 256
-// rows (one block).
+// They also stay where the workspace holds fewer ranges and they make less than 128 workgroups, and
+// below 256 rows (one block).
 bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
   const long long least = n <= 4 ? 1LL << 19 : n <= 8 ? 1LL << 20 : 1LL << 24;  // elements of A
   if (n > MNV_SKINNY_COLUMNS || m < 256 || k < 64 || (long long)m * k < least) return false;
   const int blocks = (m + 255) / 256;
-  long long splits = 512 / blocks;
+  int per, ranges;
+  auto cut = [&](long long splits) {
+    per = (int)((k + 4 * splits - 1) / (4 * splits) + 15) / 16 * 16;
+    ranges = (int)(((long long)k + 4LL * per - 1) / (4LL * per));
+  };
+  const int most = 512 / blocks;
+  int slices = k < 128 ? 1 : (k + 63) / 64;
+  if (slices > 65) slices = k > 65 * 128 ? (k + 127) / 128 : 65;
+  cut(most < 1 ? 1 : most < slices ? most : slices);
   const size_t fit = ws_floats / ((size_t)m * n);
-  if (splits > k / 64) splits = k / 64;
-  if ((size_t)splits > fit) splits = (long long)fit;
-  if (splits < 1) splits = 1;
-  const int per = (int)((k + 4 * splits - 1) / (4 * splits) + 15) / 16 * 16;
-  const int ranges = (int)(((long long)k + 4LL * per - 1) / (4LL * per));
-  if ((long long)blocks * ranges < 128 && ranges < k / 64) return false;
+  if (ranges > 1 && (size_t)ranges > fit) {
+    const long long have = fit ? (long long)fit : 1;  // one range needs no workspace
+    if (blocks * have < 128) return false;
+    cut(have);
+  }
   *plan = SgemmPlan{false, ranges, 4};
   plan->skinny = per;
   return true;

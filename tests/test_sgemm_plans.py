@@ -1,0 +1,46 @@
+"""Which kernel a product of at most 12 columns takes: host arithmetic on the extents and the
+workspace alone, so checked without a GPU."""
+import ctypes
+
+import pytest
+
+from minerva_amd import capi
+
+
+def _query(m, n, k):
+    return capi.lib().mnv_sgemm_nn_workspace_bytes(m, n, k)
+
+
+def _plan(m, n, k, ws_bytes):
+    v = [ctypes.c_int() for _ in range(3)]
+    assert capi.lib().mnv_sgemm_nn_plan(m, n, k, ctypes.c_size_t(ws_bytes), *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+def _few(plan):
+    return plan[0] == 256 and plan[2] == 4
+
+
+@pytest.mark.parametrize("m", [256, 512, 513, 1000])
+def test_ranges_do_not_depend_on_how_k_ends(m):
+    """16 k per wavefront up to 65 ranges and 32 beyond, whatever k is modulo 64, with the workspace
+    that the query asks for and with more."""
+    for k in range(2048, 8321):
+        ws = _query(m, 1, k)
+        plan = _plan(m, 1, k, ws)
+        assert _few(plan), k
+        assert plan[1] == -(-k // (64 if k <= 4160 else 128)), k
+        assert ws == plan[1] * m * 4 and _plan(m, 1, k, 1 << 40) == plan, k
+
+
+def test_few_columns_with_less_workspace():
+    """A quarter of the 512 workgroups at least, or the tiles; the ranges never need more than there is."""
+    m, n, k = 4096, 3, 5000
+    full = _plan(m, n, k, _query(m, n, k))
+    assert full == (256, 27, 4)
+    for have in range(full[1] + 1):
+        plan = _plan(m, n, k, have * m * n * 4)
+        assert _few(plan) == (have >= 8), have
+        assert not _few(plan) or plan[1] <= have
+    for m, few in ((127 * 256, False), (127 * 256 + 1, True)):  # 128 row blocks: one range, no workspace
+        assert _few(_plan(m, 1, 1000, 0)) == few and _plan(m, 1, 1000, 0)[1] == 1
