@@ -391,19 +391,25 @@ struct SgemmPlan {
 // Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), with
 // at least 16 k per wavefront, beyond 65 ranges 32 (1024 x 1 x 8192 12.2 -> 9.4 us).  The ranges are
 // whole steps of 16 k: only the wavefront at the end of k meets the kernels' cut steps.
-// The tiles stay for a small A, where the time is that of two launches
-// either way, and for more columns, where the multiplies, not A's bytes, take this kernel's time;
-// their own time does not change from 1 to 64 columns.  Before -> with this kernel, us:
-//   4 columns: 512 x 1 x 1024 6.6 -> 6.3, 1000 x 4 x 600 7.3 -> 7.3, 1000 x 1 x 4096 11.1 -> 6.6
-//   8 columns: 512 x 8 x 1024 6.9 -> 8.5, 1000 x 8 x 1000 7.8 -> 8.0, 256 x 8 x 4096 10.2 -> 8.6,
-//     4096 x 8 x 4096 24.7 -> 19.2
-//   12 columns: 1000 x 10 x 4096 12.3 -> 12.2, 4096 x 12 x 4096 24.4 -> 20.6, 9216 x 12 x 4096
-//     45.0 -> 33.4
-//   16 columns: 2000 x 16 x 2000 10.8 -> 16.9, 4096 x 16 x 4096 25.1 -> 25.4
+// The tiles stay for a small A, where the time is that of two launches either way, and for more
+// columns, where the multiplies, not A's bytes, take this kernel's time; their own time does
+// not change from 1 to 64 columns.  The transposed and fused forms share the plan, and their bits.
+// Tiles -> this kernel, us, plain / B transposed / A transposed (* where the rule keeps the tiles):
+//   4 columns: 512 x 1024 6.8 -> 6.7 / 6.8 -> 7.1 / 6.5 -> 6.2, 1000 x 1500 7.5 -> 7.3 / 7.8 -> 7.8 /
+//     7.4 -> 6.3, 1000 x 4096 11.6 -> 7.5 / 12.6 -> 8.2 / 10.5 -> 6.3
+//   8 columns: *1024 x 1024 6.9 -> 8.7 / 7.1 -> 9.3 / 6.8 -> 6.4, 256 x 4096 10.3 -> 8.7 / 11.2 -> 9.3 /
+//     10.2 -> 6.4, *768 x 3000 9.2 -> 9.7 / 9.9 -> 10.2 / 9.2 -> 7.3, 2000 x 2000 10.1 -> 10.0 / 10.7 -> 10.6 /
+//     9.9 -> 8.3, 4096 x 1000 10.3 -> 9.4 / 10.9 -> 10.0 / 10.2 -> 7.8; few k, so that a workgroup's start
+//     and end weigh more: *40000 x 100 8.9 -> 9.6 / 9.3 -> 11.4 / 8.8 -> 5.4, *30000 x 150 9.8 -> 11.1 /
+//     9.1 -> 11.6 / 10.2 -> 9.3, 100000 x 64 11.5 -> 9.7 / 11.7 -> 10.4 / 11.0 -> 6.3
+//   12 columns: *4096 x 2048 15.0 -> 15.1 / 15.0 -> 16.5 / 14.8 -> 12.4, *1024 x 8192 15.2 -> 18.9 / 15.3 ->
+//     19.4 / 15.2 -> 13.0, 4096 x 4096 24.5 -> 20.6 / 25.3 -> 24.0 / 23.7 -> 17.5, 1024 x 16384 23.1 -> 22.8 /
+//     23.3 -> 25.2 / 24.0 -> 18.9, 9216 x 4096 45.4 -> 33.3 / 47.7 -> 40.9 / 44.5 -> 34.7
+//   16 columns: *2000 x 2000 10.8 -> 16.9, *4096 x 4096 25.1 -> 25.4
 // They also stay where the workspace holds fewer ranges and they make less than 128 workgroups, and
 // below 256 rows (one block).
 bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
-  const long long least = n <= 4 ? 1LL << 19 : n <= 8 ? 1LL << 20 : 1LL << 24;  // elements of A
+  const long long least = n <= 4 ? 1LL << 19 : n > 8 ? 1LL << 24 : k >= 4096 ? 1LL << 20 : k >= 256 ? 7LL << 19 : 3LL << 21;  // elements of A
   if (n > MNV_SKINNY_COLUMNS || m < 256 || k < 64 || (long long)m * k < least) return false;
   const int blocks = (m + 255) / 256;
   int per, ranges;

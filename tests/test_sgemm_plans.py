@@ -33,6 +33,20 @@ def test_ranges_do_not_depend_on_how_k_ends(m):
         assert ws == plan[1] * m * 4 and _plan(m, 1, k, 1 << 40) == plan, k
 
 
+@pytest.mark.parametrize("n,least", [(1, 1 << 19), (4, 1 << 19), (5, 7 << 19), (8, 7 << 19), (9, 1 << 24), (12, 1 << 24)])
+def test_elements_of_the_left_operand_from_which_few_columns_have_their_kernel(n, least):
+    for m in (1024, 2048):
+        k = least // m
+        assert _few(_plan(m, n, k, 1 << 40)) and not _few(_plan(m, n, k - 1, 1 << 40)), (m, k)
+    assert not _few(_plan(4096, 13, 4096, 1 << 40)) and not _few(_plan(255, n, 1 << 20, 1 << 40))
+
+
+def test_few_columns_over_few_or_many_k():
+    assert _few(_plan(256, 8, 4096, 1 << 40)) and not _few(_plan(257, 8, 4095, 1 << 40))   # from 4096 k on, 2^20 elements
+    assert not _few(_plan(40000, 8, 100, 1 << 40)) and _few(_plan(100000, 8, 64, 1 << 40))  # below 256 k, 6 x 2^20
+    assert _few(_plan(40000, 4, 100, 1 << 40)) and not _few(_plan(40000, 4, 63, 1 << 40))
+
+
 def test_few_columns_with_less_workspace():
     """A quarter of the 512 workgroups at least, or the tiles; the ranges never need more than there is."""
     m, n, k = 4096, 3, 5000
