@@ -26,11 +26,11 @@ namespace {
 // s_i = (address of c[i*n + j0] in floats) mod 16, so that every run starts and ends on a
 // sector boundary; the tile reads 16 more columns on its left to have those values.
 //
-// ODD (with SHIFT): extents or pointers off the 16-byte grid.  The reads are 16-byte loads at
-// whatever address a column has; the shifted runs of the result are on the sector grid for
-// any n, so its stores are aligned 16-byte ones; only the vectors that a row or column end cuts
-// go element by element.  (4 bytes per access both ways before: 8191 x 8193 140 -> 89 us,
-// 1001 x 257 4.8 -> 4.2 us.)
+// ODD: extents or pointers off the 16-byte grid.  The reads are 16-byte loads at whatever
+// address a column has.  With SHIFT the runs of the result are on the sector grid for any n, so
+// its stores are aligned 16-byte ones; without, they lie where the tile does.  Only the vectors
+// that a row or column end cuts go element by element.  (4 bytes per access both ways before:
+// 8191 x 8193 140 -> 89 us, 1001 x 257 4.8 -> 4.2 us.)
 template <int TI, int TJ, int NTH, bool NT, bool SHIFT, bool ODD>
 __global__ __launch_bounds__(NTH) void mnv_transpose_vec4_kernel(
     const float* __restrict__ a, float* __restrict__ c, int m, int n, int tiles_i, int tiles_j, int diagonal) {
@@ -95,26 +95,37 @@ __global__ __launch_bounds__(NTH) void mnv_transpose_vec4_kernel(
       o.y = tile[jj + 1][r];
       o.z = tile[jj + 2][r];
       o.w = tile[jj + 3][r];
-      __builtin_nontemporal_store(o, reinterpret_cast<mnv_f4*>(c + (size_t)i * n + j));
+      if (ODD && !SHIFT) *reinterpret_cast<mnv_f4u*>(c + (size_t)i * n + j) = o;
+      else __builtin_nontemporal_store(o, reinterpret_cast<mnv_f4*>(c + (size_t)i * n + j));
     }
   }
 }
 
 template <int TI, int TJ, int NTH>
 int launch_vec4(const float* a, float* c, int m, int n, bool nt, hipStream_t s) {
-  // rows of the result off the 64-byte grid: shifted runs, by up to 15 floats, which the last
-  // tile has to reach further
   const bool odd = m % 4 != 0 || n % 4 != 0 || !mnv_aligned16(a) || !mnv_aligned16(c);
-  const bool shift = odd || n % 16 != 0 || (reinterpret_cast<uintptr_t>(c) & 63u) != 0;
-  const size_t tiles_i = mnv_ceil_div((size_t)m, TI), tiles_j = mnv_ceil_div((size_t)n + (shift ? 15 : 0), TJ);
+  // Rows of the result off the 64-byte grid: shifted runs.  Off the 16-byte grid only from four
+  // tile columns on: before, the halo and the column of tiles that the shift adds cost more than the
+  // sectors that neighbouring tiles share (shifted -> not, us: 1714285 x 7 104 -> 35, 100001 x 127
+  // 31.3 -> 19.6, 100001 x 257 44.7 -> 40.4; 100001 x 385 63.3 -> 66.7, 8191 x 8193 89 -> 111).
+  const int phase = (int)((reinterpret_cast<uintptr_t>(c) >> 2) & 15u);
+  const bool shift = odd ? n > 384 : n % 16 != 0 || phase != 0;
+  int reach = 0;  // of the largest shift, as far as the last tile has to go further
+  for (int i = 0; shift && i < 16 && i < m; ++i) {
+    const int sft = (i * (n & 15) + phase) & 15;
+    if (sft > reach) reach = sft;
+  }
+  const size_t tiles_i = mnv_ceil_div((size_t)m, TI), tiles_j = mnv_ceil_div((size_t)n + reach, TJ);
   if (tiles_i * tiles_j > 0x7fffffffULL) return MNV_ERR_INVALID;
   const int diagonal = m % 4096 == 0 && n % 4096 == 0;
   const dim3 grid((unsigned)(tiles_i * tiles_j)), block(NTH);
 #define MNV_TR_LAUNCH(NT, SHIFT, ODD)                                                                    \
   hipLaunchKernelGGL((mnv_transpose_vec4_kernel<TI, TJ, NTH, NT, SHIFT, ODD>), grid, block, 0, s, a, c, \
                      m, n, (int)tiles_i, (int)tiles_j, diagonal)
-  if (odd) {
+  if (odd && shift) {
     if (nt) MNV_TR_LAUNCH(true, true, true); else MNV_TR_LAUNCH(false, true, true);
+  } else if (odd) {
+    if (nt) MNV_TR_LAUNCH(true, false, true); else MNV_TR_LAUNCH(false, false, true);
   } else if (shift) {
     if (nt) MNV_TR_LAUNCH(true, true, false); else MNV_TR_LAUNCH(false, true, false);
   } else {
@@ -132,8 +143,9 @@ extern "C" int mnv_transpose(const float* a, float* c, int m, int n, mnv_stream_
   // past the last-level cache the source streams with non-temporal loads
   const bool nt = (size_t)m * n * sizeof(float) >= MNV_PAST_CACHE_BYTES;
   // the large tile from 128 of them on; below that the small tile's four times as many
-  // workgroups fill the chip better
+  // workgroups fill the chip better, and where an extent fits the small tile most of the large one
+  // would be empty (2400001 x 5 144 -> 44 us, 5 x 2400001 102 -> 46)
   const size_t big_tiles = mnv_ceil_div((size_t)m, 128) * mnv_ceil_div((size_t)n, 128);
-  if (big_tiles >= 128) return launch_vec4<128, 128, 1024>(a, c, m, n, nt, mnv_stream(stream));
+  if (big_tiles >= 128 && m > 64 && n > 64) return launch_vec4<128, 128, 1024>(a, c, m, n, nt, mnv_stream(stream));
   return launch_vec4<64, 64, 256>(a, c, m, n, nt, mnv_stream(stream));
 }

@@ -86,3 +86,39 @@ def test_few_columns_of_a_transposed_operand_cost_what_the_plain_form_does(gpu, 
         gpu.call("mnv_randn", d.p, ctypes.c_size_t(count), ctypes.c_uint64(5), ctypes.c_float(0), ctypes.c_float(1))
     tail = (c.p, m, n, k, ws.p, ctypes.c_size_t(ws_bytes), gpu.dev.stream)
     assert _ratio(gpu, lambda: gpu.L.mnv_sgemm_tn(a.p, b.p, None, *tail), lambda: gpu.L.mnv_sgemm_nn(a.p, b.p, *tail)) < 1.8
+
+
+def _at(d, floats):
+    return ctypes.c_void_p(d.ptr + 4 * floats)
+
+
+def _guarded(v, lead):
+    """v behind `lead` floats of 7 and in front of 5."""
+    return np.concatenate([np.full(lead, 7, np.float32), v, np.full(5, 7, np.float32)])
+
+
+# either extent within the small tile and past it, with and without 128 large tiles; three tile columns
+# of the result and one value more (shifted runs), rows that end with every shift; a result whose last
+# tile column is full with the shift (52 and 116 modulo 128)
+@pytest.mark.parametrize("m,n", [(1, 20001), (20001, 1), (3, 16387), (16387, 3), (64, 8197), (65, 16389), (16389, 64),
+                                 (16389, 65), (8191, 127), (8193, 129), (6145, 383), (6145, 384), (6145, 385), (6148, 388),
+                                 (1000, 52), (4096, 116), (2052, 1012), (33, 401), (5, 500)])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_transpose_of_narrow_matrices(gpu, m, n, off):
+    """Bit for bit, and the floats around the result untouched."""
+    say("transpose", m, n, off)
+    x = _rand(m * n, 30)
+    lead = off + 4
+    src, dst = gpu.up(_guarded(x, lead)), gpu.up(_guarded(np.zeros(m * n, np.float32), lead))
+    gpu.call("mnv_transpose", _at(src, lead), _at(dst, lead), m, n)
+    assert gpu.down(dst).tobytes() == _guarded(x.reshape(n, m).T.reshape(-1), lead).tobytes()
+
+
+@pytest.mark.parametrize("m,n", [(1714285, 7), (5, 2400001)])
+def test_transpose_of_narrow_matrices_costs_a_few_copies(gpu, m, n):
+    """Off the 16-byte grid: 35 and 46 us, copies of the same bytes 15 (large tiles: 104 and 102)."""
+    say("transpose, time", m, n)
+    a, c = gpu.empty(m * n), gpu.empty(m * n)
+    gpu.call("mnv_fill", a.p, ctypes.c_size_t(m * n), ctypes.c_float(1))
+    s = gpu.dev.stream
+    assert _ratio(gpu, lambda: gpu.L.mnv_transpose(a.p, c.p, m, n, s), lambda: gpu.L.mnv_copy(a.p, c.p, m * n, s)) < 4.5
