@@ -122,3 +122,34 @@ def test_transpose_of_narrow_matrices_costs_a_few_copies(gpu, m, n):
     gpu.call("mnv_fill", a.p, ctypes.c_size_t(m * n), ctypes.c_float(1))
     s = gpu.dev.stream
     assert _ratio(gpu, lambda: gpu.L.mnv_transpose(a.p, c.p, m, n, s), lambda: gpu.L.mnv_copy(a.p, c.p, m * n, s)) < 4.5
+
+
+# rows: one per thread and four (16), a cut last vector of each length, one and several wavefronts and
+# workgroups to a column, a last workgroup with a single row's vector (1025)
+@pytest.mark.parametrize("m", [1, 3, 15, 16, 17, 18, 19, 255, 257, 1023, 1025, 1026, 1283, 2049])
+@pytest.mark.parametrize("off", [0, 2])
+def test_broadcast_over_few_rows(gpu, m, off):
+    """Bit for bit into another matrix and in place, and the floats around the result untouched."""
+    n = 41
+    say("broadcast", m, n, off)
+    x, row, col = _rand(m * n, 31), _rand(m, 32), _rand(n, 33)
+    X, lead = x.reshape(n, m), off + 4
+    drow, dcol = gpu.up(row), gpu.up(col)
+    for name, vec, want in (("norm_sub_row", drow, X - row), ("norm_div_col", dcol, X / col[:, None])):
+        src, dst = gpu.up(_guarded(x, lead)), gpu.up(_guarded(np.zeros(m * n, np.float32), lead))
+        for to in (dst, src):
+            gpu.call("mnv_" + name, _at(src, lead), vec.p, _at(to, lead), m, n)
+            assert gpu.down(to).tobytes() == _guarded(want.reshape(-1), lead).tobytes(), name
+
+
+@pytest.mark.parametrize("m,n", [(10, 2000000), (15, 1333333), (7, 2857143)])
+def test_broadcast_over_few_rows_costs_a_few_streams(gpu, m, n):
+    """86, 60 and 136 us, adding a constant to as many values 26 (four rows per thread and the last ones
+    element by element: 316, 278 and 551)."""
+    say("broadcast, time", m, n)
+    a, c, v = gpu.empty(m * n), gpu.empty(m * n), gpu.empty(m)
+    for d, count in ((a, m * n), (v, m)):
+        gpu.call("mnv_fill", d.p, ctypes.c_size_t(count), ctypes.c_float(1))
+    s = gpu.dev.stream
+    assert _ratio(gpu, lambda: gpu.L.mnv_norm_add_row(a.p, v.p, c.p, m, n, s),
+                  lambda: gpu.L.mnv_const_add(a.p, c.p, ctypes.c_float(2), m * n, s)) < 8
