@@ -21,6 +21,7 @@ namespace {
 
 struct SumAcc {
   static constexpr int ROW_UNROLL = 2;  // columns in flight per thread in the row reducer
+  static constexpr int ROW_FEW = 32, ROW_FEW_ODD = 48;  // columns, see launch_reduce_row
   float s;
   __device__ void init() { s = 0.f; }
   __device__ void push(float v, int) { s += v; }
@@ -36,27 +37,25 @@ struct SumAcc {
 
 struct ArgAcc {
   static constexpr int ROW_UNROLL = 4;
+  static constexpr int ROW_FEW = 128, ROW_FEW_ODD = 256;
   float v;
   int idx;
   __device__ void init() {
     v = -INFINITY;
     idx = MNV_NONE;
   }
-  // Elements reach one accumulator in ascending index order.
+  // Elements reach one accumulator in ascending index order.  Selections, no branches: where few
+  // lanes have rows, all of them skipping the update is common, and each jump over it stalled the
+  // wavefront (36 x 4097 37 us, 32 x 4097 14).
   __device__ void push(float x, int i) {
-    bool take = (idx == MNV_NONE) ? (x == x) : (x > v);
-    if (take) {
-      v = x;
-      idx = i;
-    }
+    const bool take = ((idx == MNV_NONE) & (x == x)) | (x > v);  // v is -inf before the first one
+    v = take ? x : v;
+    idx = take ? i : idx;
   }
   __device__ void merge(const ArgAcc& o) {
-    bool take = (o.idx != MNV_NONE) &&
-                (idx == MNV_NONE || o.v > v || (o.v == v && o.idx < idx));
-    if (take) {
-      v = o.v;
-      idx = o.idx;
-    }
+    const bool take = (o.idx != MNV_NONE) & ((idx == MNV_NONE) | (o.v > v) | ((o.v == v) & (o.idx < idx)));
+    v = take ? o.v : v;
+    idx = take ? o.idx : idx;
   }
   __device__ ArgAcc shfl_down(int off) const {
     ArgAcc r;
@@ -190,28 +189,31 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
 // Along dimension 1: out[r] = reduce_c in[r + c*m] (stride m between elements).
 // A workgroup owns RL*W consecutive rows (128 contiguous bytes per column) and
 // splits the columns over CG thread groups; partial results meet in LDS.
+// W = 4 rows per thread; 1 for matrices of less than four rows.
 // VEC4: m and the matrix on the 16-byte grid; otherwise the same loads at the addresses the
-// columns have, and the last 1 to 3 rows element by element.  (One row per thread, 4 bytes per
-// load, one load in flight before: sums of 8191 x 8193 140 -> 128 us, 65 x 4097
-// 27 -> 8.5; the 128-byte run of an unaligned column lies in two lines, both fetched whole.)
+// columns have, and the thread whose rows the matrix ends in reduces its last four rows and keeps
+// its own.  (One row per thread, 4 bytes per load, one load in flight before: sums of 8191 x 8193
+// 140 -> 128 us, 65 x 4097 27 -> 8.5; the 128-byte run of an unaligned column lies in two lines,
+// both fetched whole.)
 // ---------------------------------------------------------------------------
-template <class Acc, class Emit, int RL, int CG, bool VEC4, bool NT>
+template <class Acc, class Emit, int RL, int CG, int W, bool VEC4, bool NT>
 __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __restrict__ in,
                                                                 float* __restrict__ out, int m,
                                                                 int n) {
-  constexpr int W = 4;
   constexpr int ROWS = RL * W;
   __shared__ Acc part[CG][ROWS + 1];
   const int rl = threadIdx.x % RL;
   const int cg = threadIdx.x / RL;
   const int r0 = blockIdx.x * ROWS + rl * W;
+  const int skip = W == 4 && !VEC4 && r0 + 3 >= m ? r0 + 4 - m : 0;  // rows that are another thread's
   Acc acc[W];
 #pragma unroll
   for (int q = 0; q < W; ++q) acc[q].init();
   if (r0 < m) {
-    if (VEC4 || r0 + 3 < m) {
+    const float* first = in + (r0 - skip);
+    if constexpr (W == 4) {
       auto ld = [&](int c) {
-        const float* at = in + (size_t)c * m + r0;
+        const float* at = first + (size_t)c * m;
         return VEC4 ? mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(at)) : mnv_ldx4u<NT>(at);
       };
       // several columns in flight per thread: with one workgroup per 32 rows there are few
@@ -226,23 +228,21 @@ __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __r
           v[u] = ld(c + u * CG);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          acc[0].push(v[u].x, c + u * CG); acc[1 % W].push(v[u].y, c + u * CG);
-          acc[2 % W].push(v[u].z, c + u * CG); acc[3 % W].push(v[u].w, c + u * CG);
+          acc[0].push(v[u].x, c + u * CG); acc[1].push(v[u].y, c + u * CG);
+          acc[2].push(v[u].z, c + u * CG); acc[3].push(v[u].w, c + u * CG);
         }
       }
       for (; c < n; c += CG) {
         mnv_f4 a = ld(c);
-        acc[0].push(a.x, c); acc[1 % W].push(a.y, c); acc[2 % W].push(a.z, c); acc[3 % W].push(a.w, c);
+        acc[0].push(a.x, c); acc[1].push(a.y, c); acc[2].push(a.z, c); acc[3].push(a.w, c);
       }
     } else {
-      for (int c = cg; c < n; c += CG)
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-          if (r0 + q < m) acc[q].push(in[(size_t)c * m + r0 + q], c);
+      for (int c = cg; c < n; c += CG) acc[0].push(first[(size_t)c * m], c);
     }
   }
 #pragma unroll
-  for (int q = 0; q < W; ++q) part[cg][rl * W + q] = acc[q];
+  for (int q = 0; q < W; ++q)
+    if (q >= skip) part[cg][rl * W + q - skip] = acc[q];
   __syncthreads();
   for (int sft = CG / 2; sft > 0; sft >>= 1) {
     if (cg < sft) {
@@ -268,16 +268,22 @@ int launch_reduce_row(const float* in, float* out, int m, int n, mnv_stream_t st
   hipStream_t s = mnv_stream(stream);
   const bool vec4 = (m % 4 == 0) && mnv_aligned16(in);
   const bool big = (size_t)m * n * sizeof(float) >= MNV_PAST_CACHE_BYTES;
-  constexpr int RL = 8, CG = 64;
-  const dim3 grid((unsigned)mnv_ceil_div((size_t)m, RL * 4)), block(RL * CG);
-  if (vec4 && big)
-    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, true>), grid, block, 0, s, in, out, m, n);
-  else if (vec4)
-    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, true, false>), grid, block, 0, s, in, out, m, n);
-  else if (big)
-    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, false, true>), grid, block, 0, s, in, out, m, n);
-  else
-    hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, false, false>), grid, block, 0, s, in, out, m, n);
+#define MNV_RR_LAUNCH(RL, CG, W, VEC4, NT)                                                            \
+  hipLaunchKernelGGL((mnv_reduce_row_kernel<Acc, Emit, RL, CG, W, VEC4, NT>),                          \
+                     dim3((unsigned)mnv_ceil_div((size_t)m, RL * W)), dim3(RL * CG), 0, s, in, out, m, n)
+  // One row per thread and fewer column groups for few columns, where the groups' sums meeting in LDS
+  // are most of the work (four rows and 64 groups -> one and 16, us: sums of 100003 x 9 5.7 -> 3.8,
+  // 100000 x 32 5.6 -> 4.4, 100003 x 33 6.6 -> 6.2, 727272 x 33 33.7 -> 37.4, 100003 x 63 9.0 -> 10.3;
+  // maxima of 255 x 9 4.0 -> 3.4, 100003 x 17 11.7 -> 5.8, 100000 x 128 17.7 -> 15.6, 15000 x 200 5.9 ->
+  // 6.4, 100003 x 129 23.5 -> 20.4, 2049 x 257 4.0 -> 5.0; four groups up to four columns: maxima of
+  // 3000001 x 1 91.6 -> 17.3).
+  if (n <= 4) MNV_RR_LAUNCH(64, 4, 1, false, false);
+  else if (n < (vec4 ? Acc::ROW_FEW : Acc::ROW_FEW_ODD)) MNV_RR_LAUNCH(32, 16, 1, false, false);
+  else if (vec4) { if (big) MNV_RR_LAUNCH(8, 64, 4, true, true); else MNV_RR_LAUNCH(8, 64, 4, true, false); }
+  else if (m < 4) MNV_RR_LAUNCH(4, 128, 1, false, false);
+  else if (big) MNV_RR_LAUNCH(8, 64, 4, false, true);
+  else MNV_RR_LAUNCH(8, 64, 4, false, false);
+#undef MNV_RR_LAUNCH
   return MNV_LAUNCH_STATUS();
 }
 

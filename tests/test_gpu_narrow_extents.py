@@ -7,7 +7,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from gpu_util import Gpu, say
+from gpu_util import Gpu, assert_bits_equal, say
 
 pytestmark = pytest.mark.gpu
 
@@ -153,3 +153,49 @@ def test_broadcast_over_few_rows_costs_a_few_streams(gpu, m, n):
     s = gpu.dev.stream
     assert _ratio(gpu, lambda: gpu.L.mnv_norm_add_row(a.p, v.p, c.p, m, n, s),
                   lambda: gpu.L.mnv_const_add(a.p, c.p, ctypes.c_float(2), m * n, s)) < 8
+
+
+# rows: one per thread, four, and a cut last vector of each length behind a full workgroup and alone; columns
+# at the sizes where the kernels change (4, 32, 48, 128 and 256), and enough for several trips of a thread
+ROW_SHAPES = [(1, 300), (2, 5), (3, 260), (5, 4), (6, 5), (7, 31), (33, 33), (34, 47), (35, 48), (36, 127), (66, 130), (67, 255),
+              (37, 256), (255, 513), (1001, 300), (4099, 6), (70001, 3)]
+
+
+@pytest.mark.parametrize("m,n", ROW_SHAPES)
+@pytest.mark.parametrize("off", [0, 1, 2])
+def test_row_reductions_with_ties_nan_and_infinities(gpu, ora, m, n, off):
+    """Maxima and arg-maxima bit for bit: many ties, zeros of both signs, NaN first in some rows and inside
+    others, rows of -inf and of NaN.  Sums of the finite values against float64: n roundings of 2^-24
+    relative to the sum of magnitudes.  The floats around the results untouched."""
+    say("row reductions", m, n, off)
+    rng = np.random.default_rng(40)
+    x = rng.integers(-2, 3, m * n).astype(np.float32)
+    x[x == 0] = np.where(rng.random(np.count_nonzero(x == 0)) < 0.5, 0.0, -0.0)
+    finite = x.copy()
+    x[rng.random(m * n) < 0.1] = np.nan
+    X = x.reshape(n, m)  # X[column, row]
+    X[0, ::3] = np.nan
+    X[:, 1::7] = -np.inf
+    X[:, 4::11] = np.nan
+    lead = off + 4
+    for name, v, want in (("reduce_max_row", x, ora.reduction(ora.MAX, x, [m, n], [1])),
+                          ("maxindex_row", x, ora.maxindex(x, [m, n], 1)), ("reduce_sum_row", finite, None)):
+        src, dst = gpu.up(_guarded(v, lead)), gpu.up(_guarded(np.zeros(m, np.float32), lead))
+        gpu.call("mnv_" + name, _at(src, lead), _at(dst, lead), m, n)
+        got = gpu.down(dst)
+        assert np.all(got[:lead] == 7) and np.all(got[lead + m:] == 7), name
+        if want is not None:
+            assert_bits_equal(got[lead:lead + m], want, name)
+        else:
+            f = finite.reshape(n, m).astype(np.float64)
+            assert np.all(np.abs(got[lead:lead + m] - f.sum(0)) <= n * 2.0 ** -24 * np.abs(f).sum(0))
+
+
+@pytest.mark.parametrize("m,n", [(3000001, 1), (1000001, 3)])
+def test_row_reductions_of_few_columns_cost_a_few_copies(gpu, m, n):
+    """17.3 us for the first, a copy of its bytes 4.5 (64 column groups: 210)."""
+    say("row maxima, time", m, n)
+    a, c, r = gpu.empty(m * n), gpu.empty(m * n), gpu.empty(m)
+    gpu.call("mnv_fill", a.p, ctypes.c_size_t(m * n), ctypes.c_float(1))
+    s = gpu.dev.stream
+    assert _ratio(gpu, lambda: gpu.L.mnv_reduce_max_row(a.p, r.p, m, n, s), lambda: gpu.L.mnv_copy(a.p, c.p, m * n, s)) < 12
