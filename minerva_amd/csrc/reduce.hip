@@ -22,6 +22,7 @@ namespace {
 struct SumAcc {
   static constexpr int ROW_UNROLL = 2;  // columns in flight per thread in the row reducer
   static constexpr int ROW_FEW = 32, ROW_FEW_ODD = 48;  // columns, see launch_reduce_row
+  static constexpr bool SKIP_IDLE = false;  // merges of idle lanes cost less than the branches around them
   float s;
   __device__ void init() { s = 0.f; }
   __device__ void push(float v, int) { s += v; }
@@ -38,6 +39,7 @@ struct SumAcc {
 struct ArgAcc {
   static constexpr int ROW_UNROLL = 4;
   static constexpr int ROW_FEW = 128, ROW_FEW_ODD = 256;
+  static constexpr bool SKIP_IDLE = true;  // 1000000 columns of 1: 136 -> 97 us
   float v;
   int idx;
   __device__ void init() {
@@ -81,55 +83,48 @@ struct EmitIndex {
 // ---------------------------------------------------------------------------
 // Along dimension 0: each of the n columns is m contiguous floats.
 // GROUP threads (one wavefront, or the whole 256-thread workgroup) share a column.
-// VEC4: every column starts on the 16-byte grid.  (Columns that do not were read 4 bytes at a
-// time before, one load in flight: sums of 8191 x 8193 53 -> 38 us.)
+// LOAD: 16-byte loads of columns on the 16-byte grid, the same at whatever address a column has
+// (4 bytes at a time, one load in flight before: sums of 8191 x 8193 53 -> 38 us), or one value
+// per lane, for columns that are short of a vector per lane anyway.
 // ---------------------------------------------------------------------------
 #define MNV_RC_THREADS 256
+enum RcLoad { RC_SINGLE, RC_ODD, RC_VEC4 };
 
-template <class Acc, class Emit, int GROUP, bool VEC4, bool NT>
+template <class Acc, class Emit, int GROUP, RcLoad LOAD, bool NT>
 __global__ __launch_bounds__(MNV_RC_THREADS) void mnv_reduce_col_kernel(
     const float* __restrict__ in, float* __restrict__ out, int m, int n) {
   constexpr int COLS = MNV_RC_THREADS / GROUP;
   __shared__ Acc part[MNV_RC_THREADS / MNV_WAVE];
   const int g = threadIdx.x / GROUP;
   const int t = threadIdx.x % GROUP;
+  const int lanes = LOAD == RC_SINGLE ? m : (m + 3) >> 2;  // lanes from here on have nothing to merge
   for (int c = blockIdx.x * COLS + g; c < n; c += gridDim.x * COLS) {
     const float* col = in + (size_t)c * m;
     Acc acc;
     acc.init();
-    if (VEC4) {
-      const mnv_f4* col4 = reinterpret_cast<const mnv_f4*>(col);
+    if (LOAD == RC_SINGLE) {
+      for (int i = t; i < m; i += GROUP) acc.push(col[i], i);
+    } else {
+      auto ld = [&](int i) {
+        return LOAD == RC_VEC4 ? mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(col) + i) : mnv_ldx4u<NT>(col + 4 * (size_t)i);
+      };
+      auto push = [&](const mnv_f4& v, int i) {
+        acc.push(v.x, 4 * i); acc.push(v.y, 4 * i + 1); acc.push(v.z, 4 * i + 2); acc.push(v.w, 4 * i + 3);
+      };
       const int m4 = m >> 2;
       int i = t;
       // two independent 16-byte loads in flight per thread
       for (; i + GROUP < m4; i += 2 * GROUP) {
-        mnv_f4 a = mnv_ldx4<NT>(col4 + i), b = mnv_ldx4<NT>(col4 + i + GROUP);
-        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
-        int j = i + GROUP;
-        acc.push(b.x, 4 * j); acc.push(b.y, 4 * j + 1); acc.push(b.z, 4 * j + 2); acc.push(b.w, 4 * j + 3);
+        const mnv_f4 a = ld(i), b = ld(i + GROUP);
+        push(a, i);
+        push(b, i + GROUP);
       }
-      if (i < m4) {
-        mnv_f4 a = mnv_ldx4<NT>(col4 + i);
-        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
-      }
-    } else {
-      // the same loads at the address the column has, then its last 1 to 3 values
-      const int m4 = m >> 2;
-      int i = t;
-      for (; i + GROUP < m4; i += 2 * GROUP) {
-        mnv_f4 a = mnv_ldx4u<NT>(col + 4 * (size_t)i), b = mnv_ldx4u<NT>(col + 4 * (size_t)(i + GROUP));
-        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
-        int j = i + GROUP;
-        acc.push(b.x, 4 * j); acc.push(b.y, 4 * j + 1); acc.push(b.z, 4 * j + 2); acc.push(b.w, 4 * j + 3);
-      }
-      if (i < m4) {
-        mnv_f4 a = mnv_ldx4u<NT>(col + 4 * (size_t)i);
-        acc.push(a.x, 4 * i); acc.push(a.y, 4 * i + 1); acc.push(a.z, 4 * i + 2); acc.push(a.w, 4 * i + 3);
-      }
-      if (4 * m4 + t < m) acc.push(col[4 * m4 + t], 4 * m4 + t);
+      if (i < m4) push(ld(i), i);
+      if (LOAD == RC_ODD && 4 * m4 + t < m) acc.push(col[4 * m4 + t], 4 * m4 + t);
     }
 #pragma unroll
-    for (int off = MNV_WAVE / 2; off > 0; off >>= 1) acc.merge(acc.shfl_down(off));
+    for (int off = MNV_WAVE / 2; off > 0; off >>= 1)
+      if (!Acc::SKIP_IDLE || off < lanes) acc.merge(acc.shfl_down(off));
     if (GROUP > MNV_WAVE) {
       const int w = threadIdx.x / MNV_WAVE;
       if ((threadIdx.x % MNV_WAVE) == 0) part[w] = acc;
@@ -150,38 +145,25 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
   if (n == 0) return MNV_OK;
   if (!in || !out || m <= 0 || n < 0) return MNV_ERR_INVALID;
   hipStream_t s = mnv_stream(stream);
-  bool vec4 = (m % 4 == 0) && mnv_aligned16(in);
+  const bool vec4 = (m % 4 == 0) && mnv_aligned16(in);
   const bool big = (size_t)m * n * sizeof(float) >= MNV_PAST_CACHE_BYTES;
+#define MNV_RC_LAUNCH(GROUP, LOAD, NT, GRID)                                                           \
+  hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, GROUP, LOAD, NT>), dim3(GRID), dim3(MNV_RC_THREADS), \
+                     0, s, in, out, m, n)
   if (m > 2048) {
-    unsigned grid = (unsigned)(n < 65536 ? n : 65536);
-    if (vec4 && big)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, true, true>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else if (vec4)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, true, false>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else if (big)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, false, true>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_RC_THREADS, false, false>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
+    const unsigned grid = (unsigned)(n < 65536 ? n : 65536);
+    if (vec4) { if (big) MNV_RC_LAUNCH(MNV_RC_THREADS, RC_VEC4, true, grid); else MNV_RC_LAUNCH(MNV_RC_THREADS, RC_VEC4, false, grid); }
+    else { if (big) MNV_RC_LAUNCH(MNV_RC_THREADS, RC_ODD, true, grid); else MNV_RC_LAUNCH(MNV_RC_THREADS, RC_ODD, false, grid); }
   } else {
-    size_t blocks = mnv_ceil_div((size_t)n, MNV_RC_THREADS / MNV_WAVE);
-    unsigned grid = (unsigned)(blocks < 65536 ? blocks : 65536);
-    if (vec4 && big)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, true, true>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else if (vec4)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, true, false>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else if (big)
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, false, true>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
-    else
-      hipLaunchKernelGGL((mnv_reduce_col_kernel<Acc, Emit, MNV_WAVE, false, false>), dim3(grid),
-                         dim3(MNV_RC_THREADS), 0, s, in, out, m, n);
+    const size_t cols = MNV_RC_THREADS / MNV_WAVE, want = mnv_ceil_div((size_t)n, cols);
+    const unsigned grid = (unsigned)(want < 65536 ? want : 65536);
+    // off the 16-byte grid one value per lane below 96 (vectors -> values, sums of 100000 columns: of 63
+    // 15.6 -> 12.4 us, 79 16.1 -> 15.7, 95 16.5 -> 16.7, 129 17.6 -> 20.3)
+    if (vec4) { if (big) MNV_RC_LAUNCH(MNV_WAVE, RC_VEC4, true, grid); else MNV_RC_LAUNCH(MNV_WAVE, RC_VEC4, false, grid); }
+    else if (m < 96) MNV_RC_LAUNCH(MNV_WAVE, RC_SINGLE, false, grid);
+    else { if (big) MNV_RC_LAUNCH(MNV_WAVE, RC_ODD, true, grid); else MNV_RC_LAUNCH(MNV_WAVE, RC_ODD, false, grid); }
   }
+#undef MNV_RC_LAUNCH
   return MNV_LAUNCH_STATUS();
 }
 

@@ -199,3 +199,42 @@ def test_row_reductions_of_few_columns_cost_a_few_copies(gpu, m, n):
     gpu.call("mnv_fill", a.p, ctypes.c_size_t(m * n), ctypes.c_float(1))
     s = gpu.dev.stream
     assert _ratio(gpu, lambda: gpu.L.mnv_reduce_max_row(a.p, r.p, m, n, s), lambda: gpu.L.mnv_copy(a.p, c.p, m * n, s)) < 12
+
+
+# values per column: one per lane (up to 64, and two for some), vectors with a cut last one (from 96 on, from
+# 2049 on by a whole workgroup), few lanes to merge
+@pytest.mark.parametrize("m,n", [(1, 9), (2, 5), (3, 300), (5, 7), (33, 33), (63, 65), (65, 11), (95, 13), (96, 6), (97, 6), (98, 5),
+                                 (255, 4), (2047, 3), (2050, 3), (8195, 2)])
+@pytest.mark.parametrize("off", [0, 1, 3])
+def test_column_reductions_with_ties_nan_and_infinities(gpu, ora, m, n, off):
+    """As above, along the columns: NaN first in some, columns of -inf and of NaN."""
+    say("column reductions", m, n, off)
+    rng = np.random.default_rng(41)
+    x = rng.integers(-2, 3, m * n).astype(np.float32)
+    x[x == 0] = np.where(rng.random(np.count_nonzero(x == 0)) < 0.5, 0.0, -0.0)
+    finite = x.copy()
+    x[rng.random(m * n) < 0.1] = np.nan
+    X = x.reshape(n, m)  # X[column, row]
+    X[::3, 0] = np.nan
+    X[1::7] = -np.inf
+    X[4::11] = np.nan
+    lead = off + 4
+    for name, v, want in (("reduce_max_col", x, ora.reduction(ora.MAX, x, [m, n], [0])),
+                          ("maxindex_col", x, ora.maxindex(x, [m, n], 0)), ("reduce_sum_col", finite, None)):
+        src, dst = gpu.up(_guarded(v, lead)), gpu.up(_guarded(np.zeros(n, np.float32), lead))
+        gpu.call("mnv_" + name, _at(src, lead), _at(dst, lead), m, n)
+        got = gpu.down(dst)
+        assert np.all(got[:lead] == 7) and np.all(got[lead + n:] == 7), name
+        if want is not None:
+            assert_bits_equal(got[lead:lead + n], want, name)
+        else:
+            f = finite.reshape(n, m).astype(np.float64)
+            assert np.all(np.abs(got[lead:lead + n] - f.sum(1)) <= m * 2.0 ** -24 * np.abs(f).sum(1))
+
+
+def test_short_columns_cost_what_aligned_ones_do(gpu):
+    """Sums of 11 and of 12 values: 82 us each (vectors at any address: 117 for 11)."""
+    n = 1000000
+    a, r, s = gpu.empty(12 * n), gpu.empty(n), gpu.dev.stream
+    gpu.call("mnv_fill", a.p, ctypes.c_size_t(12 * n), ctypes.c_float(1))
+    assert _ratio(gpu, lambda: gpu.L.mnv_reduce_sum_col(a.p, r.p, 11, n, s), lambda: gpu.L.mnv_reduce_sum_col(a.p, r.p, 12, n, s)) < 1.25
