@@ -67,15 +67,29 @@ __device__ __forceinline__ T* lane_pointer(T* p) {
 // vectors each rather than 256 with eight (more wavefronts, shorter per-thread chains): on
 // 8192 lines of 8192, operands cycled through four sets, 6.3 TB/s against 5.8 TB/s (a plain
 // copy of the same operands: 6.3 TB/s).
-// ODD: lines off the 16-byte grid, or of a length that is no multiple of four.  The same 16-byte
-// accesses at the addresses the lines have; the last 1 to 3 values of a line go element by
-// element, with -inf in the places past them, whose exponential is 0.  Exponentials and
-// quotients are the ones of the general kernel below, which made three passes over such lines,
-// 4 bytes per access (8193 lines of 8191: 314 -> 104 us; backward 233 -> 147).
-template <class LineVec>
-__device__ __forceinline__ void line_load(mnv_f4& v, const LineVec& whole, const float* p, int left, float fill) {
-  if (left >= 4) {
-    v = whole();
+// Lines off the 16-byte grid, or of a length that is no multiple of four: the same 16-byte
+// accesses at the addresses the lines have; what stands in the places past a line's end has the
+// exponential 0 (-inf).  Exponentials and quotients are the ones of the general kernel below, which
+// made three passes over such lines, 4 bytes per access (8193 lines of 8191: 314 -> 104 us; backward
+// 233 -> 147).  Of a cut last vector
+//  TAIL_EACH: the 1 to 3 values go element by element;
+//  TAIL_BACK (lines of 4 to 256 values, one vector per lane): the line's last four values are loaded, and
+//    those that another lane has are replaced: one load instead of three guarded ones (100000 lines of
+//    255 36.7 -> 32.6 us, backward 50.5 -> 49.4; with several vectors per lane every one pays the
+//    selections: of 257 54 -> 65).
+enum LineForm { ALIGNED, TAIL_EACH, TAIL_BACK };
+template <LineForm FORM, bool NT>
+__device__ __forceinline__ void line_load(mnv_f4& v, const float* p, int left, float fill) {
+  if (FORM == ALIGNED) {
+    v = mnv_ldx4<NT>(reinterpret_cast<const mnv_f4*>(p));
+  } else if (FORM == TAIL_BACK) {
+    const int skip = left < 4 ? 4 - left : 0;
+    v = mnv_ldx4u<NT>(p - skip);
+    v.x = skip > 0 ? fill : v.x;
+    v.y = skip > 1 ? fill : v.y;
+    v.z = skip > 2 ? fill : v.z;
+  } else if (left >= 4) {
+    v = mnv_ldx4u<NT>(p);
   } else {
     v.x = p[0];
     v.y = left > 1 ? p[1] : fill;
@@ -83,9 +97,16 @@ __device__ __forceinline__ void line_load(mnv_f4& v, const LineVec& whole, const
     v.w = fill;
   }
 }
+template <LineForm FORM>
 __device__ __forceinline__ void line_store(float* p, int left, mnv_f4 o) {
-  if (left >= 4) {
+  if (FORM == ALIGNED) {
+    __builtin_nontemporal_store(o, reinterpret_cast<mnv_f4*>(p));
+  } else if (left >= 4) {
     *reinterpret_cast<mnv_f4u*>(p) = o;
+  } else if (FORM == TAIL_BACK) {
+    p[left - 1] = o.w;
+    if (left > 1) p[left - 2] = o.z;
+    if (left > 2) p[left - 3] = o.y;
   } else {
     p[0] = o.x;
     if (left > 1) p[1] = o.y;
@@ -93,7 +114,7 @@ __device__ __forceinline__ void line_store(float* p, int left, mnv_f4 o) {
   }
 }
 
-template <int GROUP, int CACHE, int NTH, bool NT, bool ODD>
+template <int GROUP, int CACHE, int NTH, bool NT, LineForm FORM>
 __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     const float* __restrict__ in, float* __restrict__ out, int len, int lines) {
   __shared__ float lds[NTH / MNV_WAVE];
@@ -106,21 +127,14 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
   for (int line = blockIdx.x * LPB + (LPB > 1 ? threadIdx.x / GROUP : 0); line < lines; line += gridDim.x * LPB) {
     const float* x = lane_pointer(in + (size_t)line * len + 4 * t);
     float* y = lane_pointer(out + (size_t)line * len + 4 * t);
-    const mnv_f4* x4 = reinterpret_cast<const mnv_f4*>(x);
-    mnv_f4* y4 = reinterpret_cast<mnv_f4*>(y);
     const int left = len - 4 * t;  // values from the thread's first vector on
     mnv_f4 v[CACHE];
     // all loads first, in a loop of their own: a use inside the same guarded block would
     // make each load wait for the one before it
 #pragma unroll
     for (int u = 0; u < CACHE; ++u)
-      if (t + u * GROUP < len4) {
-        if (ODD)
-          line_load(v[u], [&] { return mnv_ldx4u<NT>(x + 4 * u * GROUP); }, x + 4 * u * GROUP, left - 4 * u * GROUP,
-                    -INFINITY);
-        else
-          v[u] = mnv_ldx4<NT>(x4 + u * GROUP);
-      }
+      if (t + u * GROUP < len4)
+        line_load<FORM, NT>(v[u], x + 4 * u * GROUP, left - 4 * u * GROUP, -INFINITY);
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < CACHE; ++u)
@@ -131,10 +145,10 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
         // exp through the hardware exp2: relative error ~1e-6 for the arguments <= 0 here
-        v[u].x = ODD ? expf(v[u].x - mx) : __expf(v[u].x - mx);
-        v[u].y = ODD ? expf(v[u].y - mx) : __expf(v[u].y - mx);
-        v[u].z = ODD ? expf(v[u].z - mx) : __expf(v[u].z - mx);
-        v[u].w = ODD ? expf(v[u].w - mx) : __expf(v[u].w - mx);
+        v[u].x = FORM != ALIGNED ? expf(v[u].x - mx) : __expf(v[u].x - mx);
+        v[u].y = FORM != ALIGNED ? expf(v[u].y - mx) : __expf(v[u].y - mx);
+        v[u].z = FORM != ALIGNED ? expf(v[u].z - mx) : __expf(v[u].z - mx);
+        v[u].w = FORM != ALIGNED ? expf(v[u].w - mx) : __expf(v[u].w - mx);
         s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
       }
     }
@@ -144,12 +158,11 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
         mnv_f4 o;
-        o.x = ODD ? v[u].x / s : v[u].x * inv;
-        o.y = ODD ? v[u].y / s : v[u].y * inv;
-        o.z = ODD ? v[u].z / s : v[u].z * inv;
-        o.w = ODD ? v[u].w / s : v[u].w * inv;
-        if (ODD) line_store(y + 4 * u * GROUP, left - 4 * u * GROUP, o);
-        else __builtin_nontemporal_store(o, y4 + u * GROUP);
+        o.x = FORM != ALIGNED ? v[u].x / s : v[u].x * inv;
+        o.y = FORM != ALIGNED ? v[u].y / s : v[u].y * inv;
+        o.z = FORM != ALIGNED ? v[u].z / s : v[u].z * inv;
+        o.w = FORM != ALIGNED ? v[u].w / s : v[u].w * inv;
+        line_store<FORM>(y + 4 * u * GROUP, left - 4 * u * GROUP, o);
       }
     }
   }
@@ -182,7 +195,7 @@ __global__ __launch_bounds__(MNV_SM_THREADS) void mnv_softmax_fwd_generic_kernel
   }
 }
 
-template <int GROUP, int CACHE, int NTH, bool ODD>
+template <int GROUP, int CACHE, int NTH, LineForm FORM>
 __global__ __launch_bounds__(NTH) void mnv_softmax_bwd_cached_kernel(
     const float* __restrict__ dy, const float* __restrict__ y, float* __restrict__ dx, int len,
     int lines) {
@@ -194,22 +207,15 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_bwd_cached_kernel(
     const float* dp = lane_pointer(dy + (size_t)line * len + 4 * t);
     const float* tp = lane_pointer(y + (size_t)line * len + 4 * t);
     float* op = lane_pointer(dx + (size_t)line * len + 4 * t);
-    const mnv_f4* d4 = reinterpret_cast<const mnv_f4*>(dp);
-    const mnv_f4* t4 = reinterpret_cast<const mnv_f4*>(tp);
-    mnv_f4* o4 = reinterpret_cast<mnv_f4*>(op);
     const int left = len - 4 * t;
     mnv_f4 d[CACHE], p[CACHE];
 #pragma unroll
     for (int u = 0; u < CACHE; ++u) {  // loads only, so that none waits for another
       if (t + u * GROUP < len4) {
         const int at = 4 * u * GROUP;
-        if (ODD) {  // zeros past the line's end: they add nothing to the sum
-          line_load(d[u], [&] { return mnv_ldx4u<false>(dp + at); }, dp + at, left - at, 0.f);
-          line_load(p[u], [&] { return mnv_ldx4u<true>(tp + at); }, tp + at, left - at, 0.f);
-        } else {
-          d[u] = d4[u * GROUP];
-          p[u] = __builtin_nontemporal_load(t4 + u * GROUP);
-        }
+        // zeros in the places past the line's end: they add nothing to the sum
+        line_load<FORM, false>(d[u], dp + at, left - at, 0.f);
+        line_load<FORM, true>(p[u], tp + at, left - at, 0.f);
       }
     }
     float dot = 0.f;
@@ -226,8 +232,7 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_bwd_cached_kernel(
         o.y = p[u].y * (d[u].y - dot);
         o.z = p[u].z * (d[u].z - dot);
         o.w = p[u].w * (d[u].w - dot);
-        if (ODD) line_store(op + 4 * u * GROUP, left - 4 * u * GROUP, o);
-        else __builtin_nontemporal_store(o, o4 + u * GROUP);
+        line_store<FORM>(op + 4 * u * GROUP, left - 4 * u * GROUP, o);
       }
     }
   }
@@ -398,16 +403,23 @@ unsigned line_grid(int lines, int lpb) {
 // 4.3 us with eight; 1023 lines of 2047, one wavefront -> 256 threads: forward 7.9 -> 5.8 us, backward 8.4 -> 5.1).
 #define MNV_SM_WIDE 512      // threads per line for lines of more than 4096 values
 #define MNV_SM_WIDE_CACHE 4  // 16-byte vectors cached per thread in that configuration
+LineForm line_form(int len, bool vec) {
+  return vec ? ALIGNED : len % 4 != 0 && len >= 4 && len <= MNV_WAVE * 4 ? TAIL_BACK : TAIL_EACH;
+}
+
 template <int GROUP, int CACHE, int NTH>
 int launch_fwd_cached(const float* in, float* out, int len, int lines, bool vec, bool nt, hipStream_t s) {
   const dim3 grid(line_grid(lines, NTH / GROUP)), block(NTH);
-#define MNV_SM_LAUNCH(NT, ODD)                                                                             \
-  hipLaunchKernelGGL((mnv_softmax_fwd_cached_kernel<GROUP, CACHE, NTH, NT, ODD>), grid, block, 0, s, in, \
+  const LineForm form = line_form(len, vec);
+#define MNV_SM_LAUNCH(NT, FORM)                                                                             \
+  hipLaunchKernelGGL((mnv_softmax_fwd_cached_kernel<GROUP, CACHE, NTH, NT, FORM>), grid, block, 0, s, in, \
                      out, len, lines)
-  if (vec) {
-    if (nt) MNV_SM_LAUNCH(true, false); else MNV_SM_LAUNCH(false, false);
-  } else {
-    if (nt) MNV_SM_LAUNCH(true, true); else MNV_SM_LAUNCH(false, true);
+  if (form == ALIGNED) {
+    if (nt) MNV_SM_LAUNCH(true, ALIGNED); else MNV_SM_LAUNCH(false, ALIGNED);
+  } else if (CACHE > 1 || form == TAIL_EACH) {
+    if (nt) MNV_SM_LAUNCH(true, TAIL_EACH); else MNV_SM_LAUNCH(false, TAIL_EACH);
+  } else if constexpr (CACHE == 1) {
+    if (nt) MNV_SM_LAUNCH(true, TAIL_BACK); else MNV_SM_LAUNCH(false, TAIL_BACK);
   }
 #undef MNV_SM_LAUNCH
   return MNV_LAUNCH_STATUS();
@@ -416,6 +428,13 @@ int launch_fwd_cached(const float* in, float* out, int len, int lines, bool vec,
 int softmax_lines_fwd(const float* in, float* out, int len, int lines, hipStream_t s) {
   const bool vec = (len % 4 == 0) && mnv_aligned16(in) && mnv_aligned16(out);
   const bool big = (size_t)len * lines * sizeof(float) >= MNV_PAST_CACHE_BYTES;
+  // short lines off the 16-byte grid: one value per lane (the general kernel) where a vector per lane
+  // leaves most lanes idle (vectors -> values, 1000000 lines: of 10 220 -> 195 us, 33 217 -> 202, 47 243 -> 277)
+  if (len % 4 != 0 && len >= 4 && len < 40) {
+    hipLaunchKernelGGL((mnv_softmax_fwd_generic_kernel<MNV_WAVE>), dim3(line_grid(lines, 4)), dim3(MNV_SM_THREADS), 0, s,
+                       in, out, len, lines, 1, (size_t)len, (size_t)1);
+    return MNV_LAUNCH_STATUS();
+  }
   if (len <= MNV_WAVE * 4) return launch_fwd_cached<MNV_WAVE, 1, MNV_SM_THREADS>(in, out, len, lines, vec, big, s);
   if (len <= MNV_WAVE * 4 * MNV_SM_CACHE / (vec ? 1 : 2))
     return launch_fwd_cached<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>(in, out, len, lines, vec, big, s);
@@ -431,18 +450,27 @@ int softmax_lines_fwd(const float* in, float* out, int len, int lines, hipStream
 template <int GROUP, int CACHE, int NTH>
 int launch_bwd_cached(const float* dy, const float* y, float* dx, int len, int lines, bool vec, hipStream_t s) {
   const dim3 grid(line_grid(lines, NTH / GROUP)), block(NTH);
-  if (vec)
-    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<GROUP, CACHE, NTH, false>), grid, block, 0, s, dy, y, dx,
-                       len, lines);
-  else
-    hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<GROUP, CACHE, NTH, true>), grid, block, 0, s, dy, y, dx,
-                       len, lines);
+  const LineForm form = line_form(len, vec);
+#define MNV_SM_LAUNCH(FORM)                                                                                   \
+  hipLaunchKernelGGL((mnv_softmax_bwd_cached_kernel<GROUP, CACHE, NTH, FORM>), grid, block, 0, s, dy, y, dx, \
+                     len, lines)
+  if (form == ALIGNED) MNV_SM_LAUNCH(ALIGNED);
+  else if (CACHE > 1 || form == TAIL_EACH) MNV_SM_LAUNCH(TAIL_EACH);
+  else if constexpr (CACHE == 1) MNV_SM_LAUNCH(TAIL_BACK);
+#undef MNV_SM_LAUNCH
   return MNV_LAUNCH_STATUS();
 }
 
 int softmax_lines_bwd(const float* dy, const float* y, float* dx, int len, int lines,
                       hipStream_t s) {
   const bool vec = (len % 4 == 0) && mnv_aligned16(dy) && mnv_aligned16(y) && mnv_aligned16(dx);
+  // as above (100000 lines: of 10 16.3 -> 15.6 us, 63 28.6 -> 19.8, 127 33.5 -> 31.6, 129 33.2 -> 35.6;
+  // 1000000 of 10 180 -> 127)
+  if (!vec && len >= 4 && len < 128) {
+    hipLaunchKernelGGL((mnv_softmax_bwd_generic_kernel<MNV_WAVE>), dim3(line_grid(lines, 4)), dim3(MNV_SM_THREADS), 0, s,
+                       dy, y, dx, len, lines, 1, (size_t)len, (size_t)1);
+    return MNV_LAUNCH_STATUS();
+  }
   if (len <= MNV_WAVE * 4) return launch_bwd_cached<MNV_WAVE, 1, MNV_SM_THREADS>(dy, y, dx, len, lines, vec, s);
   if (len <= MNV_WAVE * 4 * MNV_SM_CACHE / (vec ? 1 : 2))
     return launch_bwd_cached<MNV_WAVE, MNV_SM_CACHE, MNV_SM_THREADS>(dy, y, dx, len, lines, vec, s);

@@ -238,3 +238,68 @@ def test_short_columns_cost_what_aligned_ones_do(gpu):
     a, r, s = gpu.empty(12 * n), gpu.empty(n), gpu.dev.stream
     gpu.call("mnv_fill", a.p, ctypes.c_size_t(12 * n), ctypes.c_float(1))
     assert _ratio(gpu, lambda: gpu.L.mnv_reduce_sum_col(a.p, r.p, 11, n, s), lambda: gpu.L.mnv_reduce_sum_col(a.p, r.p, 12, n, s)) < 1.25
+
+
+def _softmax64(x):
+    with np.errstate(invalid="ignore"):
+        e = np.exp(x - x.max(1, keepdims=True))
+        return e / e.sum(1, keepdims=True)
+
+
+# lines of one value per lane, of a vector per lane and of several, around the lengths where that changes
+# (40 forward, 128 backward, 256, 1024, 4096, 8192), and shorter than a vector
+@pytest.mark.parametrize("length", [1, 2, 3, 4, 5, 10, 36, 39, 41, 126, 127, 129, 130, 131, 252, 255, 257, 259, 1022, 1027, 2050, 4097,
+                                    8191, 8194])
+@pytest.mark.parametrize("off", [0, 1, 2])
+def test_softmax_lines_off_the_16_byte_grid(gpu, ora, length, off):
+    """Against float64: the exponential's argument is rounded once (up to 10 u relative), a thread adds up to
+    length / 64 values and the threads' sums meet in a tree, (length / 64 + 32) u in all, u = 2^-24.
+    Backward: a dot product of that depth, relative to its sum of magnitudes, and three roundings.  Lines with
+    an infinity, a NaN, or nothing but -inf: NaN and zero where the oracle has them.  Both in place as
+    well, and the floats around the results untouched."""
+    lines, u, lead = 11, 2.0 ** -24, off + 4
+    say("softmax lines", length, lines, off)
+    x, dy = _rand(lines * length, 50), _rand(lines * length, 51)
+    X = x.reshape(lines, length)
+    X[3, length // 2] = np.nan
+    X[5, -1] = np.inf
+    X[7] = -np.inf
+    X[8, : length - 1] = -np.inf
+    plain = [i for i in range(lines) if i not in (3, 5, 7, 8)]
+    src, ddy, dst = gpu.up(_guarded(x, lead)), gpu.up(_guarded(dy, lead)), gpu.up(_guarded(np.zeros_like(x), lead))
+
+    def floats(d):
+        whole = gpu.down(d)
+        assert np.all(whole[:lead] == 7) and np.all(whole[lead + x.size:] == 7)
+        return whole[lead:lead + x.size].reshape(lines, length)
+
+    gpu.call("mnv_softmax_instance_fwd", _at(src, lead), _at(dst, lead), lines, length, 1, 1)
+    got = floats(dst)
+    want = _softmax64(X.astype(np.float64))
+    depth = length / 64 + 32
+    assert np.all(np.abs(got - want)[plain] <= depth * u * want[plain])
+    ref = ora.softmax_instance_fwd(x, lines, length, 1, 1).reshape(lines, length)
+    for i in (3, 5, 7, 8):
+        assert np.array_equal(np.isnan(got[i]), np.isnan(ref[i])) and np.array_equal(got[i] == 0, ref[i] == 0), i
+    gpu.call("mnv_softmax_instance_fwd", _at(src, lead), _at(src, lead), lines, length, 1, 1)
+    assert floats(src).tobytes() == got.tobytes()
+
+    gpu.call("mnv_softmax_instance_bwd", _at(ddy, lead), _at(src, lead), _at(dst, lead), lines, length, 1, 1)
+    back = floats(dst)
+    y, d = got[plain].astype(np.float64), dy.reshape(lines, length)[plain].astype(np.float64)
+    dot = (y * d).sum(1, keepdims=True)
+    bound = y * (depth * u * np.abs(y * d).sum(1, keepdims=True) + 3 * u * np.abs(d - dot))
+    assert np.all(np.abs(back[plain] - y * (d - dot)) <= bound)
+    assert np.isnan(back[3]).all() and np.isnan(back[7]).all()
+    gpu.call("mnv_softmax_instance_bwd", _at(ddy, lead), _at(src, lead), _at(ddy, lead), lines, length, 1, 1)
+    assert floats(ddy).tobytes() == back.tobytes()
+
+
+def test_short_softmax_lines_backward_cost_what_aligned_ones_do(gpu):
+    """10 and 12 values to a line: 125 and 133 us (a vector per lane for 10: 212)."""
+    n, s = 1000000, gpu.dev.stream
+    dy, y, dx = gpu.empty(12 * n), gpu.empty(12 * n), gpu.empty(12 * n)
+    for d in (dy, y):
+        gpu.call("mnv_fill", d.p, ctypes.c_size_t(12 * n), ctypes.c_float(0.1))
+    assert _ratio(gpu, lambda: gpu.L.mnv_softmax_instance_bwd(dy.p, y.p, dx.p, n, 10, 1, 1, s),
+                  lambda: gpu.L.mnv_softmax_instance_bwd(dy.p, y.p, dx.p, n, 12, 1, 1, s)) < 1.5
