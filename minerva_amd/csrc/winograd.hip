@@ -50,6 +50,7 @@
 
 #include "gemm_core.h"
 #include "winograd.h"
+#include "winograd_spans.h"
 
 namespace {
 
@@ -388,20 +389,6 @@ __global__ __launch_bounds__(256) void mnv_wino_input_kernel(const float* __rest
   wino_store_v<AL, R>(d, V + (size_t)ci * g.Pp + p, (size_t)g.Cin * g.Pp);
 }
 
-// What of the planes the 256 tiles from p0 on read, in 16-byte chunks: chunk c of plane i of
-// the tiles' images (the first one's plane is 0) is number i chunks + c, chunks = ceil(HW / 4),
-// and the tiles need the numbers [lo, hi) -- of the first and the last image only the rows that
-// hold their tiles.  A tile row th needs the plane's rows from m th - pad on, `reach` of them.
-struct WinoSpan {
-  int lo, hi;
-};
-__host__ __device__ inline WinoSpan wino_span(int th0, int th1, int images, int m, int pad, int reach, int H, int W,
-                                              int chunks) {
-  const int y0 = m * th0 - pad > 0 ? m * th0 - pad : 0;
-  const int y1 = m * th1 - pad + reach < H ? m * th1 - pad + reach : H;
-  return WinoSpan{y0 * W / 4, (images - 1) * chunks + (y1 * W + 3) / 4};
-}
-
 // Fetches that span of the planes at `src` (img_floats from one image's plane to the next's;
 // `floats`: what lies from src to the tensor's end) into LDS, number lo first.  Four 16-byte
 // loads in flight per thread; a plane's last chunk may reach into the next plane (never read
@@ -518,10 +505,6 @@ __global__ __launch_bounds__(256) void mnv_wino_output_kernel(const float* __res
         dst[at] = v;
       }
     }
-}
-
-__host__ __device__ inline WinoSpan wino_rows_span(int th0, int th1, int images, int m, int H, int W) {
-  return WinoSpan{m * th0 * W, (images - 1) * H * W + (m * (th1 + 1) < H ? m * (th1 + 1) : H) * W};
 }
 
 // The same through LDS, for planes small enough that the output rows of a workgroup's 256
@@ -913,38 +896,24 @@ int make_wino_geom(WinoGeom* g, int N, int Cin, int Cout, int Hs, int Ws, int pa
   return MNV_OK;
 }
 
-// The largest span of a launch's workgroups: span(first tile row, last tile row, images).
-template <class Span>
-int most_of_spans(const WinoGeom& g, const Span& span) {
-  const int T = g.TH * g.TW;
-  int most = 0;
-  for (long long p0 = 0; p0 < g.P; p0 += 256) {
-    const int last = p0 + 255 < g.P ? (int)p0 + 255 : g.P - 1;
-    const int img0 = (int)p0 / T, img1 = last / T;
-    const WinoSpan s = span(((int)p0 - img0 * T) / g.TW, (last - img1 * T) / g.TW, img1 - img0 + 1);
-    if (s.hi - s.lo > most) most = s.hi - s.lo;
-  }
-  return most;
-}
-
 // LDS bytes of the largest wino_span, or 0 where the planes are too large for LDS (three
 // workgroups per CU at least) or for 32-bit byte offsets.
 size_t span_lds_bytes(const WinoGeom& g, int channels, int H, int W, int m, int pad, int reach) {
   const int T = g.TH * g.TW, chunks = (H * W + 3) / 4;
   if ((255 / T + 2.0) * channels * H * W * 4.0 >= 2147483648.0) return 0;
-  const int most = most_of_spans(g, [&](int th0, int th1, int images) {
+  const int limit = 48 * 1024 / 16, most = wino_most_of_spans(g.P, g.TH, g.TW, limit, [&](int th0, int th1, int images) {
     return wino_span(th0, th1, images, m, pad, reach, H, W, chunks);
   });
-  return most <= 48 * 1024 / 16 ? (size_t)most * 16 : 0;
+  return most <= limit ? (size_t)most * 16 : 0;
 }
 
 // The same for the output rows; 0: too large for LDS.
 size_t rows_lds_bytes(const WinoGeom& g) {
   if ((255 / (g.TH * g.TW) + 2.0) * g.Hd * g.Wd >= 2147483648.0) return 0;
-  const int most = most_of_spans(g, [&](int th0, int th1, int images) {
+  const int limit = 48 * 1024 / 4, most = wino_most_of_spans(g.P, g.TH, g.TW, limit, [&](int th0, int th1, int images) {
     return wino_rows_span(th0, th1, images, g.m, g.Hd, g.Wd);
   });
-  return most <= 48 * 1024 / 4 ? (size_t)most * 4 : 0;
+  return most <= limit ? (size_t)most * 4 : 0;
 }
 
 // V of the group of images that `g` describes

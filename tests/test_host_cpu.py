@@ -117,3 +117,18 @@ def test_interface_fixture_is_what_the_extractor_writes():
     assert ip.structs(read("minerva/op/closure.h")) == want["closures"]
     assert ip.class_methods(read("minerva/device/device_manager.h"), "DeviceManager") == \
         want["classes"]["DeviceManager"]
+
+
+def test_lds_spans_of_the_minimal_filtering_transforms(tmp_path):
+    """What the transform kernels stage of the planes and the host's size for it, in the same code, on the
+    CPU: see the program's head."""
+    exe = str(tmp_path / "wino_spans_test")
+    cmd = ["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=all",
+           "-I" + os.path.join(ROOT, "minerva_amd", "csrc"), os.path.join(ROOT, "tests", "host_cpu", "wino_spans_test.cpp"),
+           "-o", exe]
+    build = subprocess.run(cmd, capture_output=True, text=True)
+    assert build.returncode == 0, build.stderr[-3000:]
+    env = dict(os.environ)
+    env.pop("LD_PRELOAD", None)
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=600, env=env)
+    assert run.returncode == 0 and run.stdout.strip() == "OK", (run.stdout + run.stderr)[-4000:]
