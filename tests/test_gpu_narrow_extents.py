@@ -303,3 +303,117 @@ def test_short_softmax_lines_backward_cost_what_aligned_ones_do(gpu):
         gpu.call("mnv_fill", d.p, ctypes.c_size_t(12 * n), ctypes.c_float(0.1))
     assert _ratio(gpu, lambda: gpu.L.mnv_softmax_instance_bwd(dy.p, y.p, dx.p, n, 10, 1, 1, s),
                   lambda: gpu.L.mnv_softmax_instance_bwd(dy.p, y.p, dx.p, n, 12, 1, 1, s)) < 1.5
+
+
+def _few(gpu, m, n, k, ws_bytes):
+    tile, ranges, groups = _plan(gpu, m, n, k, ws_bytes)
+    assert (tile, groups) == (256, 4), "the case must run the few-column kernels"
+    return ranges
+
+
+# every width the columns are rounded up to, at odd and even extents of the three lines of the rule; k ranges that
+# end in a step of 8, of 4 and in 1 to 3 values; m one row past a block
+FEW = [(1, 257, 4111), (2, 1027, 1039), (3, 300, 5002), (4, 513, 1029), (5, 257, 4109), (6, 1501, 2503), (7, 1027, 4099), (8, 4097, 1021),
+       (9, 4099, 4101), (10, 1025, 16391), (11, 9001, 1870), (12, 4097, 4098)]
+
+
+@pytest.mark.parametrize("n,m,k", FEW)
+def test_few_columns_off_the_16_byte_grid_next_to_infinities(gpu, n, m, k):
+    """Operands at 1, 2 and 3 floats past a 16-byte boundary, every float around them a NaN; a row of A and a
+    column of B that hold an infinity.  k + 1 roundings of 2^-24 against float64, and the fused forms
+    (bias and ReLU, ReLU gate, weight update) bit for bit the separate steps on the same product."""
+    say("few columns off the grid", n, m, k)
+    ws_bytes = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    _few(gpu, m, n, k, ws_bytes)
+    a, b = _rand(m * k, 60).reshape(k, m), _rand(n * k, 61).reshape(n, k)
+    a[k - 1, 0], b[n - 1, k - 1] = np.inf, -np.inf
+    ok = np.ix_(range(n - 1), range(1, m))  # rows and columns without an infinity
+    want = (b[:-1].astype(np.float64) @ a[:, 1:].astype(np.float64))
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(b[:-1]).astype(np.float64) @ np.abs(a[:, 1:]).astype(np.float64))
+    nan = np.full(4, np.nan, np.float32)
+    ws, dc = gpu.empty(ws_bytes // 4 + 1), gpu.empty(m * n)
+
+    def run(form, da, db, *extra, off, tail=()):
+        gpu.call("mnv_sgemm_" + form, _at(da, off), _at(db, off), *extra, m, n, k, *tail, ws.p, ctypes.c_size_t(ws_bytes))
+        return gpu.down(dc).reshape(n, m).copy()
+
+    first = None
+    for off in (1, 2, 3):
+        wrap = lambda v: gpu.up(np.concatenate([nan[:off], np.ascontiguousarray(v).reshape(-1), nan]))  # noqa: E731
+        da, db, dat, dbt = wrap(a), wrap(b), wrap(a.T), wrap(b.T)
+        got = run("nn", da, db, dc.p, off=off)
+        assert np.all(np.abs(got[ok] - want) <= bound)
+        assert not np.isfinite(got[:, 0]).any() and not np.isfinite(got[n - 1]).any()
+        first = got if first is None else first
+        for other in (got, run("tn", dat, db, None, dc.p, off=off), run("nt", da, dbt, dc.p, off=off)):
+            assert other.tobytes() == first.tobytes(), off
+    bias, gate, w = _rand(m, 62), _rand(m * n, 63).reshape(n, m), _rand(m * n, 64).reshape(n, m)
+    dbias, dgate, dw = gpu.up(bias), gpu.up(gate.reshape(-1)), gpu.up(w.reshape(-1))
+    with np.errstate(invalid="ignore"):
+        biased = first + bias
+        assert run("nn_bias", da, db, dbias.p, dc.p, off=3, tail=(1,)).tobytes() == np.where(biased > 0, biased, np.float32(0)).tobytes()
+        assert run("nn_relu_bwd", da, db, dgate.p, dc.p, off=3).tobytes() == np.where(gate > 0, first, np.float32(0)).tobytes()
+        sgd = run("nt_sgd", da, dbt, dw.p, ctypes.c_float(0.125), dc.p, off=3)
+        assert sgd.tobytes() == (w - np.float32(0.125) * first).tobytes()
+
+
+@pytest.mark.parametrize("m,n,k", [(4096, 3, 5000), (2050, 2, 4100), (8200, 12, 2100)])
+def test_few_columns_with_a_part_of_the_workspace(gpu, m, n, k):
+    """Fewer k ranges, down to the least that the rule accepts: within k + 1 roundings of float64 each."""
+    say("few columns, part of the workspace", m, n, k)
+    full = _few(gpu, m, n, k, gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k))
+    least = -(-128 // -(-m // 256))
+    a, b = _rand(m * k, 65), _rand(n * k, 66)
+    A, B = a.reshape(k, m).astype(np.float64), b.reshape(n, k).astype(np.float64)
+    want, bound = B @ A, (k + 1) * 2.0 ** -24 * (np.abs(B) @ np.abs(A))
+    da, db = gpu.up(a), gpu.up(b)
+    assert least < full
+    for have in sorted({least, least + 1, (least + full) // 2, full}):
+        assert _few(gpu, m, n, k, 4 * m * n * have) <= have
+        got = _bits(gpu, "nn", da, db, m, n, k, 4 * m * n * have).reshape(n, m)
+        assert np.all(np.abs(got - want) <= bound), have
+
+
+@pytest.mark.parametrize("m,n,k", [(32769, 2, 64), (33001, 1, 127), (40003, 3, 100), (66001, 4, 1000)])
+def test_few_columns_in_one_range(gpu, m, n, k):
+    """128 row blocks and more, or few k: one range, stored by the kernel itself, without a workspace."""
+    say("few columns, one range", m, n, k)
+    assert _few(gpu, m, n, k, 0) == 1
+    a, b = _rand(m * k, 67), _rand(n * k, 68)
+    A, B = a.reshape(k, m).astype(np.float64), b.reshape(n, k).astype(np.float64)
+    bound = (k + 1) * 2.0 ** -24 * (np.abs(B) @ np.abs(A))
+    da, db, dat = gpu.up(a), gpu.up(b), gpu.up(np.ascontiguousarray(a.reshape(k, m).T).reshape(-1))
+    got = _bits(gpu, "nn", da, db, m, n, k, 0)
+    assert np.all(np.abs(got.reshape(n, m) - B @ A) <= bound)
+    assert _bits(gpu, "tn", dat, db, m, n, k, 0, None).tobytes() == got.tobytes()
+
+
+def test_few_columns_of_an_operand_past_32_bit_offsets(gpu):
+    """A of 2^29 elements and more: two k panels, the second accumulated into C, both by the few-column
+    kernel.  Sampled rows against float64, k + 2 roundings."""
+    m, n, k = 70001, 3, 8192
+    assert m * k >= 1 << 29
+    first = ((1 << 29) - 1 - m) // m + 1
+    first -= first % 16
+    assert 64 <= k - first and _few(gpu, m, n, first, 0) == 1 and _few(gpu, m, n, k - first, 0) == 1
+    say("few columns, two panels", m, n, k)
+    da, db, dc = gpu.empty(m * k), gpu.up(_rand(n * k, 69)), gpu.up(np.full(m * n, np.nan, np.float32))
+    gpu.call("mnv_randn", da.p, ctypes.c_size_t(m * k), ctypes.c_uint64(70), ctypes.c_float(0), ctypes.c_float(1))
+    gpu.call("mnv_sgemm_nn", da.p, db.p, dc.p, m, n, k, None, ctypes.c_size_t(0))
+    rows = np.unique(np.concatenate([[0, 255, 256, m - 1], np.random.default_rng(71).integers(0, m, 60)]))
+    A = gpu.down(da).reshape(k, m)[:, rows].astype(np.float64)
+    B, got = gpu.down(db).reshape(n, k).astype(np.float64), gpu.down(dc).reshape(n, m)[:, rows]
+    assert np.all(np.abs(got - B @ A) <= (k + 2) * 2.0 ** -24 * (np.abs(B) @ np.abs(A)))
+
+
+@pytest.mark.parametrize("N,K,H,W", [(8192, 1, 1, 3), (4000, 3, 2, 1), (1500, 5, 1, 1)])
+def test_bias_gradient_of_several_hundred_image_groups(gpu, N, K, H, W):
+    """Up to 2048 group sums per channel, 32 to a lane: N H W roundings of 2^-24 against float64."""
+    say("bias gradient", N, K, H, W)
+    nbytes = gpu.L.mnv_conv_bwd_bias_workspace_bytes(N, K)
+    assert nbytes // (4 * K) >= 375
+    dy = _rand(N * K * H * W, 72)
+    ws, db, ddy = gpu.empty(nbytes // 4 + 1), gpu.empty(K), gpu.up(dy)
+    gpu.call("mnv_conv_bwd_bias", ddy.p, db.p, N, K, H, W, ws.p, ctypes.c_size_t(nbytes))
+    t = dy.reshape(N, K, H * W).astype(np.float64)
+    assert np.all(np.abs(gpu.down(db) - t.sum((0, 2))) <= N * H * W * 2.0 ** -24 * np.abs(t).sum((0, 2)))
