@@ -153,10 +153,12 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * range.
  * mnv_sgemm_nn_plan reports how a product of these extents is launched with a workspace of
  * that size (no counterpart in the reference, where the plan is cuBLAS's own): tile_rows is
- * 128 or 64 (square tiles) or 256 (256 x 128, or 256 rows by all of at most 12 columns), k_ranges the number of partial results reduced by a second
- * kernel (1: none), groups 4 when four wavefront groups of a workgroup share a tile and add
- * their quarters of the k range through LDS.  The plan depends on (m, n, k, workspace_bytes)
- * only, never on the operands. ---- */
+ * 128 or 64 for square tiles, 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
+ * kernels of at most 12 columns over a large A (256 rows per workgroup, 64 where A is given
+ * transposed; four wavefronts take a quarter of a k range each); k_ranges is the number of
+ * partial results reduced by a second kernel (1: none); groups is otherwise 4 when four
+ * wavefront groups of a workgroup share a tile and add their quarters of the k range through
+ * LDS.  The plan depends on (m, n, k, workspace_bytes) only, never on the operands. ---- */
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k);
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,
                       int* groups);

@@ -171,12 +171,13 @@ int launch_reduce_col(const float* in, float* out, int m, int n, mnv_stream_t st
 // Along dimension 1: out[r] = reduce_c in[r + c*m] (stride m between elements).
 // A workgroup owns RL*W consecutive rows (128 contiguous bytes per column) and
 // splits the columns over CG thread groups; partial results meet in LDS.
-// W = 4 rows per thread; 1 for matrices of less than four rows.
+// W = 4 rows per thread; 1 for few columns and for matrices of less than four rows.
 // VEC4: m and the matrix on the 16-byte grid; otherwise the same loads at the addresses the
 // columns have, and the thread whose rows the matrix ends in reduces its last four rows and keeps
-// its own.  (One row per thread, 4 bytes per load, one load in flight before: sums of 8191 x 8193
-// 140 -> 128 us, 65 x 4097 27 -> 8.5; the 128-byte run of an unaligned column lies in two lines,
-// both fetched whole.)
+// its own.  (One row per thread, 4 bytes per load, one load in flight: sums of 8191 x 8193
+// 140 us, 65 x 4097 27.4; vectors with the last rows element by element 120 and 8.3; now 75 and
+// 7.4.  At 8192 x 8192 44: the 128-byte run of an unaligned column lies in two lines, both fetched
+// whole.)
 // ---------------------------------------------------------------------------
 template <class Acc, class Emit, int RL, int CG, int W, bool VEC4, bool NT>
 __global__ __launch_bounds__(RL* CG) void mnv_reduce_row_kernel(const float* __restrict__ in,
@@ -328,9 +329,10 @@ __global__ __launch_bounds__(MNV_BIAS_THREADS) void mnv_conv_bwd_bias_kernel(
   }
 }
 
-// One wavefront per channel: its group sums arrive in one or two loads.  (One thread per
-// channel walked them one trip to memory after the other: 128 groups, 16 channels of 256 images,
-// 6.4 -> 2.3 us.)
+// One wavefront per channel, a group sum per lane and trip: one trip up to 64 groups, 32 at most (2048
+// groups, one channel of 8192 images).  (One thread per channel walked them one trip to memory after
+// the other: 64 groups, 16 channels of 256 images, 6.4 -> 2.3 us; with its first kernel, 8192 images of
+// one 3 x 3 channel 126 -> 10.9.)
 __global__ __launch_bounds__(256) void mnv_conv_bwd_bias_finish_kernel(
     const float* __restrict__ partial, float* __restrict__ bias_diff, int K, int groups) {
   const int k = blockIdx.x * (256 / MNV_WAVE) + threadIdx.x / MNV_WAVE, lane = threadIdx.x % MNV_WAVE;

@@ -385,7 +385,7 @@ struct SgemmPlan {
   int splits;
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
-  int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel, with this many k per wavefront
+  int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
 };
 
 // Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), with

@@ -62,8 +62,8 @@ __device__ __forceinline__ T* lane_pointer(T* p) {
 
 // One line per GROUP threads of an NTH-thread workgroup (GROUP = one wavefront or the whole
 // workgroup); the line (len <= GROUP*4*CACHE) is cached in registers.
-// Stores are non-temporal; NT: so are the loads (inputs of 256 MB and more, which no cache
-// holds until the next operator).  Lines of up to 8192 values take 512 threads with four
+// Aligned lines are stored non-temporally; NT: the loads are non-temporal (inputs of 256 MB and more,
+// which no cache holds until the next operator).  Lines of up to 8192 values take 512 threads with four
 // vectors each rather than 256 with eight (more wavefronts, shorter per-thread chains): on
 // 8192 lines of 8192, operands cycled through four sets, 6.3 TB/s against 5.8 TB/s (a plain
 // copy of the same operands: 6.3 TB/s).
@@ -71,7 +71,9 @@ __device__ __forceinline__ T* lane_pointer(T* p) {
 // accesses at the addresses the lines have; what stands in the places past a line's end has the
 // exponential 0 (-inf).  Exponentials and quotients are the ones of the general kernel below, which
 // made three passes over such lines, 4 bytes per access (8193 lines of 8191: 314 -> 104 us; backward
-// 233 -> 147).  Of a cut last vector
+// 233 -> 147): expf and a division per element, where aligned lines take the hardware's exp2 and one
+// reciprocal, so the last bits of a forward result depend on the alignment of its line.  Of a cut
+// last vector
 //  TAIL_EACH: the 1 to 3 values go element by element;
 //  TAIL_BACK (lines of 4 to 256 values, one vector per lane): the line's last four values are loaded, and
 //    those that another lane has are replaced: one load instead of three guarded ones (100000 lines of
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
 #pragma unroll
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
-        // exp through the hardware exp2: relative error ~1e-6 for the arguments <= 0 here
+        // aligned lines: exp through the hardware exp2, relative error ~1e-6 for the arguments <= 0 here
         v[u].x = FORM != ALIGNED ? expf(v[u].x - mx) : __expf(v[u].x - mx);
         v[u].y = FORM != ALIGNED ? expf(v[u].y - mx) : __expf(v[u].y - mx);
         v[u].z = FORM != ALIGNED ? expf(v[u].z - mx) : __expf(v[u].z - mx);
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(NTH) void mnv_softmax_fwd_cached_kernel(
       }
     }
     s = group_sum<GROUP>(s, lds);
-    const float inv = 1.0f / s;  // one reciprocal per thread instead of a division per element
+    const float inv = 1.0f / s;  // aligned lines: one reciprocal per thread instead of a division per element
 #pragma unroll
     for (int u = 0; u < CACHE; ++u) {
       if (t + u * GROUP < len4) {
