@@ -156,9 +156,14 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * 128 or 64 for square tiles, 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
  * kernels of at most 12 columns over a large A (256 rows per workgroup, 64 where A is given
  * transposed; four wavefronts take a quarter of a k range each); k_ranges is the number of
- * partial results reduced by a second kernel (1: none); groups is otherwise 4 when four
- * wavefront groups of a workgroup share a tile and add their quarters of the k range through
- * LDS.  The plan depends on (m, n, k, workspace_bytes) only, never on the operands. ---- */
+ * partial results reduced by a second kernel (1: none); groups is otherwise 4 when a workgroup
+ * has a CU to itself: four wavefront groups that share a 64 x 64 tile and add their quarters of the
+ * k range through LDS, or the eight wavefronts of a 128 x 128 tile.  The plan depends on (m, n, k,
+ * workspace_bytes) only, never on the operands.
+ * Tiles of 128 and 256 rows (groups 1, and 4 with 128) multiply on the bf16 matrix cores, every fp32
+ * value in three bf16 parts: the error against exact arithmetic is that of fp32 sums with fewer
+ * roundings, about 0.4 times that of one fused multiply-add per k; infinities, NaN and values
+ * from 2^111 on give what fp32 arithmetic gives, slower. ---- */
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k);
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,
                       int* groups);

@@ -178,6 +178,18 @@ template <class P>
 struct MnvCPreload<P, std::enable_if_t<P::C_PRELOAD>> {
   static constexpr bool value = true;
 };
+// Tiles of the bf16 matrix cores (MnvSplitTile, gemm_split.h); the launches below take either kind.
+template <class T, class = void>
+struct MnvIsSplit {
+  static constexpr bool value = false;
+};
+template <class T>
+struct MnvIsSplit<T, std::enable_if_t<T::SPLIT>> {
+  static constexpr bool value = true;
+};
+template <class T, class P, bool SK>
+__global__ void mnv_gemm_split_kernel(P prob, int tiles_m, int tiles_n, int slabs_per_split, float* __restrict__ partial,
+                                      int tail_begin, int tail_z);
 template <int NOFF>
 __device__ __forceinline__ void mnv_fetch_vec(mnv_rsrc r, const unsigned (&off)[NOFF],
                                               unsigned soff, float (&v)[4]) {
@@ -270,6 +282,34 @@ __device__ __forceinline__ void mnv_partial_group_mn(int group, int& m, int& n) 
   const int i = q / (T::TN * 4), j = (q / 4) % T::TN, g = q % 4;
   m = (wave % T::WGM) * T::WM + i * 32 + lane % 32;
   n = (wave / T::WGM) * T::WN + j * 32 + (lane / 32) * 4 + 8 * g;
+}
+// Hands a group's four sums to the policy's store (a tile of the bf16 cores keeps four rows of
+// one column together).
+template <class T, class P>
+__device__ __forceinline__ void mnv_partial_store(const P& prob, int m0, int n0, int group, mnv_f4 s) {
+  int m, n;
+  if constexpr (MnvIsSplit<T>::value) {
+    const int q = group / T::NT, t = group - q * T::NT;
+    const int wave = t / MNV_WAVE, lane = t % MNV_WAVE, j = q / 4, r = q % 4;
+    const int block = wave / T::WGM * T::TN + j, col = lane / 16 * 4 + r;
+    m = m0 + wave % T::WGM * T::WM + 4 * (lane % 16);
+    n = n0 + (P::B_KFAST ? block * 16 + col : block / 4 * 64 + block % 4 + 4 * col);
+    if (n >= prob.N) return;
+    if (m + 0 < prob.M) prob.c_store(m + 0, n, s.x);
+    if (m + 1 < prob.M) prob.c_store(m + 1, n, s.y);
+    if (m + 2 < prob.M) prob.c_store(m + 2, n, s.z);
+    if (m + 3 < prob.M) prob.c_store(m + 3, n, s.w);
+  } else {
+    mnv_partial_group_mn<T>(group, m, n);
+    m += m0;
+    n += n0;
+    if (m < prob.M) {
+      if (n + 0 < prob.N) prob.c_store(m, n + 0, s.x);
+      if (n + 1 < prob.N) prob.c_store(m, n + 1, s.y);
+      if (n + 2 < prob.N) prob.c_store(m, n + 2, s.z);
+      if (n + 3 < prob.N) prob.c_store(m, n + 3, s.w);
+    }
+  }
 }
 template <class T, class P, int G = 1, bool SK = false, int PF = 1>
 __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MIN_WAVES) void mnv_gemm_kernel(
@@ -786,16 +826,7 @@ __global__ __launch_bounds__(256) void mnv_gemm_tail_reduce_kernel(P prob,
       const mnv_f4 v = *reinterpret_cast<const mnv_f4*>(p + (size_t)z * TILE + e);
       s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
-    int m, n;
-    mnv_partial_group_mn<T>(e / 4, m, n);
-    m += m0;
-    n += n0;
-    if (m < prob.M) {
-      if (n + 0 < prob.N) prob.c_store(m, n + 0, s.x);
-      if (n + 1 < prob.N) prob.c_store(m, n + 1, s.y);
-      if (n + 2 < prob.N) prob.c_store(m, n + 2, s.z);
-      if (n + 3 < prob.N) prob.c_store(m, n + 3, s.w);
-    }
+    mnv_partial_store<T>(prob, m0, n0, e / 4, s);
   }
 }
 
@@ -874,16 +905,7 @@ __global__ __launch_bounds__(256) void mnv_gemm_streamk_reduce_kernel(P prob,
         s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
       }
     }
-    int m, n;
-    mnv_partial_group_mn<T>(e / 4, m, n);
-    m += m0;
-    n += n0;
-    if (m < prob.M) {
-      if (n + 0 < prob.N) prob.c_store(m, n + 0, s.x);
-      if (n + 1 < prob.N) prob.c_store(m, n + 1, s.y);
-      if (n + 2 < prob.N) prob.c_store(m, n + 2, s.z);
-      if (n + 3 < prob.N) prob.c_store(m, n + 3, s.w);
-    }
+    mnv_partial_store<T>(prob, m0, n0, e / 4, s);
   }
 }
 
@@ -944,6 +966,12 @@ static inline int mnv_pick_splits(long long tiles, int slabs, int max_splits, do
   return best;
 }
 
+template <class T, class P, int G, bool SK, int PF>
+static auto mnv_gemm_entry() {
+  if constexpr (MnvIsSplit<T>::value) return &mnv_gemm_split_kernel<T, P, SK>;
+  else return &mnv_gemm_kernel<T, P, G, SK, PF>;
+}
+
 // Host-side launch of one tile configuration.  `splits` > 1 needs
 // splits*M*N*sizeof(float) bytes at `workspace`.
 // `tail_bytes`: bytes at `workspace` that a launch without k ranges may use for the partial
@@ -963,14 +991,15 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
   // race only repeats the same call).
   static std::atomic<bool> attr_set[64];
   const size_t tile_bytes = G * T::lds_bytes(P::A_KFAST, P::B_KFAST);
-  const size_t lds_limit = (G > 1 ? 160 : 64) * 1024;
+  const size_t lds_limit = (G > 1 || MnvIsSplit<T>::value ? 160 : 64) * 1024;
+  const auto kernel = mnv_gemm_entry<T, P, G, false, PF>();
   if (G > 1 && prob.extra_lds_bytes()) return MNV_ERR_INVALID;  // groups use every tile buffer
   if (tile_bytes + prob.extra_lds_bytes() > 48 * 1024) {
     int dev = 0;
     MNV_HIP_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) return MNV_ERR_INVALID;
     if (!attr_set[dev].load(std::memory_order_acquire)) {
-      MNV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(&mnv_gemm_kernel<T, P, G, false, PF>),
+      MNV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit));
       attr_set[dev].store(true, std::memory_order_release);
     }
@@ -978,12 +1007,11 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
   const size_t lds_bytes = tile_bytes + prob.extra_lds_bytes();
   if (lds_bytes > lds_limit) return MNV_ERR_INVALID;
   MnvTailPlan tail{tiles_m * tiles_n, 1};
-  if (G == 1 && splits == 1 && T::MIN_WAVES == 4 && workspace && tail_bytes)
+  if (G == 1 && splits == 1 && (T::MIN_WAVES == 4 || MnvIsSplit<T>::value) && workspace && tail_bytes)
     tail = mnv_tail_plan((long long)tiles_m * tiles_n, total_slabs, (size_t)T::BM * T::BNU,
                          tail_bytes / sizeof(float));
   const int tail_tiles = tiles_m * tiles_n - tail.begin;
-  hipLaunchKernelGGL((mnv_gemm_kernel<T, P, G, false, PF>),
-                     dim3(tail.begin + tail_tiles * tail.z, 1, splits), dim3(T::NT * G), lds_bytes,
+  hipLaunchKernelGGL(kernel, dim3(tail.begin + tail_tiles * tail.z, 1, splits), dim3(T::NT * G), lds_bytes,
                      s, prob, tiles_m, tiles_n, per, reinterpret_cast<float*>(workspace),
                      tail.begin, tail.z);
   int rc = MNV_LAUNCH_STATUS();
@@ -1021,18 +1049,20 @@ static int mnv_gemm_streamk_launch(const P& prob, void* workspace, size_t ws_byt
   const int tiles_m = (prob.M + T::BM - 1) / T::BM, tiles_n = (prob.N + T::BNU - 1) / T::BNU;
   const long long tiles = (long long)tiles_m * tiles_n;
   const size_t lds_bytes = T::lds_bytes(P::A_KFAST, P::B_KFAST) + prob.extra_lds_bytes();
+  const size_t lds_limit = (MnvIsSplit<T>::value ? 160 : 64) * 1024;
   if (!workspace || prob.total_slabs <= 0 || tiles > 0x7fffffffLL / prob.total_slabs ||
-      lds_bytes > 64 * 1024)
+      lds_bytes > lds_limit)
     return MNV_OK;
   int dev = 0;
   MNV_HIP_TRY(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) return MNV_ERR_INVALID;
-  const void* fn = reinterpret_cast<const void*>(&mnv_gemm_kernel<T, P, 1, true, PF>);
+  const auto kernel = mnv_gemm_entry<T, P, 1, true, PF>();
+  const void* fn = reinterpret_cast<const void*>(kernel);
   // (LDS bytes << 8 | workgroups per CU) of the last query on each device
   static std::atomic<unsigned long long> cached[64];
   static std::atomic<bool> attr_set[64];
   if (lds_bytes > 48 * 1024 && !attr_set[dev].load(std::memory_order_acquire)) {
-    MNV_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+    MNV_HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_limit));
     attr_set[dev].store(true, std::memory_order_release);
   }
   unsigned long long c = cached[dev].load(std::memory_order_relaxed);
@@ -1071,7 +1101,7 @@ static int mnv_gemm_streamk_launch(const P& prob, void* workspace, size_t ws_byt
     *done = true;
     return MNV_OK;
   }
-  hipLaunchKernelGGL((mnv_gemm_kernel<T, P, 1, true, PF>), dim3(launched), dim3(T::NT), lds_bytes, s,
+  hipLaunchKernelGGL(kernel, dim3(launched), dim3(T::NT), lds_bytes, s,
                      prob, tiles_m, tiles_n, chunk, reinterpret_cast<float*>(workspace), aligned, 1);
   int rc = MNV_LAUNCH_STATUS();
   if (rc) return rc;

@@ -1,12 +1,13 @@
 // SGEMM C{m,n} = A{m,k} * B{k,n}, column-major, no transposes, alpha 1 / beta 0:
 // the product Minerva's MatMult asks for (reference minerva/op/impl/basic.cpp:150-173;
 // cublasSgemm call at minerva/op/impl/cuda/cuda_perform.cu:66-70).
-// Built on the fp32 MFMA core in gemm_core.h; A is fetched x-fast (m contiguous),
-// B k-fast (k contiguous).  Products with too few output tiles to fill 256 CUs split
-// the k range over blockIdx.z when the caller lends a workspace.
+// Built on the matrix cores, in bf16 parts (gemm_split.h) for products of enough work and with the
+// fp32 instruction (gemm_core.h) for the others; A is fetched x-fast (m contiguous), B k-fast (k
+// contiguous).  Products with too few output tiles to fill 256 CUs split the k range over
+// blockIdx.z when the caller lends a workspace.
 #include <mutex>
 
-#include "gemm_core.h"
+#include "gemm_split.h"
 
 // Split-k partial sums of mnv_sgemm_nn_static: one array per GPU the library is loaded on,
 // held until the process ends.  In host code the name `scratch` is only a handle for
@@ -59,6 +60,10 @@ struct SgemmNN {
   int relu;
   const float* sgd_w;
   float sgd_scale;
+  // Column tiles that are dealt m-tile by m-tile together, so that the 32 tiles an XCD works on
+  // at a time are not all the rows of one column (see launch_split).
+  static constexpr bool N_GROUPED = true;
+  int n_group;
   struct Res {
     mnv_rsrc a, b;
   };
@@ -364,15 +369,16 @@ SgemmNN<K4, TA, TB> make_sgemm(const float* a, const float* b, float* c, int m, 
   p.lda = e.lda ? e.lda : (TA ? k : m); p.ldb = e.ldb ? e.ldb : (TB ? n : k); p.ldc = e.ldc ? e.ldc : m;
   p.accumulate = e.accumulate;
   p.sgd_w = e.sgd_w; p.sgd_scale = e.sgd_scale;
+  p.n_group = 1;
   p.set_bk(16);
   return p;
 }
 
-typedef MnvGemmTile<128, 128, 16, 2, 2> TileBig;
 typedef MnvGemmTile<64, 64, 16, 2, 2> TileSmall;
-// Eight wavefronts of 64 x 64 (512 threads, two workgroups per CU): a quarter fewer bytes
-// fetched and staged per multiply than TileBig, the same reads from LDS.
-typedef MnvGemmTile<256, 128, 16, 4, 2> TileTall;
+// Of the bf16 parts: two workgroups per CU, one, and one with twice the rows.
+typedef MnvSplitTile<128, 128, 2, 4, 1> SplitPair;
+typedef MnvSplitTile<128, 128, 2, 4, 2> SplitOne;
+typedef MnvSplitTile<256, 128, 4, 2, 2> SplitTall;
 #define MNV_SGEMM_MAX_SPLITS 16
 
 // Tile shape and number of k ranges for an (m,n,k) product given `ws_floats` floats of
@@ -385,6 +391,7 @@ struct SgemmPlan {
   int splits;
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
+  bool split = false; // 128 x 128 and 256 x 128 tiles: in bf16 parts
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
 };
 
@@ -430,6 +437,53 @@ bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
   *plan = SgemmPlan{false, ranges, 4};
   plan->skinny = per;
   return true;
+}
+
+// Microseconds of a product on 128 x 128 tiles in bf16 parts with z k ranges: a step of 32 k takes
+// 1.13 where a CU has one workgroup (SplitOne), 1.3 of the CU's time for each where it has several
+// (SplitPair); about 3 for a workgroup's first loads and last stores, 4 for the reduction of
+// the k ranges beside its bytes.
+double split_cost(int m, int n, int k, int z) {
+  const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
+  const long long per_cu = (tiles * z + mnv_cu_count() - 1) / mnv_cu_count();
+  const int slabs = (k + 15) / 16, steps = ((slabs + z - 1) / z + 1) / 2;
+  const double work = per_cu == 1 ? 1.13 * steps + 3.0 : 1.3 * per_cu * steps + 3.0 * (double)((per_cu + 1) / 2);
+  return work + (z > 1 ? 4.0 + 8.0 * (double)m * n * z / 6e6 : 0.0);
+}
+
+// Which products run in bf16 parts.  Those planned on large tiles do, with the k ranges of their
+// plan where it wants workgroups of four wavefront groups, one per CU, and otherwise with those that
+// split_cost prefers.  Those planned on 64 x 64 tiles do where split_cost puts them at 90% of the
+// plan's cost (in slabs of a 128 x 128 tile, about 0.83 us) or less.  64 x 64 tiles themselves stay with the
+// fp32 instruction: the cut of their operands takes 4.3 vector instructions per matrix instruction.
+// us, fp32 instruction -> bf16 parts (* where the rule keeps the former):
+//   4096 x 4096 x 4096 941 -> 601, 4096 x 9216 x 256 161 -> 110, 4096 x 4096 x 256 69 -> 51,
+//   4096 x 256 x 9216 156 -> 109, 9216 x 256 x 4096 165 -> 121, 2048 x 2048 x 2048 152 -> 88,
+//   4096 x 1000 x 1000 76 -> 48, 4096 x 100 x 4096 47 -> 32, 200 x 3000 x 4000 67 -> 48, 1500 x 1500 x 1500
+//   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
+//   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
+//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0
+void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* plan) {
+  if (plan->tall || (!plan->small && plan->groups == 4)) {
+    plan->split = true;
+    return;
+  }
+  if (plan->groups == 4 || m <= 64 || n <= 64) return;
+  const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
+  const size_t fit = ws_floats / ((size_t)m * n);
+  const int slabs = (k + 15) / 16;
+  int best_z = 1;
+  double best = split_cost(m, n, k, 1);
+  for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * mnv_cu_count(); ++z) {
+    const double c = split_cost(m, n, k, z);
+    if (c < 0.97 * best) {
+      best = c;
+      best_z = z;
+    }
+  }
+  if (plan->small && best > 0.9 * 0.83 * cost) return;
+  *plan = SgemmPlan{false, best_z};
+  plan->split = true;
 }
 
 SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
@@ -493,14 +547,14 @@ SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
     }
   }
   // Large products whose 256 x 128 tiles fill the chip's two-per-CU slots in whole rounds
-  // (at least 95% of the multiplies of all rounds are the product's own): measured back to
-  // back, 4096^3 0.956 -> 0.940 ms, 8192 x 4096 x 8192 3.85 -> 3.74 ms.  Every element is summed
+  // (at least 95% of the multiplies of all rounds are the product's own).  Every element is summed
   // over k in the same order as on the 128 x 128 tile: the same bits.
   if (!best.small && best.splits == 1 && best.groups == 1 && m >= 256 && slabs >= 32) {
     const long long tiles = (long long)((m + 255) / 256) * ((n + 127) / 128);
     const long long slots = 2LL * mnv_cu_count(), rounds = (tiles + slots - 1) / slots;
     if ((double)m * n >= 0.95 * (double)(rounds * slots) * 256.0 * 128.0) best.tall = true;
   }
+  plan_split(m, n, k, ws_floats, best_cost, &best);
   return best;
 }
 
@@ -538,17 +592,26 @@ int launch_skinny_columns(const SgemmPlan& plan, const SgemmNN<K4, TA, TB>& p, v
   return mnv_gemm_reduce_launch(p, part, plan.splits, s);
 }
 
+// In bf16 parts.  Groups of up to eight column tiles, as many as divide them: 4096^3 on 256 x 128
+// tiles reads 12 panels for 32 tiles where whole columns read 18.
+template <class P>
+int launch_split(const SgemmPlan& plan, P p, void* workspace, size_t tail_bytes, hipStream_t s) {
+  const int tiles_n = (p.N + 127) / 128;
+  while (p.n_group < 8 && tiles_n % (2 * p.n_group) == 0) p.n_group *= 2;
+  if (plan.tall) return mnv_gemm_launch<SplitTall>(p, 1, workspace, s);
+  const long long tiles = (long long)((p.M + 127) / 128) * tiles_n;
+  return tiles * plan.splits <= mnv_cu_count() ? mnv_gemm_launch<SplitOne>(p, plan.splits, workspace, s)
+                                               : mnv_gemm_launch<SplitPair>(p, plan.splits, workspace, s, tail_bytes);
+}
+
 // A launch without k ranges may use the workspace for the partial tiles of a cut tail.
 template <class P>
 int launch_plan(const SgemmPlan& plan, const P& p, void* workspace, size_t workspace_bytes,
                 hipStream_t s) {
-  if (plan.tall) return mnv_gemm_launch<TileTall>(p, 1, workspace, s);
-  if (plan.groups == 4)
-    return plan.small ? mnv_gemm_launch<TileSmall, 4>(p, plan.splits, workspace, s)
-                      : mnv_gemm_launch<TileBig, 4>(p, plan.splits, workspace, s);
   const size_t tail_bytes = plan.splits == 1 && workspace ? workspace_bytes : 0;
-  return plan.small ? mnv_gemm_launch<TileSmall>(p, plan.splits, workspace, s, tail_bytes)
-                    : mnv_gemm_launch<TileBig>(p, plan.splits, workspace, s, tail_bytes);
+  if (plan.split) return launch_split(plan, p, workspace, tail_bytes, s);
+  if (plan.groups == 4) return mnv_gemm_launch<TileSmall, 4>(p, plan.splits, workspace, s);
+  return mnv_gemm_launch<TileSmall>(p, plan.splits, workspace, s, tail_bytes);
 }
 
 // Bytes a product without k ranges wants for the partial tiles of its cut tail.

@@ -1,0 +1,166 @@
+"""The matrix products that run in bf16 parts (csrc/gemm_split.h): at the edges of their tiles and
+k steps, with each operand transposed, with every epilogue, against float64 element by element; and
+with operands that have no such parts (infinities, NaN, values from 2^111 on) or hardly any
+(denormals), where they must do what fp32 arithmetic does."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_util import Gpu, assert_bits_equal, normwise, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return Gpu()
+
+
+def _plan(gpu, m, n, k, ws_bytes):
+    v = [ctypes.c_int() for _ in range(3)]
+    assert gpu.L.mnv_sgemm_nn_plan(m, n, k, ctypes.c_size_t(ws_bytes), *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+def _bound(A, B):
+    """Element-wise: the sum of a1 b1 is rounded at every eight k, in two sets of accumulators and (k
+    ranges) their sums, each time by at most one unit in the last place (the instruction cuts) of a partial sum of
+    |a||b|; what the cut into parts leaves out is 3 x 2^-25 of every product."""
+    k = A.shape[1]
+    return (k / 8 + 24) * 2.0 ** -23 * (np.abs(B) @ np.abs(A).T)
+
+
+def _products(gpu, A, B, workspace=True):
+    """C{m,n} by the three entry points; A is {m,k}, B {n,k} here (float32)."""
+    m, k = A.shape
+    n = B.shape[0]
+    a, at = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(np.ascontiguousarray(A).reshape(-1))
+    b, bt = gpu.up(np.ascontiguousarray(B).reshape(-1)), gpu.up(np.ascontiguousarray(B.T).reshape(-1))
+    nb = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k) if workspace else 0
+    ws = gpu.empty(nb // 4 + 1)
+    out = {}
+    for name, args in (("nn", (a, b)), ("tn", (at, b)), ("nt", (a, bt))):
+        c = gpu.up(np.full(m * n + 4, np.float32(7.5), np.float32))
+        extra = (None,) if name == "tn" else ()
+        gpu.call("mnv_sgemm_" + name, args[0].p, args[1].p, *extra, c.p, m, n, k, ws.p if nb else None, ctypes.c_size_t(nb))
+        got = gpu.down(c)
+        assert (got[m * n:] == 7.5).all(), "wrote past C"
+        out[name] = got[:m * n].reshape(n, m)
+    return out
+
+
+def _rand(shape, seed, relu=False):
+    x = np.random.default_rng(seed).standard_normal(shape).astype(np.float32)
+    return np.maximum(x, 0) if relu else x
+
+
+SHAPES = [  # m, n, k: what the tile, the k step (32), the slab (16) and the planner divide them into
+    (2048, 2048, 96),      # whole tiles, three steps, two workgroups per CU
+    (2561, 2047, 97),      # one past and one short of a tile, one k in the last slab: an odd step
+    (3841, 2177, 33), (3968, 1985, 31), (2500, 2500, 17),  # one slab and a bit, and less than a step
+    (2303, 3073, 112),     # the second half of the last step is missing
+    (1793, 2047, 1001),    # one workgroup per CU
+    (200, 3000, 4001),     # k ranges
+    (4095, 4096, 515),     # 256 x 128 tiles
+]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("workspace", [True, False])
+def test_products_in_parts_against_float64(gpu, m, n, k, workspace):
+    ws = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k) if workspace else 0
+    tile = _plan(gpu, m, n, k, ws)
+    if workspace:
+        assert tile[0] in (128, 256), "the case is meant to run in parts"
+    A, B = _rand((m, k), m + k, relu=True), _rand((n, k), n)
+    say("product in parts", m, n, k, "plan", tile)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    want, bound = B64 @ A64.T, _bound(A64, B64)
+    got = _products(gpu, A, B, workspace)
+    for name, c in got.items():
+        bad = np.abs(c - want) > bound
+        assert not bad.any(), "%s: %d elements, first %s" % (name, int(bad.sum()), np.argwhere(bad)[0])
+    assert_bits_equal(got["tn"], got["nn"], "A given transposed")
+
+
+@pytest.mark.parametrize("m,n,k", [(2561, 2047, 97), (1793, 2047, 1001), (200, 3000, 4001), (4095, 4096, 515)])
+def test_products_in_parts_next_to_values_without_parts(gpu, m, n, k):
+    """Infinities, NaN and finite values that a bf16 part or the scale in front of it cannot hold: the
+    result is infinite, NaN or finite where float32 arithmetic has it so (inf times 1, which has
+    two zero parts, is inf), and finite ones are as close as elsewhere."""
+    rng = np.random.default_rng(k)
+    A, B = _rand((m, k), 11), _rand((n, k), 12)
+    B[:, 3] = 1.0  # meets the infinities of A: parts 1, 0, 0
+    A[5, 3], A[m - 1, 3], A[m // 2, 3] = np.inf, -np.inf, np.nan
+    A[7, k - 1] = np.float32(3.4e38)   # rounds to infinity in bf16; its products stay finite
+    B[:, k - 1] = rng.uniform(0.25, 0.5, n).astype(np.float32)
+    B[n - 1, 0], A[:, 0] = np.float32(2.0 ** 120), np.float32(2.0 ** -20) * rng.uniform(1, 2, m).astype(np.float32)
+    B[2, 1], A[9, 1] = np.inf, 0.0     # inf times 0
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        want = B64 @ A64.T
+        # the redone blocks add in the order of fp32 arithmetic: one rounding per k
+        bound = (k + 8) * 2.0 ** -24 * (np.abs(B64) @ np.abs(A64).T)
+    say("product in parts next to infinities", m, n, k)
+    for name, c in _products(gpu, A, B).items():
+        assert np.array_equal(np.isnan(c), np.isnan(want)), name
+        inf = np.isinf(want)
+        assert np.array_equal(np.isinf(c), inf) and np.array_equal(c[inf] > 0, want[inf] > 0), name
+        fin = np.isfinite(want)
+        assert (np.abs(c[fin] - want[fin]) <= bound[fin]).all(), name
+
+
+def test_products_in_parts_of_denormals(gpu):
+    """The smallest operands keep all their bits: denormals times values near 1, and normal values whose
+    third part would be below the smallest bf16 number but for the scale."""
+    m, n, k = 2048, 2048, 96
+    rng = np.random.default_rng(3)
+    A = (rng.integers(1, 1 << 23, (m, k)) * 2.0 ** -149).astype(np.float32)   # denormals
+    A[m // 2:] = (_rand((m - m // 2, k), 5) * np.float32(2.0 ** -112)).astype(np.float32)
+    B = (_rand((n, k), 6) * np.float32(2.0 ** 30)).astype(np.float32)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    want, bound = B64 @ A64.T, _bound(A64, B64)
+    say("product in parts of denormals")
+    for name, c in _products(gpu, A, B).items():
+        assert (np.abs(c - want) <= bound).all(), name
+        assert normwise(c[:, :m // 2], want[:, :m // 2]) <= 1e-6, name
+
+
+def test_products_in_parts_are_no_less_exact_than_one_rounding_per_k(gpu):
+    """2-norm of the error against float64, for a left operand from a ReLU (whose zeros a sum of one
+    rounding per k gets for nothing): below what such a sum has, computed here in float32."""
+    m, n, k = 2048, 2048, 576
+    A, B = _rand((m, k), 21, relu=True), _rand((n, k), 22)
+    want = B[:64].astype(np.float64) @ A.astype(np.float64).T
+    acc = np.zeros((64, m), np.float32)
+    for q in range(k):  # a fused multiply-add per k
+        acc = (acc.astype(np.float64) + np.outer(B[:64, q].astype(np.float64), A[:, q].astype(np.float64))).astype(np.float32)
+    ref = np.linalg.norm(acc - want)
+    for name, c in _products(gpu, A, B).items():
+        assert np.linalg.norm(c[:64] - want) <= 0.6 * ref, name
+
+
+def test_epilogues_of_products_in_parts(gpu):
+    """Bias, ReLU, gate and update on a product in parts have the bits of the separate operators."""
+    m, n, k = 2562, 2047, 100
+    A, B = _rand((m, k), 31), _rand((n, k), 32)
+    rng = np.random.default_rng(33)
+    bias, gate, w = (rng.standard_normal(s).astype(np.float32) for s in (m, m * n, m * n))
+    nb = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    assert _plan(gpu, m, n, k, nb)[0] == 128
+    plain = _products(gpu, A, B)["nn"].reshape(-1)
+    ws, c = gpu.empty(nb // 4 + 1), gpu.empty(m * n)
+    a, b = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(B.reshape(-1))
+    at, bt = gpu.up(A.reshape(-1)), gpu.up(np.ascontiguousarray(B.T).reshape(-1))
+    tail = (m, n, k)
+    wsz = (ws.p, ctypes.c_size_t(nb))
+    say("epilogues of products in parts")
+    dbias, dgate, dw = gpu.up(bias), gpu.up(gate), gpu.up(w)
+    gpu.call("mnv_sgemm_nn_bias", a.p, b.p, dbias.p, c.p, *tail, 1, *wsz)
+    biased = (plain.reshape(n, m) + bias).reshape(-1)
+    assert_bits_equal(gpu.down(c), np.where(biased > 0, biased, np.float32(0)), "bias and ReLU")
+    gpu.call("mnv_sgemm_tn", at.p, b.p, dgate.p, c.p, *tail, *wsz)
+    assert_bits_equal(gpu.down(c), np.where(gate > 0, plain, np.float32(0)), "gate")
+    gpu.call("mnv_sgemm_nt_sgd", a.p, bt.p, dw.p, ctypes.c_float(0.25), c.p, *tail, *wsz)
+    assert_bits_equal(gpu.down(c), w - np.float32(0.25) * plain, "update")
