@@ -12,7 +12,7 @@
 // al x al tile (al = m + r - 1),
 //     M[xi,nu][co][p] = sum_ci U[xi,nu][co][ci] * V[xi,nu][ci][p],      p = (image, tile row, tile col)
 // with U = G g G^T (filters), V = B^T d B (input tiles) and the outputs Y = A^T M A.  The
-// products run as ONE launch of the fp32 MFMA core (gemm_core.h): the point is folded into the
+// products run as ONE launch of the matrix core kernel (gemm_split.h): the point is folded into the
 // column index, n = point * Coutp + co, and a workgroup picks the V panel of its point once, in
 // block_init.  Semantics are those of conv.hip: the forward pass correlates with the flipped
 // filter (cuDNN's CUDNN_CONVOLUTION as selected at minerva/op/impl/cuda/cuda_perform.cu:227-264),
@@ -48,7 +48,7 @@
 #include <mutex>
 #include <vector>
 
-#include "gemm_core.h"
+#include "gemm_split.h"
 #include "winograd.h"
 #include "winograd_spans.h"
 
@@ -803,7 +803,13 @@ struct WinoGradGemm {
   }
 };
 
-typedef MnvGemmTile<128, 128, 16, 2, 2> TileBig;
+// The products' tile, two workgroups per CU.  The k of these products is short (96 to 384) and their
+// output long, so a workgroup's first loads and last stores weigh: the 256 x 128 tile, one
+// workgroup per CU and the faster one for a long k, takes 2.2% more time over the training step at batch
+// 256 and 4.4% more over the three passes of 128 -> 256 channels on 32 x 56 x 56.  Against the
+// fp32 instruction on 128 x 128 tiles, us: 12544 x 64 * 256 x 96 395 -> 350, 2304 x 49 * 384 x 256
+// 185 -> 134, filter gradients of conv2-5 at batch 256 1062 -> 815 in all.
+typedef MnvSplitTile<128, 128, 2, 4, 1> TileBig;
 
 // Measurement aid (mnv_conv_winograd_profile): while it is on, every launch of the products
 // is bracketed by an event pair on its stream, so that a benchmark can time the MFMA kernel of
@@ -1035,13 +1041,6 @@ int wino_conv(const WinoGeom& g0, const float* src, const float* filter, const f
   return MNV_OK;
 }
 
-// Slabs the filter-gradient products' loads run ahead (see mnv_gemm_kernel): two; the kernel
-// still holds four workgroups per CU (conv2 / conv4 at batch 256: 387 -> 377 us on average).
-#ifndef MNV_WINO_SK_PF
-#define MNV_WINO_SK_PF 2
-#endif
-// (the forward / data-gradient products gain nothing from it: 388 / 474 / 435 against 388 / 474 /
-// 426 us.)
 template <int AL, int R>
 int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_diff, float* filter_diff,
                      int N, int images, int accumulate, const float* sgd_w, float sgd_scale,
@@ -1063,7 +1062,7 @@ int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_d
     plan[0] = 128;
     plan[1] = 1;
     plan[2] = 0;
-    return mnv_gemm_streamk_launch<TileBig, MNV_WINO_SK_PF>(p, w, sk_bytes, s, &done, plan + 2);
+    return mnv_gemm_streamk_launch<TileBig>(p, w, sk_bytes, s, &done, plan + 2);
   }
   int rc;
   const size_t per_bottom = (size_t)C * g.Hs * g.Ws, per_top = (size_t)K * g.Hd * g.Wd;
@@ -1084,7 +1083,7 @@ int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_d
     bool done = false;
     hipEvent_t e0, e1;
     const bool timed = profile_begin(&e0, &e1, s);
-    rc = mnv_gemm_streamk_launch<TileBig, MNV_WINO_SK_PF>(p, w, sk_bytes, s, &done);
+    rc = mnv_gemm_streamk_launch<TileBig>(p, w, sk_bytes, s, &done);
     if (!rc && !done) rc = mnv_gemm_launch<TileBig>(p, 1, nullptr, s);
     if (timed) profile_end(e0, e1, s, 1, 2.0 * AL * AL * K * C * g.P);
     if (rc) return rc;

@@ -164,3 +164,37 @@ def test_epilogues_of_products_in_parts(gpu):
     assert_bits_equal(gpu.down(c), np.where(gate > 0, plain, np.float32(0)), "gate")
     gpu.call("mnv_sgemm_nt_sgd", a.p, bt.p, dw.p, ctypes.c_float(0.25), c.p, *tail, *wsz)
     assert_bits_equal(gpu.down(c), w - np.float32(0.25) * plain, "update")
+
+
+@pytest.mark.parametrize("C,K,tile", [(96, 136, 4), (64, 256, 5), (40, 130, 3)])
+def test_filtering_passes_of_values_without_parts(gpu, C, K, tile):
+    """The minimal-filtering passes multiply transformed tensors in parts: inputs scaled by 2^100 and more, whose
+    transforms have none, give the scaled results of ordinary ones to the rounding of the sums."""
+    N, H = 6, 13
+    p = (N, C, K, H, H, 1, 1, 1, 1, 3, 3)
+    if C % 16:
+        p = (N, 48, K, H, H, 1, 1, 1, 1, 3, 3)
+    C = p[1]
+    rng = np.random.default_rng(C + K)
+    x, w, b = (rng.standard_normal(s).astype(np.float32) for s in (N * C * H * H, K * C * 9, K))
+    dy = rng.standard_normal(N * K * H * H).astype(np.float32)
+    up, down = np.float32(2.0 ** 112), np.float32(2.0 ** -30)
+    mode = gpu.L.mnv_conv_winograd_mode(tile)
+    try:
+        nb = max(gpu.L.mnv_conv_fwd_workspace_bytes(*p), gpu.L.mnv_conv_bwd_filter_workspace_bytes(*p))
+        ws = gpu.empty(nb // 4 + 1)
+        top, fd = gpu.empty(N * K * H * H), gpu.empty(K * C * 9)
+
+        def passes(sx, sw, sd):
+            say("filtering passes", p, "tile mode", tile, "scale", float(sx))
+            dx, dw, db, ddy = (gpu.up(v) for v in (x * sx, w * sw, b * sx * sw, dy * sd))
+            gpu.call("mnv_conv_fwd", dx.p, dw.p, db.p, top.p, *p, ws.p, ctypes.c_size_t(nb))
+            gpu.call("mnv_conv_bwd_filter", dx.p, ddy.p, fd.p, *p, ws.p, ctypes.c_size_t(nb))
+            return gpu.down(top).astype(np.float64) / (float(sx) * float(sw)), gpu.down(fd).astype(np.float64) / (float(sx) * float(sd))
+
+        one = np.float32(1)
+        ordinary, scaled = passes(one, one, one), passes(up, down, down)
+    finally:
+        gpu.L.mnv_conv_winograd_mode(mode)
+    for got, want in zip(scaled, ordinary):
+        assert np.isfinite(got).all() and normwise(got, want) <= 2e-5
