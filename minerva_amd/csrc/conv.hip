@@ -1,5 +1,6 @@
-// Convolution forward, backward-data and backward-filter as implicit GEMMs on the fp32
-// MFMA core (gemm_core.h).  Semantics: cuDNN v2 CUDNN_CONVOLUTION (flipped filter),
+// Convolution forward, backward-data and backward-filter as implicit GEMMs on the matrix cores:
+// with the fp32 instruction (gemm_core.h) or, where that is the faster one, in bf16 parts
+// (gemm_split.h).  Semantics: cuDNN v2 CUDNN_CONVOLUTION (flipped filter),
 // zero padding, NCHW / KCRS bytes, as selected by the reference at
 // minerva/op/impl/cuda/cuda_perform.cu:227-318:
 //   top[n,k,i,j] = bias[k] + sum_{c,r,s} bottom[n,c,i*sv-ph+r,j*sh-pw+s] * filter[k,c,R-1-r,S-1-s]
@@ -13,7 +14,7 @@
 // tensor, so result stores are coalesced, and no im2col buffer exists in HBM.
 // Roofline: fp32 MFMA, 2*N*Ho*Wo*K*C*R*S algorithmic flops per pass.
 
-#include "gemm_core.h"
+#include "gemm_split.h"
 #include "winograd.h"
 
 namespace {
@@ -736,6 +737,14 @@ int launch_tile(int tile, const P& p, int splits, void* ws, hipStream_t s, size_
 }
 const int kTileM[4] = {64, 128, 128, 128}, kTileN[4] = {64, 128, 96, 32};
 
+// In bf16 parts.  128 x 128 tiles with a CU to themselves: the gathers' offsets need the registers
+// (four 4-byte loads per vector; on the tile with two workgroups per CU they spill, 490 against
+// 415 us for 96 -> 256 channels under 5 x 5 filters on 64 x 27 x 27).  96-column tiles: two
+// workgroups of four wavefronts per CU.
+typedef MnvSplitTile<128, 128, 2, 4, 2> SplitOne;
+typedef MnvSplitTile<128, 128, 2, 4, 1> SplitPair;
+typedef MnvSplitTile<128, 96, 2, 2, 1> Split96;
+
 // The filter gradient: few output tiles and a very long k.  On the large tiles it runs as
 // one launch of as many workgroups as the chip holds, every one with the same number of
 // k-slabs (stream-k: aligned k ranges of every tile, the rest in shares; see mnv_gemm_kernel),
@@ -750,7 +759,13 @@ const int kTileM[4] = {64, 128, 128, 128}, kTileN[4] = {64, 128, 96, 32};
 #endif
 // `plan` (optional): nothing is launched; plan[0] = rows of the tile, plan[1] = k ranges,
 // plan[2] = workgroups of the stream-k launch (0: k ranges).
-template <class P>
+// `parts`: in bf16 parts where the workspace holds the partial tiles (unpadded layers, whose
+// gathered operand comes four k at a time; of the padded ones, one k per lane, the fetch by fours and the cut
+// together take what the faster instruction gains: 53 -> 46 us for 256 -> 384 under 3 x 3 on
+// 10 x 13 x 13, 60 -> 59 for 384 -> 384, 129 -> 143 for 128 -> 256 on 32 x 56 x 56 at stride 2).  3 -> 96
+// under 11 x 11, stride 4, 256 / 50 / 10 images of 227 x 227: 537 -> 386, 101 -> 89, 38 -> 34 us; 256 ->
+// 256 under 1 x 1 on 16 x 28 x 28 40 -> 30.
+template <bool PARTS = false, class P>
 int launch_filter_gradient(int tile, const P& p, int splits, void* ws, size_t ws_bytes, hipStream_t s,
                            int* plan = nullptr) {
   if (plan) {
@@ -761,8 +776,19 @@ int launch_filter_gradient(int tile, const P& p, int splits, void* ws, size_t ws
   if (tile == 1 || tile == 2) {
     bool done = false;
     int* wgs = plan ? plan + 2 : nullptr;
-    const int rc = tile == 1 ? mnv_gemm_streamk_launch<TileBig, MNV_SK_PF>(p, ws, ws_bytes, s, &done, wgs)
-                             : mnv_gemm_streamk_launch<Tile96, MNV_SK_PF>(p, ws, ws_bytes, s, &done, wgs);
+    int rc = MNV_OK;
+    if constexpr (PARTS) {
+      // Few tiles have long ranges, which the pair works off faster (96 -> 256 under 3 x 3 on 64 x 28 x
+      // 28, 14 tiles: 146 us, 152 with one workgroup per CU); many need twice the partial tiles for it
+      // (22 -> 1408 under 5 x 5 on 17 x 17 x 17, 55 tiles: 54 and 53), and short ranges do not
+      // repay twice the workgroups at all.
+      const bool pair = (long long)((p.M + 127) / 128) * ((p.N + 127) / 128) < 32;
+      if (tile == 2) rc = mnv_gemm_streamk_launch<Split96>(p, ws, ws_bytes, s, &done, wgs);
+      else if (pair) rc = mnv_gemm_streamk_launch<SplitPair>(p, ws, ws_bytes, s, &done, wgs);
+      if (!rc && !done && tile == 1) rc = mnv_gemm_streamk_launch<SplitOne>(p, ws, ws_bytes, s, &done, wgs);
+    }
+    if (!rc && !done) rc = tile == 1 ? mnv_gemm_streamk_launch<TileBig, MNV_SK_PF>(p, ws, ws_bytes, s, &done, wgs)
+                                   : mnv_gemm_streamk_launch<Tile96, MNV_SK_PF>(p, ws, ws_bytes, s, &done, wgs);
     if (rc || done) {
       if (plan && done) plan[1] = 1;
       return rc;
@@ -787,6 +813,57 @@ size_t tail_workspace_bytes(int tile, int m, int n, int slabs) {
 int wide_tile(int n) {
   int pad128 = (n + 127) / 128 * 128, pad96 = (n + 95) / 96 * 96;
   return pad96 * 10 < pad128 * 9 ? 2 : 1;
+}
+
+// Which forward and data-gradient products run in bf16 parts, and in how many k ranges (0: not).
+// From 0.7 GFLOP on where the estimate is below that of the fp32 tiles: a step of 32 k takes 1.6 us
+// on SplitOne, 1.7 on Split96 alone on its CU and 1.26 of the CU's time beside another; about 3 for
+// a workgroup's first loads and last stores, 4 for the reduction of the k ranges beside its bytes; the
+// fp32 instruction 115 TFLOP/s on the large tiles, 80 and 11 us on 64 x 64.
+// us with the filter's permutation, fp32 instruction -> bf16 parts, forward: 96 -> 256 under 5 x 5 on 27 x 27,
+// 1 / 2 / 10 / 64 images 27 -> 25 / 41 -> 32 / 123 -> 77 / 523 -> 415; 384 -> 384 under 3 x 3 on
+// 13 x 13, 2 / 10 images 31 -> 28 / 70 -> 48; 128 -> 256 on 32 x 56 x 56 547 -> 430, stride 2 188 -> 164;
+// 256 -> 256 under 1 x 1 on 16 x 28 x 28 33 -> 24; 3 -> 96 under 11 x 11, stride 4, 227 x 227, 10 / 256
+// images 40 -> 38 / 572 -> 537; data gradients: 96 <- 256 of 10 images 131 -> 84, 256 <- 384 54 -> 40.
+// Left: 256 -> 384 of one image (0.3 GFLOP) 19 -> 21, 64 -> 128 under 1 x 1, stride 2 (0.2) 9.5 -> 10.3.
+int split_ranges(int m, int n, int slabs, int tile, size_t ws_floats) {
+  const double flop = 2.0 * m * n * slabs * 16.0;
+  if (n <= 64 || m < 128 || flop < 7e8) return 0;
+  const bool narrow = wide_tile(n) == 2;
+  const long long tiles = (long long)((m + 127) / 128) * (narrow ? (n + 95) / 96 : (n + 127) / 128);
+  const long long cus = mnv_cu_count();
+  const size_t fit = ws_floats / ((size_t)m * n);
+  double best = tile == 0 ? flop / 80e6 + 11.0 : flop / 115e6;
+  best *= 0.95;
+  int z_best = 0;
+  for (int z = 1; z <= 32; ++z) {
+    if (z > 1 && ((size_t)z > fit || slabs / z < 4 || tiles * z > 4 * cus)) break;
+    const long long per_cu = (tiles * z + cus - 1) / cus;
+    const int steps = ((slabs + z - 1) / z + 1) / 2;
+    double cost = narrow ? (per_cu == 1 ? 1.7 : 1.26 * per_cu) * steps + 3.0 * (double)((per_cu + 1) / 2)
+                         : per_cu * (1.6 * steps + 3.0);
+    if (z > 1) cost += 4.0 + 8.0 * (double)m * n * z / 6e6;
+    if (cost < best * (z_best ? 0.97 : 1.0)) {
+      best = cost;
+      z_best = z;
+    }
+  }
+  return z_best;
+}
+
+// Forward and data gradient: in bf16 parts or, with `splits` k ranges, on the fp32 tile.
+template <class P>
+int launch_direct(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t ws_bytes) {
+  if (const int z = split_ranges(p.M, p.N, p.total_slabs, tile, ws_bytes / sizeof(float)))
+    return wide_tile(p.N) == 2 ? mnv_gemm_launch<Split96>(p, z, ws, s, ws_bytes)
+                               : mnv_gemm_launch<SplitOne>(p, z, ws, s, ws_bytes);
+  return launch_tile(tile, p, splits, ws, s, ws_bytes);
+}
+
+// Bytes of the k ranges' partial results in bf16 parts.
+size_t split_bytes(int tile, int m, int n, int slabs) {
+  const int z = split_ranges(m, n, slabs, tile, (size_t)-1);
+  return z > 1 ? (size_t)z * m * n * sizeof(float) : 0;
 }
 
 int make_geom(ConvGeom* g, int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh,
@@ -903,6 +980,8 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
   const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, (g.CRS + 15) / 16);
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
+  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, (g.CRS + 15) / 16);
+  if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
   if (mnv_wino_images(N, C, K, H, W, ph, pw, R, S, sv, sh, (size_t)-1)) {
     const size_t w = mnv_wino_workspace_bytes(N, C, K, H, W, ph, pw, R);
     if (w > need) need = w;
@@ -943,11 +1022,11 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
     rc = permute_filter(filter, wp, K, C, g.RS, false, s);
     if (rc) return rc;
     ConvFwd<true> p{bottom, wp, bias, top, g, gm, gn, gk, g.RS * (C / 16), C / 16, relu};
-    return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
   }
   if (np) {
     ConvFwdNP p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, gk >= 16 ? gk / 16 : 1, relu};
-    return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
   }
   ConvFwd<false> p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, 1, relu};
   return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
@@ -997,6 +1076,8 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
   const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, (K * g.RS + 15) / 16);
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
+  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, (K * g.RS + 15) / 16);
+  if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
   if (mnv_wino_images(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R, S, sv, sh, (size_t)-1)) {
     const size_t w = mnv_wino_workspace_bytes(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R);
     if (w > need) need = w;
@@ -1031,7 +1112,7 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
     rc = permute_filter(filter, wq, K, C, g.RS, true, s);
     if (rc) return rc;
     ConvBwdData<true> p{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * (K / 16), K / 16, gate};
-    return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
   }
   ConvBwdData<false> p{top_diff, filter, bottom_diff, g, gm, gn, gk, (gk + 15) / 16, 1, gate};
   return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
@@ -1132,7 +1213,7 @@ static int conv_bwd_filter_impl(const float* bottom, const float* top_diff, floa
   if (tile != 0 && ph == 0 && pw == 0 && (size_t)PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<true> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                               PP / 16, PP, 1, mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale};
-    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient<true>(tile, p, splits, workspace, workspace_bytes, s, plan);
   }
   if (tile != 0 && C % 128 == 0 && (size_t)PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<false, 1> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),

@@ -63,7 +63,7 @@ struct MnvSplitTile {
   static constexpr int A_BYTES = 3 * plane(BM), B_BYTES = 3 * plane(BN), BUF_BYTES = A_BYTES + B_BYTES;
   static constexpr size_t lds_bytes(bool, bool) { return (size_t)BUFS * BUF_BYTES; }
   static constexpr int MIN_WAVES = NT / 256 * (3 - BUFS);  // per SIMD
-  static_assert(TM == 4 && WM % 16 == 0 && WN % 16 == 0 && BM % 64 == 0 && BN % 64 == 0, "four blocks of rows per wavefront");
+  static_assert(TM == 4 && WM % 16 == 0 && WN % 16 == 0 && BM % 64 == 0 && BN % 32 == 0, "four blocks of rows per wavefront");
 };
 
 // two values (consecutive k of one x) as three pairs of bf16, the largest first

@@ -6,6 +6,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 from gpu_util import Gpu, assert_bits_equal, normwise, say
 
@@ -198,3 +199,84 @@ def test_filtering_passes_of_values_without_parts(gpu, C, K, tile):
         gpu.L.mnv_conv_winograd_mode(mode)
     for got, want in zip(scaled, ordinary):
         assert np.isfinite(got).all() and normwise(got, want) <= 2e-5
+
+
+DIRECT = [  # N, C, K, H, W, pad, stride, filter
+    (10, 96, 256, 27, 27, 2, 1, 5),    # k ranges; 96 columns in the data gradient
+    (3, 48, 130, 57, 55, 1, 1, 3),     # an odd number of slabs, two columns in the last tile
+    (9, 16, 200, 41, 43, 0, 1, 3),     # one slab per tap, no padding
+    (12, 3, 96, 131, 127, 0, 4, 11),   # the channels of an image, every k its own gather
+    (8, 400, 136, 33, 33, 0, 1, 1),
+    (8, 64, 192, 61, 59, 1, 2, 3),     # 96-column tiles
+    (1, 256, 80, 70, 67, 1, 1, 3),     # one image, a tile that is not full
+]
+
+
+@pytest.mark.parametrize("case", DIRECT, ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("infinite", [False, True])
+def test_direct_convolutions_in_parts_against_float64(gpu, case, infinite):
+    """The implicit products of the convolutions, forward, data and filter gradient, with all of the
+    workspace, with what the permuted filter alone takes, and (forward) with none; once with an
+    infinity among the inputs, which reaches the outputs that it reaches in exact arithmetic."""
+    N, C, K, H, W, pad, st, R = case
+    p = (N, C, K, H, W, pad, pad, st, st, R, R)
+    Ho, Wo = (H + 2 * pad - R) // st + 1, (W + 2 * pad - R) // st + 1
+    rng = np.random.default_rng(sum(case))
+    x, w, b, dy = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (K, C, R, R), (K,), (N, K, Ho, Wo)))
+    if infinite:
+        x[N - 1, C // 2, H // 2, W // 2] = np.inf
+        dy[0, K - 1, Ho // 3, Wo // 3] = -np.inf
+    x64, w64, dy64 = (torch.from_numpy(v).double() for v in (x, w, dy))
+
+    def passes(x, w, dy):
+        xs, ws = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        y = torch.nn.functional.conv2d(xs, ws.flip(2, 3), None, st, pad)
+        dx, dw = torch.autograd.grad(y, (xs, ws), dy)
+        return [v.detach().numpy() for v in (y, dx, dw)]
+
+    # |sum| <= (roundings) 2^-23 sum |a||b|: one per eight k, those of the k ranges, and in fp32
+    # arithmetic next to an infinity one of 2^-24 per k
+    fin = [torch.nan_to_num(v, posinf=0.0, neginf=0.0) for v in (x64, dy64)]
+    size = passes(fin[0].abs(), w64.abs(), fin[1].abs())
+    want = passes(x64, w64, dy64) if not infinite else None
+    if infinite:  # where the infinity goes, with its sign; torch's products would mix it with zeros
+        base = passes(fin[0], w64, fin[1])
+        mark_x, mark_dy = torch.isinf(x64).double() * torch.sign(x64), torch.isinf(dy64).double() * torch.sign(dy64)
+        reach = [torch.nn.functional.conv2d(mark_x, w64.flip(2, 3), None, st, pad).numpy(),
+                 passes(fin[0], w64, mark_dy)[1]]
+        # every tap of the marked pixel and every pixel of the marked gradient meets one finite value
+        dw_x, dw_dy = passes(mark_x, w64, fin[1])[2], passes(fin[0], w64, mark_dy)[2]
+        reach.append(dw_x)
+        both = (dw_x != 0) & (dw_dy != 0) & (np.sign(dw_x) != np.sign(dw_dy))
+        reach[2] = np.where(dw_dy != 0, dw_dy, reach[2])
+        want = []
+        for v, r in zip(base, reach):
+            v = v.copy()
+            v[r != 0] = np.inf * np.sign(r[r != 0])
+            want.append(v)
+        want[2][both] = np.nan
+    bias = np.broadcast_to(b.astype(np.float64)[None, :, None, None], want[0].shape)
+    want[0] = want[0] + bias
+    ks = (C * R * R, K * R * R, N * Ho * Wo)
+    bound = [(k / 8 + 64 if not infinite else k + 64) * 2.0 ** -23 * v for k, v in zip(ks, size)]
+    bound[0] = bound[0] + np.abs(bias) * 2.0 ** -20
+    dx_, dw_, db_, ddy = (gpu.up(np.ascontiguousarray(v).reshape(-1)) for v in (x, w, b, dy))
+    mode = gpu.L.mnv_conv_winograd_mode(0)
+    try:
+        jobs = [("fwd", want[0], bound[0], gpu.L.mnv_conv_fwd_workspace_bytes(*p), w.size * 4),
+                ("bwd_data", want[1], bound[1], gpu.L.mnv_conv_bwd_data_workspace_bytes(*p), w.size * 4),
+                ("bwd_filter", want[2], bound[2], gpu.L.mnv_conv_bwd_filter_workspace_bytes(*p), 0)]
+        for name, ref, tol, full, small in jobs:
+            ws, out = gpu.empty(full // 4 + 1), gpu.empty(ref.size)
+            for nb in ((full, small, 0) if name == "fwd" else (full, small)):
+                say("direct convolution", case, name, "workspace", nb, "infinite", infinite)
+                args = {"fwd": (dx_.p, dw_.p, db_.p), "bwd_data": (ddy.p, dw_.p), "bwd_filter": (dx_.p, ddy.p)}[name]
+                gpu.call("mnv_conv_" + name, *args, out.p, *p, ws.p if nb else None, ctypes.c_size_t(nb))
+                got = gpu.down(out).reshape(ref.shape)
+                assert np.array_equal(np.isnan(got), np.isnan(ref)), (name, nb)
+                inf = np.isinf(ref)
+                assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf] > 0, ref[inf] > 0), (name, nb)
+                ok = np.isfinite(ref)
+                assert (np.abs(got[ok] - ref[ok]) <= tol[ok]).all(), (name, nb, float(np.max(np.abs(got[ok] - ref[ok]) / tol[ok])))
+    finally:
+        gpu.L.mnv_conv_winograd_mode(mode)
