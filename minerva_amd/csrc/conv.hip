@@ -268,6 +268,66 @@ struct ConvFwdNP {
   }
 };
 
+// The same with the filter's rows cut into groups of four taps, for filters whose rows are a multiple
+// of four taps long or one short of it (11: 12 slots for 11 taps): a vector is then four neighbouring
+// pixels and four neighbouring filter values, one 16-byte load (4-byte aligned) each, where the
+// flat order's vectors straddle filter rows and take a 4-byte load per pixel.  The order of the
+// slots of a group is that of the pixels, against that of the taps.  A row's last group ends with the
+// row as well and so begins with a tap that the group before it has: its slot 3 reads as 0 in both operands.
+// The table holds, for every group, the pixel's and the filter's byte offset, bit 0 of the first
+// marking a last group with a slot to clear.  3 -> 96 channels under 11 x 11 at stride 4 on 256 x 227 x
+// 227: 555 us with the fp32 instruction, 537 in parts in the flat order, 498 so.
+struct ConvFwdRows : ConvFwdNP {
+  static constexpr int B_NOFF = 1;
+  int groups, per_row;  // C * R * per_row, ceil(S / 4); K, total_slabs and spp count the slots
+  MnvFastDiv d_per_row, d_R;
+  struct Res {
+    mnv_rsrc a, b;
+    const unsigned* tab;  // LDS: [total_slabs * 4][2]
+  };
+  static bool takes(int S) { return S >= 4 && (S % 4 == 0 || (S % 4 == 3 && S >= 7)); }
+  __device__ void make_res(Res& r) const {
+    r.a = mnv_make_rsrc(bottom, (unsigned)(g.N * g.C * g.HW) * 4u);
+    r.b = mnv_make_rsrc(filter, (unsigned)(g.K * g.CRS) * 4u);
+    r.tab = nullptr;
+  }
+  size_t extra_lds_bytes() const { return (size_t)total_slabs * 8 * sizeof(unsigned); }
+  __device__ void block_init(Res& r, float* extra, int, int) const {
+    unsigned* tab = reinterpret_cast<unsigned*>(extra);
+    r.tab = tab;
+    for (int i = threadIdx.x; i < total_slabs * 4; i += blockDim.x) {
+      const int row = mnv_fastdiv(i, d_per_row), q = i - row * per_row;  // filter row (c, r'), group in it
+      const int c = mnv_fastdiv(row, d_R), rp = row - c * g.R;
+      const int first = q == per_row - 1 ? g.S - 4 : 4 * q;            // the group's first tap s'
+      const unsigned pixel = (unsigned)(c * g.HW + (g.R - 1 - rp) * g.W + g.S - 4 - first) * 4u;
+      tab[2 * i] = i < groups ? pixel | (first != 4 * q ? 1u : 0u) : MNV_OOB;
+      tab[2 * i + 1] = i < groups ? (unsigned)(row * g.S + first) * 4u : MNV_OOB;
+    }
+  }
+  __device__ void a_init(const Res&, AState&, int) const {}
+  __device__ void b_init(const Res&, BState&, int) const {}
+  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[1], int period, int s, int kl,
+                         float (&v)[4]) const {
+    const unsigned t = r.tab[2 * ((period * spp + s) * 4 + (kl >> 2))];
+    const unsigned one[1] = {off[0] + (t & ~1u)};
+    mnv_fetch_vec<1>(r.a, one, 0, v);
+    v[3] = t & 1u ? 0.f : v[3];
+  }
+  __device__ void b_period(const BState&, unsigned (&off)[1], int n, int, int) const {
+    off[0] = n < N ? (unsigned)(n * g.CRS) * 4u : MNV_OOB;
+  }
+  __device__ void b_load(const Res& r, const BState&, const unsigned (&off)[1], int period, int s, int kl,
+                         float (&v)[4]) const {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 t = *reinterpret_cast<const u2*>(__builtin_assume_aligned(r.tab + 2 * ((period * spp + s) * 4 + (kl >> 2)), 8));
+    const unsigned one[1] = {(off[0] | t.y) & MNV_OOB ? MNV_OOB : off[0] + t.y};
+    float f[4];
+    mnv_fetch_vec<1>(r.b, one, 0, f);
+    v[0] = f[3]; v[1] = f[2]; v[2] = f[1];
+    v[3] = t.x & 1u ? 0.f : f[0];
+  }
+};
+
 // ------------------------------------------------------------ backward data
 // FAST additionally means both strides are 1, so every (row, col) of the shifted window
 // is a real output position.
@@ -819,12 +879,13 @@ int wide_tile(int n) {
 // From 0.7 GFLOP on where the estimate is below that of the fp32 tiles: a step of 32 k takes 1.6 us
 // on SplitOne, 1.7 on Split96 alone on its CU and 1.26 of the CU's time beside another; about 3 for
 // a workgroup's first loads and last stores, 4 for the reduction of the k ranges beside its bytes; the
-// fp32 instruction 115 TFLOP/s on the large tiles, 80 and 11 us on 64 x 64.
+// fp32 instruction 115 TFLOP/s on the large tiles where a CU has four of them or more (fewer as
+// in mnv_pick_splits), 80 and 11 us on 64 x 64.
 // us with the filter's permutation, fp32 instruction -> bf16 parts, forward: 96 -> 256 under 5 x 5 on 27 x 27,
 // 1 / 2 / 10 / 64 images 27 -> 25 / 41 -> 32 / 123 -> 77 / 523 -> 415; 384 -> 384 under 3 x 3 on
 // 13 x 13, 2 / 10 images 31 -> 28 / 70 -> 48; 128 -> 256 on 32 x 56 x 56 547 -> 430, stride 2 188 -> 164;
 // 256 -> 256 under 1 x 1 on 16 x 28 x 28 33 -> 24; 3 -> 96 under 11 x 11, stride 4, 227 x 227, 10 / 256
-// images 40 -> 38 / 572 -> 537; data gradients: 96 <- 256 of 10 images 131 -> 84, 256 <- 384 54 -> 40.
+// images 39 -> 35 / 555 -> 498; 64 -> 128 under 3 x 3, no padding, on 32 x 28 x 28 57 -> 35; data gradients: 96 <- 256 of 10 images 131 -> 84, 256 <- 384 54 -> 40.
 // Left: 256 -> 384 of one image (0.3 GFLOP) 19 -> 21, 64 -> 128 under 1 x 1, stride 2 (0.2) 9.5 -> 10.3.
 int split_ranges(int m, int n, int slabs, int tile, size_t ws_floats) {
   const double flop = 2.0 * m * n * slabs * 16.0;
@@ -833,7 +894,9 @@ int split_ranges(int m, int n, int slabs, int tile, size_t ws_floats) {
   const long long tiles = (long long)((m + 127) / 128) * (narrow ? (n + 95) / 96 : (n + 127) / 128);
   const long long cus = mnv_cu_count();
   const size_t fit = ws_floats / ((size_t)m * n);
-  double best = tile == 0 ? flop / 80e6 + 11.0 : flop / 115e6;
+  static const double rate[5] = {1.0, 0.45, 0.75, 0.92, 1.0};
+  const long long resident = (tiles + cus - 1) / cus;
+  double best = tile == 0 ? flop / 80e6 + 11.0 : flop / 115e6 / rate[resident < 4 ? resident : 4];
   best *= 0.95;
   int z_best = 0;
   for (int z = 1; z <= 32; ++z) {
@@ -851,12 +914,16 @@ int split_ranges(int m, int n, int slabs, int tile, size_t ws_floats) {
   return z_best;
 }
 
+template <class P>
+int launch_parts(const P& p, int z, void* ws, hipStream_t s, size_t ws_bytes) {
+  return wide_tile(p.N) == 2 ? mnv_gemm_launch<Split96>(p, z, ws, s, ws_bytes)
+                             : mnv_gemm_launch<SplitOne>(p, z, ws, s, ws_bytes);
+}
 // Forward and data gradient: in bf16 parts or, with `splits` k ranges, on the fp32 tile.
 template <class P>
 int launch_direct(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t ws_bytes) {
   if (const int z = split_ranges(p.M, p.N, p.total_slabs, tile, ws_bytes / sizeof(float)))
-    return wide_tile(p.N) == 2 ? mnv_gemm_launch<Split96>(p, z, ws, s, ws_bytes)
-                               : mnv_gemm_launch<SplitOne>(p, z, ws, s, ws_bytes);
+    return launch_parts(p, z, ws, s, ws_bytes);
   return launch_tile(tile, p, splits, ws, s, ws_bytes);
 }
 
@@ -1026,6 +1093,20 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
   }
   if (np) {
     ConvFwdNP p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, gk >= 16 ? gk / 16 : 1, relu};
+    // four taps of a filter row at a time where its rows divide so
+    const size_t part_bytes = part ? workspace_bytes - used : 0;
+    const int z = split_ranges(gm, gn, p.total_slabs, tile, part_bytes / sizeof(float));
+    if (z && ConvFwdRows::takes(S)) {
+      ConvFwdRows q{};
+      static_cast<ConvFwdNP&>(q) = p;
+      q.per_row = (S + 3) / 4;
+      q.groups = C * R * q.per_row;
+      q.K = 4 * q.groups;
+      q.total_slabs = q.spp = (q.groups + 3) / 4;
+      q.d_per_row = mnv_fastdiv_make(q.per_row);
+      q.d_R = mnv_fastdiv_make(R);
+      return launch_parts(q, z, part, s, part_bytes);
+    }
     return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
   }
   ConvFwd<false> p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, 1, relu};

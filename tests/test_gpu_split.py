@@ -206,6 +206,8 @@ DIRECT = [  # N, C, K, H, W, pad, stride, filter
     (3, 48, 130, 57, 55, 1, 1, 3),     # an odd number of slabs, two columns in the last tile
     (9, 16, 200, 41, 43, 0, 1, 3),     # one slab per tap, no padding
     (12, 3, 96, 131, 127, 0, 4, 11),   # the channels of an image, every k its own gather
+    (6, 7, 70, 83, 85, 0, 1, 8),       # whole groups of four taps; 96-column tiles
+    (5, 9, 130, 77, 80, 0, 2, 7),      # one tap short of them, an odd number of channels
     (8, 400, 136, 33, 33, 0, 1, 1),
     (8, 64, 192, 61, 59, 1, 2, 3),     # 96-column tiles
     (1, 256, 80, 70, 67, 1, 1, 3),     # one image, a tile that is not full
