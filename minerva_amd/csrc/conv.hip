@@ -34,14 +34,16 @@ __device__ __forceinline__ int unpack_x(int p) { return (int)(short)(p & 0xffff)
 // Every policy comes in two addressing flavours (see the contract in gemm_core.h):
 //   FAST   : the reduction index is ordered (filter tap, channel) and a period is one tap,
 //            so the im2col offsets and their bounds tests are computed once per tap and a
-//            slab of 16 channels only advances a uniform scalar offset.  Needs the channel
-//            count of the reduction to be a multiple of 16 (and unit stride for the data
-//            gradient).
+//            slab of 16 channels only advances a uniform scalar offset.  Takes the channels
+//            of the reduction 16 at a time (and unit stride for the data gradient); PAD: their
+//            count is no multiple of 16, the permuted filter is padded with zeros to one and
+//            the missing channels of the last slab of a tap read as 0 too (not as the next
+//            image, whose infinities the zeros would turn into NaN).
 //   generic: the reduction index is the flat (channel, tap) order, one period per slab.
 // The two orders only differ in the order the products are summed.
 
 // ------------------------------------------------------------------ forward
-template <bool FAST>
+template <bool FAST, bool PAD = false>
 struct ConvFwd {
   static constexpr bool A_KFAST = false, B_KFAST = true;
   static constexpr int A_NOFF = 4, B_NOFF = FAST ? 1 : 4;
@@ -61,7 +63,7 @@ struct ConvFwd {
   struct BState {};
   __device__ void make_res(Res& r) const {
     r.a = mnv_make_rsrc(bottom, (unsigned)(g.N * g.C * g.HW) * 4u);
-    r.b = mnv_make_rsrc(filter, (unsigned)(g.K * g.CRS) * 4u);
+    r.b = mnv_make_rsrc(filter, (unsigned)(FAST ? N * g.RS * spp * 16 : g.K * g.CRS) * 4u);
   }
   __device__ void a_init(const Res& res, AState& st, int m) const {
 #pragma unroll
@@ -100,19 +102,26 @@ struct ConvFwd {
       off[q] = ok ? (unsigned)(st.off[q] + koff) * 4u : MNV_OOB;
     }
   }
-  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[4], int, int s, int,
+  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[4], int, int s, int kl,
                          float (&v)[4]) const {
-    mnv_fetch_vec<4>(r.a, off, FAST ? (unsigned)s * 16u * (unsigned)g.HW * 4u : 0u, v);
+    const unsigned slab = FAST ? (unsigned)s * 16u * (unsigned)g.HW * 4u : 0u;
+    if (PAD) {
+      const bool ok = s * 16 + kl < g.C;
+      const unsigned in[4] = {ok ? off[0] : MNV_OOB, ok ? off[1] : MNV_OOB, ok ? off[2] : MNV_OOB, ok ? off[3] : MNV_OOB};
+      mnv_fetch_vec<4>(r.a, in, slab, v);
+    } else {
+      mnv_fetch_vec<4>(r.a, off, slab, v);
+    }
   }
   size_t extra_lds_bytes() const { return 0; }
   __device__ void block_init(Res&, float*, int, int) const {}
   // generic: `filter` is the caller's tensor [n][c][r'][s'], element (k, n) at n*CRS + k.
-  // FAST: `filter` is the permuted copy [n][r's'][c], so the 4 channels of a vector are
+  // FAST: `filter` is the permuted copy [n][r's'][c, padded to 16], so the 4 channels of a vector are
   // one 16-byte load and consecutive slabs are consecutive memory.
   __device__ void b_period(const BState&, unsigned (&off)[B_NOFF], int n, int kl,
                            int period) const {
     if (FAST) {
-      off[0] = (n < N) ? (unsigned)(n * g.CRS + period * g.C + kl) * 4u : MNV_OOB;
+      off[0] = (n < N) ? (unsigned)((n * g.RS + period) * spp * 16 + kl) * 4u : MNV_OOB;
     } else {
 #pragma unroll
       for (int q = 0; q < B_NOFF; ++q) {
@@ -331,7 +340,7 @@ struct ConvFwdRows : ConvFwdNP {
 // ------------------------------------------------------------ backward data
 // FAST additionally means both strides are 1, so every (row, col) of the shifted window
 // is a real output position.
-template <bool FAST>
+template <bool FAST, bool PAD = false>
 struct ConvBwdData {
   static constexpr bool A_KFAST = false, B_KFAST = true;
   static constexpr int A_NOFF = 4, B_NOFF = FAST ? 1 : 4;
@@ -352,7 +361,7 @@ struct ConvBwdData {
   struct BState {};
   __device__ void make_res(Res& r) const {
     r.a = mnv_make_rsrc(top_diff, (unsigned)(g.N * g.K * g.HoWo) * 4u);
-    r.b = mnv_make_rsrc(filter, (unsigned)(g.K * g.CRS) * 4u);
+    r.b = mnv_make_rsrc(filter, (unsigned)(FAST ? N * g.RS * spp * 16 : g.K * g.CRS) * 4u);
   }
   __device__ void a_init(const Res& res, AState& st, int m) const {
 #pragma unroll
@@ -397,17 +406,24 @@ struct ConvBwdData {
       }
     }
   }
-  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[4], int, int s, int,
+  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[4], int, int s, int kl,
                          float (&v)[4]) const {
-    mnv_fetch_vec<4>(r.a, off, FAST ? (unsigned)s * 16u * (unsigned)g.HoWo * 4u : 0u, v);
+    const unsigned slab = FAST ? (unsigned)s * 16u * (unsigned)g.HoWo * 4u : 0u;
+    if (PAD) {
+      const bool ok = s * 16 + kl < g.K;
+      const unsigned in[4] = {ok ? off[0] : MNV_OOB, ok ? off[1] : MNV_OOB, ok ? off[2] : MNV_OOB, ok ? off[3] : MNV_OOB};
+      mnv_fetch_vec<4>(r.a, in, slab, v);
+    } else {
+      mnv_fetch_vec<4>(r.a, off, slab, v);
+    }
   }
   size_t extra_lds_bytes() const { return 0; }
   __device__ void block_init(Res&, float*, int, int) const {}
-  // B[kk, c] = filter[ko, c, r', s'].  FAST reads the permuted copy [c][r's'][ko].
+  // B[kk, c] = filter[ko, c, r', s'].  FAST reads the permuted copy [c][r's'][ko, padded to 16].
   __device__ void b_period(const BState&, unsigned (&off)[B_NOFF], int n, int kl,
                            int period) const {
     if (FAST) {
-      off[0] = (n < N) ? (unsigned)((n * g.RS + period) * g.K + kl) * 4u : MNV_OOB;
+      off[0] = (n < N) ? (unsigned)((n * g.RS + period) * spp * 16 + kl) * 4u : MNV_OOB;
     } else {
       int k = period * 16 + kl;
       int ko = mnv_fastdiv(k, g.d_RS);
@@ -730,33 +746,26 @@ struct ConvBwdFilterFast {
   }
 };
 
-// Filter permutations for the FAST policies (a few MB at most, one pass):
+// Filter permutations for the FAST policies (a few MB at most, one pass); the last dimension is
+// padded with zeros to `width`:
 //   to_rsc: out[k][r's'][c] = in[k][c][r's']      (forward)
 //   to_crk: out[c][r's'][k] = in[k][c][r's']      (data gradient)
 __global__ __launch_bounds__(256) void mnv_filter_permute_kernel(const float* __restrict__ in,
                                                                  float* __restrict__ out, int K,
-                                                                 int C, int RS, bool to_crk) {
-  const int total = K * C * RS;
+                                                                 int C, int RS, int width, bool to_crk) {
+  const int total = (to_crk ? C : K) * RS * width;
   for (int o = blockIdx.x * 256 + threadIdx.x; o < total; o += gridDim.x * 256) {
-    int k, c, rs;
-    if (to_crk) {
-      k = o % K;
-      rs = (o / K) % RS;
-      c = o / (K * RS);
-    } else {
-      c = o % C;
-      rs = (o / C) % RS;
-      k = o / (C * RS);
-    }
-    out[o] = in[(k * C + c) * RS + rs];
+    const int last = o % width, rs = (o / width) % RS, first = o / (width * RS);
+    const int k = to_crk ? last : first, c = to_crk ? first : last;
+    out[o] = last < (to_crk ? K : C) ? in[(k * C + c) * RS + rs] : 0.f;
   }
 }
 
-int permute_filter(const float* in, float* out, int K, int C, int RS, bool to_crk, hipStream_t s) {
-  int total = K * C * RS;
+int permute_filter(const float* in, float* out, int K, int C, int RS, int width, bool to_crk, hipStream_t s) {
+  int total = (to_crk ? C : K) * RS * width;
   int blocks = (total + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(mnv_filter_permute_kernel, dim3(blocks), dim3(256), 0, s, in, out, K, C, RS,
+  hipLaunchKernelGGL(mnv_filter_permute_kernel, dim3(blocks), dim3(256), 0, s, in, out, K, C, RS, width,
                      to_crk);
   return MNV_LAUNCH_STATUS();
 }
@@ -1008,6 +1017,35 @@ int small_tile_splits(int tile, int m, int n, int slabs, size_t ws_floats) {
 // (when the fast policy applies) first, then, 256-byte aligned, the partial results.
 size_t align256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
+// The reduction's channel count as the FAST policies take it, a multiple of 16, or 0 where the
+// generic ones are to be used; `others` x RS x channels is the permuted filter.  Padding pays where it
+// adds up to 60%, or any amount within one slab: data gradients of 64 x 28 x 28 under 3 x 3, generic -> padded, 20
+// channels 35 -> 30 us, 8 15.1 -> 14.3, but 17 26 -> 29.
+int fast_channels(int channels, int others, int RS) {
+  const int width = (channels + 15) / 16 * 16;
+  const bool pays = width == 16 ? channels >= 8 : 5 * width <= 8 * channels;
+  return pays && (long long)others * RS * width <= (1LL << 29) - 1 ? width : 0;
+}
+// the no-padding policy reads the filter where it is; for a small problem the extra launch that
+// permutes the filter for the fast policy would cost more than it gains
+bool unpadded_table(const ConvGeom& g) { return g.ph == 0 && g.pw == 0 && g.CRS <= 4096; }
+// Forward, channels padded: only in bf16 parts, the generic gathers are as fast on the fp32
+// instruction.  200 -> 200 channels under 3 x 3 on 16 x 14 x 14 61 -> 34 us, 64 x 28 x 28 470 -> 380, under 5 x 5 on
+// 16 x 28 x 28 629 -> 214; without parts 24 -> 24 on 64 x 28 x 28 31 -> 33, 8 -> 8 10 -> 15.
+int fwd_channels(const ConvGeom& g) {
+  const int m = g.N * g.HoWo, tile = pick_tile(m, g.K);
+  const bool off = g.C % 16 != 0;
+  if (unpadded_table(g) && (tile == 0 || tile == 3 || off)) return 0;
+  const int width = fast_channels(g.C, g.K, g.RS);
+  return off && width && !split_ranges(m, g.K, g.RS * (width / 16), tile, (size_t)-1) ? 0 : width;
+}
+// Data gradient: the generic gathers also divide by the strides and lose at every size.  200 <- 200
+// channels under 3 x 3 on 16 x 14 x 14 65 -> 34 us, 64 x 28 x 28 612 -> 375, under 5 x 5 on 16 x 28 x 28 838 -> 216;
+// 40 <- 40 on 16 x 14 x 14 16.2 -> 13.7.
+int bwd_data_channels(const ConvGeom& g) {
+  return g.sv == 1 && g.sh == 1 ? fast_channels(g.K, g.C, g.RS) : 0;
+}
+
 // k ranges of the filter gradient: up to 256, and up to 512 for outputs of at most 16384
 // elements, whose partial results cost next to nothing (the MNIST CNN's filters: its step
 // 0.28 -> 0.25 ms; conv1 of the AlexNet shape with 341 ranges instead of 255: 0.50 -> 0.54 ms).
@@ -1041,13 +1079,14 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
                                    int sh, int R, int S) {
   ConvGeom g;
   if (make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S)) return 0;
-  const size_t permuted = C % 16 == 0 ? (size_t)K * g.CRS * sizeof(float) : 0;
-  const int gm = N * g.HoWo, gn = K;
-  const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, (g.CRS + 15) / 16, (size_t)-1);
-  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, (g.CRS + 15) / 16);
+  const int width = fwd_channels(g);
+  const size_t permuted = (size_t)K * g.RS * width * sizeof(float);
+  const int gm = N * g.HoWo, gn = K, slabs = width ? g.RS * (width / 16) : (g.CRS + 15) / 16;
+  const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, slabs, (size_t)-1);
+  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs);
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
-  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, (g.CRS + 15) / 16);
+  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);
   if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
   if (mnv_wino_images(N, C, K, H, W, ph, pw, R, S, sv, sh, (size_t)-1)) {
     const size_t w = mnv_wino_workspace_bytes(N, C, K, H, W, ph, pw, R);
@@ -1073,23 +1112,27 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
     return mnv_wino_conv(bottom, filter, bias, nullptr, top, N, C, K, H, W, ph, pw, R, 0, relu, images,
                          workspace, workspace_bytes, s);
   const int tile = pick_tile(gm, gn);
-  const size_t permuted_bytes = (size_t)K * g.CRS * sizeof(float);
-  // the no-padding policy reads the filter where it is; for a small problem the extra
-  // launch that permutes the filter for the fast policy would cost more than it gains
-  const bool np = ph == 0 && pw == 0 && gk <= 4096;
-  const bool fast = C % 16 == 0 && workspace && workspace_bytes >= permuted_bytes &&
-                    !(np && (tile == 0 || tile == 3));
+  int width = fwd_channels(g);
+  const size_t permuted_bytes = (size_t)K * g.RS * width * sizeof(float);
+  const bool np = unpadded_table(g);
+  if (!workspace || workspace_bytes < permuted_bytes) width = 0;
+  const bool fast = width != 0;
   // what is left of the workspace after the permuted filter holds the partial results
   const size_t used = fast ? align256(permuted_bytes) : 0;
   float* part = workspace && workspace_bytes > used ? reinterpret_cast<float*>(static_cast<char*>(workspace) + used) : nullptr;
-  const int splits = small_tile_splits(tile, gm, gn, (gk + 15) / 16,
+  const int splits = small_tile_splits(tile, gm, gn, fast ? g.RS * (width / 16) : (gk + 15) / 16,
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wp = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wp, K, C, g.RS, false, s);
+    rc = permute_filter(filter, wp, K, C, g.RS, width, false, s);
     if (rc) return rc;
-    ConvFwd<true> p{bottom, wp, bias, top, g, gm, gn, gk, g.RS * (C / 16), C / 16, relu};
-    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    const int spp = width / 16;
+    const size_t part_bytes = part ? workspace_bytes - used : 0;
+    if (width != C)
+      return launch_direct(tile, ConvFwd<true, true>{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}, splits,
+                           part, s, part_bytes);
+    return launch_direct(tile, ConvFwd<true>{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}, splits, part, s,
+                         part_bytes);
   }
   if (np) {
     ConvFwdNP p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, gk >= 16 ? gk / 16 : 1, relu};
@@ -1151,13 +1194,14 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
                                         int sv, int sh, int R, int S) {
   ConvGeom g;
   if (make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S)) return 0;
-  const size_t permuted = (sv == 1 && sh == 1 && K % 16 == 0) ? (size_t)K * g.CRS * sizeof(float) : 0;
-  const int gm = N * g.HW, gn = C;
-  const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, (K * g.RS + 15) / 16, (size_t)-1);
-  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, (K * g.RS + 15) / 16);
+  const int width = bwd_data_channels(g);
+  const size_t permuted = (size_t)C * g.RS * width * sizeof(float);
+  const int gm = N * g.HW, gn = C, slabs = width ? g.RS * (width / 16) : (K * g.RS + 15) / 16;
+  const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, slabs, (size_t)-1);
+  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs);
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
-  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, (K * g.RS + 15) / 16);
+  const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);
   if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
   if (mnv_wino_images(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R, S, sv, sh, (size_t)-1)) {
     const size_t w = mnv_wino_workspace_bytes(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R);
@@ -1182,18 +1226,24 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
     return mnv_wino_conv(top_diff, filter, nullptr, gate, bottom_diff, N, K, C, g.Ho, g.Wo, R - 1 - ph,
                          S - 1 - pw, R, 1, 0, images, workspace, workspace_bytes, s);
   const int tile = pick_tile(gm, gn);
-  const size_t permuted_bytes = (size_t)K * g.CRS * sizeof(float);
-  const bool fast = sv == 1 && sh == 1 && K % 16 == 0 && workspace && workspace_bytes >= permuted_bytes;
+  const int width = bwd_data_channels(g);
+  const size_t permuted_bytes = (size_t)C * g.RS * width * sizeof(float);
+  const bool fast = width && workspace && workspace_bytes >= permuted_bytes;
   const size_t used = fast ? align256(permuted_bytes) : 0;
   float* part = workspace && workspace_bytes > used ? reinterpret_cast<float*>(static_cast<char*>(workspace) + used) : nullptr;
-  const int splits = small_tile_splits(tile, gm, gn, (gk + 15) / 16,
+  const int splits = small_tile_splits(tile, gm, gn, fast ? g.RS * (width / 16) : (gk + 15) / 16,
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wq = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wq, K, C, g.RS, true, s);
+    rc = permute_filter(filter, wq, K, C, g.RS, width, true, s);
     if (rc) return rc;
-    ConvBwdData<true> p{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * (K / 16), K / 16, gate};
-    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    const int spp = width / 16;
+    const size_t part_bytes = part ? workspace_bytes - used : 0;
+    if (width != K)
+      return launch_direct(tile, ConvBwdData<true, true>{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate},
+                           splits, part, s, part_bytes);
+    return launch_direct(tile, ConvBwdData<true>{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate}, splits,
+                         part, s, part_bytes);
   }
   ConvBwdData<false> p{top_diff, filter, bottom_diff, g, gm, gn, gk, (gk + 15) / 16, 1, gate};
   return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);

@@ -282,3 +282,56 @@ def test_direct_convolutions_in_parts_against_float64(gpu, case, infinite):
                 assert (np.abs(got[ok] - ref[ok]) <= tol[ok]).all(), (name, nb, float(np.max(np.abs(got[ok] - ref[ok]) / tol[ok])))
     finally:
         gpu.L.mnv_conv_winograd_mode(mode)
+
+
+CHANNELS = [  # N, C, K, H, W, pad, stride, filter: channels of the reduction 16 at a time, the last ones padded
+    (2, 8, 9, 7, 7, 1, 1, 3),         # half of a slab; 128 x 32 tiles with k ranges
+    (3, 17, 24, 12, 11, 1, 1, 3),     # one channel in the last slab
+    (3, 15, 31, 9, 20, 1, 2, 3),      # one short of a slab; strided, the data gradient by the generic gathers
+    (2, 40, 88, 33, 31, 2, 1, 5),     # 64 x 64 tiles
+    (3, 72, 136, 57, 50, 1, 1, 3),    # in parts
+    (3, 104, 200, 40, 41, 0, 1, 3),   # no padding: 96-column tiles in the data gradient
+]
+
+
+@pytest.mark.parametrize("case", CHANNELS, ids=lambda c: "x".join(map(str, c)))
+def test_channels_off_the_multiples_of_16(gpu, case):
+    """Forward and data gradient with all of the workspace, with just the permuted filter's, and with one
+    byte less.  The last image is all infinities: it must not reach the images before it, whose
+    missing channels lie where its first ones are."""
+    N, C, K, H, W, pad, st, R = case
+    p = (N, C, K, H, W, pad, pad, st, st, R, R)
+    Ho, Wo = (H + 2 * pad - R) // st + 1, (W + 2 * pad - R) // st + 1
+    rng = np.random.default_rng(sum(case))
+    x, w, b, dy = (rng.standard_normal(s).astype(np.float32) for s in ((N, C, H, W), (K, C, R, R), (K,), (N, K, Ho, Wo)))
+    x[N - 1], dy[N - 1] = np.inf, np.inf
+    conv, m = torch.nn.functional, N - 1
+    x64, w64, dy64 = (torch.from_numpy(v).double() for v in (x[:m], w.copy(), dy[:m]))
+
+    def passes(x, w, dy):
+        dx = conv.conv_transpose2d(dy, w.flip(2, 3), None, st, pad, ((H + 2 * pad - R) % st, (W + 2 * pad - R) % st))
+        return conv.conv2d(x, w.flip(2, 3), None, st, pad).numpy(), dx.numpy()
+
+    want, size = passes(x64, w64, dy64), passes(x64.abs(), w64.abs(), dy64.abs())
+    want = want[0] + b.astype(np.float64)[None, :, None, None], want[1]
+    assert want[0].shape == (m, K, Ho, Wo) and want[1].shape == (m, C, H, W)
+    # one rounding per k at most, those of the k ranges, the bias
+    bound = [(k * R * R + 64) * 2.0 ** -23 * v + 1e-6 for k, v in zip((C, K), size)]
+    d = {n: gpu.up(np.ascontiguousarray(v).reshape(-1)) for n, v in (("x", x), ("w", w), ("b", b), ("dy", dy))}
+    mode = gpu.L.mnv_conv_winograd_mode(0)
+    try:
+        for name, args, ref, tol, count, inner in (("fwd", ("x", "w", "b"), want[0], bound[0], K, C),
+                                                   ("bwd_data", ("dy", "w"), want[1], bound[1], C, K)):
+            full = getattr(gpu.L, "mnv_conv_%s_workspace_bytes" % name)(*p)
+            permuted = count * R * R * ((inner + 15) // 16 * 16) * 4
+            per_image = ref[0].size
+            for nb in (full, permuted, permuted - 1):
+                say("channels off 16", case, name, "workspace", nb)
+                out, ws = gpu.up(np.full(N * per_image + 4, np.float32(7.5), np.float32)), gpu.empty(max(full, nb) // 4 + 1)
+                gpu.call("mnv_conv_" + name, *[d[a].p for a in args], out.p, *p, ws.p, ctypes.c_size_t(nb))
+                got = gpu.down(out)
+                assert (got[N * per_image:] == 7.5).all(), "wrote past the result"
+                got = got[:m * per_image].reshape(ref.shape)
+                assert (np.abs(got - ref) <= tol).all(), (name, nb, float(np.nanmax(np.abs(got - ref) / tol)))
+    finally:
+        gpu.L.mnv_conv_winograd_mode(mode)
