@@ -11,8 +11,9 @@ shapes under one name and only the grid tells them apart.
       per run), plus, where their counters are present, the derived columns
         cycles     = GRBM_GUI_ACTIVE / 8                        (the counter sums the eight XCDs)
         MFMA busy  = SQ_VALU_MFMA_BUSY_CYCLES / (cycles * SIMDs) (one v_mfma_f32_32x32x2_f32 holds
-                                                                  the pipe 64 cycles)
-        other VALU = (SQ_INSTS_VALU - SQ_VALU_MFMA_BUSY_CYCLES / 64) * 4 / (cycles * SIMDs)
+                                                                  the pipe 64 cycles, one
+                                                                  v_mfma_f32_16x16x32_bf16 16)
+        other VALU = (SQ_INSTS_VALU - SQ_VALU_MFMA_BUSY_CYCLES / 64 or 16) * 4 / (cycles * SIMDs)
         waves/SIMD = SQ_WAVE_CYCLES * 4 / (cycles * SIMDs)        (the counter ticks every 4 cycles)
         waiting    = SQ_WAIT_INST_ANY / SQ_WAVE_CYCLES            (share of a wavefront's life spent
                                                                   waiting for an instruction to issue)
@@ -34,6 +35,7 @@ SIMDS = 256 * 4  # MI355X: 256 CUs x 4 SIMDs
 def short(name):
     name = re.sub(r"\(anonymous namespace\)::", "", name)
     name = re.sub(r"MnvGemmTile<(\d+), (\d+), (\d+), \d+, \d+, \d+, (\d+)>", r"T\1x\4x\3", name)
+    name = re.sub(r"MnvSplitTile<(\d+), \d+, \d+, \d+, (\d+), (\d+)>", r"Parts\1x\3b\2", name)  # in bf16 parts
     name = re.sub(r"^void ", "", name)
     return re.sub(r"\(.*$", "", name)
 
@@ -123,7 +125,8 @@ def counter_table(rows, trace=None, min_cycles=20000, show=None):
             elif name == "MFMA busy":
                 cells.append("%11.1f%%" % (100 * d.get("SQ_VALU_MFMA_BUSY_CYCLES", 0) / (cyc * SIMDS)))
             elif name == "other VALU":
-                other = d.get("SQ_INSTS_VALU", 0) - d.get("SQ_VALU_MFMA_BUSY_CYCLES", 0) / 64.0
+                per = 16.0 if "Parts" in k else 64.0
+                other = d.get("SQ_INSTS_VALU", 0) - d.get("SQ_VALU_MFMA_BUSY_CYCLES", 0) / per
                 cells.append("%11.1f%%" % (100 * other * 4.0 / (cyc * SIMDS)))
             elif name == "waves/SIMD":
                 cells.append("%12.2f" % (d.get("SQ_WAVE_CYCLES", 0) * 4.0 / (cyc * SIMDS)))
