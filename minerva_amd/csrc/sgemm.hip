@@ -392,6 +392,7 @@ struct SgemmPlan {
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
   bool split = false; // 128 x 128 and 256 x 128 tiles: in bf16 parts
+  int lend = 0;       // k ranges that the caller is to lend a workspace for, where more than `splits`
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
 };
 
@@ -481,8 +482,14 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* p
       best_z = z;
     }
   }
-  if (plan->small && best > 0.9 * 0.83 * cost) return;
+  // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
+  // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6).
+  if (plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
+  // with less than the 64 x 64 tiles' k ranges want the comparison above would be with another plan
+  // (978 x 1316 x 3098: 93 us became 108)
+  const int lend = best_z > 1 ? plan->splits : 0;
   *plan = SgemmPlan{false, best_z};
+  plan->lend = lend;
   plan->split = true;
 }
 
@@ -707,7 +714,8 @@ extern "C" {
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   const SgemmPlan plan = plan_sgemm(m, n, k, (size_t)-1);
-  return plan.splits > 1 ? (size_t)plan.splits * m * n * sizeof(float) : sgemm_tail_bytes(plan, m, n, k);
+  const int ranges = plan.lend > plan.splits ? plan.lend : plan.splits;
+  return ranges > 1 ? (size_t)ranges * m * n * sizeof(float) : sgemm_tail_bytes(plan, m, n, k);
 }
 
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,
