@@ -159,7 +159,8 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * partial results reduced by a second kernel (1: none); groups is otherwise 4 when a workgroup
  * has a CU to itself: four wavefront groups that share a 64 x 64 tile and add their quarters of the
  * k range through LDS, or the eight wavefronts of a 128 x 128 tile.  The plan depends on (m, n, k,
- * workspace_bytes) only, never on the operands.
+ * workspace_bytes) only, never on the operands.  mnv_sgemm_nn_workspace_bytes is what the partial
+ * results of the plan of an unlimited workspace need, so that lending it gives that plan.
  * Tiles of 128 and 256 rows (groups 1, and 4 with 128) multiply on the bf16 matrix cores, every fp32
  * value in three bf16 parts: the error against exact arithmetic is that of fp32 sums with fewer
  * roundings, about 0.4 times that of one fused multiply-add per k; infinities, NaN and values

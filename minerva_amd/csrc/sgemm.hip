@@ -392,7 +392,6 @@ struct SgemmPlan {
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
   bool split = false; // 128 x 128 and 256 x 128 tiles: in bf16 parts
-  int lend = 0;       // k ranges that the caller is to lend a workspace for, where more than `splits`
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
 };
 
@@ -485,15 +484,12 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* p
   // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
   // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6).
   if (plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
-  // with less than the 64 x 64 tiles' k ranges want the comparison above would be with another plan
-  // (978 x 1316 x 3098: 93 us became 108)
-  const int lend = best_z > 1 ? plan->splits : 0;
   *plan = SgemmPlan{false, best_z};
-  plan->lend = lend;
   plan->split = true;
 }
 
-SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
+// The cheapest of the plans whose partial results fit `ws_floats`.
+SgemmPlan plan_within(int m, int n, int k, size_t ws_floats) {
   const int slabs = (k + 15) / 16;
   const size_t mn = (size_t)m * n;
   const double per_split = 8.0 * (double)mn / 6e6 / 1.2;
@@ -563,6 +559,30 @@ SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   }
   plan_split(m, n, k, ws_floats, best_cost, &best);
   return best;
+}
+
+// The plan of an unlimited workspace.  A plan of the fp32 instruction is planned again within what its
+// own partial results need, until that changes nothing: alternatives with more k ranges have
+// then lost them (0.1% of products of random extents change).  One in bf16 parts stands, it won against the
+// best that the others can be.
+SgemmPlan plan_unlimited(int m, int n, int k) {
+  SgemmPlan plan = plan_within(m, n, k, (size_t)-1);
+  while (!plan.split) {
+    const SgemmPlan next = plan_within(m, n, k, plan.splits > 1 ? (size_t)plan.splits * m * n : 0);
+    const bool same = next.split == plan.split && next.small == plan.small && next.splits == plan.splits && next.groups == plan.groups;
+    plan = next;
+    if (same) break;
+  }
+  return plan;
+}
+
+// The plan of an unlimited workspace wherever its own partial results fit, so that the bytes the
+// query asks for give the plan that the query was made for.  Planned within those bytes
+// instead, the plans that lost against it would have fewer k ranges, one of them would win, and 1500 x
+// 1500 x 1501 would stay on grouped 64 x 64 tiles (72 us with a large workspace, 88 with the queried one).
+SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
+  const SgemmPlan plan = plan_unlimited(m, n, k);
+  return plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n) ? plan : plan_within(m, n, k, ws_floats);
 }
 
 template <int NC, bool TB, class P>
@@ -713,9 +733,8 @@ extern "C" {
 
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  const SgemmPlan plan = plan_sgemm(m, n, k, (size_t)-1);
-  const int ranges = plan.lend > plan.splits ? plan.lend : plan.splits;
-  return ranges > 1 ? (size_t)ranges * m * n * sizeof(float) : sgemm_tail_bytes(plan, m, n, k);
+  const SgemmPlan plan = plan_unlimited(m, n, k);
+  return plan.splits > 1 ? (size_t)plan.splits * m * n * sizeof(float) : sgemm_tail_bytes(plan, m, n, k);
 }
 
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,

@@ -1,6 +1,7 @@
-"""Which kernel a product of at most 12 columns takes: host arithmetic on the extents and the
-workspace alone, so checked without a GPU."""
+"""Which kernel a product takes, those of at most 12 columns above all: host arithmetic on the extents
+and the workspace alone, so checked without a GPU."""
 import ctypes
+import random
 
 import pytest
 
@@ -58,3 +59,33 @@ def test_few_columns_with_less_workspace():
         assert not _few(plan) or plan[1] <= have
     for m, few in ((127 * 256, False), (127 * 256 + 1, True)):  # 128 row blocks: one range, no workspace
         assert _few(_plan(m, 1, 1000, 0)) == few and _plan(m, 1, 1000, 0)[1] == 1
+
+
+def _extents(count):
+    rng = random.Random(6)
+    span = lambda low, high: int(low * (high / low) ** rng.random())
+    return [(span(16, 4097), span(16, 4097), span(32, 4097)) for _ in range(count)]
+
+
+NAMED = [  # planned with k ranges on the large tiles by one of the two instructions and without by the other
+    (3530, 2630, 3872), (2921, 3395, 3933), (3372, 3896, 3982), (1500, 1500, 1501), (978, 1316, 3098), (9216, 256, 4096),
+]
+
+
+def test_the_queried_workspace_gives_the_plan_of_an_unlimited_one():
+    """A caller that lends what the query asks for gets the plan that the query was made for, and the
+    query asks for the partial results of that plan and no more."""
+    for m, n, k in NAMED + _extents(6000):
+        ws, most = _query(m, n, k), _plan(m, n, k, 1 << 40)
+        assert _plan(m, n, k, ws) == most, (m, n, k, ws)
+        slabs = -(-k // 16)
+        if most[1] > 1 and not _few(most):  # the launch rounds the planned ranges to equal ones
+            planned = ws // (4 * m * n)
+            assert ws == planned * 4 * m * n and -(-slabs // -(-slabs // planned)) == most[1], (m, n, k, ws)
+
+
+def test_a_plan_without_k_ranges_needs_no_workspace():
+    for m, n, k in NAMED + _extents(6000):
+        most = _plan(m, n, k, 1 << 40)
+        if most[1] == 1:
+            assert _plan(m, n, k, 0) == most, (m, n, k)
