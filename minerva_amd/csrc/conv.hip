@@ -867,15 +867,6 @@ int launch_filter_gradient(int tile, const P& p, int splits, void* ws, size_t ws
   return launch_tile(tile, p, splits, ws, s);
 }
 
-// Bytes the large tiles' launches want for the partial tiles of a cut tail (0: no tail).
-size_t tail_workspace_bytes(int tile, int m, int n, int slabs) {
-  if (tile != 1 && tile != 2) return 0;
-  const long long tiles = (long long)((m + kTileM[tile] - 1) / kTileM[tile]) * ((n + kTileN[tile] - 1) / kTileN[tile]);
-  const size_t tile_floats = (size_t)kTileM[tile] * kTileN[tile];
-  const MnvTailPlan t = mnv_tail_plan(tiles, slabs, tile_floats, (size_t)-1 / sizeof(float));
-  return t.z > 1 ? (size_t)(tiles - t.begin) * t.z * tile_floats * sizeof(float) : 0;
-}
-
 // 128-row tiles: 96 columns wide when that leaves clearly fewer idle columns than 128
 // (an output 96 or 192 wide), since the narrower tile does a little less work per byte
 // staged.
@@ -934,6 +925,19 @@ int launch_direct(int tile, const P& p, int splits, void* ws, hipStream_t s, siz
   if (const int z = split_ranges(p.M, p.N, p.total_slabs, tile, ws_bytes / sizeof(float)))
     return launch_parts(p, z, ws, s, ws_bytes);
   return launch_tile(tile, p, splits, ws, s, ws_bytes);
+}
+
+// Bytes the large tiles' launches want for the partial tiles of a cut tail (0: no tail); `parts`: the
+// policy is one that launch_direct takes.
+size_t tail_workspace_bytes(int tile, int m, int n, int slabs, bool parts) {
+  if (tile != 1 && tile != 2) return 0;
+  const int z = parts ? split_ranges(m, n, slabs, tile, (size_t)-1) : 0;
+  if (z > 1) return 0;
+  const long long tiles = (long long)((m + kTileM[tile] - 1) / kTileM[tile]) * ((n + kTileN[tile] - 1) / kTileN[tile]);
+  const size_t tile_floats = (size_t)kTileM[tile] * kTileN[tile];
+  const MnvTailPlan t = mnv_tail_plan(tiles, slabs, tile_floats, (size_t)-1 / sizeof(float),
+                                      !z ? MnvTailCost{} : tile == 2 ? Split96::TAIL : SplitOne::TAIL);
+  return t.z > 1 ? (size_t)(tiles - t.begin) * t.z * tile_floats * sizeof(float) : 0;
 }
 
 // Bytes of the k ranges' partial results in bf16 parts.
@@ -1083,7 +1087,7 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
   const size_t permuted = (size_t)K * g.RS * width * sizeof(float);
   const int gm = N * g.HoWo, gn = K, slabs = width ? g.RS * (width / 16) : (g.CRS + 15) / 16;
   const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, slabs, (size_t)-1);
-  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs);
+  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs, width || unpadded_table(g));
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
   const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);
@@ -1198,7 +1202,7 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
   const size_t permuted = (size_t)C * g.RS * width * sizeof(float);
   const int gm = N * g.HW, gn = C, slabs = width ? g.RS * (width / 16) : (K * g.RS + 15) / 16;
   const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, slabs, (size_t)-1);
-  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs);
+  const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs, width);
   size_t need = tail ? align256(permuted) + tail
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
   const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);

@@ -178,14 +178,21 @@ template <class P>
 struct MnvCPreload<P, std::enable_if_t<P::C_PRELOAD>> {
   static constexpr bool value = true;
 };
+// What mnv_tail_plan prices a cut tail with, in us of a CU's time: a slab of a workgroup, and its first
+// loads and last stores.  slab 0: not priced.
+struct MnvTailCost {
+  double slab = 0.0, start = 0.0;
+};
 // Tiles of the bf16 matrix cores (MnvSplitTile, gemm_split.h); the launches below take either kind.
 template <class T, class = void>
 struct MnvIsSplit {
   static constexpr bool value = false;
+  static constexpr MnvTailCost tail{};
 };
 template <class T>
 struct MnvIsSplit<T, std::enable_if_t<T::SPLIT>> {
   static constexpr bool value = true;
+  static constexpr MnvTailCost tail = T::TAIL;
 };
 template <class T, class P, bool SK>
 __global__ void mnv_gemm_split_kernel(P prob, int tiles_m, int tiles_n, int slabs_per_split, float* __restrict__ partial,
@@ -916,11 +923,17 @@ __global__ __launch_bounds__(256) void mnv_gemm_streamk_reduce_kernel(P prob,
 // with about three small workgroups per CU (two to four measured alike: conv2 data gradient
 // 1.77 -> 1.74 / 1.71 / 1.70 ms, conv5 forward 0.71 -> 0.66 ms with any of them), at least
 // eight slabs each, and only as far as the workspace holds the partial tiles.
+// A kernel with one or two workgroups per CU whose slabs take half the time gains less and pays the
+// same for it: there the cut is priced (`cost`), with 2 us for the second launch and 0.46 us per MB
+// of partial tiles for writing and reading them (fitted to 264 products and 34 convolutions, of which 4 lose
+// more than 2% by the cut and 5 more than 3% without it).  In bf16 parts, uncut -> cut, us: 3909 x 1954 x 260 (496
+// tiles) 31 -> 49, 2716 x 2401 x 242 27 -> 39, 2307 x 3549 x 528 (532) 72 -> 59; convolutions, 352 -> 208 channels under 1 x 1
+// on 30 x 47 x 22 52 -> 64, data gradient 280 <- 232 under 3 x 3 on 51 x 30 x 30 451 -> 372.
 struct MnvTailPlan {
   int begin, z;
 };
 static inline MnvTailPlan mnv_tail_plan(long long tiles, int slabs, size_t tile_floats,
-                                        size_t ws_floats) {
+                                        size_t ws_floats, const MnvTailCost& cost = MnvTailCost{}) {
   const int cus = mnv_cu_count();
   const MnvTailPlan none{(int)(tiles < 0x7fffffff ? tiles : 0x7fffffff), 1};
   if (tiles < cus || tiles > 0x3fffffff) return none;
@@ -934,6 +947,11 @@ static inline MnvTailPlan mnv_tail_plan(long long tiles, int slabs, size_t tile_
   const size_t fit = ws_floats / ((size_t)rem * tile_floats);
   if ((size_t)z > fit) z = (int)fit;
   if (z < 2) return none;
+  if (cost.slab > 0.0) {
+    const int parts = (rem * z + cus - 1) / cus, len = (slabs + z - 1) / z;  // of the fullest CU, for one more tile
+    const double partial_mb = 1e-6 * sizeof(float) * (double)rem * z * (double)tile_floats;
+    if (cost.slab * (parts * len - slabs) + cost.start * (parts - 1) + 2.0 + 0.46 * partial_mb >= 0.0) return none;
+  }
   return MnvTailPlan{(int)(tiles - rem), z};
 }
 
@@ -1009,7 +1027,7 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
   MnvTailPlan tail{tiles_m * tiles_n, 1};
   if (G == 1 && splits == 1 && (T::MIN_WAVES == 4 || MnvIsSplit<T>::value) && workspace && tail_bytes)
     tail = mnv_tail_plan((long long)tiles_m * tiles_n, total_slabs, (size_t)T::BM * T::BNU,
-                         tail_bytes / sizeof(float));
+                         tail_bytes / sizeof(float), MnvIsSplit<T>::tail);
   const int tail_tiles = tiles_m * tiles_n - tail.begin;
   hipLaunchKernelGGL(kernel, dim3(tail.begin + tail_tiles * tail.z, 1, splits), dim3(T::NT * G), lds_bytes,
                      s, prob, tiles_m, tiles_n, per, reinterpret_cast<float*>(workspace),

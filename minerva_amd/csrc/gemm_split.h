@@ -63,6 +63,8 @@ struct MnvSplitTile {
   static constexpr int A_BYTES = 3 * plane(BM), B_BYTES = 3 * plane(BN), BUF_BYTES = A_BYTES + B_BYTES;
   static constexpr size_t lds_bytes(bool, bool) { return (size_t)BUFS * BUF_BYTES; }
   static constexpr int MIN_WAVES = NT / 256 * (3 - BUFS);  // per SIMD
+  // One workgroup per CU as the gathers of the convolutions run on it, two on 96 and 128 columns (see mnv_tail_plan).
+  static constexpr MnvTailCost TAIL = BUFS == 2 ? MnvTailCost{0.8, 3.0} : BNU == 96 ? MnvTailCost{1.1, 1.5} : MnvTailCost{0.72, 1.5};
   static_assert(TM == 4 && WM % 16 == 0 && WN % 16 == 0 && BM % 64 == 0 && BN % 32 == 0, "four blocks of rows per wavefront");
 };
 

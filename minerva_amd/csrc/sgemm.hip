@@ -646,7 +646,8 @@ size_t sgemm_tail_bytes(const SgemmPlan& plan, int m, int n, int k) {
   if (plan.splits != 1 || plan.groups != 1 || plan.tall) return 0;
   const int bm = plan.small ? 64 : 128;
   const long long tiles = (long long)((m + bm - 1) / bm) * ((n + bm - 1) / bm);
-  const MnvTailPlan t = mnv_tail_plan(tiles, (k + 15) / 16, (size_t)bm * bm, (size_t)-1 / sizeof(float));
+  const MnvTailPlan t = mnv_tail_plan(tiles, (k + 15) / 16, (size_t)bm * bm, (size_t)-1 / sizeof(float),
+                                      plan.split ? SplitPair::TAIL : MnvTailCost{});
   return t.z > 1 ? (size_t)(tiles - t.begin) * t.z * bm * bm * sizeof(float) : 0;
 }
 

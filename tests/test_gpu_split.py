@@ -64,6 +64,7 @@ SHAPES = [  # m, n, k: what the tile, the k step (32), the slab (16) and the pla
     (1793, 2047, 1001),    # one workgroup per CU
     (200, 3000, 4001),     # k ranges
     (4095, 4096, 515),     # 256 x 128 tiles
+    (2307, 3549, 530),     # the tiles past two per CU cut into k ranges
 ]
 
 

@@ -89,3 +89,13 @@ def test_a_plan_without_k_ranges_needs_no_workspace():
         most = _plan(m, n, k, 1 << 40)
         if most[1] == 1:
             assert _plan(m, n, k, 0) == most, (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,cut", [
+    (3909, 1954, 260, False), (2716, 2401, 242, False),  # two tiles per CU, short k: all at once
+    (2307, 3549, 528, True), (3530, 2630, 3872, True),   # a few tiles more than that
+    (1298, 4851, 1634, False), (4096, 4096, 256, False), # many parts of long ranges; nothing left over
+])
+def test_products_in_parts_cut_their_tail_where_the_partial_tiles_cost_less(m, n, k, cut):
+    assert _plan(m, n, k, 1 << 40) == (128, 1, 1)
+    assert (_query(m, n, k) > 0) == cut
