@@ -1072,7 +1072,7 @@ int bwd_filter_splits(int m, int n, int k, size_t ws_floats) {
   if (max_splits > slabs / 8) max_splits = slabs / 8;
   size_t fit = ws_floats / ((size_t)m * n);
   if ((size_t)max_splits > fit) max_splits = (int)fit;
-  return mnv_pick_splits(tiles, slabs, max_splits);
+  return mnv_pick_splits(tiles, slabs, max_splits, mnv_cu_count());
 }
 
 }  // namespace

@@ -964,10 +964,9 @@ static inline MnvTailPlan mnv_tail_plan(long long tiles, int slabs, size_t tile_
 // `per_split` (optional) is what every additional k range costs for writing and re-reading
 // its partial result, in the same unit (one slab of one workgroup); `cost_out` receives the
 // estimate of the chosen count so that callers can compare tile shapes.
-static inline int mnv_pick_splits(long long tiles, int slabs, int max_splits, double per_split = 0.0,
+static inline int mnv_pick_splits(long long tiles, int slabs, int max_splits, int cus, double per_split = 0.0,
                                   double* cost_out = nullptr) {
   static const double rate[5] = {1.0, 0.45, 0.75, 0.92, 1.0};
-  const int cus = mnv_cu_count();
   if (max_splits < 1) max_splits = 1;
   int best = 1;
   double best_cost = 0;

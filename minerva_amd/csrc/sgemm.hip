@@ -443,9 +443,9 @@ bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
 // 1.13 where a CU has one workgroup (SplitOne), 1.3 of the CU's time for each where it has several
 // (SplitPair); about 3 for a workgroup's first loads and last stores, 4 for the reduction of
 // the k ranges beside its bytes.
-double split_cost(int m, int n, int k, int z) {
+double split_cost(int m, int n, int k, int z, int cus) {
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
-  const long long per_cu = (tiles * z + mnv_cu_count() - 1) / mnv_cu_count();
+  const long long per_cu = (tiles * z + cus - 1) / cus;
   const int slabs = (k + 15) / 16, steps = ((slabs + z - 1) / z + 1) / 2;
   const double work = per_cu == 1 ? 1.13 * steps + 3.0 : 1.3 * per_cu * steps + 3.0 * (double)((per_cu + 1) / 2);
   return work + (z > 1 ? 4.0 + 8.0 * (double)m * n * z / 6e6 : 0.0);
@@ -463,7 +463,7 @@ double split_cost(int m, int n, int k, int z) {
 //   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
 //   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
 //   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0
-void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* plan) {
+void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {
   if (plan->tall || (!plan->small && plan->groups == 4)) {
     plan->split = true;
     return;
@@ -473,9 +473,9 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* p
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
   int best_z = 1;
-  double best = split_cost(m, n, k, 1);
-  for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * mnv_cu_count(); ++z) {
-    const double c = split_cost(m, n, k, z);
+  double best = split_cost(m, n, k, 1, cus);
+  for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus; ++z) {
+    const double c = split_cost(m, n, k, z, cus);
     if (c < 0.97 * best) {
       best = c;
       best_z = z;
@@ -488,8 +488,9 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, SgemmPlan* p
   plan->split = true;
 }
 
-// The cheapest of the plans whose partial results fit `ws_floats`.
-SgemmPlan plan_within(int m, int n, int k, size_t ws_floats) {
+// The cheapest of the plans whose partial results fit `ws_floats`.  `cus`: the device's, asked for once per
+// call, since the query takes about 0.05 us and the plans below weigh some fifty launches.
+SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
   const int slabs = (k + 15) / 16;
   const size_t mn = (size_t)m * n;
   const double per_split = 8.0 * (double)mn / 6e6 / 1.2;
@@ -503,10 +504,10 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats) {
     if (max_splits > slabs / 4) max_splits = slabs / 4;
     const size_t fit = mn ? ws_floats / mn : 0;
     if ((size_t)max_splits > fit) max_splits = (int)fit;
-    if (tiles >= 4LL * mnv_cu_count() || slabs < 8) max_splits = 1;  // one per resident workgroup
+    if (tiles >= 4LL * cus || slabs < 8) max_splits = 1;  // one per resident workgroup
     const double unit = small ? 0.31 : 1.0;
     double cost;
-    const int splits = mnv_pick_splits(tiles, slabs, max_splits, per_split / unit, &cost);
+    const int splits = mnv_pick_splits(tiles, slabs, max_splits, cus, per_split / unit, &cost);
     cost *= unit;
     const bool forced = small ? (m <= 64 || n <= 64) : false;
     if (small == 0 || forced || cost < best_cost) {
@@ -554,10 +555,10 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats) {
   // over k in the same order as on the 128 x 128 tile: the same bits.
   if (!best.small && best.splits == 1 && best.groups == 1 && m >= 256 && slabs >= 32) {
     const long long tiles = (long long)((m + 255) / 256) * ((n + 127) / 128);
-    const long long slots = 2LL * mnv_cu_count(), rounds = (tiles + slots - 1) / slots;
+    const long long slots = 2LL * cus, rounds = (tiles + slots - 1) / slots;
     if ((double)m * n >= 0.95 * (double)(rounds * slots) * 256.0 * 128.0) best.tall = true;
   }
-  plan_split(m, n, k, ws_floats, best_cost, &best);
+  plan_split(m, n, k, ws_floats, best_cost, cus, &best);
   return best;
 }
 
@@ -565,10 +566,10 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats) {
 // own partial results need, until that changes nothing: alternatives with more k ranges have
 // then lost them (0.1% of products of random extents change).  One in bf16 parts stands, it won against the
 // best that the others can be.
-SgemmPlan plan_unlimited(int m, int n, int k) {
-  SgemmPlan plan = plan_within(m, n, k, (size_t)-1);
+SgemmPlan plan_unlimited(int m, int n, int k, int cus) {
+  SgemmPlan plan = plan_within(m, n, k, (size_t)-1, cus);
   while (!plan.split) {
-    const SgemmPlan next = plan_within(m, n, k, plan.splits > 1 ? (size_t)plan.splits * m * n : 0);
+    const SgemmPlan next = plan_within(m, n, k, plan.splits > 1 ? (size_t)plan.splits * m * n : 0, cus);
     const bool same = next.split == plan.split && next.small == plan.small && next.splits == plan.splits && next.groups == plan.groups;
     plan = next;
     if (same) break;
@@ -581,8 +582,9 @@ SgemmPlan plan_unlimited(int m, int n, int k) {
 // instead, the plans that lost against it would have fewer k ranges, one of them would win, and 1500 x
 // 1500 x 1501 would stay on grouped 64 x 64 tiles (72 us with a large workspace, 88 with the queried one).
 SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
-  const SgemmPlan plan = plan_unlimited(m, n, k);
-  return plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n) ? plan : plan_within(m, n, k, ws_floats);
+  const int cus = mnv_cu_count();
+  const SgemmPlan plan = plan_unlimited(m, n, k, cus);
+  return plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n) ? plan : plan_within(m, n, k, ws_floats, cus);
 }
 
 template <int NC, bool TB, class P>
@@ -734,7 +736,7 @@ extern "C" {
 
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  const SgemmPlan plan = plan_unlimited(m, n, k);
+  const SgemmPlan plan = plan_unlimited(m, n, k, mnv_cu_count());
   return plan.splits > 1 ? (size_t)plan.splits * m * n * sizeof(float) : sgemm_tail_bytes(plan, m, n, k);
 }
 
