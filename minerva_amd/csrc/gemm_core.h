@@ -111,10 +111,11 @@ struct MnvFetchMap {
 //        tid / 16 + 16 j.  a_init is called once, for row tid / 16, and
 //   void a_load_lanek(const Res&, const AState&, int period, int s, int kl, float (&v)[AV][4]) const;
 //        loads element j (row tid / 16 + 16 j, k = kl) into v[j / 4][j % 4]; a_period is unused
-//   optional, for a right operand whose loads may fetch values that must read as 0 and that are
+//   optional, for an operand whose loads may fetch values that must read as 0 and that are
 //   cheaper to clear once they have arrived: static constexpr bool B_STASH_FIX = true;
 //   void b_stash_fix(int period, int s, int kl, float (&v)[4]) const;   called on every vector of
 //        slab s of that period right before the vector is written to LDS
+//   (A_STASH_FIX and a_stash_fix likewise)
 //   optional, for an output whose m direction is contiguous in memory:
 //   static constexpr bool C_STORE4 = true;
 //   void c_store4(int m, int n, const float (&v)[4]) const;   the elements (m .. m + 3, n); m is a
@@ -151,6 +152,14 @@ struct MnvBStashFix {
 };
 template <class P>
 struct MnvBStashFix<P, std::enable_if_t<P::B_STASH_FIX>> {
+  static constexpr bool value = true;
+};
+template <class P, class = void>
+struct MnvAStashFix {
+  static constexpr bool value = false;
+};
+template <class P>
+struct MnvAStashFix<P, std::enable_if_t<P::A_STASH_FIX>> {
   static constexpr bool value = true;
 };
 #define MNV_STORE4_MAX_SLABS 64
@@ -462,6 +471,11 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
     constexpr int set = decltype(SET)::value;
     float* a = As + buf * ATILE;
     float* bb = Bs + buf * BTILE;
+    static_assert(!LK || !MnvAStashFix<P>::value, "vectors of one k per lane");
+    if constexpr (MnvAStashFix<P>::value) {
+#pragma unroll
+      for (int p = 0; p < T::AV; ++p) prob.a_stash_fix(period_of_set[set], s_of_set[set], MapA::k(tid, p), ra[set][p]);
+    }
     if constexpr (MnvBStashFix<P>::value) {
 #pragma unroll
       for (int p = 0; p < T::BV; ++p) prob.b_stash_fix(period_of_set[set], s_of_set[set], MapB::k(tid, p), rb[set][p]);

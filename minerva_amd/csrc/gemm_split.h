@@ -177,6 +177,7 @@ __device__ __forceinline__ void mnv_split_redo(const P& prob, const typename P::
         float v[4];
         prob.a_period(st, off, m, kl, period);
         prob.a_load(res, st, off, period, s, kl, v);
+        if constexpr (MnvAStashFix<P>::value) prob.a_stash_fix(period, s, kl, v);
         if (P::A_KFAST) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) av[i][q] = v[q];
@@ -338,6 +339,11 @@ __global__ __launch_bounds__(T::NT, T::MIN_WAVES) void mnv_gemm_split_kernel(P p
       held_scale = live ? MNV_SPLIT_SCALE : 0.f;
     };
     auto stash_a = [&](int at, int from, int to) {
+      if constexpr (MnvAStashFix<P>::value) {
+        static_assert(P::A_KFAST, "pieces are vectors");
+#pragma unroll
+        for (int p = from; p < to; ++p) prob.a_stash_fix(held_period, held_s, MapA::k(g, p), ra[p]);
+      }
       MapA::stash(mnv_split_lds + at, g, sub, held_scale, ra, from, to);
     };
     auto stash_b = [&](int at) {

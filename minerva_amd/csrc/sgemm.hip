@@ -30,16 +30,18 @@ namespace {
 //  x-fast: a vector that reaches past the last row (column) brings values of the next one;
 //    they are summed into accumulators that are never stored.
 //  k-fast: a vector that reaches past K brings values that would be summed.  K4 (K % 4 == 0):
-//    there is none.  Otherwise B's vectors of the last, partial slab are cleared past K on
-//    their way to LDS (b_stash_fix: a uniform branch per slab; an infinity there times the
-//    other operand's 0 would not be 0), and a transposed A keeps four 4-byte loads.
+//    there is none.  Otherwise the vectors of the last, partial slab are cleared past K on
+//    their way to LDS (a_stash_fix, b_stash_fix: a uniform branch per slab; an infinity there
+//    times the other operand's 0 would not be 0).
 // Four 4-byte loads per vector, which odd extents took before, keep four times as many
 // load instructions in a slab: 1001 x 250 x 4099 41.0 -> 28.5 us, 4099 x 4099 x 1023
-// 292 -> 272, 10 x 256 x 256 9.4 -> 7.3; the same bits.
+// 292 -> 272, 10 x 256 x 256 9.4 -> 7.3; the same bits.  A transposed, in bf16 parts, where they also
+// spill into the loop: 2230 x 2410 x 1302 173 -> 108 us, 2675 x 3691 x 237 64 -> 42 (fp32
+// instruction 155 and 55).
 template <bool K4, bool TA = false, bool TB = false>
 struct SgemmNN {
   static constexpr bool A_KFAST = TA, B_KFAST = !TB;
-  static constexpr int A_NOFF = TA && !K4 ? 4 : 1, B_NOFF = 1;
+  static constexpr int A_NOFF = 1, B_NOFF = 1;
   const float* __restrict__ A;
   const float* __restrict__ B;
   float* __restrict__ C;
@@ -83,7 +85,7 @@ struct SgemmNN {
     if (TA) {
       const unsigned base = ((unsigned)m * (unsigned)lda + (unsigned)k) * 4u;
 #pragma unroll
-      for (int q = 0; q < A_NOFF; ++q) off[q] = ((m < M) & (k + q < K)) ? base + 4u * q : MNV_OOB;
+      for (int q = 0; q < A_NOFF; ++q) off[q] = ((m < M) & (k < K)) ? base + 4u * q : MNV_OOB;
     } else {
       const unsigned base = ((unsigned)k * (unsigned)lda + (unsigned)m) * 4u;
 #pragma unroll
@@ -111,7 +113,8 @@ struct SgemmNN {
                          int, float (&v)[4]) const {
     mnv_fetch_vec<B_NOFF>(r.b, off, (unsigned)s * (unsigned)bk * (TB ? (unsigned)ldb : 1u) * 4u, v);
   }
-  static constexpr bool B_STASH_FIX = !K4 && !TB;
+  static constexpr bool A_STASH_FIX = !K4 && TA, B_STASH_FIX = !K4 && !TB;
+  __device__ void a_stash_fix(int period, int s, int kl, float (&v)[4]) const { b_stash_fix(period, s, kl, v); }
   __device__ void b_stash_fix(int period, int, int kl, float (&v)[4]) const {
     if (period == (K >= bk ? 1 : 0)) {  // the partial slab
       const int rest = K % bk;

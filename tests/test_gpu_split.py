@@ -113,6 +113,20 @@ def test_products_in_parts_next_to_values_without_parts(gpu, m, n, k):
         assert (np.abs(c[fin] - want[fin]) <= bound[fin]).all(), name
 
 
+@pytest.mark.parametrize("m,n,k", [(2561, 2047, 97), (1793, 2047, 1002), (200, 3000, 4003), (257, 300, 145), (70, 90, 3)])
+def test_rows_that_begin_with_infinities(gpu, m, n, k):
+    """With k off the multiples of 4 the last vector of a row of A given transposed (a column of B) runs into
+    the next row (column): what it brings from there must not reach the row's own results."""
+    A, B = _rand((m, k), 61), _rand((n, k), 62)
+    A[1::2, :3], B[1::2, :3] = np.inf, np.nan
+    A64, B64 = A[::2].astype(np.float64), B[::2].astype(np.float64)
+    want, bound = B64 @ A64.T, (k + 8) * 2.0 ** -24 * (np.abs(B64) @ np.abs(A64).T)
+    say("rows that begin with infinities", m, n, k)
+    for name, c in _products(gpu, A, B).items():
+        assert (np.abs(c[::2, ::2] - want) <= bound).all(), name
+        assert np.isnan(c[1::2]).all() and not np.isfinite(c[:, 1::2]).any(), name
+
+
 def test_products_in_parts_of_denormals(gpu):
     """The smallest operands keep all their bits: denormals times values near 1, and normal values whose
     third part would be below the smallest bf16 number but for the scale."""

@@ -1,7 +1,11 @@
 """Which kernel a product takes, those of at most 12 columns above all: host arithmetic on the extents
 and the workspace alone, so checked without a GPU."""
 import ctypes
+import os
 import random
+import re
+import struct
+import subprocess
 import time
 
 import pytest
@@ -115,3 +119,40 @@ def test_weighing_many_launches_costs_little_host_time():
             best = min(best, time.perf_counter() - t)
         return best
     assert min(fastest(256, 256, 784) / fastest(10, 256, 256) for _ in range(3)) <= 2.5
+
+
+def _device_code(path):
+    """The code objects in a library's bundles."""
+    data, magic, at = open(path, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (at := data.find(magic, at)) >= 0:
+        pos = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", data, pos - 8)[0]):
+            offset, size, chars = struct.unpack_from("<QQQ", data, pos)
+            name = data[pos + 24:pos + 24 + chars]
+            pos += 24 + chars
+            if b"gfx950" in name:
+                yield data[at + offset:at + offset + size]
+        at += len(magic)
+
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+def test_products_in_parts_keep_their_loop_in_registers(tmp_path):
+    """Two workgroups per CU leave 128 registers.  The few that do not fit are those of the result's
+    addresses, outside the loop; with a fetch of four loads per vector, which a transposed A of a k off
+    the multiples of 4 once took, there were 17 and the loop waited for them."""
+    found = 0
+    for i, image in enumerate(_device_code(capi.LIB_PATH)):
+        if b"mnv_gemm_split_kernel" not in image or b"SgemmNN" not in image:
+            continue
+        co = tmp_path / ("%d.co" % i)
+        co.write_bytes(image)
+        notes = subprocess.run([READELF, "--notes", str(co)], capture_output=True, text=True, check=True).stdout
+        for kernel in notes.split(".agpr_count")[1:]:
+            name = re.search(r"\.name: +(\S+)", kernel).group(1)
+            if "mnv_gemm_split_kernel" in name and "SgemmNN" in name:
+                found += 1
+                assert int(re.search(r"\.vgpr_spill_count: +(\d+)", kernel).group(1)) <= 8, name
+    assert found == 18  # three tiles, six forms of the operands
