@@ -96,6 +96,14 @@ def test_a_plan_without_k_ranges_needs_no_workspace():
             assert _plan(m, n, k, 0) == most, (m, n, k)
 
 
+@pytest.mark.parametrize("m,n,k", [(307, 270, 143), (78, 382, 127), (2271, 261, 215), (3059, 183, 194), (329, 1452, 164)])
+def test_short_products_stay_on_small_tiles_without_k_ranges(m, n, k):
+    """A few slabs of k: the 64 x 64 tiles without ranges beat those with ranges, which the tiles in parts
+    are weighed against first, and the tiles in parts."""
+    for ws in (0, _query(m, n, k), 1 << 40):
+        assert _plan(m, n, k, ws) == (64, 1, 1)
+
+
 @pytest.mark.parametrize("m,n,k,cut", [
     (3909, 1954, 260, False), (2716, 2401, 242, False),  # two tiles per CU, short k: all at once
     (2307, 3549, 528, True), (3530, 2630, 3872, True),   # a few tiles more than that
