@@ -444,13 +444,15 @@ bool plan_skinny(int m, int n, int k, size_t ws_floats, SgemmPlan* plan) {
 
 // Microseconds of a product on 128 x 128 tiles in bf16 parts with z k ranges: a step of 32 k takes
 // 1.13 where a CU has one workgroup (SplitOne), 1.3 of the CU's time for each where it has several
-// (SplitPair); about 3 for a workgroup's first loads and last stores, 4 for the reduction of
+// (SplitPair); about 3 for a workgroup's first loads and last stores, 4 where up to three steps of
+// a CU's one workgroup leave nothing to hide them behind (2871 x 1047 x 42 8.9 us with the fp32 instruction, 10.3 in parts; of 680 products of 36 to 700 k,
+// 12 lost 7 to 16% to it with 3, 4 with 4, by up to 8%, and 3 gained that much less); 4 for the reduction of
 // the k ranges beside its bytes.
 double split_cost(int m, int n, int k, int z, int cus) {
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
   const long long per_cu = (tiles * z + cus - 1) / cus;
   const int slabs = (k + 15) / 16, steps = ((slabs + z - 1) / z + 1) / 2;
-  const double work = per_cu == 1 ? 1.13 * steps + 3.0 : 1.3 * per_cu * steps + 3.0 * (double)((per_cu + 1) / 2);
+  const double work = per_cu == 1 ? 1.13 * steps + (steps <= 3 ? 4.0 : 3.0) : 1.3 * per_cu * steps + 3.0 * (double)((per_cu + 1) / 2);
   return work + (z > 1 ? 4.0 + 8.0 * (double)m * n * z / 6e6 : 0.0);
 }
 

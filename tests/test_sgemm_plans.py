@@ -104,6 +104,14 @@ def test_short_products_stay_on_small_tiles_without_k_ranges(m, n, k):
         assert _plan(m, n, k, ws) == (64, 1, 1)
 
 
+@pytest.mark.parametrize("m,n,k,rows", [
+    (2871, 1047, 42, 64), (603, 3437, 70, 64), (1519, 1490, 36, 64),     # one workgroup per CU, nothing to overlap
+    (3189, 2290, 49, 128), (2882, 2636, 172, 128), (2015, 1742, 107, 128),
+])
+def test_products_of_few_steps(m, n, k, rows):
+    assert _plan(m, n, k, 0) == (rows, 1, 1)
+
+
 @pytest.mark.parametrize("m,n,k,cut", [
     (3909, 1954, 260, False), (2716, 2401, 242, False),  # two tiles per CU, short k: all at once
     (2307, 3549, 528, True), (3530, 2630, 3872, True),   # a few tiles more than that
