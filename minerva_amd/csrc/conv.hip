@@ -1022,13 +1022,25 @@ int small_tile_splits(int tile, int m, int n, int slabs, size_t ws_floats) {
 size_t align256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
 // The reduction's channel count as the FAST policies take it, a multiple of 16, or 0 where the
-// generic ones are to be used; `others` x RS x channels is the permuted filter.  Padding pays where it
-// adds up to 60%, or any amount within one slab: data gradients of 64 x 28 x 28 under 3 x 3, generic -> padded, 20
-// channels 35 -> 30 us, 8 15.1 -> 14.3, but 17 26 -> 29.
-int fast_channels(int channels, int others, int RS) {
+// generic ones are to be used; `others` x RS x channels is the permuted filter, `rows` those of the product.
+// Padding pays where it adds up to 60%, or up to 100% within one slab (33% on 128 and more of the 64 x 64
+// tiles, which 33 columns and more take): data gradients of 64 x 28 x 28 under 3 x 3, generic -> padded, 20 channels 35 -> 30 us, 8 15.1 -> 14.3,
+// but 17 26 -> 29; 40 <- 8 under 5 x 5 17 -> 21 on 16 x 28 x 28, 13.5 -> 12.5 on 14 x 14, forward 8 -> 88 on 64 x 28 x 28 35 -> 41.
+// Few tiles wait for one slab after the other, 1.5 us for a generic one and 0.65 for a padded one, which has to
+// repay the launch that permutes the filter too (data gradients of 12 channels, 1 to 16 images of 14 x 14 or 28 x 28: under
+// 1 x 1 <- 8, 1 slab each, 5.2 -> 6.4; <- 24, 2, 6.8 -> 6.8; <- 40, 3, 8.3 -> 7.5; under 3 x 3 <- 8, 5 and 9, 11.2 -> 11.7; <- 12,
+// 7 and 9, 14.4 -> 12.2).  With tiles to fill the chip, two per CU, a single slab still does not, two do (312 <- 24
+// on 50 x 23 x 14 24 -> 19).
+int fast_channels(int channels, int others, int RS, long long rows) {
   const int width = (channels + 15) / 16 * 16;
-  const bool pays = width == 16 ? channels >= 8 : 5 * width <= 8 * channels;
-  return pays && (long long)others * RS * width <= (1LL << 29) - 1 ? width : 0;
+  const long long tiles = (rows + 63) / 64 * ((others + 63) / 64);
+  const bool wide = others > 32;
+  if (width == 16 ? channels < (wide && tiles >= 128 ? 12 : 8) : 5 * width > 8 * channels) return 0;
+  if (width != channels) {
+    const long long slabs = ((long long)channels * RS + 15) / 16, padded = (long long)RS * (width / 16);
+    if (tiles < 512 ? 7 * slabs <= 3 * padded + (wide ? 14 : 10) : slabs < 2) return 0;
+  }
+  return (long long)others * RS * width <= (1LL << 29) - 1 ? width : 0;
 }
 // the no-padding policy reads the filter where it is; for a small problem the extra launch that
 // permutes the filter for the fast policy would cost more than it gains
@@ -1040,14 +1052,14 @@ int fwd_channels(const ConvGeom& g) {
   const int m = g.N * g.HoWo, tile = pick_tile(m, g.K);
   const bool off = g.C % 16 != 0;
   if (unpadded_table(g) && (tile == 0 || tile == 3 || off)) return 0;
-  const int width = fast_channels(g.C, g.K, g.RS);
+  const int width = fast_channels(g.C, g.K, g.RS, m);
   return off && width && !split_ranges(m, g.K, g.RS * (width / 16), tile, (size_t)-1) ? 0 : width;
 }
-// Data gradient: the generic gathers also divide by the strides and lose at every size.  200 <- 200
+// Data gradient: the generic gathers also divide by the strides and lose wherever padding pays.  200 <- 200
 // channels under 3 x 3 on 16 x 14 x 14 65 -> 34 us, 64 x 28 x 28 612 -> 375, under 5 x 5 on 16 x 28 x 28 838 -> 216;
 // 40 <- 40 on 16 x 14 x 14 16.2 -> 13.7.
 int bwd_data_channels(const ConvGeom& g) {
-  return g.sv == 1 && g.sh == 1 ? fast_channels(g.K, g.C, g.RS) : 0;
+  return g.sv == 1 && g.sh == 1 ? fast_channels(g.K, g.C, g.RS, (long long)g.N * g.HW) : 0;
 }
 
 // k ranges of the filter gradient: up to 256, and up to 512 for outputs of at most 16384

@@ -1,0 +1,36 @@
+"""Which data gradients and forward passes have their channels padded to the multiples of 16: host
+arithmetic on the extents alone, seen from the workspace that holds the padded filter."""
+import pytest
+
+from minerva_amd import capi
+
+
+def _query(direction, N, C, K, H, W, pad, R):
+    return getattr(capi.lib(), "mnv_conv_%s_workspace_bytes" % direction)(N, C, K, H, W, pad, pad, 1, 1, R, R)
+
+
+@pytest.mark.parametrize("dims,padded", [  # N, C, K, H, W, pad, R; the reduction runs over K
+    ((1, 8, 8, 14, 14, 0, 1), False), ((4, 24, 24, 14, 14, 0, 1), False),     # one and two slabs: the permutation's launch
+    ((64, 8, 12, 28, 28, 0, 1), False),                                       # costs more than they do
+    ((50, 312, 24, 23, 14, 0, 1), True),                                      # or does not, over many tiles
+    ((1, 24, 40, 14, 14, 0, 1), True), ((1, 40, 40, 14, 14, 0, 1), False),    # three slabs; 64 x 64 tiles
+    ((16, 8, 8, 14, 14, 1, 3), False), ((64, 8, 8, 28, 28, 1, 3), True), ((1, 8, 12, 14, 14, 1, 3), True),
+    ((4, 8, 8, 14, 14, 2, 5), True), ((16, 40, 8, 28, 28, 2, 5), False),      # twice the work,
+    ((2, 40, 8, 28, 28, 2, 5), True),                                         # of few tiles
+    ((64, 24, 17, 28, 28, 1, 3), False), ((64, 24, 20, 28, 28, 1, 3), True),
+])
+def test_channels_of_small_data_gradients_are_padded_where_it_pays(dims, padded):
+    N, C, K, H, W, pad, R = dims
+    filter_bytes = 4 * C * R * R * ((K + 15) // 16 * 16)
+    ws = _query("bwd_data", *dims)
+    partial = 4 * N * H * W * C  # what k ranges ask for, in whole results
+    if padded:
+        assert ws >= filter_bytes and (ws - filter_bytes) % partial in (0, (256 - filter_bytes) % 256)
+    else:
+        assert ws % partial == 0
+
+
+@pytest.mark.parametrize("C,padded", [(8, False), (9, False), (12, True), (24, True)])
+def test_channels_of_forward_passes_are_padded_where_it_pays(C, padded):
+    dims = (64, C, 88, 28, 28, 2, 5)
+    assert (_query("fwd", *dims) >= 4 * 88 * 25 * ((C + 15) // 16 * 16)) == padded
