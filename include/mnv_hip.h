@@ -163,8 +163,9 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * results of the plan of an unlimited workspace need, so that lending it gives that plan.
  * Tiles of 128 and 256 rows (groups 1, and 4 with 128) multiply on the bf16 matrix cores, every fp32
  * value in three bf16 parts: the error against exact arithmetic is that of fp32 sums with fewer
- * roundings, about 0.4 times that of one fused multiply-add per k; infinities, NaN and values
- * from 2^111 on give what fp32 arithmetic gives, slower. ---- */
+ * roundings, for dense operands about 0.4 times that of one fused multiply-add per k; a sum of a
+ * single product is within 2^-23 of it (fp32 arithmetic: 2^-24).  Infinities, NaN, values from
+ * 2^111 and running sums from 2^96 on give what fp32 arithmetic gives, slower. ---- */
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k);
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,
                       int* groups);

@@ -1,7 +1,7 @@
-// fp32 products on the bf16 matrix cores of gfx950, no less exact than on the fp32 ones.
+// fp32 products on the bf16 matrix cores of gfx950, with fewer roundings than on the fp32 ones.
 //
-// A value x is cut into three bf16 numbers, x = x1 + x2 + x3 with |x2| <= 2^-9 |x| and
-// |x3| <= 2^-18 |x|; their 3 x 8 significant bits hold all 24 of x.  A product a b is then
+// A value x is cut into three bf16 numbers, x = x1 + x2 + x3 with |x2| <= 2^-8 |x| and
+// |x3| <= 2^-17 |x|; their 3 x 8 significant bits hold all 24 of x.  A product a b is then
 //   a1 b1 + (a1 b2 + a2 b1) + (a1 b3 + a2 b2 + a3 b1)
 // and three terms of at most 2^-25 |a b| each that are left out (with all nine the error against
 // float64 is the same to three digits).  The bf16 matrix instruction multiplies exactly and adds
@@ -12,13 +12,21 @@
 // rounding of the full sum for 8 k.  Error against float64 (2-norm, relative), fp32 instruction /
 // this: k = 32 1.0e-7 / 0.4e-7, 576 4.3e-7 / 1.4e-7, 4096 11.3e-7 / 4.0e-7; with a left operand
 // from a ReLU, whose zeros cost the fp32 sum nothing, 4096 8.3e-7 / 3.2e-7.  (One set of
-// accumulators for all six: 9.9e-7 and 9.6e-7, the second worse than the fp32 instruction.)
+// accumulators for all six: 9.9e-7 and 9.6e-7, the second worse than the fp32 instruction.)  Two kinds of
+// sums gain nothing.  One of a single term (a one-hot or diagonal operand) is within 2^-23 and not
+// 2^-24 of it, for the three terms left out (rms 2.53e-8 / 2.60e-8; 0 and 1 times a value stay exact).  One
+// of positive terms only, where the fp32 kernel had four wavefronts sum a quarter of the k each: uniform
+// operands 4096^3 8.4e-7 / 3.0e-7 (one chain), 2048^3 1.6e-7 / 2.2e-7, 3837 x 2065 x 4394 2.4e-7 / 3.4e-7 (both from a
+// ReLU 1.3e-7 / 3.3e-7).  Folding the sums every 512 k into a third set of accumulators mends half of these
+// (of 70 random extents of uniform operands 21 were worse than the fp32 kernel, and 10 with it): only one workgroup per
+// CU leaves registers for it, and it costs up to 9% (1215 x 1372 x 3540 81 -> 88 us).
 //
 // Range.  Operands are multiplied by 2^16 before the cut, so that the last bit of the smallest
 // denormal is still a bf16 denormal, and the product by 2^-32 after the sum.  An operand from
 // 2^111 on, or an infinity or NaN, makes x2 an infinity or a NaN where fp32 arithmetic may have
-// a finite or an infinite result (inf * 1: 1 = 1 + 0 + 0, and inf * 0 is NaN): a wavefront
-// whose sums are not all finite multiplies its block again with the fp32 instruction.
+// a finite or an infinite result (inf * 1: 1 = 1 + 0 + 0, and inf * 0 is NaN), and a
+// running sum from 2^96 on overflows: a wavefront whose sums are not all finite multiplies its block
+// again with the fp32 instruction.
 //
 // Data path: HBM -> registers (the policies' fetches, gemm_core.h) -> cut -> three bf16 planes
 // in LDS -> v_mfma_f32_16x16x32_bf16.  A step of the main loop is two 16-deep slabs of the

@@ -157,6 +157,25 @@ def test_products_in_parts_are_no_less_exact_than_one_rounding_per_k(gpu):
         assert np.linalg.norm(c[:64] - want) <= 0.6 * ref, name
 
 
+@pytest.mark.parametrize("m,n,k", [(2048, 2048, 96), (1793, 2047, 1001), (4095, 4096, 515)])
+def test_sums_of_one_term(gpu, m, n, k):
+    """A sum whose other terms are zero has no rounding of a running value to gain from.  What is left is
+    that of the result, 2^-24, which the fp32 instruction has too, and the three products of parts that are
+    left out: |second part| <= 2^-8, |third| <= 2^-17 of a value, 2 x 2^-25 and 2^-34 of the product
+    (the sums of the small parts, at 2^-8, add less than 2^-28)."""
+    rng = np.random.default_rng(k)
+    hot, value, B = rng.integers(0, k, m), _rand(m, 43), _rand((n, k), 42)
+    A = np.zeros((m, k), np.float32)
+    A[np.arange(m), hot] = value
+    want = B[:, hot].astype(np.float64) * value.astype(np.float64)
+    say("sums of one term", m, n, k)
+    for name, c in _products(gpu, A, B).items():
+        assert (np.abs(c - want) <= (2.0 ** -23 + 2.0 ** -28) * np.abs(want)).all(), name
+    A[np.arange(m), hot] = 1.0  # 1 = 1 + 0 + 0: times a value, its three parts and their sum
+    for name, c in _products(gpu, A, B).items():
+        assert_bits_equal(c, B[:, hot], name)
+
+
 def test_epilogues_of_products_in_parts(gpu):
     """Bias, ReLU, gate and update on a product in parts have the bits of the separate operators."""
     m, n, k = 2562, 2047, 100
