@@ -63,7 +63,7 @@ SHAPES = [  # m, n, k: what the tile, the k step (32), the slab (16) and the pla
     (2303, 3073, 112),     # the second half of the last step is missing
     (1793, 2047, 1001),    # one workgroup per CU
     (200, 3000, 4001),     # k ranges
-    (4095, 4096, 515),     # 256 x 128 tiles
+    (4095, 4096, 515), (4093, 4095, 514),  # 256 x 128 tiles
     (2307, 3549, 530),     # the tiles past two per CU cut into k ranges
 ]
 
@@ -176,14 +176,14 @@ def test_sums_of_one_term(gpu, m, n, k):
         assert_bits_equal(c, B[:, hot], name)
 
 
-def test_epilogues_of_products_in_parts(gpu):
+@pytest.mark.parametrize("m,n,k,rows", [(2562, 2047, 100, 128), (4094, 4095, 514, 256)])
+def test_epilogues_of_products_in_parts(gpu, m, n, k, rows):
     """Bias, ReLU, gate and update on a product in parts have the bits of the separate operators."""
-    m, n, k = 2562, 2047, 100
     A, B = _rand((m, k), 31), _rand((n, k), 32)
     rng = np.random.default_rng(33)
     bias, gate, w = (rng.standard_normal(s).astype(np.float32) for s in (m, m * n, m * n))
     nb = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
-    assert _plan(gpu, m, n, k, nb)[0] == 128
+    assert _plan(gpu, m, n, k, nb)[0] == rows
     plain = _products(gpu, A, B)["nn"].reshape(-1)
     ws, c = gpu.empty(nb // 4 + 1), gpu.empty(m * n)
     a, b = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(B.reshape(-1))
