@@ -12,7 +12,8 @@
 //   backward filter: C[(c,r',s'), k]    = sum_{(n,i,j)}    gather(bottom) * top_diff   (k range split)
 // In every case the GEMM "m" dimension is the one that is contiguous in the output
 // tensor, so result stores are coalesced, and no im2col buffer exists in HBM.
-// Roofline: fp32 MFMA, 2*N*Ho*Wo*K*C*R*S algorithmic flops per pass.
+// Roofline: 2*N*Ho*Wo*K*C*R*S algorithmic flops per pass, at 157.3 TFLOP/s with the fp32 instruction and 419.4
+// in parts (six bf16 products of 2516.6).
 
 #include "gemm_split.h"
 #include "winograd.h"

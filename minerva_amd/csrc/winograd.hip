@@ -943,8 +943,9 @@ size_t vm_bytes(const WinoGeom& g, int images) {
   const size_t pp = ((size_t)images * g.TH * g.TW + 3) / 4 * 4, points = (size_t)g.al * g.al;
   return align256(points * pp * g.Cin * sizeof(float)) + align256(points * pp * g.Coutp * sizeof(float));
 }
-// partial tiles of the filter gradient's equal-shares launch: at most four workgroups per CU,
-// a partial tile each and one more per output tile
+// partial tiles of the filter gradient's equal-shares launch: a partial tile for each workgroup and one
+// more per output tile.  Room for four workgroups per CU, of which the launch in bf16 parts takes two: the
+// size decides which layers a given workspace holds.
 size_t grad_sk_bytes(const WinoGeom& g) {
   const long long tiles = (long long)((g.Cin + 127) / 128) * (g.al * g.al * g.Coutp / 128);
   return (size_t)(4 * mnv_cu_count() + tiles) * 128 * 128 * sizeof(float);
@@ -987,7 +988,9 @@ bool plan_geom(WinoGeom* g, int* mode_out, int N, int Cin, int Cout, int Hs, int
 //            the products: 157 TFLOP/s x k / (k + 64 slab-equivalents of prologue and store),
 //            k = Cin for forward / data gradient, 0.85 for the filter gradient's long k
 //            (Cin' = Cin rounded up to the 128-row tile there).
-// Checked against the batch-256 layers: 96 -> 256 channels under 5 x 5 filters 0.46 estimated,
+// The rates are those of the fp32 instruction on both sides; in bf16 parts either is faster (products 145
+// TFLOP/s at k = 96 to 384, direct 138 for 96 -> 256 under 5 x 5 on 64 x 27 x 27), and where the line then lies has not
+// been measured.  Checked against the batch-256 layers as they were: 96 -> 256 channels under 5 x 5 filters 0.46 estimated,
 // 0.43 measured; 256 -> 384 under 3 x 3 on 13 x 13 planes 0.65 / 0.63.  Layers of 128 channels
 // and fewer stay direct: the transforms alone cost what the multiplies save.
 bool pays(const WinoGeom& g, int images, bool filter_gradient) {
