@@ -161,7 +161,7 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * k range through LDS, or the eight wavefronts of a 128 x 128 tile.  The plan depends on (m, n, k,
  * workspace_bytes) only, never on the operands.  mnv_sgemm_nn_workspace_bytes is what the partial
  * results of the plan of an unlimited workspace need, so that lending it gives that plan.
- * Tiles of 128 and 256 rows (groups 1, and 4 with 128) multiply on the bf16 matrix cores, every fp32
+ * Tiles of 128 and 256 rows (groups 1, and 4 with 128) multiply on the bf16 matrix cores if k > 16, every fp32
  * value in three bf16 parts: the error against exact arithmetic is that of fp32 sums with fewer
  * roundings, for dense operands about 0.4 times that of one fused multiply-add per k; a sum of a
  * single product is within 2^-23 of it (fp32 arithmetic: 2^-24).  Infinities, NaN, values from

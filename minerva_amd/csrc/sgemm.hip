@@ -378,6 +378,7 @@ SgemmNN<K4, TA, TB> make_sgemm(const float* a, const float* b, float* c, int m, 
 }
 
 typedef MnvGemmTile<64, 64, 16, 2, 2> TileSmall;
+typedef MnvGemmTile<128, 128, 16, 2, 2> TileBig;  // products of one slab (see plan_split)
 // Of the bf16 parts: two workgroups per CU, one, and one with twice the rows.
 typedef MnvSplitTile<128, 128, 2, 4, 1> SplitPair;
 typedef MnvSplitTile<128, 128, 2, 4, 2> SplitOne;
@@ -394,7 +395,7 @@ struct SgemmPlan {
   int splits;
   int groups = 1;  // 4: workgroups of four wavefront groups that share a tile's k range
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
-  bool split = false; // 128 x 128 and 256 x 128 tiles: in bf16 parts
+  bool split = false; // in bf16 parts (256 x 128 tiles always, 128 x 128 ones but for a single slab)
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
 };
 
@@ -474,6 +475,10 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, Sge
     return;
   }
   if (plan->groups == 4 || m <= 64 || n <= 64) return;
+  // One slab fills half of a step, and what such a product takes is the time of its stores, which the fp32 kernel, with
+  // twice the workgroups per CU, spreads better (fp32 instruction / parts, us: k = 16 4096 x 4096 16.4 / 18.9, 4096 x 9216
+  // 30.0 / 33.7, k = 17 20.4 / 18.3, 38.9 / 32.4).  Those planned on 64 x 64 tiles gain as little by parts as they lose.
+  if (k <= 16 && !plan->small) return;
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
@@ -650,7 +655,8 @@ int launch_plan(const SgemmPlan& plan, const P& p, void* workspace, size_t works
   const size_t tail_bytes = plan.splits == 1 && workspace ? workspace_bytes : 0;
   if (plan.split) return launch_split(plan, p, workspace, tail_bytes, s);
   if (plan.groups == 4) return mnv_gemm_launch<TileSmall, 4>(p, plan.splits, workspace, s);
-  return mnv_gemm_launch<TileSmall>(p, plan.splits, workspace, s, tail_bytes);
+  return plan.small ? mnv_gemm_launch<TileSmall>(p, plan.splits, workspace, s, tail_bytes)
+                    : mnv_gemm_launch<TileBig>(p, plan.splits, workspace, s, tail_bytes);
 }
 
 // Bytes a product without k ranges wants for the partial tiles of its cut tail.

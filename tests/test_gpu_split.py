@@ -113,6 +113,22 @@ def test_products_in_parts_next_to_values_without_parts(gpu, m, n, k):
         assert (np.abs(c[fin] - want[fin]) <= bound[fin]).all(), name
 
 
+@pytest.mark.parametrize("m,n,k", [(4093, 4099, 13), (4096, 4096, 16), (4099, 5003, 1)])
+def test_products_of_one_slab_round_as_the_fp32_instruction(gpu, m, n, k):
+    """Up to 16 k the large tiles stay with the fp32 instruction: one rounding per k."""
+    A, B = _rand((m, k), 71), _rand((n, k), 72)
+    assert _plan(gpu, m, n, k, 0) == (128, 1, 1)
+    say("products of one slab", m, n, k)
+    got = _products(gpu, A, B)
+    A64, B64 = A.astype(np.float64), B.astype(np.float64)
+    want, bound = B64 @ A64.T, k * 2.0 ** -24 * (np.abs(B64) @ np.abs(A64).T)
+    for name, c in got.items():
+        assert (np.abs(c - want) <= bound).all(), name
+        assert_bits_equal(c, got["nn"], name)
+        if k == 1:
+            assert_bits_equal(c, np.outer(B, A), name)
+
+
 @pytest.mark.parametrize("m,n,k", [(2561, 2047, 97), (1793, 2047, 1002), (200, 3000, 4003), (257, 300, 145), (70, 90, 3)])
 def test_rows_that_begin_with_infinities(gpu, m, n, k):
     """With k off the multiples of 4 the last vector of a row of A given transposed (a column of B) runs into
