@@ -1024,22 +1024,28 @@ size_t align256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
 // The reduction's channel count as the FAST policies take it, a multiple of 16, or 0 where the
 // generic ones are to be used; `others` x RS x channels is the permuted filter, `rows` those of the product.
-// Padding pays where it adds up to 60%, or up to 100% within one slab (33% on 128 and more of the 64 x 64
-// tiles, which 33 columns and more take): data gradients of 64 x 28 x 28 under 3 x 3, generic -> padded, 20 channels 35 -> 30 us, 8 15.1 -> 14.3,
-// but 17 26 -> 29; 40 <- 8 under 5 x 5 17 -> 21 on 16 x 28 x 28, 13.5 -> 12.5 on 14 x 14, forward 8 -> 88 on 64 x 28 x 28 35 -> 41.
+// Data gradients unless said otherwise, us, generic -> padded.
+// Padding pays where it adds up to 60% (64 x 28 x 28 under 3 x 3, 20 channels 35 -> 30, but 17 26 -> 29), within one
+// slab up to 100% (8 channels 15.1 -> 14.3) while the outputs are at most 32.  On 128 and more of the 64 x 64 tiles that
+// more outputs take it may add 40%, in bf16 parts 60% (10 channels to 200, 16 x 28 x 28 under 3 x 3 25.3 -> 16.5,
+// under 5 x 5 51.6 -> 28.7, but without parts on 16 x 14 x 14 20.8 -> 22.5; 8 to 40 on 16 x 28 x 28 17.2 -> 21.0; forward 8 to 128 on
+// 64 x 28 x 28 46.7 -> 64.8, and in a few sizes that fill one round of the CUs the other way: 8 to 104 on 32 x 28 x 28 43 -> 29).
 // Few tiles wait for one slab after the other, 1.5 us for a generic one and 0.65 for a padded one, which has to
-// repay the launch that permutes the filter too (data gradients of 12 channels, 1 to 16 images of 14 x 14 or 28 x 28: under
-// 1 x 1 <- 8, 1 slab each, 5.2 -> 6.4; <- 24, 2, 6.8 -> 6.8; <- 40, 3, 8.3 -> 7.5; under 3 x 3 <- 8, 5 and 9, 11.2 -> 11.7; <- 12,
-// 7 and 9, 14.4 -> 12.2).  With tiles to fill the chip, two per CU, a single slab still does not, two do (312 <- 24
-// on 50 x 23 x 14 24 -> 19).
+// repay the launch that permutes the filter too (to 12 channels, 1 to 16 images of 14 x 14 or 28 x 28: under 1 x 1 from 8, 1
+// slab each, 5.2 -> 6.4; from 24, 2, 6.8 -> 6.8; from 40, 3, 8.3 -> 7.5; under 3 x 3 from 8, 5 and 9, 11.2 -> 11.7; from 12, 7 and 9,
+// 14.4 -> 12.2).  With tiles to fill the chip, two per CU, a single slab still does not, two do (24 to 312 on 50 x 23 x 14
+// 24 -> 19).
 int fast_channels(int channels, int others, int RS, long long rows) {
   const int width = (channels + 15) / 16 * 16;
-  const long long tiles = (rows + 63) / 64 * ((others + 63) / 64);
-  const bool wide = others > 32;
-  if (width == 16 ? channels < (wide && tiles >= 128 ? 12 : 8) : 5 * width > 8 * channels) return 0;
   if (width != channels) {
+    const long long tiles = (rows + 63) / 64 * ((others + 63) / 64);
     const long long slabs = ((long long)channels * RS + 15) / 16, padded = (long long)RS * (width / 16);
-    if (tiles < 512 ? 7 * slabs <= 3 * padded + (wide ? 14 : 10) : slabs < 2) return 0;
+    const bool wide = others > 32;
+    if (width > 16 ? 5 * width > 8 * channels : channels < 8) return 0;
+    if (width == 16 && wide && tiles >= 128 && 5 * padded > 7 * slabs &&
+        (5 * padded > 8 * slabs || !split_ranges((int)rows, others, (int)padded, pick_tile((int)rows, others), (size_t)-1)))
+      return 0;
+    if (tiles < 512 ? 7 * slabs <= 3 * padded + (wide ? 15 : 10) : slabs < 2) return 0;
   }
   return (long long)others * RS * width <= (1LL << 29) - 1 ? width : 0;
 }

@@ -17,6 +17,9 @@ def _query(direction, N, C, K, H, W, pad, R):
     ((16, 8, 8, 14, 14, 1, 3), False), ((64, 8, 8, 28, 28, 1, 3), True), ((1, 8, 12, 14, 14, 1, 3), True),
     ((4, 8, 8, 14, 14, 2, 5), True), ((16, 40, 8, 28, 28, 2, 5), False),      # twice the work,
     ((2, 40, 8, 28, 28, 2, 5), True),                                         # of few tiles
+    ((16, 200, 10, 28, 28, 1, 3), True), ((32, 104, 10, 28, 28, 2, 5), True),  # 60% more work, in parts
+    ((16, 40, 10, 28, 28, 2, 5), False), ((16, 256, 10, 14, 14, 2, 5), False), ((64, 200, 8, 28, 28, 1, 3), False),
+    ((4, 40, 10, 14, 14, 1, 3), False),
     ((64, 24, 17, 28, 28, 1, 3), False), ((64, 24, 20, 28, 28, 1, 3), True),
 ])
 def test_channels_of_small_data_gradients_are_padded_where_it_pays(dims, padded):
