@@ -472,6 +472,145 @@ struct ConvBwdData {
   }
 };
 
+// Strides above 1.  An input position is met by the filter taps of one class modulo the stride per dimension
+// only, 1 / (sv sh) of them; the generic policy multiplies all, zeros but for that share.  Here the positions are
+// taken class by class ("phase"): each is a product of its own, the unit-stride correlation of top_diff with
+// every sv-th row and sh-th column of the filter, and all of them are one launch, those with the most taps first.
+// Row class rho = 0 .. sv - 1 meets the taps r' = rho + sv t (R-1-r of the filter); its rows are y = a + sv u
+// with a = (R - 1 - ph - rho) mod sv, and they meet output row u + i0 + t.  Columns likewise.  Every phase has
+// `phase_rows` rows of the product, (image, u, v) and what fills up to whole tiles; rows past a phase's own read 0
+// and are not stored.  `filter` is the permuted copy [c][taps, phase by phase][k, padded to 16] (PAD as above).
+// What bounds it is what bounds the unit-stride gathers (a trip to memory per slab on the small tiles), and the stores,
+// which leave every sh-th float of a row.
+template <bool PAD>
+struct ConvBwdDataPhases {
+  static constexpr bool A_KFAST = false, B_KFAST = true, PHASED = true;
+  static constexpr int A_NOFF = 4, B_NOFF = 1;
+  const float* __restrict__ top_diff;
+  const float* __restrict__ filter;
+  float* __restrict__ bottom_diff;
+  ConvGeom g;
+  int M, N, total_slabs, spp;      // sv * sh * phase_rows, C, most taps of a phase * spp
+  const float* __restrict__ gate;  // as in ConvBwdData
+  int phase_rows;
+  // of class 0: its first row / column, and the output row / column that this one meets with its first tap
+  int a0, b0, i00, j00;
+  // H, W, R, S = stride * quotient + rest: the first `rest` classes have one row, column, tap more
+  int hq, hr, wq, wr, rq, rr, sq, sr;
+  MnvFastDiv d_rows, d_plane[4], d_width[2], d_taps[2];  // by [rows more * 2 + columns more], [columns more], [taps more]
+  struct Phase {
+    int a, b, i0, j0, rows_more, cols_more, taps, taps_per_row, tap0;
+    MnvFastDiv d_taps_per_row;
+  };
+  struct Res {
+    mnv_rsrc a, b;
+    Phase ph;
+    int row0, end;  // the phase's own rows of the product
+  };
+  struct AState {
+    int off[4], yx[4], taps_per_row;
+    MnvFastDiv d_taps_per_row;
+  };
+  struct BState {
+    unsigned off;
+  };
+  __device__ Phase phase(int q) const {
+    const int rho = mnv_fastdiv(q, g.d_sh), sigma = q - rho * g.sh;
+    Phase p;
+    p.a = a0 - rho;
+    p.i0 = i00;
+    if (p.a < 0) p.a += g.sv, ++p.i0;
+    p.b = b0 - sigma;
+    p.j0 = j00;
+    if (p.b < 0) p.b += g.sh, ++p.j0;
+    p.rows_more = p.a < hr;
+    p.cols_more = p.b < wr;
+    const int taps_per_column = rq + (rho < rr);
+    p.taps_per_row = sq + (sigma < sr);
+    p.taps = taps_per_column * p.taps_per_row;
+    p.tap0 = (rho * rq + (rho < rr ? rho : rr)) * g.S + taps_per_column * (sigma * sq + (sigma < sr ? sigma : sr));
+    p.d_taps_per_row = sigma < sr ? d_taps[1] : d_taps[0];
+    return p;
+  }
+  __device__ int rows(const Phase& p) const { return g.N * (hq + p.rows_more) * (wq + p.cols_more); }
+  __device__ int phase_slabs(int m0) const {
+    const int q = mnv_fastdiv(m0, d_rows);
+    const Phase p = phase(q);
+    return m0 - q * phase_rows < rows(p) ? p.taps * spp : 0;
+  }
+  // (image, u, v) of a row of the phase
+  __device__ void place(const Phase& p, int row, int& img, int& u, int& v) const {
+    const int w = wq + p.cols_more;
+    img = mnv_fastdiv(row, p.rows_more ? (p.cols_more ? d_plane[3] : d_plane[2]) : p.cols_more ? d_plane[1] : d_plane[0]);
+    const int pos = row - img * (hq + p.rows_more) * w;
+    u = mnv_fastdiv(pos, p.cols_more ? d_width[1] : d_width[0]);
+    v = pos - u * w;
+  }
+  __device__ void make_res(Res& r) const {
+    r.a = mnv_make_rsrc(top_diff, (unsigned)(g.N * g.K * g.HoWo) * 4u);
+    r.b = mnv_make_rsrc(filter, (unsigned)(N * g.RS * spp * 16) * 4u);
+  }
+  size_t extra_lds_bytes() const { return 0; }
+  __device__ void block_init(Res& r, float*, int m0, int) const {
+    const int q = mnv_fastdiv(m0, d_rows);
+    r.ph = phase(q);
+    r.row0 = q * phase_rows;
+    r.end = r.row0 + rows(r.ph);
+  }
+  __device__ void a_init(const Res& r, AState& st, int m) const {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      int img, u, v;
+      place(r.ph, m + q - r.row0, img, u, v);
+      const int i = u + r.ph.i0, j = v + r.ph.j0;
+      st.off[q] = img * g.K * g.HoWo + i * g.Wo + j;
+      st.yx[q] = m + q < r.end ? pack_yx(i, j) : pack_yx(MNV_FAR, MNV_FAR);
+    }
+    st.taps_per_row = r.ph.taps_per_row;
+    st.d_taps_per_row = r.ph.d_taps_per_row;
+  }
+  __device__ void b_init(const Res& r, BState& st, int n) const {
+    st.off = n < N ? (unsigned)((n * g.RS + r.ph.tap0) * spp * 16) * 4u : MNV_OOB;
+  }
+  // period = tap of the phase, kl = output channel within the slab
+  __device__ void a_period(const AState& st, unsigned (&off)[4], int, int kl, int period) const {
+    const int rp = mnv_fastdiv(period, st.d_taps_per_row), sp = period - rp * st.taps_per_row;
+    const int koff = kl * g.HoWo + rp * g.Wo + sp;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int i = unpack_y(st.yx[q]) + rp, j = unpack_x(st.yx[q]) + sp;
+      const bool ok = ((unsigned)i < (unsigned)g.Ho) & ((unsigned)j < (unsigned)g.Wo);
+      off[q] = ok ? (unsigned)(st.off[q] + koff) * 4u : MNV_OOB;
+    }
+  }
+  __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[4], int, int s, int kl, float (&v)[4]) const {
+    const unsigned slab = (unsigned)s * 16u * (unsigned)g.HoWo * 4u;
+    if (PAD) {
+      const bool ok = s * 16 + kl < g.K;
+      const unsigned in[4] = {ok ? off[0] : MNV_OOB, ok ? off[1] : MNV_OOB, ok ? off[2] : MNV_OOB, ok ? off[3] : MNV_OOB};
+      mnv_fetch_vec<4>(r.a, in, slab, v);
+    } else {
+      mnv_fetch_vec<4>(r.a, off, slab, v);
+    }
+  }
+  __device__ void b_period(const BState& st, unsigned (&off)[1], int, int kl, int period) const {
+    off[0] = st.off + (unsigned)(period * spp * 16 + kl) * 4u;  // past the filter for MNV_OOB
+  }
+  __device__ void b_load(const Res& r, const BState&, const unsigned (&off)[1], int, int s, int, float (&v)[4]) const {
+    mnv_fetch_vec<1>(r.b, off, (unsigned)s * 64u, v);
+  }
+  __device__ void c_store(int m, int n, float x) const {
+    const int q = mnv_fastdiv(m, d_rows), row = m - q * phase_rows;
+    const Phase p = phase(q);
+    if (row >= rows(p)) return;
+    int img, u, v;
+    place(p, row, img, u, v);
+    const size_t at = ((size_t)img * N + n) * g.HW + (p.a + g.sv * u) * g.W + p.b + g.sh * v;
+    if (gate) x = gate[at] > 0.f ? x : 0.f;
+    bottom_diff[at] = x;
+  }
+};
+
 // ---------------------------------------------------------- backward filter
 struct ConvBwdFilter {
   static constexpr bool A_KFAST = true, B_KFAST = true;
@@ -750,24 +889,32 @@ struct ConvBwdFilterFast {
 // Filter permutations for the FAST policies (a few MB at most, one pass); the last dimension is
 // padded with zeros to `width`:
 //   to_rsc: out[k][r's'][c] = in[k][c][r's']      (forward)
-//   to_crk: out[c][r's'][k] = in[k][c][r's']      (data gradient)
+//   to_crk: out[c][r's'][k] = in[k][c][r's']      (data gradient; with strides above 1 the taps class by
+//           class of (r' mod sv, s' mod sh), see ConvBwdDataPhases)
 __global__ __launch_bounds__(256) void mnv_filter_permute_kernel(const float* __restrict__ in,
                                                                  float* __restrict__ out, int K,
-                                                                 int C, int RS, int width, bool to_crk) {
-  const int total = (to_crk ? C : K) * RS * width;
+                                                                 int C, int R, int S, int width, bool to_crk, int sv, int sh) {
+  const int RS = R * S, total = (to_crk ? C : K) * RS * width;
   for (int o = blockIdx.x * 256 + threadIdx.x; o < total; o += gridDim.x * 256) {
-    const int last = o % width, rs = (o / width) % RS, first = o / (width * RS);
+    const int last = o % width, first = o / (width * RS);
+    int rs = (o / width) % RS;
+    if (sv > 1 || sh > 1) {
+      int rho = 0, sigma = 0, rows = (R + sv - 1) / sv, cols = (S + sh - 1) / sh;
+      while (rs >= rows * S) rs -= rows * S, ++rho, rows = (R - rho + sv - 1) / sv;
+      while (rs >= rows * cols) rs -= rows * cols, ++sigma, cols = (S - sigma + sh - 1) / sh;
+      rs = (rho + sv * (rs / cols)) * S + sigma + sh * (rs % cols);
+    }
     const int k = to_crk ? last : first, c = to_crk ? first : last;
     out[o] = last < (to_crk ? K : C) ? in[(k * C + c) * RS + rs] : 0.f;
   }
 }
 
-int permute_filter(const float* in, float* out, int K, int C, int RS, int width, bool to_crk, hipStream_t s) {
-  int total = (to_crk ? C : K) * RS * width;
+int permute_filter(const float* in, float* out, int K, int C, int R, int S, int width, bool to_crk, hipStream_t s,
+                   int sv = 1, int sh = 1) {
+  int total = (to_crk ? C : K) * R * S * width;
   int blocks = (total + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(mnv_filter_permute_kernel, dim3(blocks), dim3(256), 0, s, in, out, K, C, RS, width,
-                     to_crk);
+  hipLaunchKernelGGL(mnv_filter_permute_kernel, dim3(blocks), dim3(256), 0, s, in, out, K, C, R, S, width, to_crk, sv, sh);
   return MNV_LAUNCH_STATUS();
 }
 
@@ -790,7 +937,7 @@ typedef MnvGemmTile<128, 64, 16, 4, 1, 0, 32> TileThin;
 typedef MnvGemmTile<256, 128, 16, 4, 2> TileTall;
 template <class P>
 int launch_tile(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t tail_bytes = 0) {
-  if constexpr (P::A_KFAST == false && P::B_NOFF == 1) {
+  if constexpr (P::A_KFAST == false && P::B_NOFF == 1 && !MnvPhased<P>::value) {
     if (tile == 1 && splits == 1) {
       const long long tiles = (long long)((p.M + 255) / 256) * ((p.N + 127) / 128);
       const long long slots = 2LL * mnv_cu_count(), rounds = (tiles + slots - 1) / slots;
@@ -1069,6 +1216,50 @@ int bwd_data_channels(const ConvGeom& g) {
   return g.sv == 1 && g.sh == 1 ? fast_channels(g.K, g.C, g.RS, (long long)g.N * g.HW) : 0;
 }
 
+// The data gradient of strides above 1, phase by phase (ConvBwdDataPhases).  us, generic gathers -> phases, at stride 2: 344 <- 112 channels under
+// 5 x 5 on 104 x 15 x 45 1780 -> 249, 264 <- 216 on 45 x 33 x 38 2293 -> 453, 128 <- 128 under 1 x 1 on 88 x 15 x 20 32 -> 31, 320 <- 96
+// under 3 x 3 on 41 x 14 x 29 191 -> 64, 48 <- 184 on 17 x 16 x 15 26.6 -> 19.1.  Few tiles of few slabs are bound by one
+// trip to memory after the other, 1.45 us for a generic slab and 0.65 for one of a phase, and pay for the launch that permutes the filter,
+// 5.5 us in all: 11 channels under 1 x 1 5.0 -> 10.2, 70 10.3 -> 10.9, 16 under 3 x 3 15.1 -> 9.7.  Error against float64: large products 0.2 to 0.6
+// of what it was (bf16 parts now); on the fp32 tiles that of the sums' own length, the fewer k ranges of which make it
+// 1.0 to 1.9 times what the generic ranges had (2.0e-7 against 1.1e-7 at 1728 products, as for a unit stride).
+struct PhasePlan {
+  int width = 0;  // channels as the policy takes them; 0: the generic gathers
+  int tile = 0, parts = 0, splits = 1, phase_rows = 0, slabs = 0;  // parts > 0: bf16 parts with that many k ranges
+  size_t filter_bytes = 0, rows = 0;
+  size_t partial_bytes(int n) const { return parts > 1 || splits > 1 ? (size_t)(parts ? parts : splits) * rows * n * sizeof(float) : 0; }
+};
+PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
+  PhasePlan p;
+  if (g.sv == 1 && g.sh == 1) return p;
+  const int width = (g.K + 15) / 16 * 16, spp = width / 16;
+  const long long phases = (long long)g.sv * g.sh;
+  const long long most = (long long)g.N * ((g.H + g.sv - 1) / g.sv) * ((g.W + g.sh - 1) / g.sh);  // rows of a phase
+  p.filter_bytes = (size_t)g.C * g.RS * width * sizeof(float);
+  if ((long long)g.C * g.RS * width > (1LL << 29) - 1 || ws_bytes < p.filter_bytes) return p;
+  const size_t left = ws_bytes > align256(p.filter_bytes) ? (ws_bytes - align256(p.filter_bytes)) / sizeof(float) : 0;
+  // what the launch shapes are chosen by: a product of all positions and the mean extent of k
+  const int m = g.N * g.HW, mean = (int)(((long long)g.RS * spp + phases - 1) / phases);
+  p.tile = pick_tile(m, g.C);
+  p.slabs = ((g.R + g.sv - 1) / g.sv) * ((g.S + g.sh - 1) / g.sh) * spp;
+  auto rows_on = [&](int tile_rows) {
+    p.phase_rows = (int)((most + tile_rows - 1) / tile_rows * tile_rows);
+    p.rows = (size_t)p.phase_rows * phases;
+  };
+  rows_on(128);
+  p.parts = split_ranges(m, g.C, mean, p.tile, left / (p.rows ? p.rows : 1) * m);
+  if (!p.parts) {
+    rows_on(kTileM[p.tile]);
+    p.splits = small_tile_splits(p.tile, (int)p.rows, g.C, p.slabs, left);
+  }
+  // the tiles' rows, and channels, are filled up: not where that multiplies more than the generic gathers
+  if ((long long)p.rows * width >= (long long)m * g.K * phases || p.rows > 0x3fffffff) return p;
+  const long long tiles = (m + 63LL) / 64 * ((g.C + 63) / 64), slabs = ((long long)g.K * g.RS + 15) / 16;
+  if (tiles < 512 ? 11 * slabs <= 5 * p.slabs + 42 : slabs < 2) return p;
+  p.width = width;
+  return p;
+}
+
 // k ranges of the filter gradient: up to 256, and up to 512 for outputs of at most 16384
 // elements, whose partial results cost next to nothing (the MNIST CNN's filters: its step
 // 0.28 -> 0.25 ms; conv1 of the AlexNet shape with 341 ranges instead of 255: 0.50 -> 0.54 ms).
@@ -1147,7 +1338,7 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wp = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wp, K, C, g.RS, width, false, s);
+    rc = permute_filter(filter, wp, K, C, R, S, width, false, s);
     if (rc) return rc;
     const int spp = width / 16;
     const size_t part_bytes = part ? workspace_bytes - used : 0;
@@ -1217,6 +1408,11 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
                                         int sv, int sh, int R, int S) {
   ConvGeom g;
   if (make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S)) return 0;
+  const PhasePlan phases = phase_plan(g, (size_t)-1);
+  if (phases.width) {
+    const size_t partial = phases.partial_bytes(C);
+    return partial ? align256(phases.filter_bytes) + partial : phases.filter_bytes;
+  }
   const int width = bwd_data_channels(g);
   const size_t permuted = (size_t)C * g.RS * width * sizeof(float);
   const int gm = N * g.HW, gn = C, slabs = width ? g.RS * (width / 16) : (K * g.RS + 15) / 16;
@@ -1231,6 +1427,40 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
     if (w > need) need = w;
   }
   return need;
+}
+
+static int bwd_data_phases(const float* top_diff, const float* filter, const float* gate, float* bottom_diff, const ConvGeom& g,
+                           const PhasePlan& plan, void* workspace, hipStream_t s) {
+  float* permuted = static_cast<float*>(workspace);
+  float* part = plan.partial_bytes(g.C) ? reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(plan.filter_bytes)) : nullptr;
+  const int rc = permute_filter(filter, permuted, g.K, g.C, g.R, g.S, plan.width, true, s, g.sv, g.sh);
+  if (rc) return rc;
+  auto launch = [&](auto p) {
+    p.top_diff = top_diff; p.filter = permuted; p.bottom_diff = bottom_diff; p.gate = gate;
+    p.g = g;
+    p.M = (int)plan.rows; p.N = g.C; p.total_slabs = plan.slabs; p.spp = plan.width / 16;
+    p.phase_rows = plan.phase_rows;
+    // class 0 holds the tap r' = 0, which meets output row i at input row i sv - ph + R - 1
+    auto first = [](int reach, int stride, int* at, int* out) {
+      *at = (reach % stride + stride) % stride;
+      *out = (*at - reach) / stride;
+    };
+    first(g.R - 1 - g.ph, g.sv, &p.a0, &p.i00);
+    first(g.S - 1 - g.pw, g.sh, &p.b0, &p.j00);
+    p.hq = g.H / g.sv; p.hr = g.H % g.sv; p.wq = g.W / g.sh; p.wr = g.W % g.sh;
+    p.rq = g.R / g.sv; p.rr = g.R % g.sv; p.sq = g.S / g.sh; p.sr = g.S % g.sh;
+    p.d_rows = mnv_fastdiv_make(p.phase_rows);
+    for (int more = 0; more < 4; ++more) {
+      const int plane = (p.hq + more / 2) * (p.wq + more % 2);  // 0: no position is in such a class
+      p.d_plane[more] = mnv_fastdiv_make(plane ? plane : 1);
+    }
+    for (int more = 0; more < 2; ++more) {
+      p.d_width[more] = mnv_fastdiv_make(p.wq + more ? p.wq + more : 1);
+      p.d_taps[more] = mnv_fastdiv_make(p.sq + more ? p.sq + more : 1);
+    }
+    return plan.parts ? launch_parts(p, plan.parts, part, s, 0) : launch_tile(plan.tile, p, plan.splits, part, s);
+  };
+  return plan.width != g.K ? launch(ConvBwdDataPhases<true>{}) : launch(ConvBwdDataPhases<false>{});
 }
 
 static int conv_bwd_data_impl(const float* top_diff, const float* filter, const float* gate,
@@ -1248,6 +1478,10 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
                                          workspace && mnv_aligned16(workspace) ? workspace_bytes : 0))
     return mnv_wino_conv(top_diff, filter, nullptr, gate, bottom_diff, N, K, C, g.Ho, g.Wo, R - 1 - ph,
                          S - 1 - pw, R, 1, 0, images, workspace, workspace_bytes, s);
+  if (sv > 1 || sh > 1) {
+    const PhasePlan plan = phase_plan(g, workspace ? workspace_bytes : 0);
+    if (plan.width) return bwd_data_phases(top_diff, filter, gate, bottom_diff, g, plan, workspace, s);
+  }
   const int tile = pick_tile(gm, gn);
   const int width = bwd_data_channels(g);
   const size_t permuted_bytes = (size_t)C * g.RS * width * sizeof(float);
@@ -1258,7 +1492,7 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wq = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wq, K, C, g.RS, width, true, s);
+    rc = permute_filter(filter, wq, K, C, R, S, width, true, s);
     if (rc) return rc;
     const int spp = width / 16;
     const size_t part_bytes = part ? workspace_bytes - used : 0;

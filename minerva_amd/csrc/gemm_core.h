@@ -131,6 +131,11 @@ struct MnvFetchMap {
 //        tiles (tiles_n is a multiple of n_group), so that the column tiles that read the
 //        same A panel run next to each other; without it all m-tiles of one column tile come
 //        first (the B panel is shared).  Not for stream-k launches.
+//   optional, for a product whose rows fall into equal runs of `phase_rows` (a multiple of the tile's
+//   rows; M is a multiple of it) with k extents of their own: static constexpr bool PHASED = true;
+//   int phase_rows;  int phase_slabs(int m0) const;   slabs of the tile whose first row is m0, total_slabs at most
+//        Tiles are dealt run by run, so that the order of the runs is the order of the launch (the
+//        longest first), and k ranges cut a tile's own slabs.  Not for stream-k launches and cut tails.
 //   optional, for a store that combines the product with a value read from memory:
 //   static constexpr bool C_PRELOAD = true;
 //   bool c_preload_on() const;                   uniform: whether this launch reads
@@ -177,6 +182,14 @@ struct MnvNGrouped {
 };
 template <class P>
 struct MnvNGrouped<P, std::enable_if_t<P::N_GROUPED>> {
+  static constexpr bool value = true;
+};
+template <class P, class = void>
+struct MnvPhased {
+  static constexpr bool value = false;
+};
+template <class P>
+struct MnvPhased<P, std::enable_if_t<P::PHASED>> {
   static constexpr bool value = true;
 };
 template <class P, class = void>
@@ -228,10 +241,18 @@ __device__ __forceinline__ int mnv_tile_remap(int t, int total) {
   return t < per_xcd * 8 ? (t % 8) * per_xcd + t / 8 : t;
 }
 
-// Tile coordinates of the (remapped) tile index b.
+// Tile coordinates of tile vb of the launch order.
 template <class P>
-__device__ __forceinline__ void mnv_tile_coords(const P& prob, int b, int tiles_m, int& tile_m,
-                                                int& tile_n) {
+__device__ __forceinline__ void mnv_tile_coords(const P& prob, int vb, int tile_rows, int tiles_m, int tiles_n,
+                                                int& tile_m, int& tile_n) {
+  if constexpr (MnvPhased<P>::value) {
+    const int across = prob.phase_rows / tile_rows, per = across * tiles_n;
+    const int phase = vb / per, b = mnv_tile_remap(vb - phase * per, per);
+    tile_n = b / across;
+    tile_m = phase * across + (b - tile_n * across);
+    return;
+  }
+  const int b = mnv_tile_remap(vb, tiles_m * tiles_n);
   if constexpr (MnvNGrouped<P>::value) {
     const int per = tiles_m * prob.n_group;
     const int grp = b / per, r = b - grp * per;
@@ -240,6 +261,17 @@ __device__ __forceinline__ void mnv_tile_coords(const P& prob, int b, int tiles_
   } else {
     tile_m = b % tiles_m;
     tile_n = b / tiles_m;
+  }
+}
+// Slabs of the tile at row m0, and of each of its k ranges.
+template <class P>
+__device__ __forceinline__ int mnv_tile_slabs(const P& prob, int m0, int& slabs_per_split) {
+  if constexpr (MnvPhased<P>::value) {
+    const int own = prob.phase_slabs(m0);
+    slabs_per_split = (own + (int)gridDim.z - 1) / (int)gridDim.z;
+    return own;
+  } else {
+    return prob.total_slabs;
   }
 }
 
@@ -378,19 +410,21 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
       vb = (int)(sk_u / sk_rest);
     }
   }
-  const int b = SK ? vb : mnv_tile_remap(vb, tiles_m * tiles_n);
   int tile_m, tile_n;
   if constexpr (SK) {
-    tile_m = b % tiles_m;
-    tile_n = b / tiles_m;
+    tile_m = vb % tiles_m;
+    tile_n = vb / tiles_m;
   } else {
-    mnv_tile_coords(prob, b, tiles_m, tile_m, tile_n);
+    mnv_tile_coords(prob, vb, T::BM, tiles_m, tiles_n, tile_m, tile_n);
   }
   const int m0 = tile_m * T::BM, n0 = tile_n * T::BNU;
 
+  static_assert(!MnvPhased<P>::value || (!SK && G == 1), "whole tiles or whole k ranges");
+  const int total_slabs = mnv_tile_slabs(prob, m0, slabs_per_split);
   int slab_begin = blockIdx.z * slabs_per_split;
   int slab_end = slab_begin + slabs_per_split;
-  if (slab_end > prob.total_slabs) slab_end = prob.total_slabs;
+  if (slab_end > total_slabs) slab_end = total_slabs;
+  if (slab_begin > slab_end) slab_begin = slab_end;
   if constexpr (SK) {
     if (sk_aligned) {
       if ((int)gridDim.x == tiles_m * tiles_n * tail_begin) {  // no remaining workgroups: even cuts
@@ -836,9 +870,8 @@ __global__ __launch_bounds__(256) void mnv_gemm_tail_reduce_kernel(P prob,
                                                                    int tiles_m, int tiles_n,
                                                                    int tail_begin, int tail_z) {
   constexpr int TILE = T::BM * T::BNU;
-  const int b = mnv_tile_remap(tail_begin + (int)blockIdx.y, tiles_m * tiles_n);
   int tile_m, tile_n;
-  mnv_tile_coords(prob, b, tiles_m, tile_m, tile_n);
+  mnv_tile_coords(prob, tail_begin + (int)blockIdx.y, T::BM, tiles_m, tiles_n, tile_m, tile_n);
   const int m0 = tile_m * T::BM, n0 = tile_n * T::BNU;
   const float* p = partial + (size_t)blockIdx.y * tail_z * TILE;
   for (int e = (blockIdx.x * 256 + threadIdx.x) * 4; e < TILE; e += gridDim.x * 256 * 4) {
@@ -1038,7 +1071,7 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
   const size_t lds_bytes = tile_bytes + prob.extra_lds_bytes();
   if (lds_bytes > lds_limit) return MNV_ERR_INVALID;
   MnvTailPlan tail{tiles_m * tiles_n, 1};
-  if (G == 1 && splits == 1 && (T::MIN_WAVES == 4 || MnvIsSplit<T>::value) && workspace && tail_bytes)
+  if (G == 1 && splits == 1 && !MnvPhased<P>::value && (T::MIN_WAVES == 4 || MnvIsSplit<T>::value) && workspace && tail_bytes)
     tail = mnv_tail_plan((long long)tiles_m * tiles_n, total_slabs, (size_t)T::BM * T::BNU,
                          tail_bytes / sizeof(float), MnvIsSplit<T>::tail);
   const int tail_tiles = tiles_m * tiles_n - tail.begin;
@@ -1047,11 +1080,13 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
                      tail.begin, tail.z);
   int rc = MNV_LAUNCH_STATUS();
   if (rc) return rc;
-  if (tail.z > 1) {
-    hipLaunchKernelGGL((mnv_gemm_tail_reduce_kernel<T, P>), dim3(T::BM * T::BNU / 1024, tail_tiles),
-                       dim3(256), 0, s, prob, reinterpret_cast<const float*>(workspace), tiles_m,
-                       tiles_n, tail.begin, tail.z);
-    return MNV_LAUNCH_STATUS();
+  if constexpr (!MnvPhased<P>::value) {
+    if (tail.z > 1) {
+      hipLaunchKernelGGL((mnv_gemm_tail_reduce_kernel<T, P>), dim3(T::BM * T::BNU / 1024, tail_tiles),
+                         dim3(256), 0, s, prob, reinterpret_cast<const float*>(workspace), tiles_m,
+                         tiles_n, tail.begin, tail.z);
+      return MNV_LAUNCH_STATUS();
+    }
   }
   if (splits > 1) {
     rc = mnv_gemm_reduce_launch(prob, reinterpret_cast<const float*>(workspace), splits, s);

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(T::NT, T::MIN_WAVES) void mnv_gemm_split_kernel(P p
     }
   }
   for (;;) {  // SK: one pass per segment; otherwise a single pass that ends in a return
-    int vb = blockIdx.x, tail_part = -1, b, tile_m, tile_n, slab_begin, slab_end;
+    int vb = blockIdx.x, tail_part = -1, tile_m, tile_n, slab_begin, slab_end;
     if constexpr (SK) {
       if (sk_aligned) {
         const int z = sk_p / tiles;
@@ -277,22 +277,23 @@ __global__ __launch_bounds__(T::NT, T::MIN_WAVES) void mnv_gemm_split_kernel(P p
         const long long left = sk_end - sk_u;
         slab_end = left < prob.total_slabs - slab_begin ? slab_begin + (int)left : prob.total_slabs;
       }
-      b = vb;
-      tile_m = b % tiles_m;
-      tile_n = b / tiles_m;
+      tile_m = vb % tiles_m;
+      tile_n = vb / tiles_m;
     } else {
-      int begin = blockIdx.z * slabs_per_split, per = slabs_per_split;
       if (tail_z > 1 && vb >= tail_begin) {
         const int i = vb - tail_begin, tl = i / tail_z;
         tail_part = i - tl * tail_z;
         vb = tail_begin + tl;
-        per = (prob.total_slabs + tail_z - 1) / tail_z;
+      }
+      mnv_tile_coords(prob, vb, T::BM, tiles_m, tiles_n, tile_m, tile_n);
+      const int total_slabs = mnv_tile_slabs(prob, tile_m * T::BM, slabs_per_split);
+      int per = slabs_per_split, begin = blockIdx.z * per;
+      if (tail_part >= 0) {
+        per = (total_slabs + tail_z - 1) / tail_z;
         begin = tail_part * per;
       }
-      slab_begin = begin < prob.total_slabs ? begin : prob.total_slabs;
-      slab_end = begin + per < prob.total_slabs ? begin + per : prob.total_slabs;
-      b = mnv_tile_remap(vb, tiles);
-      mnv_tile_coords(prob, b, tiles_m, tile_m, tile_n);
+      slab_begin = begin < total_slabs ? begin : total_slabs;
+      slab_end = begin + per < total_slabs ? begin + per : total_slabs;
     }
     const int m0 = tile_m * T::BM, n0 = tile_n * T::BNU;
 
