@@ -153,7 +153,8 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * range.
  * mnv_sgemm_nn_plan reports how a product of these extents is launched with a workspace of
  * that size (no counterpart in the reference, where the plan is cuBLAS's own): tile_rows is
- * 128 or 64 for square tiles, 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
+ * 128 or 64 for square tiles (64 with k_ranges and groups 1 also for the 32 x 32 and 16 x 16 tiles of small
+ * products, whose wavefronts share the k range), 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
  * kernels of at most 12 columns over a large A (256 rows per workgroup, 64 where A is given
  * transposed; four wavefronts take a quarter of a k range each); k_ranges is the number of
  * partial results reduced by a second kernel (1: none); groups is otherwise 4 when a workgroup

@@ -5,6 +5,7 @@
 // fp32 instruction (gemm_core.h) for the others; A is fetched x-fast (m contiguous), B k-fast (k
 // contiguous).  Products with too few output tiles to fill 256 CUs split the k range over
 // blockIdx.z when the caller lends a workspace.
+#include <cmath>
 #include <mutex>
 
 #include "gemm_split.h"
@@ -354,6 +355,106 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_tn_kernel(P prob, int k_
   }
 }
 
+// Small products: T x T tiles (16 or 32) of the result, one per workgroup, whose W wavefronts share the k range.  A 64 x 64 tile
+// of the core takes 0.24 us of a CU's matrix cores per 16 k and leaves most CUs without one; four or sixteen times as
+// many tiles spread the same multiplies over them, and the k ranges meet in LDS, not in memory and a second launch.
+// No operand passes through LDS: a lane loads what it multiplies, 16 bytes along k (a k-fast operand) or 4 bytes a k
+// (x-fast, neighbouring lanes at neighbouring addresses), 32 k at a time, the next 32 in flight under the multiplies
+// (96 in flight: no faster).  Of instruction t, lane group h (of 64 / T) takes k = 4 h + t of each run of 4 * 64 / T, in every
+// form, so that the transposed forms have the bits of transposing first.  The wavefronts' sums are added in the order of k.
+// k past K: an x-fast operand reads 0 past its end, a k-fast one is cleared; rows and columns past the result's may
+// read anything inside the operand and are not stored.
+// What bounds it: a launch and two trips to memory, 3 us; from one tile per CU on the operands' way from L2
+// (128 or 256 bytes per k and tile).  An XCD works on neighbouring tiles across the shorter side of the result, so that its
+// L2 fetches an eighth of the longer operand (4021 x 169 x 731 on 32 x 32 tiles 25 -> 17 us, 2093 x 198 x 3376 on 16 x 16 147 -> 55).
+// us, tiles of the core -> this: 17 x 53 x 124 6.5 -> 3.5, 256 x 256 x 784 9.1 -> 3.9, 10 x 256 x 256 6.8 -> 3.4, 512 x 512 x 512
+// 13.0 -> 5.5, 1421 x 284 x 488 14.1 -> 8.6, 1001 x 250 x 4099 28.2 -> 24; 300 random products of up to
+// 4096 in every extent 0.65 of the time.
+// Error against float64: 2 W sums per value, 0.83 of what it was over 300 random products, none more than 1.1 times.
+template <class P, int T, int W>
+__global__ __launch_bounds__(W * MNV_WAVE) void mnv_sgemm_small_kernel(P prob, int tiles_m, int tiles_n, int k_per_wave) {
+  constexpr int H = MNV_WAVE / T, RUN = 4 * H, VECS = 32 / RUN, REGS = T * T / MNV_WAVE;
+  typedef float Acc __attribute__((ext_vector_type(REGS)));
+  __shared__ float red[W * T * T];
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
+  const int x = lane % T, h = lane / T;
+  const int tile = mnv_tile_remap((int)blockIdx.x, tiles_m * tiles_n);
+  const bool tall = tiles_m > tiles_n;
+  const int across = tall ? tiles_n : tiles_m, outer = tile / across, inner = tile - outer * across;
+  const int m0 = (tall ? outer : inner) * T, n0 = (tall ? inner : outer) * T;
+  typename P::Res res;
+  prob.make_res(res);
+  const unsigned lda = (unsigned)prob.lda * 4u, ldb = (unsigned)prob.ldb * 4u;
+  const unsigned a_off = P::A_KFAST ? (m0 + x < prob.M ? (unsigned)(m0 + x) * lda + (unsigned)h * 16u : MNV_OOB)
+                                    : (unsigned)h * 4u * lda + (unsigned)(m0 + x) * 4u;
+  const unsigned b_off = P::B_KFAST ? (n0 + x < prob.N ? (unsigned)(n0 + x) * ldb + (unsigned)h * 16u : MNV_OOB)
+                                    : (unsigned)h * 4u * ldb + (unsigned)(n0 + x) * 4u;
+  auto fetch = [&](mnv_rsrc r, unsigned off, unsigned ld, auto KFAST, int k, float (&v)[VECS][4]) {
+#pragma unroll
+    for (int j = 0; j < VECS; ++j) {
+      if constexpr (decltype(KFAST)::value) {
+        const unsigned one[1] = {off};
+        mnv_fetch_vec<1>(r, one, (unsigned)(k + RUN * j) * 4u, v[j]);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          v[j][t] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)((unsigned)(k + RUN * j + t) * ld), 0));
+      }
+    }
+  };
+  typedef std::integral_constant<bool, P::A_KFAST> AFast;
+  typedef std::integral_constant<bool, P::B_KFAST> BFast;
+  int k = wave * k_per_wave;
+  const int k_end = k + k_per_wave < prob.K ? k + k_per_wave : prob.K;
+  Acc acc[2] = {0.f, 0.f};  // of the even and the odd fetches: half the length of the sums
+  float a[2][VECS][4], b[2][VECS][4];
+  if (k < k_end) {
+    fetch(res.a, a_off, lda, AFast{}, k, a[0]);
+    fetch(res.b, b_off, ldb, BFast{}, k, b[0]);
+  }
+  auto step = [&](auto SET) {
+    constexpr int set = decltype(SET)::value;
+    fetch(res.a, a_off, lda, AFast{}, k + 32, a[set ^ 1]);  // past the range: not multiplied
+    fetch(res.b, b_off, ldb, BFast{}, k + 32, b[set ^ 1]);
+    if (k + 32 > prob.K) {
+#pragma unroll
+      for (int j = 0; j < VECS; ++j)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const bool on = k + RUN * j + 4 * h + t < prob.K;
+          if (P::A_KFAST) a[set][j][t] = on ? a[set][j][t] : 0.f;
+          if (P::B_KFAST) b[set][j][t] = on ? b[set][j][t] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < VECS; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (T == 32) acc[set] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], acc[set], 0, 0, 0);
+        else acc[set] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], acc[set], 0, 0, 0);
+      }
+    k += 32;
+  };
+  int steps = (k_end - k + 31) / 32;
+  for (; steps >= 2; steps -= 2) {
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+  }
+  if (steps > 0) step(std::integral_constant<int, 0>{});
+  // register r of lane (x, h): row x, column 4 h + r % 4 + 8 (r / 4)
+#pragma unroll
+  for (int r = 0; r < REGS; ++r) red[wave * T * T + (4 * h + r % 4 + 8 * (r / 4)) * T + x] = acc[0][r] + acc[1][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < T * T; e += W * MNV_WAVE) {
+    float sum = red[e];
+#pragma unroll
+    for (int w = 1; w < W; ++w) sum += red[w * T * T + e];
+    const int m = m0 + e % T, n = n0 + e / T;
+    if (m < prob.M && n < prob.N) prob.c_store(m, n, sum);
+  }
+}
+
 struct SgemmEpilogue {
   const float* bias;
   const float* gate;
@@ -384,6 +485,7 @@ typedef MnvSplitTile<128, 128, 2, 4, 1> SplitPair;
 typedef MnvSplitTile<128, 128, 2, 4, 2> SplitOne;
 typedef MnvSplitTile<256, 128, 4, 2, 2> SplitTall;
 #define MNV_SGEMM_MAX_SPLITS 16
+const long long kSmallOperand = (1LL << 29) - 1;  // floats that mnv_sgemm_small_kernel's offsets reach
 
 // Tile shape and number of k ranges for an (m,n,k) product given `ws_floats` floats of
 // scratch.  Both shapes are priced with the occupancy model of mnv_pick_splits, in units of
@@ -397,6 +499,8 @@ struct SgemmPlan {
   bool tall = false;  // 256 x 128 tiles (no k ranges, one wavefront group)
   bool split = false; // in bf16 parts (256 x 128 tiles always, 128 x 128 ones but for a single slab)
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
+  int tile = 0;       // 16, 32: mnv_sgemm_small_kernel with `groups` wavefronts
+  double us = 0.0;    // the estimate of one on 64 x 64 or larger tiles
 };
 
 // Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), with
@@ -571,7 +675,32 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
     if ((double)m * n >= 0.95 * (double)(rounds * slots) * 256.0 * 128.0) best.tall = true;
   }
   plan_split(m, n, k, ws_floats, best_cost, cus, &best);
+  // in us, fitted to 500 random products of up to 3 GFLOP (10% off, rms)
+  best.us = best.split ? split_cost(m, n, k, best.splits, cus) : best.groups == 4 ? (k % 4 ? 0.92 : 0.84) * best_cost : 0.77 * best_cost + 0.5;
   return best;
+}
+
+// A plan on the small kernel's tiles where that is estimated at less than 90% of `plan`: 3 us, and the larger of what the
+// fullest CU multiplies and what all tiles take from L2, 1.49 and 1.95 us per 1000 k of a 16 x 16 tile on every CU, 4.36 and
+// 4.81 of a 32 x 32 one (5.2 from 2048 k on); beyond the eight or five workgroups that a CU holds, 2.5 us for each further round.
+// From 2048 k on 16 x 16 tiles take up to 1.4 times their estimate (292 x 243 x 3361 14.8 -> 21.7; 49 x 98 x 3847 11.7 -> 9.8) and are
+// left to the k ranges.  Measured on 500 products with every shape: 0.593 of the time, the fastest of all throughout
+// 0.575; seven lost 4 to 20% (555 x 2773 x 156 10.7 -> 11.6, 677 x 84 x 3060 14.5 -> 15.3).  Four wavefronts for many tiles, eight for few.
+// The kernel reads an x-fast operand up to 95 k past its end: its offsets have to stay below 2^31.
+void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
+  // (products in parts are the more exact ones)
+  if (plan->skinny || plan->split || (k + 96LL) * m > kSmallOperand || (k + 96LL) * n > kSmallOperand) return;
+  auto cost = [&](int t, double own, double all, int resident) {
+    const double per_cu = (double)((m + t - 1LL) / t) * ((n + t - 1) / t) / cus;
+    const double work = all * per_cu > own * ceil(per_cu) ? all * per_cu : own * ceil(per_cu);
+    return 3.0 + work * 1e-3 * k + (per_cu > resident ? 2.5 * (per_cu / resident - 1.0) : 0.0);
+  };
+  const double c16 = k <= 2048 ? cost(16, 1.49, 1.95, 8) : 1e30, c32 = cost(32, k > 2048 ? 5.2 : 4.36, k > 2048 ? 5.2 : 4.81, 5);
+  if ((c16 < c32 ? c16 : c32) >= 0.9 * plan->us) return;
+  *plan = SgemmPlan{true, 1};
+  plan->tile = c16 < c32 ? 16 : 32;
+  const bool many = plan->tile == 16 ? (long long)m * n > 512 * cus : (m + 31LL) / 32 * ((n + 31) / 32) >= cus;
+  plan->groups = many ? 4 : 8;
 }
 
 // The plan of an unlimited workspace.  A plan is planned again within what its own partial results need,
@@ -589,6 +718,7 @@ SgemmPlan plan_unlimited(int m, int n, int k, int cus) {
     plan = next;
     if (same) break;
   }
+  plan_small(m, n, k, cus, &plan);
   return plan;
 }
 
@@ -598,8 +728,11 @@ SgemmPlan plan_unlimited(int m, int n, int k, int cus) {
 // 1500 x 1501 would stay on grouped 64 x 64 tiles (72 us with a large workspace, 88 with the queried one).
 SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   const int cus = mnv_cu_count();
-  const SgemmPlan plan = plan_unlimited(m, n, k, cus);
-  return plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n) ? plan : plan_within(m, n, k, ws_floats, cus);
+  SgemmPlan plan = plan_unlimited(m, n, k, cus);
+  if (plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n)) return plan;
+  plan = plan_within(m, n, k, ws_floats, cus);
+  plan_small(m, n, k, cus, &plan);
+  return plan;
 }
 
 template <int NC, bool TB, class P>
@@ -636,6 +769,20 @@ int launch_skinny_columns(const SgemmPlan& plan, const SgemmNN<K4, TA, TB>& p, v
   return mnv_gemm_reduce_launch(p, part, plan.splits, s);
 }
 
+template <int T, int W, class P>
+int launch_small(const P& p, hipStream_t s) {
+  const int tiles_m = (p.M + T - 1) / T, tiles_n = (p.N + T - 1) / T;
+  hipLaunchKernelGGL((mnv_sgemm_small_kernel<P, T, W>), dim3(tiles_m * tiles_n), dim3(W * MNV_WAVE), 0, s, p, tiles_m, tiles_n,
+                     (p.K + 32 * W - 1) / (32 * W) * 32);
+  return MNV_LAUNCH_STATUS();
+}
+
+template <bool TA, bool TB>
+int launch_small_tiles(const SgemmPlan& plan, const SgemmNN<true, TA, TB>& p, hipStream_t s) {
+  if (plan.tile == 16) return plan.groups == 4 ? launch_small<16, 4>(p, s) : launch_small<16, 8>(p, s);
+  return plan.groups == 4 ? launch_small<32, 4>(p, s) : launch_small<32, 8>(p, s);
+}
+
 // In bf16 parts.  Groups of up to eight column tiles, as many as divide them: 4096^3 on 256 x 128
 // tiles reads 12 panels for 32 tiles where whole columns read 18.
 template <class P>
@@ -661,7 +808,7 @@ int launch_plan(const SgemmPlan& plan, const P& p, void* workspace, size_t works
 
 // Bytes a product without k ranges wants for the partial tiles of its cut tail.
 size_t sgemm_tail_bytes(const SgemmPlan& plan, int m, int n, int k) {
-  if (plan.splits != 1 || plan.groups != 1 || plan.tall) return 0;
+  if (plan.splits != 1 || plan.groups != 1 || plan.tall || plan.tile) return 0;
   const int bm = plan.small ? 64 : 128;
   const long long tiles = (long long)((m + bm - 1) / bm) * ((n + bm - 1) / bm);
   const MnvTailPlan t = mnv_tail_plan(tiles, (k + 15) / 16, (size_t)bm * bm, (size_t)-1 / sizeof(float),
@@ -692,8 +839,10 @@ int scratch_address(float** out) {
 int sgemm_nn_impl(const float* a, const float* b, float* c, int m, int n, int k, void* workspace,
                   size_t workspace_bytes, hipStream_t s,
                   const SgemmEpilogue& e = SgemmEpilogue{nullptr, nullptr, 0}) {
-  const SgemmPlan plan = plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
+  // a panel of larger matrices has their pitches, which the small kernel's reach is not planned for
+  const SgemmPlan plan = e.lda ? plan_within(m, n, k, 0, mnv_cu_count()) : plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
   if (plan.skinny) return launch_skinny_columns(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, s);
+  if (plan.tile) return launch_small_tiles(plan, make_sgemm<true>(a, b, c, m, n, k, e), s);
   if (k % 4 == 0) return launch_plan(plan, make_sgemm<true>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
   return launch_plan(plan, make_sgemm<false>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
 }
@@ -705,6 +854,7 @@ int sgemm_t_impl(const float* a, const float* b, float* c, int m, int n, int k, 
                  size_t workspace_bytes, hipStream_t s, const SgemmEpilogue& e) {
   const SgemmPlan plan = plan_sgemm(m, n, k, workspace ? workspace_bytes / sizeof(float) : 0);
   if (plan.skinny) return launch_skinny_columns(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, s);
+  if (plan.tile) return launch_small_tiles(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), s);
   // with both operands x-fast no vector runs along k
   if ((!TA && TB) || k % 4 == 0)
     return launch_plan(plan, make_sgemm<true, TA, TB>(a, b, c, m, n, k, e), workspace, workspace_bytes, s);
@@ -760,7 +910,7 @@ int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_row
   *tile_rows = plan.tall || plan.skinny ? 256 : plan.small ? 64 : 128;
   const int slabs = (k + 15) / 16, per = (slabs + plan.splits - 1) / plan.splits;
   *k_ranges = plan.skinny ? plan.splits : (slabs + per - 1) / per;  // as the launch rounds it: ranges of equal length
-  *groups = plan.groups;
+  *groups = plan.tile ? 1 : plan.groups;
   return MNV_OK;
 }
 
