@@ -312,7 +312,7 @@ int mnv_conv_bwd_filter(const float* bottom, const float* top_diff, float* filte
                         mnv_stream_t stream);
 /* How mnv_conv_bwd_filter launches a problem with a workspace of `workspace_bytes` on the
  * current device (no reference counterpart: cuDNN chooses its algorithm out of sight,
- * cuda_perform.cu:293-318): rows of the output tile (64 or 128); the k ranges the reduction
+ * cuda_perform.cu:293-318): rows of the output tile (32, 64 or 128); the k ranges the reduction
  * over images and positions is cut into, each with a partial result in the workspace (1: none);
  * and, when the launch instead has as many workgroups as the chip holds at once, each with the
  * same number of k-slabs ("stream-k": aligned k ranges of every tile, the rest in shares;

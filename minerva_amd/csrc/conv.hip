@@ -114,6 +114,8 @@ struct ConvFwd {
       mnv_fetch_vec<4>(r.a, off, slab, v);
     }
   }
+  __device__ int channels() const { return g.C; }
+  __device__ int channel_floats() const { return g.HW; }
   size_t extra_lds_bytes() const { return 0; }
   __device__ void block_init(Res&, float*, int, int) const {}
   // generic: `filter` is the caller's tensor [n][c][r'][s'], element (k, n) at n*CRS + k.
@@ -418,6 +420,8 @@ struct ConvBwdData {
       mnv_fetch_vec<4>(r.a, off, slab, v);
     }
   }
+  __device__ int channels() const { return g.K; }
+  __device__ int channel_floats() const { return g.HoWo; }
   size_t extra_lds_bytes() const { return 0; }
   __device__ void block_init(Res&, float*, int, int) const {}
   // B[kk, c] = filter[ko, c, r', s'].  FAST reads the permuted copy [c][r's'][ko, padded to 16].
@@ -484,7 +488,7 @@ struct ConvBwdData {
 // which leave every sh-th float of a row.
 template <bool PAD>
 struct ConvBwdDataPhases {
-  static constexpr bool A_KFAST = false, B_KFAST = true, PHASED = true;
+  static constexpr bool A_KFAST = false, B_KFAST = true, PHASED = true, PADDED = PAD;
   static constexpr int A_NOFF = 4, B_NOFF = 1;
   const float* __restrict__ top_diff;
   const float* __restrict__ filter;
@@ -550,6 +554,8 @@ struct ConvBwdDataPhases {
     r.a = mnv_make_rsrc(top_diff, (unsigned)(g.N * g.K * g.HoWo) * 4u);
     r.b = mnv_make_rsrc(filter, (unsigned)(N * g.RS * spp * 16) * 4u);
   }
+  __device__ int channels() const { return g.K; }
+  __device__ int channel_floats() const { return g.HoWo; }
   size_t extra_lds_bytes() const { return 0; }
   __device__ void block_init(Res& r, float*, int m0, int) const {
     const int q = mnv_fastdiv(m0, d_rows);
@@ -608,6 +614,28 @@ struct ConvBwdDataPhases {
     const size_t at = ((size_t)img * N + n) * g.HW + (p.a + g.sv * u) * g.W + p.b + g.sh * v;
     if (gate) x = gate[at] > 0.f ? x : 0.f;
     bottom_diff[at] = x;
+  }
+};
+
+// The fast gathers of B, four channels of one position to a vector: for mnv_gemm_small_kernel.
+template <class B, bool PAD>
+struct ConvOneRow : B {
+  typedef B StoredBy;
+  static constexpr bool A_KFAST = true;
+  static constexpr int A_NOFF = 1;
+  __device__ void a_period(const typename B::AState& st, unsigned (&off)[1], int m, int kl, int period) const {
+    unsigned rows[4];  // of m and the three rows after it, which are not used
+    B::a_period(st, rows, m, kl, period);
+    off[0] = rows[0];
+  }
+  __device__ void a_load(const typename B::Res& r, const typename B::AState&, const unsigned (&off)[1], int, int s, int kl,
+                         float (&v)[4]) const {
+    const unsigned plane = (unsigned)this->channel_floats() * 4u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const unsigned at = !PAD || s * 16 + kl + q < this->channels() ? off[0] : MNV_OOB;
+      v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r.a, (int)at, (int)((unsigned)(s * 16 + q) * plane), 0));
+    }
   }
 };
 
@@ -982,9 +1010,10 @@ typedef MnvSplitTile<128, 96, 2, 2, 1> Split96;
 // 10 x 13 x 13, 60 -> 59 for 384 -> 384, 129 -> 143 for 128 -> 256 on 32 x 56 x 56 at stride 2).  3 -> 96
 // under 11 x 11, stride 4, 256 / 50 / 10 images of 227 x 227: 537 -> 386, 101 -> 89, 38 -> 34 us; 256 ->
 // 256 under 1 x 1 on 16 x 28 x 28 40 -> 30.
-template <bool PARTS = false, class P>
+// `small(&done)`: the launch on the small tiles, for what does not run in equal shares.
+template <bool PARTS = false, class P, class Small>
 int launch_filter_gradient(int tile, const P& p, int splits, void* ws, size_t ws_bytes, hipStream_t s,
-                           int* plan = nullptr) {
+                           int* plan, const Small& small) {
   if (plan) {
     plan[0] = kTileM[tile];
     plan[1] = splits;
@@ -1011,7 +1040,9 @@ int launch_filter_gradient(int tile, const P& p, int splits, void* ws, size_t ws
       return rc;
     }
   }
-  if (plan) return MNV_OK;
+  bool done = false;
+  const int rc = small(&done);
+  if (rc || done || plan) return rc;
   return launch_tile(tile, p, splits, ws, s);
 }
 
@@ -1094,6 +1125,19 @@ size_t split_bytes(int tile, int m, int n, int slabs) {
   return z > 1 ? (size_t)z * m * n * sizeof(float) : 0;
 }
 
+// Forward and data gradient on the small tiles (mnv_gemm_small_kernel) instead of `tile` with as many k ranges as it takes: the
+// number of their own, 0: not.  `slabs`: of the small tiles and of the others.  A slab of a 64 x 64 or
+// 128 x 32 tile takes 0.28 or 0.46 us of a CU, and 0.3 at least.  Products in bf16 parts, the more exact ones, stay.
+// us: 24 -> 32 channels under 3 x 3 on 19 x 44 x 12 12.3 -> 5.8, 80 -> 32 under 5 x 5, stride 2, on 59 x 48 x 20 82 -> 36,
+// data gradient 32 <- 160 under 3 x 3 on 4 x 53 x 52 34 -> 21, 40 <- 48 on 7 x 14 x 41 13.8 -> 7.7.
+const MnvSmallCost kSmallGather{0.0992, 2.8, 2.0, 0.0}, kSmallFilter{0.1824, 4.3, 1.4, 3.9};
+int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats);
+// where their vectors' offsets (channel planes, rows past the last) stay within 32 bits
+bool small_reach(const ConvGeom& g) {
+  const long long lim = (1LL << 28) - 1;
+  return (long long)g.N * g.C * g.HW <= lim && (long long)g.N * g.K * g.HoWo <= lim && (long long)g.K * g.CRS <= lim;
+}
+
 int make_geom(ConvGeom* g, int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh,
               int R, int S) {
   if (N <= 0 || C <= 0 || K <= 0 || H <= 0 || W <= 0 || ph < 0 || pw < 0 || sv <= 0 ||
@@ -1165,6 +1209,16 @@ int small_tile_splits(int tile, int m, int n, int slabs, size_t ws_floats) {
   return want < 2 ? 1 : (int)want;
 }
 
+int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats) {
+  if ((tile != 0 && tile != 3) || tile_rows > 0x7fffffff) return 0;
+  const int splits = small_tile_splits(tile, (int)tile_rows, n, slabs, (size_t)-1);
+  const long long tiles = (tile_rows + kTileM[tile] - 1) / kTileM[tile] * ((n + kTileN[tile] - 1) / kTileN[tile]);
+  const double slab = (tile == 0 ? 0.28 : 0.46) * (double)tiles * splits / mnv_cu_count();
+  double against = fixed + (slab > 0.3 ? slab : 0.3) * ((slabs + splits - 1) / splits);
+  if (splits > 1) against += (tile == 0 ? 2.6 : 3.0) + (tile == 0 ? 1.6 : 0.7) * 8.0 * (double)tile_rows * n * splits / 6e6;
+  return mnv_small_ranges(rows, n, small_slabs, ws_floats, kSmallGather, against);
+}
+
 // Workspace layout of the forward and data-gradient convolutions: the permuted filter
 // (when the fast policy applies) first, then, 256-byte aligned, the partial results.
 size_t align256(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
@@ -1209,6 +1263,29 @@ int fwd_channels(const ConvGeom& g) {
   const int width = fast_channels(g.C, g.K, g.RS, m);
   return off && width && !split_ranges(m, g.K, g.RS * (width / 16), tile, (size_t)-1) ? 0 : width;
 }
+// The forward pass on the small tiles: their k ranges (0: not), and the channels of the permuted filter
+// (0: the filter as it is).  From 16 channels on the generic gathers of padded layers are left for the permuted filter.
+struct SmallForward {
+  int z = 0, width = 0;
+  size_t filter_bytes = 0;
+};
+SmallForward small_forward(const ConvGeom& g, size_t ws_bytes) {
+  SmallForward p;
+  const int m = g.N * g.HoWo, tile = pick_tile(m, g.K), width = fwd_channels(g);
+  if (!small_reach(g)) return p;
+  const int slabs = width ? g.RS * (width / 16) : (g.CRS + 15) / 16;
+  if ((width || unpadded_table(g)) && split_ranges(m, g.K, slabs, tile, (size_t)-1)) return p;
+  p.width = width || unpadded_table(g) || g.C < 16 ? width : fast_channels(g.C, g.K, g.RS, m);
+  if (!p.width && !unpadded_table(g)) return p;
+  p.filter_bytes = (size_t)g.K * g.RS * p.width * sizeof(float);
+  if (p.filter_bytes > ws_bytes) return p;
+  const size_t left = ws_bytes > align256(p.filter_bytes) ? (ws_bytes - align256(p.filter_bytes)) / sizeof(float) : 0;
+  p.z = small_gather_ranges(m, g.K, p.width ? g.RS * (p.width / 16) : slabs, tile, m, slabs, 1.0, left);
+  return p;
+}
+size_t small_bytes(size_t filter_bytes, int z, size_t results) {
+  return z > 1 ? align256(filter_bytes) + z * results * sizeof(float) : filter_bytes;
+}
 // Data gradient: the generic gathers also divide by the strides and lose wherever padding pays.  200 <- 200
 // channels under 3 x 3 on 16 x 14 x 14 65 -> 34 us, 64 x 28 x 28 612 -> 375, under 5 x 5 on 16 x 28 x 28 838 -> 216;
 // 40 <- 40 on 16 x 14 x 14 16.2 -> 13.7.
@@ -1226,6 +1303,7 @@ int bwd_data_channels(const ConvGeom& g) {
 struct PhasePlan {
   int width = 0;  // channels as the policy takes them; 0: the generic gathers
   int tile = 0, parts = 0, splits = 1, phase_rows = 0, slabs = 0;  // parts > 0: bf16 parts with that many k ranges
+  bool small = false;  // the small tiles with `splits`
   size_t filter_bytes = 0, rows = 0;
   size_t partial_bytes(int n) const { return parts > 1 || splits > 1 ? (size_t)(parts ? parts : splits) * rows * n * sizeof(float) : 0; }
 };
@@ -1251,6 +1329,14 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
   if (!p.parts) {
     rows_on(kTileM[p.tile]);
     p.splits = small_tile_splits(p.tile, (int)p.rows, g.C, p.slabs, left);
+    const size_t tile_rows = p.rows;
+    rows_on(MNV_SMALL_TILE);
+    if (const int z = small_reach(g) ? small_gather_ranges((long long)p.rows, g.C, mean, p.tile, (long long)tile_rows, mean, 2.0, left) : 0) {
+      p.small = true;
+      p.splits = z;
+    } else {
+      rows_on(kTileM[p.tile]);
+    }
   }
   // the tiles' rows, and channels, are filled up: not where that multiplies more than the generic gathers
   if ((long long)p.rows * width >= (long long)m * g.K * phases || p.rows > 0x3fffffff) return p;
@@ -1258,6 +1344,16 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
   if (tiles < 512 ? 11 * slabs <= 5 * p.slabs + 42 : slabs < 2) return p;
   p.width = width;
   return p;
+}
+
+// The data gradient of unit strides on the small tiles: their k ranges, 0: not.
+int small_bwd_data(const ConvGeom& g, int width, size_t ws_bytes) {
+  const size_t filter_bytes = (size_t)g.C * g.RS * width * sizeof(float);
+  if (!width || filter_bytes > ws_bytes || !small_reach(g)) return 0;
+  const int m = g.N * g.HW, tile = pick_tile(m, g.C), slabs = g.RS * (width / 16);
+  if (split_ranges(m, g.C, slabs, tile, (size_t)-1)) return 0;
+  const size_t left = ws_bytes > align256(filter_bytes) ? (ws_bytes - align256(filter_bytes)) / sizeof(float) : 0;
+  return small_gather_ranges(m, g.C, slabs, tile, m, slabs, 2.0, left);
 }
 
 // k ranges of the filter gradient: up to 256, and up to 512 for outputs of at most 16384
@@ -1273,7 +1369,7 @@ int bwd_filter_tile(int m, int n) {
   return (m <= 64 || n <= 64) ? 0 : wide_tile(n);
 }
 
-int bwd_filter_splits(int m, int n, int k, size_t ws_floats) {
+int bwd_filter_splits(int m, int n, int k, size_t ws_floats, double* cost = nullptr) {
   const int tile = bwd_filter_tile(m, n);
   const int bm = kTileM[tile], bn = kTileN[tile];
   long long tiles = (long long)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
@@ -1282,7 +1378,35 @@ int bwd_filter_splits(int m, int n, int k, size_t ws_floats) {
   if (max_splits > slabs / 8) max_splits = slabs / 8;
   size_t fit = ws_floats / ((size_t)m * n);
   if ((size_t)max_splits > fit) max_splits = (int)fit;
-  return mnv_pick_splits(tiles, slabs, max_splits, mnv_cu_count());
+  return mnv_pick_splits(tiles, slabs, max_splits, mnv_cu_count(), 0.0, cost);
+}
+
+// The filter gradient on the small tiles instead of k ranges of the others: their number, 0: not; `slabs` as the policies with a
+// table of positions count them.  In us, an estimate of mnv_pick_splits is worth 0.47, 0.74, 0.51 and 0.39 on the four tiles, beside 1.3,
+// 2.6, 4.5 and 3.6 and the partial results at 3.3, 3.9, 3 and 5.6 TB/s (10% off, rms, on 194 layers).
+// us: 352 <- 48 channels under 3 x 3, stride 2, on 2 x 27 x 36 22.8 -> 11.0, 344 <- 40 under 5 x 5 on 43 x 13 25 -> 10,
+// 64 <- 288 on 7 x 26 x 19 48 -> 36.
+int small_filter_ranges(const ConvGeom& g, int slabs, size_t ws_floats) {
+  static const double fixed[4] = {1.3, 2.6, 4.5, 3.6}, unit[4] = {0.468, 0.738, 0.507, 0.385}, bytes[4] = {1.83, 1.55, 1.98, 1.07};
+  if (!small_reach(g)) return 0;
+  double cost;
+  const int tile = bwd_filter_tile(g.CRS, g.K), z = bwd_filter_splits(g.CRS, g.K, g.N * g.HoWo, (size_t)-1, &cost);
+  const double against = fixed[tile] + unit[tile] * cost + (z > 1 ? bytes[tile] * 8.0 * (double)g.CRS * g.K * z / 6e6 : 0.0);
+  return mnv_small_ranges(g.CRS, g.K, slabs, ws_floats, kSmallFilter, against);
+}
+// Positions of an image, as those policies pad them, and whether the table of `taps` taps fits beside the tiles.
+int filter_positions(const ConvGeom& g) { return (g.HoWo + 15) / 16 * 16; }
+bool filter_table(const ConvGeom& g, int taps) { return (size_t)taps * filter_positions(g) * 4 <= 24 * 1024; }
+// Taps whose rows, in (tap, channel) order, meet one tile of `rows`, over all tiles: 1 when `rows` divides
+// C, never more than (rows + C - 1) / C + 1.
+int filter_taps(const ConvGeom& g, int rows) {
+  int taps = 1;
+  for (int m0 = 0; m0 < g.CRS; m0 += rows) {
+    const int last = (m0 + rows - 1 < g.CRS ? m0 + rows - 1 : g.CRS - 1) / g.C;
+    if (last - m0 / g.C + 1 > taps) taps = last - m0 / g.C + 1;
+    if (m0 / rows >= g.C) break;  // the pattern of m0 % C repeats after C tiles
+  }
+  return taps;
 }
 
 }  // namespace
@@ -1293,6 +1417,9 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
                                    int sh, int R, int S) {
   ConvGeom g;
   if (make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S)) return 0;
+  const SmallForward small = small_forward(g, (size_t)-1);
+  const bool wino = mnv_wino_images(N, C, K, H, W, ph, pw, R, S, sv, sh, (size_t)-1);
+  if (small.z && !wino) return small_bytes(small.filter_bytes, small.z, (size_t)N * g.HoWo * K);
   const int width = fwd_channels(g);
   const size_t permuted = (size_t)K * g.RS * width * sizeof(float);
   const int gm = N * g.HoWo, gn = K, slabs = width ? g.RS * (width / 16) : (g.CRS + 15) / 16;
@@ -1302,7 +1429,7 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
   const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);
   if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
-  if (mnv_wino_images(N, C, K, H, W, ph, pw, R, S, sv, sh, (size_t)-1)) {
+  if (wino) {
     const size_t w = mnv_wino_workspace_bytes(N, C, K, H, W, ph, pw, R);
     if (w > need) need = w;
   }
@@ -1325,6 +1452,21 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
                                          workspace && mnv_aligned16(workspace) ? workspace_bytes : 0))
     return mnv_wino_conv(bottom, filter, bias, nullptr, top, N, C, K, H, W, ph, pw, R, 0, relu, images,
                          workspace, workspace_bytes, s);
+  if (const SmallForward small = small_forward(g, workspace ? workspace_bytes : 0); small.z) {
+    float* wp = static_cast<float*>(workspace);
+    float* part = small.z > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(small.filter_bytes)) : nullptr;
+    if (!small.width)
+      return mnv_gemm_small_launch(ConvFwdNP{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, gk >= 16 ? gk / 16 : 1, relu},
+                                   small.z, part, s);
+    rc = permute_filter(filter, wp, K, C, R, S, small.width, false, s);
+    if (rc) return rc;
+    const int spp = small.width / 16;
+    if (small.width != C)
+      return mnv_gemm_small_launch(ConvOneRow<ConvFwd<true, true>, true>{{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}},
+                                   small.z, part, s);
+    return mnv_gemm_small_launch(ConvOneRow<ConvFwd<true>, false>{{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}},
+                                 small.z, part, s);
+  }
   const int tile = pick_tile(gm, gn);
   int width = fwd_channels(g);
   const size_t permuted_bytes = (size_t)K * g.RS * width * sizeof(float);
@@ -1415,6 +1557,8 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
   }
   const int width = bwd_data_channels(g);
   const size_t permuted = (size_t)C * g.RS * width * sizeof(float);
+  const bool wino = mnv_wino_images(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R, S, sv, sh, (size_t)-1);
+  if (const int z = wino ? 0 : small_bwd_data(g, width, (size_t)-1)) return small_bytes(permuted, z, (size_t)N * g.HW * C);
   const int gm = N * g.HW, gn = C, slabs = width ? g.RS * (width / 16) : (K * g.RS + 15) / 16;
   const int splits = small_tile_splits(pick_tile(gm, gn), gm, gn, slabs, (size_t)-1);
   const size_t tail = tail_workspace_bytes(pick_tile(gm, gn), gm, gn, slabs, width);
@@ -1422,7 +1566,7 @@ size_t mnv_conv_bwd_data_workspace_bytes(int N, int C, int K, int H, int W, int 
                      : splits > 1 ? align256(permuted) + (size_t)splits * gm * gn * sizeof(float) : permuted;
   const size_t parts = split_bytes(pick_tile(gm, gn), gm, gn, slabs);
   if (parts && align256(permuted) + parts > need) need = align256(permuted) + parts;
-  if (mnv_wino_images(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R, S, sv, sh, (size_t)-1)) {
+  if (wino) {
     const size_t w = mnv_wino_workspace_bytes(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R);
     if (w > need) need = w;
   }
@@ -1457,6 +1601,11 @@ static int bwd_data_phases(const float* top_diff, const float* filter, const flo
     for (int more = 0; more < 2; ++more) {
       p.d_width[more] = mnv_fastdiv_make(p.wq + more ? p.wq + more : 1);
       p.d_taps[more] = mnv_fastdiv_make(p.sq + more ? p.sq + more : 1);
+    }
+    if (plan.small) {
+      ConvOneRow<decltype(p), decltype(p)::PADDED> q;
+      static_cast<decltype(p)&>(q) = p;
+      return mnv_gemm_small_launch(q, plan.splits, part, s);
     }
     return plan.parts ? launch_parts(p, plan.parts, part, s, 0) : launch_tile(plan.tile, p, plan.splits, part, s);
   };
@@ -1496,6 +1645,13 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
     if (rc) return rc;
     const int spp = width / 16;
     const size_t part_bytes = part ? workspace_bytes - used : 0;
+    if (const int z = small_bwd_data(g, width, workspace_bytes)) {
+      if (width != K)
+        return mnv_gemm_small_launch(ConvOneRow<ConvBwdData<true, true>, true>{{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate}},
+                                     z, part, s);
+      return mnv_gemm_small_launch(ConvOneRow<ConvBwdData<true>, false>{{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate}},
+                                   z, part, s);
+    }
     if (width != K)
       return launch_direct(tile, ConvBwdData<true, true>{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate},
                            splits, part, s, part_bytes);
@@ -1558,6 +1714,9 @@ size_t mnv_conv_bwd_filter_workspace_bytes(int N, int C, int K, int H, int W, in
     const size_t sk = (size_t)(4 * mnv_cu_count() + tiles) * kTileM[tile] * kTileN[tile] * sizeof(float);
     if (tiles <= 4LL * mnv_cu_count() && sk > bytes) bytes = sk;
   }
+  const int small = filter_table(g, ph || pw ? filter_taps(g, MNV_SMALL_TILE) : 1)
+                        ? small_filter_ranges(g, N * (filter_positions(g) / 16), (size_t)-1) : 0;
+  if (small > 1 && (size_t)small * g.CRS * K * sizeof(float) > bytes) bytes = (size_t)small * g.CRS * K * sizeof(float);
   if (mnv_wino_grad_images(N, C, K, H, W, ph, pw, R, S, sv, sh, (size_t)-1)) {
     const size_t w = mnv_wino_grad_workspace_bytes(N, C, K, H, W, ph, pw, R);
     if (w > bytes) bytes = w;
@@ -1587,46 +1746,57 @@ static int conv_bwd_filter_impl(const float* bottom, const float* top_diff, floa
   const int tile = bwd_filter_tile(gm, gn);
   // Fast addressing: rows in (tap, channel) order with per-tap offset tables in LDS.  The
   // tables of all taps a 128-row tile touches must fit beside the tiles.
-  const int PP = (g.HoWo + 15) / 16 * 16;
-  // Taps whose rows meet one 128-row tile, over all tiles (rows are in (tap, channel) order
-  // and tiles start at multiples of 128): 1 when 128 divides C, 2 for C = 96, never more than
-  // (128 + C - 1) / C + 1.  Sized exactly, conv2's tables (C = 96, 27 x 27 positions) take
-  // 5.9 KB instead of 8.8 KB, which is what lets four workgroups share a CU's 160 KB of LDS.
-  int taps_per_block = 1;
-  for (int m0 = 0; m0 < gm; m0 += 128) {
-    const int last = (m0 + 127 < gm ? m0 + 127 : gm - 1) / C;
-    if (last - m0 / C + 1 > taps_per_block) taps_per_block = last - m0 / C + 1;
-    if (m0 / 128 >= C) break;  // the pattern of m0 % C repeats after C tiles
-  }
+  const int PP = filter_positions(g);
+  // Sized exactly, conv2's tables (C = 96, 27 x 27 positions) take 5.9 KB instead of 8.8 KB, which is what
+  // lets four workgroups share a CU's 160 KB of LDS.
+  const int taps_per_block = filter_taps(g, 128);
+  // On the small tiles, where they are the faster ones: sets `done`.
+  auto small = [&](bool* done) -> int {
+    const bool np = ph == 0 && pw == 0;
+    const int taps = np ? 1 : filter_taps(g, MNV_SMALL_TILE), slabs = N * (PP / 16);
+    const int z = filter_table(g, taps) ? small_filter_ranges(g, slabs, workspace ? workspace_bytes / sizeof(float) : 0) : 0;
+    *done = z > 0;
+    if (!z) return MNV_OK;
+    if (plan) {
+      plan[0] = MNV_SMALL_TILE;
+      plan[1] = z;
+      return MNV_OK;
+    }
+    if (np)
+      return mnv_gemm_small_launch(ConvBwdFilterFast<true>{bottom, top_diff, filter_diff, g, gm, gn, gk, slabs, PP / 16, PP, 1,
+                                                           mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale}, z, workspace, s);
+    return mnv_gemm_small_launch(ConvBwdFilterFast<false>{bottom, top_diff, filter_diff, g, gm, gn, gk, slabs, PP / 16, PP, taps,
+                                                          mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale}, z, workspace, s);
+  };
   if (tile != 0 && ph == 0 && pw == 0 && (size_t)PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<true> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                               PP / 16, PP, 1, mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale};
-    return launch_filter_gradient<true>(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient<true>(tile, p, splits, workspace, workspace_bytes, s, plan, small);
   }
   if (tile != 0 && C % 128 == 0 && (size_t)PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<false, 1> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                                   PP / 16, PP, 1, mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale};
-    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan, small);
   }
   if (tile != 0 && C % 16 == 0 && taps_per_block == 2 && (size_t)taps_per_block * PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<false, 3> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                                   PP / 16, PP, taps_per_block, mnv_fastdiv_make(C), accumulate,
                                   sgd_w, sgd_scale};
-    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan, small);
   }
   if (tile != 0 && C % 16 == 0 && (size_t)taps_per_block * PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<false, 2> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                                   PP / 16, PP, taps_per_block, mnv_fastdiv_make(C), accumulate,
                                   sgd_w, sgd_scale};
-    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan, small);
   }
   if (tile != 0 && (size_t)taps_per_block * PP * 4 <= 24 * 1024) {
     ConvBwdFilterFast<false> p{bottom, top_diff, filter_diff, g, gm, gn, gk, N * (PP / 16),
                                PP / 16, PP, taps_per_block, mnv_fastdiv_make(C), accumulate, sgd_w, sgd_scale};
-    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+    return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan, small);
   }
   ConvBwdFilter p{bottom, top_diff, filter_diff, g, gm, gn, gk, (gk + 15) / 16, 1, accumulate, sgd_w, sgd_scale};
-  return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan);
+  return launch_filter_gradient(tile, p, splits, workspace, workspace_bytes, s, plan, small);
 }
 
 int mnv_conv_bwd_filter(const float* bottom, const float* top_diff, float* filter_diff, int N,

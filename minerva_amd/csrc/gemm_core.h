@@ -200,6 +200,16 @@ template <class P>
 struct MnvCPreload<P, std::enable_if_t<P::C_PRELOAD>> {
   static constexpr bool value = true;
 };
+// A policy that only fetches differently from another and shares its store names that one, StoredBy: their
+// partial results are then added by the same kernel.
+template <class P, class = void>
+struct MnvStoredBy {
+  typedef P type;
+};
+template <class P>
+struct MnvStoredBy<P, std::void_t<typename P::StoredBy>> {
+  typedef typename P::StoredBy type;
+};
 // What mnv_tail_plan prices a cut tail with, in us of a CU's time: a slab of a workgroup, and its first
 // loads and last stores.  slab 0: not priced.
 struct MnvTailCost {
@@ -795,6 +805,129 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
   }  // for (;;)
 }
 
+// Small tiles for products that the tiles above leave most CUs without, or in k ranges that cost more to add than to
+// multiply: T x T, one per workgroup, whose W wavefronts share the workgroup's k range.  No operand passes through LDS: a lane fetches the four k of a vector for its own row and its
+// own column through the policy (both operands k-fast), three slabs ahead, and multiplies them; lane group h (of 64 / T)
+// holds the k 4 h .. 4 h + 3 of each run of 4 * 64 / T.  The wavefronts' sums (two per value, of the even and the odd slabs) are
+// added in LDS in the order of k, or left as a partial result per k range of blockIdx.z.  Neighbouring tiles
+// across the shorter side of the result share an XCD.  What bounds it, and where it is taken: mnv_small_ranges.
+#define MNV_SMALL_TILE 32
+template <class P, int T, int W>
+__global__ __launch_bounds__(W * MNV_WAVE) void mnv_gemm_small_kernel(P prob, int tiles_m, int tiles_n, int slabs_per_split,
+                                                                      float* __restrict__ partial) {
+  static_assert(P::A_KFAST && P::B_KFAST && !MnvALaneK<P>::value, "vectors of four k");
+  constexpr int H = MNV_WAVE / T, RUN = 4 * H, VECS = 16 / RUN, REGS = T * T / MNV_WAVE;
+  typedef float Acc __attribute__((ext_vector_type(REGS)));
+  extern __shared__ float mnv_small_lds[];  // W tiles of sums, then the policy's
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
+  const int x = lane % T, h = lane / T;
+  int tile_m, tile_n;
+  if constexpr (MnvPhased<P>::value) {
+    mnv_tile_coords(prob, (int)blockIdx.x, T, tiles_m, tiles_n, tile_m, tile_n);
+  } else {
+    const int tile = mnv_tile_remap((int)blockIdx.x, tiles_m * tiles_n);
+    const bool tall = tiles_m > tiles_n;
+    const int across = tall ? tiles_n : tiles_m, outer = tile / across, inner = tile - outer * across;
+    tile_m = tall ? outer : inner;
+    tile_n = tall ? inner : outer;
+  }
+  const int m0 = tile_m * T, n0 = tile_n * T;
+  const int total_slabs = mnv_tile_slabs(prob, m0, slabs_per_split);
+  int begin = blockIdx.z * slabs_per_split, end = begin + slabs_per_split;
+  if (end > total_slabs) end = total_slabs;
+  if (begin > end) begin = end;
+  const int per = (end - begin + W - 1) / W;
+  begin += wave * per;
+  if (begin > end) begin = end;
+  if (end > begin + per) end = begin + per;
+
+  typename P::Res res;
+  prob.make_res(res);
+  prob.block_init(res, mnv_small_lds + W * T * T, m0, n0);
+  typename P::AState ast;
+  typename P::BState bst;
+  prob.a_init(res, ast, m0 + x);
+  prob.b_init(res, bst, n0 + x);
+  unsigned aoff[VECS][P::A_NOFF], boff[VECS][P::B_NOFF];
+  int period = begin / prob.spp, s = begin - period * prob.spp;
+  auto new_period = [&]() {
+#pragma unroll
+    for (int j = 0; j < VECS; ++j) {
+      prob.a_period(ast, aoff[j], m0 + x, RUN * j + 4 * h, period);
+      prob.b_period(bst, boff[j], n0 + x, RUN * j + 4 * h, period);
+    }
+  };
+  float a[4][VECS][4], b[4][VECS][4];
+  int period_of[4] = {}, s_of[4] = {};
+  auto fetch = [&](auto SET) {
+    constexpr int set = decltype(SET)::value;
+    period_of[set] = period;
+    s_of[set] = s;
+#pragma unroll
+    for (int j = 0; j < VECS; ++j) {
+      prob.a_load(res, ast, aoff[j], period, s, RUN * j + 4 * h, a[set][j]);
+      prob.b_load(res, bst, boff[j], period, s, RUN * j + 4 * h, b[set][j]);
+    }
+    if (++s == prob.spp) {
+      s = 0;
+      ++period;
+      new_period();
+    }
+  };
+  Acc acc[2] = {0.f, 0.f};
+  __syncthreads();  // block_init may have written LDS
+  typedef std::integral_constant<int, 0> Set0;
+  typedef std::integral_constant<int, 1> Set1;
+  typedef std::integral_constant<int, 2> Set2;
+  typedef std::integral_constant<int, 3> Set3;
+  if (begin < end) {
+    new_period();
+    fetch(Set0{});
+    fetch(Set1{});
+    fetch(Set2{});
+  }
+  auto step = [&](auto SET) {
+    constexpr int set = decltype(SET)::value;
+    fetch(std::integral_constant<int, (set + 3) % 4>{});  // past the range: not multiplied
+#pragma unroll
+    for (int j = 0; j < VECS; ++j) {
+      if constexpr (MnvAStashFix<P>::value) prob.a_stash_fix(period_of[set], s_of[set], RUN * j + 4 * h, a[set][j]);
+      if constexpr (MnvBStashFix<P>::value) prob.b_stash_fix(period_of[set], s_of[set], RUN * j + 4 * h, b[set][j]);
+    }
+#pragma unroll
+    for (int j = 0; j < VECS; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (T == 32) acc[set & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], acc[set & 1], 0, 0, 0);
+        else acc[set & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], acc[set & 1], 0, 0, 0);
+      }
+  };
+  int steps = end - begin;
+  for (; steps >= 4; steps -= 4) {
+    step(Set0{});
+    step(Set1{});
+    step(Set2{});
+    step(Set3{});
+  }
+  if (steps > 0) step(Set0{});
+  if (steps > 1) step(Set1{});
+  if (steps > 2) step(Set2{});
+  // register r of lane (x, h): row x, column 4 h + r % 4 + 8 (r / 4)
+#pragma unroll
+  for (int r = 0; r < REGS; ++r) mnv_small_lds[wave * T * T + (4 * h + r % 4 + 8 * (r / 4)) * T + x] = acc[0][r] + acc[1][r];
+  __syncthreads();
+  for (int e = threadIdx.x; e < T * T; e += W * MNV_WAVE) {
+    float sum = mnv_small_lds[e];
+#pragma unroll
+    for (int w = 1; w < W; ++w) sum += mnv_small_lds[w * T * T + e];
+    const int m = m0 + e % T, n = n0 + e / T;
+    if (m < prob.M && n < prob.N) {
+      if (gridDim.z > 1) partial[((size_t)blockIdx.z * prob.N + n) * prob.M + m] = sum;
+      else prob.c_store(m, n, sum);
+    }
+  }
+}
+
 // Sums the per-split partial results in a fixed order (deterministic) and hands each
 // element to the policy's store.  ZL threads share one output element: thread z of them
 // adds the partial results z, z + ZL, z + 2 ZL, ... and the ZL sums are added in order
@@ -1092,6 +1225,55 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
     rc = mnv_gemm_reduce_launch(prob, reinterpret_cast<const float*>(workspace), splits, s);
   }
   return rc;
+}
+
+// Number of k ranges with which an m x n product of `slabs` takes the small tiles, four wavefronts each; 0: it does not, their
+// estimate is not below 87% of `against`, us of the launch that they compete with, or the partial results of its ranges
+// do not fit.  A slab of a tile takes 0.1 us of a CU for the convolutions' passes over positions, 0.18 for
+// the filter gradients, whose rows are scattered over channel planes (`slab_us`); from one tile per CU on those of all
+// CUs add up, and a tile's time is that of its own before; beyond the five workgroups that a CU holds, 3.4 us a round; `reduce_us` and
+// `byte_factor` (of 6 TB/s) for the reduction of the k ranges.  `fixed`: beside what the competitor has too.  Fitted to 260
+// layers of up to 12 GFLOP with 1 to 64 ranges (15 to 20% off, rms): by this rule their forward passes, data and filter gradients
+// take 0.83, 0.83 and 0.88 of the time, with the fastest ranges throughout 0.81, 0.81 and 0.85.  Sixteen-row tiles
+// (0.90, 0.92, 0.93 by themselves) and eight wavefronts add 1%.
+struct MnvSmallCost {
+  double slab_us, reduce_us, byte_factor, fixed;
+};
+static inline int mnv_small_ranges(long long m, int n, int slabs, size_t ws_floats, const MnvSmallCost& c, double against) {
+  const long long tiles = (m + MNV_SMALL_TILE - 1) / MNV_SMALL_TILE * ((n + MNV_SMALL_TILE - 1) / MNV_SMALL_TILE);
+  const int cus = mnv_cu_count();
+  if (tiles > 0x3fffffff) return 0;
+  double best = 0.87 * against;
+  int best_z = 0;
+  for (int z = 1; z <= 32 && (z == 1 || (tiles * z <= 8LL * cus && slabs / z >= 8 && (size_t)z <= ws_floats / ((size_t)m * n))); z *= 2) {
+    const double per_cu = (double)tiles * z / cus, own = 0.93 * (double)((tiles * z + cus - 1) / cus);
+    double cost = c.fixed + c.slab_us * (per_cu > own ? per_cu : own) * slabs / z + (per_cu > 5.0 ? 3.4 * (per_cu / 5.0 - 1.0) : 0.0);
+    if (z > 1) cost += c.reduce_us + c.byte_factor * 8.0 * (double)m * n * z / 6e6;
+    if (cost < best * (best_z ? 0.97 : 1.0)) {
+      best = cost;
+      best_z = z;
+    }
+  }
+  return best_z;
+}
+
+// Host-side launch of the small tiles; `splits` > 1 needs splits * M * N floats at `workspace`.
+template <class P>
+static int mnv_gemm_small_launch(const P& prob, int splits, void* workspace, hipStream_t s) {
+  constexpr int T = MNV_SMALL_TILE, W = 4;
+  const int tiles_m = (prob.M + T - 1) / T, tiles_n = (prob.N + T - 1) / T;
+  if (splits > prob.total_slabs) splits = prob.total_slabs;
+  if (splits < 1) splits = 1;
+  const int per = (prob.total_slabs + splits - 1) / splits;
+  splits = per > 0 ? (prob.total_slabs + per - 1) / per : 1;
+  const size_t lds = W * T * T * sizeof(float) + prob.extra_lds_bytes();
+  if ((long long)tiles_m * tiles_n > 0x7fffffffLL || splits > 65535 || lds > 64 * 1024) return MNV_ERR_INVALID;
+  hipLaunchKernelGGL((mnv_gemm_small_kernel<P, T, W>), dim3(tiles_m * tiles_n, 1, splits), dim3(W * MNV_WAVE), lds, s, prob,
+                     tiles_m, tiles_n, per, reinterpret_cast<float*>(workspace));
+  const int rc = MNV_LAUNCH_STATUS();
+  if (rc || splits == 1) return rc;
+  const typename MnvStoredBy<P>::type& stored = prob;
+  return mnv_gemm_reduce_launch(stored, reinterpret_cast<const float*>(workspace), splits, s);
 }
 
 // Stream-k launch of one tile configuration (see mnv_gemm_kernel): as many workgroups as the

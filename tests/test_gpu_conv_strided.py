@@ -50,15 +50,15 @@ def test_strided_data_gradient_matches_the_oracle(gpu, p):
 
 @pytest.mark.parametrize("share", [0.0, 0.4, 0.999, 1.5])
 def test_any_workspace_gives_the_gradient(gpu, share):
-    """The queried bytes give k ranges; fewer give fewer ranges, or the generic gathers where the
-    permuted filter has no room."""
+    """The queried bytes, fewer, which give fewer k ranges or the generic gathers where the
+    permuted filter has no room, and more."""
     p = (13, 24, 232, 49, 19, 0, 0, 2, 2, 3, 3)
     N, C, K, H, W = p[:5]
     cv = Conv(gpu, *p)
     dy, w = _rand(N * K * cv.Ho * cv.Wo, 7), _rand(K * C * 9, 8)
     query = gpu.L.mnv_conv_bwd_data_workspace_bytes(*p)
     filter_bytes = 4 * C * 9 * 240
-    assert query > filter_bytes
+    assert query >= filter_bytes
     nbytes = int(share * query) if share else filter_bytes
     ddy, dw, out = gpu.up(dy), gpu.up(w), gpu.up(np.full(N * C * H * W, np.nan, np.float32))
     ws = gpu.empty(nbytes // 4 + 1)
