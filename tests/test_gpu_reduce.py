@@ -1,6 +1,8 @@
 """GPU parity of reductions, arg-max, softmax and transpose against the CPU oracle.
 Bit-exact: max, arg-max indices (ties, NaN), transpose.  Normwise <= 1e-4: sums and
 softmax forward/backward."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -244,3 +246,21 @@ def test_large_operand_paths_8192x8192(gpu):
     assert_bits_equal(gpu.down(dz), (x.reshape(n, m) + vec[:, None]).ravel(), "norm_add_col 8192")
     gpu.call("mnv_norm_add_row", dx.p, dv.p, dz.p, m, n)   # res[r + c*m] = x[r + c*m] + vec[r]
     assert_bits_equal(gpu.down(dz), (x.reshape(n, m) + vec[None, :]).ravel(), "norm_add_row 8192")
+
+
+@pytest.mark.parametrize("N,K,H,W", [(5, 3, 2, 2), (7, 5, 1, 5), (9, 17, 3, 9), (64, 2, 16, 16), (65, 3, 16, 16), (128, 2, 32, 16),
+                                     (1, 2, 255, 257), (4, 3, 1, 3), (300, 2, 7, 31)])
+def test_bias_gradients_of_short_channels(gpu, N, K, H, W):
+    """One workgroup per channel up to 16384 vectors of four, two launches beyond: planes of 4 values and
+    more on and off the multiples of 4, one vector short of and past a round, and the infinities of other channels."""
+    rng = np.random.default_rng(N * K + H)
+    dy = rng.standard_normal((N, K, H * W)).astype(np.float32)
+    dy[0, 0, 0] = np.inf
+    d, out = gpu.up(dy.reshape(-1)), gpu.up(np.full(K, np.nan, np.float32))
+    nbytes = gpu.L.mnv_conv_bwd_bias_workspace_bytes(N, K)
+    ws = gpu.empty(nbytes // 4 + 1)
+    gpu.call("mnv_conv_bwd_bias", d.p, out.p, N, K, H, W, ws.p, ctypes.c_size_t(nbytes))
+    got, want = gpu.down(out), dy.astype(np.float64).sum((0, 2))
+    assert got[0] == np.inf
+    # a tree of sums: at most 64 roundings of 2^-24 of sums within the sum of the magnitudes
+    assert np.all(np.abs(got[1:] - want[1:]) <= 64 * 2.0 ** -24 * np.abs(dy[:, 1:].astype(np.float64)).sum((0, 2)))
