@@ -57,7 +57,7 @@ HipDevice::~HipDevice() {
   data_store_.reset();  // before the streams: the deallocator uses the device
   for (size_t i = 0; i < kParallelism; ++i) {
     if (workspace_[i]) mnv_free(workspace_[i]);
-    if (staging_[i]) mnv_host_free(staging_[i]);
+    if (staging_[i].base) mnv_host_free(staging_[i].base);
     mnv_stream_destroy(streams_[i]);
   }
 }
@@ -150,8 +150,13 @@ void HipDevice::EnsureWorkspace(int thrid, size_t bytes) {
 }
 
 void HipDevice::EnsureStaging(int thrid) {
-  if (staging_[thrid]) return;
-  Ok(mnv_host_malloc(&staging_[thrid], kStagingBytes), "pinned staging");
+  StagingArea& area = staging_[thrid];
+  std::lock_guard<std::mutex> lock(area.mutex);
+  if (area.base) return;
+  void* p = nullptr;
+  Ok(mnv_host_malloc(&p, kStagingBytes), "pinned staging");
+  area.base = static_cast<char*>(p);
+  area.half = kStagingBytes / 2;
 }
 
 // ThreadedDevice::Execute plus what dataflow mode needs: waits for producers on other
@@ -229,8 +234,7 @@ void HipDevice::DoExecute(const DataList& in, const DataList& out, PhysicalOp& o
   ctx.workspace_bytes = workspace_bytes_[thrid];
   if (!capturing_) {
     EnsureStaging(thrid);
-    ctx.staging = staging_[thrid];
-    ctx.staging_bytes = kStagingBytes;
+    ctx.staging = &staging_[thrid];
   }
   Timed t{std::string(), nullptr, nullptr};
   bool timed = profile_ && !capturing_;
@@ -330,15 +334,22 @@ void HipDevice::CopyToHost(float* dst, uint64_t data_id, size_t floats) {
   const char* src = reinterpret_cast<const char*>(data_store_->GetData(data_id));
   char* out = reinterpret_cast<char*>(dst);
   const size_t bytes = floats * sizeof(float), half = kStagingBytes / 2;
-  if (bytes <= half) {
-    Ok(mnv_memcpy_d2h(out, src, bytes, streams_[0]), "copy to host");
-    Ok(mnv_stream_sync(streams_[0]), "copy to host sync");
-    return;
-  }
-  // large results come back through the pinned staging area, the DMA engine filling one
+  // results come back through the pinned staging area, large ones with the DMA engine filling one
   // half while the CPU empties the other into the caller's pageable buffer
   EnsureStaging(0);
-  char* stage = static_cast<char*>(staging_[0]);
+  std::lock_guard<std::mutex> lock(staging_[0].mutex);
+  if (bytes <= half) {
+    char* at = nullptr;
+    Ok(staging_[0].Take(bytes, streams_[0], &at), "copy to host staging");
+    Ok(mnv_memcpy_d2h(at, src, bytes, streams_[0]), "copy to host");
+    Ok(mnv_stream_sync(streams_[0]), "copy to host sync");
+    staging_[0].Drained();
+    std::memcpy(out, at, bytes);
+    return;
+  }
+  Ok(mnv_stream_sync(streams_[0]), "copy to host sync");  // uploads that the area still holds
+  staging_[0].Drained();
+  char* stage = staging_[0].base;
   void* filled[2] = {nullptr, nullptr};
   Ok(mnv_event_create_ordering(&filled[0]), "event create");
   Ok(mnv_event_create_ordering(&filled[1]), "event create");
@@ -377,8 +388,9 @@ void HipDevice::CopyFromHostOn(int thrid, uint64_t data_id, const float* src, si
   Activate();
   EnsureStaging(thrid);
   Ok(StagedHostToDevice(data_store_->GetData(data_id), src, floats * sizeof(float), streams_[thrid],
-                        staging_[thrid], kStagingBytes),
+                        &staging_[thrid]),
      "copy from host");
+  Ok(mnv_stream_sync(streams_[thrid]), "copy from host sync");
 }
 
 void* HipDevice::StreamMarker(int thrid) {

@@ -20,6 +20,7 @@
 #include <unordered_map>
 
 #include "device.h"
+#include "staged_copy.h"
 #include "op_dispatch.h"
 
 namespace minerva {
@@ -130,7 +131,7 @@ class HipDevice : public ThreadedDevice {
   std::array<void*, kParallelism> streams_{};
   std::array<void*, kParallelism> workspace_{};
   std::array<size_t, kParallelism> workspace_bytes_{};
-  std::array<void*, kParallelism> staging_{};  // pinned host memory, allocated at first use
+  std::array<StagingArea, kParallelism> staging_;  // pinned host memory, allocated at first use
   std::mutex local_mutex_;  // guards produced_
   struct Timed {
     std::string name;

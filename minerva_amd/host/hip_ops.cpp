@@ -484,12 +484,10 @@ void Select(const DataList& inputs, const DataList& outputs, SelectClosure& c, c
 void ArrayLoader(const DataList& outputs, ArrayLoaderClosure& closure, const Context& ctx) {
   MNV_CHECK_EQ(outputs.size(), 1u) << "(array loader) #outputs wrong";
   MNV_CHECK(closure.data) << "probably already executed";
-  // on the operator's own stream (the reference uses the default stream, cuda.cpp:595); large
-  // pageable buffers go through the stream's pinned staging area; synchronised, because the
-  // host buffer must outlive the copy
+  // on the operator's own stream (the reference uses the default stream, cuda.cpp:595), through the
+  // stream's pinned staging area, so that the host buffer need not outlive the copy
   const size_t bytes = outputs[0].size_.Prod() * sizeof(float);
-  Ok(StagedHostToDevice(outputs[0].data_, closure.data.get(), bytes, ctx.stream, ctx.staging,
-                        ctx.staging_bytes),
+  Ok(StagedHostToDevice(outputs[0].data_, closure.data.get(), bytes, ctx.stream, ctx.staging),
      "array loader");
   closure.data.reset();
 }
