@@ -572,22 +572,30 @@ double split_cost(int m, int n, int k, int z, int cus) {
 //   4096 x 1000 x 1000 76 -> 48, 4096 x 100 x 4096 47 -> 32, 200 x 3000 x 4000 67 -> 48, 1500 x 1500 x 1500
 //   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
 //   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
-//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0
+//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.  From 65 tiles of 128 x 128 on the grouped ones are
+//   weighed too, at 0.84 us per unit of their estimate: 341 x 3956 x 1002 41 -> 34, 2177 x 1155 x 3047 201 -> 129, 3106 x
+//   1474 x 2652 226 -> 162, 768 x 2173 x 715 32 -> 31; 120 random products that it moves 0.82 of the time, half the error.
 void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {
   if (plan->tall || (!plan->small && plan->groups == 4)) {
     plan->split = true;
     return;
   }
-  if (plan->groups == 4 || m <= 64 || n <= 64) return;
+  if (m <= 64 || n <= 64) return;
   // One slab fills half of a step, and what such a product takes is the time of its stores, which the fp32 kernel, with
   // twice the workgroups per CU, spreads better (fp32 instruction / parts, us: k = 16 4096 x 4096 16.4 / 18.9, 4096 x 9216
   // 30.0 / 33.7, k = 17 20.4 / 18.3, 38.9 / 32.4).  Those planned on 64 x 64 tiles gain as little by parts as they lose.
   if (k <= 16 && !plan->small) return;
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
+  if (plan->groups == 4 && tiles <= 64) return;
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
   int best_z = 1;
   double best = split_cost(m, n, k, 1, cus);
+  // of tiles that a cut tail spreads evenly
+  if (plan->groups == 4 && mnv_tail_plan(tiles, slabs, 128 * 128, (size_t)-1 / sizeof(float), SplitPair::TAIL).z > 1) {
+    const double cut = 1.3 * ((double)tiles / cus + 0.25) * ((slabs + 1) / 2) + 6.0;
+    if (cut < best) best = cut;
+  }
   for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus; ++z) {
     const double c = split_cost(m, n, k, z, cus);
     if (c < 0.97 * best) {
@@ -597,7 +605,7 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, Sge
   }
   // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
   // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6).
-  if (plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
+  if (plan->groups == 4 ? best > 0.9 * 0.84 * cost : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
   *plan = SgemmPlan{false, best_z};
   plan->split = true;
 }
