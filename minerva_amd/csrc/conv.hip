@@ -286,9 +286,9 @@ struct ConvFwdNP {
 // flat order's vectors straddle filter rows and take a 4-byte load per pixel.  The order of the
 // slots of a group is that of the pixels, against that of the taps.  A row's last group ends with the
 // row as well and so begins with a tap that the group before it has: its slot 3 reads as 0 in both operands.
-// The table holds, for every group, the pixel's and the filter's byte offset, bit 0 of the first
-// marking a last group with a slot to clear.  3 -> 96 channels under 11 x 11 at stride 4 on 256 x 227 x
-// 227: 555 us with the fp32 instruction, 537 in parts in the flat order, 498 so.
+// The table holds, for every group, the byte offsets of its pixels and its filter values.  3 -> 96 channels under 11 x 11
+// at stride 4 on 256 x 227 x
+// 227: 555 us with the fp32 instruction, 537 in parts in the flat order, 432 so.
 struct ConvFwdRows : ConvFwdNP {
   static constexpr int B_NOFF = 1;
   int groups, per_row;  // C * R * per_row, ceil(S / 4); K, total_slabs and spp count the slots
@@ -312,7 +312,7 @@ struct ConvFwdRows : ConvFwdNP {
       const int c = mnv_fastdiv(row, d_R), rp = row - c * g.R;
       const int first = q == per_row - 1 ? g.S - 4 : 4 * q;            // the group's first tap s'
       const unsigned pixel = (unsigned)(c * g.HW + (g.R - 1 - rp) * g.W + g.S - 4 - first) * 4u;
-      tab[2 * i] = i < groups ? pixel | (first != 4 * q ? 1u : 0u) : MNV_OOB;
+      tab[2 * i] = i < groups ? pixel : MNV_OOB;
       tab[2 * i + 1] = i < groups ? (unsigned)(row * g.S + first) * 4u : MNV_OOB;
     }
   }
@@ -321,9 +321,21 @@ struct ConvFwdRows : ConvFwdNP {
   __device__ void a_load(const Res& r, const AState&, const unsigned (&off)[1], int period, int s, int kl,
                          float (&v)[4]) const {
     const unsigned t = r.tab[2 * ((period * spp + s) * 4 + (kl >> 2))];
-    const unsigned one[1] = {off[0] + (t & ~1u)};
+    const unsigned one[1] = {off[0] + t};
     mnv_fetch_vec<1>(r.a, one, 0, v);
-    v[3] = t & 1u ? 0.f : v[3];
+  }
+  // What a row's last group has to clear is cleared on the way to LDS, and the filter's vector is reversed
+  // there: made where it is loaded, every step waited for its own loads (256 images of 3 x 227 x 227 467 -> 432 us, 50 100 -> 96; the same bits).
+  static constexpr bool A_STASH_FIX = true, B_STASH_FIX = true;
+  __device__ bool cut(int period, int s, int kl) const {
+    const int i = (period * spp + s) * 4 + (kl >> 2);
+    return g.S % 4 != 0 && i - mnv_fastdiv(i, d_per_row) * per_row == per_row - 1;
+  }
+  __device__ void a_stash_fix(int period, int s, int kl, float (&v)[4]) const { v[3] = cut(period, s, kl) ? 0.f : v[3]; }
+  __device__ void b_stash_fix(int period, int s, int kl, float (&v)[4]) const {
+    const float first = v[0], second = v[1];
+    v[0] = v[3]; v[1] = v[2]; v[2] = second;
+    v[3] = cut(period, s, kl) ? 0.f : first;
   }
   __device__ void b_period(const BState&, unsigned (&off)[1], int n, int, int) const {
     off[0] = n < N ? (unsigned)(n * g.CRS) * 4u : MNV_OOB;
@@ -333,10 +345,7 @@ struct ConvFwdRows : ConvFwdNP {
     typedef unsigned u2 __attribute__((ext_vector_type(2)));
     const u2 t = *reinterpret_cast<const u2*>(__builtin_assume_aligned(r.tab + 2 * ((period * spp + s) * 4 + (kl >> 2)), 8));
     const unsigned one[1] = {(off[0] | t.y) & MNV_OOB ? MNV_OOB : off[0] + t.y};
-    float f[4];
-    mnv_fetch_vec<1>(r.b, one, 0, f);
-    v[0] = f[3]; v[1] = f[2]; v[2] = f[1];
-    v[3] = t.x & 1u ? 0.f : f[0];
+    mnv_fetch_vec<1>(r.b, one, 0, v);
   }
 };
 
