@@ -810,6 +810,10 @@ struct WinoGradGemm {
 // fp32 instruction on 128 x 128 tiles, us: 12544 x 64 * 256 x 96 395 -> 350, 2304 x 49 * 384 x 256
 // 185 -> 134, filter gradients of conv2-5 at batch 256 1062 -> 815 in all.
 typedef MnvSplitTile<128, 128, 2, 4, 1> TileBig;
+// The filter gradient's k is long: four wavefronts of 64 x 64 read a third less of LDS per product than eight
+// of 64 x 32.  96 -> 256 of 5 x 5 on 27 x 27, 50 / 256 images, 151.9 -> 140.0 / 601 -> 595 us with the transforms;
+// 128 -> 256 of 3 x 3 on 32 x 56 x 56 207 -> 202.  The short products of the other passes lose 1 to 2 % by it.
+typedef MnvSplitTile<128, 128, 2, 2, 1> TileGrad;
 
 // Measurement aid (mnv_conv_winograd_profile): while it is on, every launch of the products
 // is bracketed by an event pair on its stream, so that a benchmark can time the MFMA kernel of
@@ -1065,7 +1069,7 @@ int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_d
     plan[0] = 128;
     plan[1] = 1;
     plan[2] = 0;
-    return mnv_gemm_streamk_launch<TileBig>(p, w, sk_bytes, s, &done, plan + 2);
+    return mnv_gemm_streamk_launch<TileGrad>(p, w, sk_bytes, s, &done, plan + 2);
   }
   int rc;
   const size_t per_bottom = (size_t)C * g.Hs * g.Ws, per_top = (size_t)K * g.Hd * g.Wd;
@@ -1086,8 +1090,8 @@ int wino_filter_grad(const WinoGeom& g0, const float* bottom, const float* top_d
     bool done = false;
     hipEvent_t e0, e1;
     const bool timed = profile_begin(&e0, &e1, s);
-    rc = mnv_gemm_streamk_launch<TileBig>(p, w, sk_bytes, s, &done);
-    if (!rc && !done) rc = mnv_gemm_launch<TileBig>(p, 1, nullptr, s);
+    rc = mnv_gemm_streamk_launch<TileGrad>(p, w, sk_bytes, s, &done);
+    if (!rc && !done) rc = mnv_gemm_launch<TileGrad>(p, 1, nullptr, s);
     if (timed) profile_end(e0, e1, s, 1, 2.0 * AL * AL * K * C * g.P);
     if (rc) return rc;
   }
