@@ -572,9 +572,11 @@ double split_cost(int m, int n, int k, int z, int cus) {
 //   4096 x 1000 x 1000 76 -> 48, 4096 x 100 x 4096 47 -> 32, 200 x 3000 x 4000 67 -> 48, 1500 x 1500 x 1500
 //   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
 //   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
-//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.  From 65 tiles of 128 x 128 on the grouped ones are
-//   weighed too, at 0.84 us per unit of their estimate: 341 x 3956 x 1002 41 -> 34, 2177 x 1155 x 3047 201 -> 129, 3106 x
-//   1474 x 2652 226 -> 162, 768 x 2173 x 715 32 -> 31; 120 random products that it moves 0.82 of the time, half the error.
+//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.  Beyond 16 tiles of 128 x 128, whose 16 k ranges at most make no
+//   more workgroups than CUs, the grouped ones are weighed too, at 0.84 us per unit of their estimate: 341 x 3956 x 1002 41 -> 34,
+//   2177 x 1155 x 3047 201 -> 129, 3106 x 1474 x 2652 226 -> 162, 1340 x 599 x 3458 70 -> 49, 200 x 3319 x 2055 44 -> 33, 2048 x 300 x 3000
+//   43 -> 35; 120 random products of 65 tiles and more that it moves 0.82 of the time, half the error, 60 of fewer 0.78 and 0.40.  Grouped tiles of exactly one per CU
+//   are the plan that the inner products of 256 columns are documented to have and stay (*4096 x 256 x 4096 74 -> 56).
 void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {
   if (plan->tall || (!plan->small && plan->groups == 4)) {
     plan->split = true;
@@ -586,7 +588,7 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, Sge
   // 30.0 / 33.7, k = 17 20.4 / 18.3, 38.9 / 32.4).  Those planned on 64 x 64 tiles gain as little by parts as they lose.
   if (k <= 16 && !plan->small) return;
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
-  if (plan->groups == 4 && tiles <= 64) return;
+  if (plan->groups == 4 && (tiles * MNV_SGEMM_MAX_SPLITS <= cus || (plan->splits == 1 && (m + 63LL) / 64 * ((n + 63) / 64) == cus))) return;
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
   int best_z = 1;
@@ -604,8 +606,9 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, Sge
     }
   }
   // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
-  // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6).
-  if (plan->groups == 4 ? best > 0.9 * 0.84 * cost : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
+  // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6), of under 20 us to the small and the
+  // grouped tiles (3312 x 73 x 1235 15.0 -> 18.0, 143 x 2058 x 1764 19.6 -> 21.2).
+  if (plan->groups == 4 ? best > 0.9 * 0.84 * cost || (best_z > 1 && best < 20.0) : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
   *plan = SgemmPlan{false, best_z};
   plan->split = true;
 }
