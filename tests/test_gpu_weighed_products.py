@@ -1,0 +1,49 @@
+"""Products that leave grouped 64 x 64 tiles for 128 x 128 ones in bf16 parts: which do, and their parity against float64
+with the queried workspace, with part of it and without."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from minerva_amd import capi
+
+
+def _plan(m, n, k, ws):
+    v = [ctypes.c_int() for _ in range(3)]
+    assert capi.lib().mnv_sgemm_nn_plan(m, n, k, ctypes.c_size_t(ws), *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+# 17 to 63 tiles of 128 x 128 with k ranges, ragged in every extent; 65 and more, with and without ranges
+MOVED = [(1340, 599, 3458), (2500, 200, 2048), (2048, 300, 3000), (341, 3956, 1002), (2177, 1155, 3047)]
+# at most 16 tiles; one grouped tile per CU; ranges of under 20 us
+STAY = [(200, 1000, 4099), (500, 500, 3000), (1000, 256, 4096), (4096, 256, 4096), (3312, 73, 1235), (143, 2058, 1764)]
+
+
+@pytest.mark.parametrize("m,n,k", MOVED)
+def test_products_weighed_against_the_parts(m, n, k):
+    assert _plan(m, n, k, capi.lib().mnv_sgemm_nn_workspace_bytes(m, n, k))[0::2] == (128, 1)
+
+
+@pytest.mark.parametrize("m,n,k", STAY)
+def test_products_that_stay_on_small_tiles(m, n, k):
+    assert _plan(m, n, k, 1 << 40)[0] == 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", MOVED)
+def test_weighed_products_against_float64(m, n, k):
+    from gpu_util import Gpu, say
+    gpu = Gpu()
+    rng = np.random.default_rng(k)
+    A, B = rng.standard_normal((m, k), np.float32), rng.standard_normal((k, n), np.float32)
+    # sums of k products round at most k times, by 2^-24 of sums within |A||B|; the parts leave out 3 x 2^-25 of a product
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    bound = (k + 8) * 2.0 ** -24 * (np.abs(A) @ np.abs(B)).astype(np.float64)
+    a, b = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(np.ascontiguousarray(B.T).reshape(-1))
+    full = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    for ws in (full, full // 2, 0):
+        say("weighed product", m, n, k, "workspace", ws, "plan", _plan(m, n, k, ws))
+        c, scratch = gpu.up(np.full(m * n, np.nan, np.float32)), gpu.up(np.full(max(1, ws // 4), np.nan, np.float32))
+        gpu.call("mnv_sgemm_nn", a.p, b.p, c.p, m, n, k, scratch.p, ctypes.c_size_t(ws))
+        assert np.all(np.abs(gpu.down(c).reshape(n, m).T - exact) <= bound), ws
