@@ -1324,6 +1324,8 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
   const long long most = (long long)g.N * ((g.H + g.sv - 1) / g.sv) * ((g.W + g.sh - 1) / g.sh);  // rows of a phase
   p.filter_bytes = (size_t)g.C * g.RS * width * sizeof(float);
   if ((long long)g.C * g.RS * width > (1LL << 29) - 1 || ws_bytes < p.filter_bytes) return p;
+  // rows of all phases on the tallest tile: within an int, for tiny phases by the million are not
+  if (phases > 0x3fffffff / ((most + 127) / 128 * 128)) return p;
   const size_t left = ws_bytes > align256(p.filter_bytes) ? (ws_bytes - align256(p.filter_bytes)) / sizeof(float) : 0;
   // what the launch shapes are chosen by: a product of all positions and the mean extent of k
   const int m = g.N * g.HW, mean = (int)(((long long)g.RS * spp + phases - 1) / phases);
@@ -1348,7 +1350,7 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
     }
   }
   // the tiles' rows, and channels, are filled up: not where that multiplies more than the generic gathers
-  if ((long long)p.rows * width >= (long long)m * g.K * phases || p.rows > 0x3fffffff) return p;
+  if ((long long)p.rows * width >= (long long)m * g.K * phases) return p;
   const long long tiles = (m + 63LL) / 64 * ((g.C + 63) / 64), slabs = ((long long)g.K * g.RS + 15) / 16;
   if (tiles < 512 ? 11 * slabs <= 5 * p.slabs + 42 : slabs < 2) return p;
   p.width = width;

@@ -37,3 +37,17 @@ def test_channels_of_small_data_gradients_are_padded_where_it_pays(dims, padded)
 def test_channels_of_forward_passes_are_padded_where_it_pays(C, padded):
     dims = (64, C, 88, 28, 28, 2, 5)
     assert (_query("fwd", *dims) >= 4 * 88 * 25 * ((C + 15) // 16 * 16)) == padded
+
+
+@pytest.mark.parametrize("dims", [  # N, C, K, H, W, ph, pw, sv, sh, R, S
+    (1, 32, 256, 2, 2, 1, 1, 65536, 65536, 3, 3), (1, 16, 16, 1, 1, 0, 0, 8192, 4096, 1, 1),
+    (1, 1, 64, 8192, 4096, 0, 0, 8192, 4096, 1, 1), (1, 2, 16, 15000, 15000, 0, 0, 15000, 15000, 1, 1),
+    (1, 32, 256, 2, 2, 1, 1, 2 ** 31 - 1, 2 ** 31 - 1, 3, 3),
+])
+def test_strides_of_millions_of_classes_have_a_workspace(dims):
+    """A data gradient of strides sv x sh takes its positions in sv * sh classes, whose rows, each class
+    filled up to whole tiles, may be more than an int holds."""
+    N, C, K, H, W, ph, pw, sv, sh, R, S = dims
+    ws = capi.lib().mnv_conv_bwd_data_workspace_bytes(*dims)
+    # no more than the permuted filter and some partial results
+    assert ws <= 4 * C * R * S * ((K + 15) // 16 * 16) + 256 + 64 * 4 * N * H * W * C
