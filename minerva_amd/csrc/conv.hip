@@ -490,7 +490,8 @@ struct ConvBwdData {
 // taken class by class ("phase"): each is a product of its own, the unit-stride correlation of top_diff with
 // every sv-th row and sh-th column of the filter, and all of them are one launch, those with the most taps first.
 // Row class rho = 0 .. sv - 1 meets the taps r' = rho + sv t (R-1-r of the filter); its rows are y = a + sv u
-// with a = (R - 1 - ph - rho) mod sv, and they meet output row u + i0 + t.  Columns likewise.  Every phase has
+// with a = (R - 1 - ph - rho) mod sv, and they meet output row u + i0 + t.  Columns likewise.  Where a stride is beyond the
+// plane, only the classes with a position are taken, by a: stride 20 over 2 x 2 planes has 4 phases, not 400.  Every phase has
 // `phase_rows` rows of the product, (image, u, v) and what fills up to whole tiles; rows past a phase's own read 0
 // and are not stored.  `filter` is the permuted copy [c][taps, phase by phase][k, padded to 16] (PAD as above).
 // What bounds it is what bounds the unit-stride gathers (a trip to memory per slab on the small tiles), and the stores,
@@ -503,14 +504,15 @@ struct ConvBwdDataPhases {
   const float* __restrict__ filter;
   float* __restrict__ bottom_diff;
   ConvGeom g;
-  int M, N, total_slabs, spp;      // sv * sh * phase_rows, C, most taps of a phase * spp
+  int M, N, total_slabs, spp;      // phases * phase_rows, C, most taps of a phase * spp
   const float* __restrict__ gate;  // as in ConvBwdData
   int phase_rows;
   // of class 0: its first row / column, and the output row / column that this one meets with its first tap
   int a0, b0, i00, j00;
   // H, W, R, S = stride * quotient + rest: the first `rest` classes have one row, column, tap more
   int hq, hr, wq, wr, rq, rr, sq, sr;
-  MnvFastDiv d_rows, d_plane[4], d_width[2], d_taps[2];  // by [rows more * 2 + columns more], [columns more], [taps more]
+  int col_classes;  // phases = row classes * col_classes
+  MnvFastDiv d_cols, d_rows, d_plane[4], d_width[2], d_taps[2];  // by [rows more * 2 + columns more], [columns more], [taps more]
   struct Phase {
     int a, b, i0, j0, rows_more, cols_more, taps, taps_per_row, tap0;
     MnvFastDiv d_taps_per_row;
@@ -528,7 +530,9 @@ struct ConvBwdDataPhases {
     unsigned off;
   };
   __device__ Phase phase(int q) const {
-    const int rho = mnv_fastdiv(q, g.d_sh), sigma = q - rho * g.sh;
+    int rho = mnv_fastdiv(q, d_cols), sigma = q - rho * col_classes;
+    if (g.sv > g.H) rho = rho <= a0 ? a0 - rho : a0 - rho + g.sv;
+    if (g.sh > g.W) sigma = sigma <= b0 ? b0 - sigma : b0 - sigma + g.sh;
     Phase p;
     p.a = a0 - rho;
     p.i0 = i00;
@@ -936,9 +940,9 @@ __global__ __launch_bounds__(256) void mnv_filter_permute_kernel(const float* __
     const int last = o % width, first = o / (width * RS);
     int rs = (o / width) % RS;
     if (sv > 1 || sh > 1) {
-      int rho = 0, sigma = 0, rows = (R + sv - 1) / sv, cols = (S + sh - 1) / sh;
-      while (rs >= rows * S) rs -= rows * S, ++rho, rows = (R - rho + sv - 1) / sv;
-      while (rs >= rows * cols) rs -= rows * cols, ++sigma, cols = (S - sigma + sh - 1) / sh;
+      int rho = 0, sigma = 0, rows = (R - 1) / sv + 1, cols = (S - 1) / sh + 1;
+      while (rs >= rows * S) rs -= rows * S, ++rho, rows = (R - rho - 1) / sv + 1;
+      while (rs >= rows * cols) rs -= rows * cols, ++sigma, cols = (S - sigma - 1) / sh + 1;
       rs = (rho + sv * (rs / cols)) * S + sigma + sh * (rs % cols);
     }
     const int k = to_crk ? last : first, c = to_crk ? first : last;
@@ -1316,21 +1320,23 @@ struct PhasePlan {
   size_t filter_bytes = 0, rows = 0;
   size_t partial_bytes(int n) const { return parts > 1 || splits > 1 ? (size_t)(parts ? parts : splits) * rows * n * sizeof(float) : 0; }
 };
+// Classes of a dimension's positions modulo the stride that hold one.
+long long phase_classes(int stride, int extent) { return stride < extent ? stride : extent; }
 PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
   PhasePlan p;
   if (g.sv == 1 && g.sh == 1) return p;
   const int width = (g.K + 15) / 16 * 16, spp = width / 16;
-  const long long phases = (long long)g.sv * g.sh;
-  const long long most = (long long)g.N * ((g.H + g.sv - 1) / g.sv) * ((g.W + g.sh - 1) / g.sh);  // rows of a phase
+  const long long phases = phase_classes(g.sv, g.H) * phase_classes(g.sh, g.W);
+  const long long most = (long long)g.N * ((g.H - 1) / g.sv + 1) * ((g.W - 1) / g.sh + 1);  // rows of a phase
   p.filter_bytes = (size_t)g.C * g.RS * width * sizeof(float);
   if ((long long)g.C * g.RS * width > (1LL << 29) - 1 || ws_bytes < p.filter_bytes) return p;
   // rows of all phases on the tallest tile: within an int, for tiny phases by the million are not
   if (phases > 0x3fffffff / ((most + 127) / 128 * 128)) return p;
   const size_t left = ws_bytes > align256(p.filter_bytes) ? (ws_bytes - align256(p.filter_bytes)) / sizeof(float) : 0;
   // what the launch shapes are chosen by: a product of all positions and the mean extent of k
-  const int m = g.N * g.HW, mean = (int)(((long long)g.RS * spp + phases - 1) / phases);
+  p.slabs = ((g.R - 1) / g.sv + 1) * ((g.S - 1) / g.sh + 1) * spp;
+  const int m = g.N * g.HW, mean = (int)std::min<long long>(((long long)g.RS * spp + phases - 1) / phases, p.slabs);
   p.tile = pick_tile(m, g.C);
-  p.slabs = ((g.R + g.sv - 1) / g.sv) * ((g.S + g.sh - 1) / g.sh) * spp;
   auto rows_on = [&](int tile_rows) {
     p.phase_rows = (int)((most + tile_rows - 1) / tile_rows * tile_rows);
     p.rows = (size_t)p.phase_rows * phases;
@@ -1597,13 +1603,15 @@ static int bwd_data_phases(const float* top_diff, const float* filter, const flo
     p.phase_rows = plan.phase_rows;
     // class 0 holds the tap r' = 0, which meets output row i at input row i sv - ph + R - 1
     auto first = [](int reach, int stride, int* at, int* out) {
-      *at = (reach % stride + stride) % stride;
+      *at = reach % stride < 0 ? reach % stride + stride : reach % stride;
       *out = (*at - reach) / stride;
     };
     first(g.R - 1 - g.ph, g.sv, &p.a0, &p.i00);
     first(g.S - 1 - g.pw, g.sh, &p.b0, &p.j00);
     p.hq = g.H / g.sv; p.hr = g.H % g.sv; p.wq = g.W / g.sh; p.wr = g.W % g.sh;
     p.rq = g.R / g.sv; p.rr = g.R % g.sv; p.sq = g.S / g.sh; p.sr = g.S % g.sh;
+    p.col_classes = (int)phase_classes(g.sh, g.W);
+    p.d_cols = mnv_fastdiv_make(p.col_classes);
     p.d_rows = mnv_fastdiv_make(p.phase_rows);
     for (int more = 0; more < 4; ++more) {
       const int plane = (p.hq + more / 2) * (p.wq + more % 2);  // 0: no position is in such a class

@@ -51,3 +51,17 @@ def test_strides_of_millions_of_classes_have_a_workspace(dims):
     ws = capi.lib().mnv_conv_bwd_data_workspace_bytes(*dims)
     # no more than the permuted filter and some partial results
     assert ws <= 4 * C * R * S * ((K + 15) // 16 * 16) + 256 + 64 * 4 * N * H * W * C
+
+
+@pytest.mark.parametrize("dims,rows", [  # N, C, K, H, W, ph, pw, sv, sh, R, S; rows of the classes that hold a position
+    ((2254, 64, 264, 3, 2, 1, 0, 8, 4, 2, 1), 0), ((929, 64, 240, 2, 4, 2, 2, 7, 5, 2, 1), 0), ((1057, 48, 200, 2, 4, 0, 2, 8, 1, 1, 1), 0),
+    ((32, 16, 224, 5, 2, 0, 0, 1, 7, 5, 2), 2 * 160),
+])
+def test_classes_without_a_position_take_no_workspace(dims, rows):
+    """Strides beyond the plane: of the sv * sh classes only min(sv, H) * min(sh, W) hold a position, and only
+    those are rows of the product (0: no partial results, one range of each class)."""
+    C, K, R, S = dims[1], dims[2], dims[9], dims[10]
+    filter_bytes = 4 * C * R * S * ((K + 15) // 16 * 16)
+    ws = capi.lib().mnv_conv_bwd_data_workspace_bytes(*dims)
+    assert ws >= filter_bytes and filter_bytes % 256 == 0
+    assert (ws == filter_bytes) if not rows else (ws > filter_bytes and (ws - filter_bytes) % (4 * rows * C) == 0)

@@ -48,6 +48,28 @@ def test_strided_data_gradient_matches_the_oracle(gpu, p):
         assert normwise(cv.bwd_data(dy, w, workspace), ref) <= TOL
 
 
+BEYOND = [  # strides beyond the plane in one direction or both: fewer classes than sv * sh
+    (64, 64, 64, 2, 2, 1, 1, 20, 20, 3, 3),
+    (17, 24, 344, 5, 3, 1, 0, 1, 6, 5, 2),
+    (32, 16, 224, 5, 2, 0, 0, 1, 7, 5, 2),      # k ranges
+    (9, 33, 40, 1, 37, 0, 1, 2, 2, 1, 3),       # one row
+    (7, 20, 48, 3, 4, 2, 3, 5, 4, 4, 5),        # the other direction's stride is the plane's extent
+    (700, 64, 128, 3, 2, 1, 2, 4, 8, 5, 5),
+    (900, 96, 256, 3, 2, 1, 1, 4, 4, 3, 3),     # bf16 parts
+]
+
+
+@pytest.mark.parametrize("p", BEYOND, ids=lambda p: "-".join(map(str, p)))
+def test_strides_beyond_the_plane_match_the_oracle(gpu, p):
+    N, C, K, H, W, ph, pw, sv, sh, R, S = p
+    say("strides beyond the plane", p)
+    cv = Conv(gpu, *p)
+    dy, w = _rand(N * K * cv.Ho * cv.Wo, 5), _rand(K * C * R * S, 6)
+    ref = ora.conv_bwd_data(dy, w, *p)
+    for workspace in (True, False):
+        assert normwise(cv.bwd_data(dy, w, workspace), ref) <= TOL
+
+
 @pytest.mark.parametrize("share", [0.0, 0.4, 0.999, 1.5])
 def test_any_workspace_gives_the_gradient(gpu, share):
     """The queried bytes, fewer, which give fewer k ranges or the generic gathers where the
