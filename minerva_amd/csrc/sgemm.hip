@@ -367,12 +367,16 @@ __global__ __launch_bounds__(256) void mnv_sgemm_skinny_tn_kernel(P prob, int k_
 // What bounds it: a launch and two trips to memory, 3 us; from one tile per CU on the operands' way from L2
 // (128 or 256 bytes per k and tile).  An XCD works on neighbouring tiles across the shorter side of the result, so that its
 // L2 fetches an eighth of the longer operand (4021 x 169 x 731 on 32 x 32 tiles 25 -> 17 us, 2093 x 198 x 3376 on 16 x 16 147 -> 55).
-// us, tiles of the core -> this: 17 x 53 x 124 6.5 -> 3.5, 256 x 256 x 784 9.1 -> 3.9, 10 x 256 x 256 6.8 -> 3.4, 512 x 512 x 512
-// 13.0 -> 5.5, 1421 x 284 x 488 14.1 -> 8.6, 1001 x 250 x 4099 28.2 -> 24; 300 random products of up to
-// 4096 in every extent 0.65 of the time.
-// Error against float64: 2 W sums per value, 0.83 of what it was over 300 random products, none more than 1.1 times.
+// us, tiles of the core -> this: 17 x 53 x 124 6.8 -> 3.1, 256 x 256 x 784 9.4 -> 4.3, 10 x 256 x 256 6.8 -> 3.3, 512 x 512 x 512
+// 13.1 -> 5.9, 1421 x 284 x 488 14.4 -> 9.3, 1001 x 250 x 4099 29.3 -> 24.1; 283 random products of up to
+// 4096 in every extent 0.59 of the time.
+// Error against float64: a wavefront adds runs of 32 k up, each run under the next one's instructions, so that no sum is longer than
+// 32 products or its own runs: 0.69 of the core's (of k ranges where it had them) over those 283 products of normal operands, none above
+// 1.01 times; uniform ones 0.70, and 0.91 where both come from a ReLU (1.18 at most), whose zeros cost a plain sum nothing.
+// With one sum each for the even and the odd fetches instead, 0.81 and up to 1.11, and 55 of the uniform products worse by up to 1.24;
+// 1001 x 250 x 4099 2.99e-7 -> 1.54e-7, 25.3 us with the eight wavefronts that it then needed.
 template <class P, int T, int W>
-__global__ __launch_bounds__(W * MNV_WAVE) void mnv_sgemm_small_kernel(P prob, int tiles_m, int tiles_n, int k_per_wave) {
+__global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_sgemm_small_kernel(P prob, int tiles_m, int tiles_n, int k_per_wave) {
   constexpr int H = MNV_WAVE / T, RUN = 4 * H, VECS = 32 / RUN, REGS = T * T / MNV_WAVE;
   typedef float Acc __attribute__((ext_vector_type(REGS)));
   __shared__ float red[W * T * T];
@@ -407,7 +411,7 @@ __global__ __launch_bounds__(W * MNV_WAVE) void mnv_sgemm_small_kernel(P prob, i
   typedef std::integral_constant<bool, P::B_KFAST> BFast;
   int k = wave * k_per_wave;
   const int k_end = k + k_per_wave < prob.K ? k + k_per_wave : prob.K;
-  Acc acc[2] = {0.f, 0.f};  // of the even and the odd fetches: half the length of the sums
+  Acc sum = 0.f, run[2] = {0.f, 0.f};  // runs of 32 k
   float a[2][VECS][4], b[2][VECS][4];
   if (k < k_end) {
     fetch(res.a, a_off, lda, AFast{}, k, a[0]);
@@ -431,8 +435,10 @@ __global__ __launch_bounds__(W * MNV_WAVE) void mnv_sgemm_small_kernel(P prob, i
     for (int j = 0; j < VECS; ++j)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        if constexpr (T == 32) acc[set] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], acc[set], 0, 0, 0);
-        else acc[set] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], acc[set], 0, 0, 0);
+        const Acc before = j == 0 && t == 0 ? Acc(0.f) : run[set];
+        if constexpr (T == 32) run[set] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
+        else run[set] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
+        if (j == 0 && t == 1) sum += run[set ^ 1];  // the run before, under this one's instructions
       }
     k += 32;
   };
@@ -441,10 +447,15 @@ __global__ __launch_bounds__(W * MNV_WAVE) void mnv_sgemm_small_kernel(P prob, i
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
   }
-  if (steps > 0) step(std::integral_constant<int, 0>{});
+  if (steps > 0) {
+    step(std::integral_constant<int, 0>{});
+    sum += run[0];
+  } else {
+    sum += run[1];
+  }
   // register r of lane (x, h): row x, column 4 h + r % 4 + 8 (r / 4)
 #pragma unroll
-  for (int r = 0; r < REGS; ++r) red[wave * T * T + (4 * h + r % 4 + 8 * (r / 4)) * T + x] = acc[0][r] + acc[1][r];
+  for (int r = 0; r < REGS; ++r) red[wave * T * T + (4 * h + r % 4 + 8 * (r / 4)) * T + x] = sum[r];
   __syncthreads();
   for (int e = threadIdx.x; e < T * T; e += W * MNV_WAVE) {
     float sum = red[e];
@@ -710,9 +721,7 @@ void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
   if ((c16 < c32 ? c16 : c32) >= 0.9 * plan->us) return;
   *plan = SgemmPlan{true, 1};
   plan->tile = c16 < c32 ? 16 : 32;
-  // four wavefronts for many tiles; past 2048 k eight, the sums of the grouped tiles' length (1001 x 250 x 4099: error 4.1e-7 with
-  // four, 2.9e-7 with eight and before, 23.6 and 24.8 us)
-  const bool many = plan->tile == 16 ? (long long)m * n > 512 * cus : k <= 2048 && (m + 31LL) / 32 * ((n + 31) / 32) >= cus;
+  const bool many = plan->tile == 16 ? (long long)m * n > 512 * cus : (m + 31LL) / 32 * ((n + 31) / 32) >= cus;
   plan->groups = many ? 4 : 8;
 }
 
