@@ -154,7 +154,8 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
  * mnv_sgemm_nn_plan reports how a product of these extents is launched with a workspace of
  * that size (no counterpart in the reference, where the plan is cuBLAS's own): tile_rows is
  * 128 or 64 for square tiles (64 with k_ranges and groups 1 also for the 32 x 32 and 16 x 16 tiles of small
- * products, whose wavefronts share the k range), 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
+ * products, whose wavefronts share the k range: mnv_sgemm_nn_small_plan tells them apart, with the rows of
+ * such a tile and its wavefronts, 4 or 8, or 0 and 0 for any other plan), 256 with groups 1 for 256 x 128 tiles, and 256 with groups 4 for the
  * kernels of at most 12 columns over a large A (256 rows per workgroup, 64 where A is given
  * transposed; four wavefronts take a quarter of a k range each); k_ranges is the number of
  * partial results reduced by a second kernel (1: none); groups is otherwise 4 when a workgroup
@@ -170,6 +171,7 @@ int mnv_maxindex_row(const float* in, float* out, int m, int n, mnv_stream_t str
 size_t mnv_sgemm_nn_workspace_bytes(int m, int n, int k);
 int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* k_ranges,
                       int* groups);
+int mnv_sgemm_nn_small_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* wavefronts);
 int mnv_sgemm_nn(const float* a, const float* b, float* c, int m, int n, int k,
                  void* workspace, size_t workspace_bytes, mnv_stream_t stream);
 
@@ -310,6 +312,19 @@ int mnv_conv_bwd_filter(const float* bottom, const float* top_diff, float* filte
                         int stride_vertical, int stride_horizontal, int filter_height,
                         int filter_width, void* workspace, size_t workspace_bytes,
                         mnv_stream_t stream);
+/* How mnv_conv_fwd and mnv_conv_bwd_data launch a problem with a workspace of `workspace_bytes` (aligned to 16 bytes) on
+ * the current device, as the next query does for the filter gradient: rows of the output tile (32, 64, 128 or
+ * 256; 0: minimal filtering); the k ranges of the reduction, each with a partial result in the workspace (1: none);
+ * whether it multiplies in bf16 parts; and the classes of input positions, modulo the strides, that the data gradient takes as
+ * products of one launch (1: not by classes).  For a batch that runs as several launches, the plan of the
+ * first.  They launch nothing. */
+int mnv_conv_fwd_plan(int num_images, int bottom_num_channels, int top_num_channels, int bottom_height, int bottom_width,
+                      int pad_height, int pad_width, int stride_vertical, int stride_horizontal, int filter_height,
+                      int filter_width, size_t workspace_bytes, int* tile_rows, int* k_ranges, int* parts);
+int mnv_conv_bwd_data_plan(int num_images, int bottom_num_channels, int top_num_channels, int bottom_height,
+                           int bottom_width, int pad_height, int pad_width, int stride_vertical, int stride_horizontal,
+                           int filter_height, int filter_width, size_t workspace_bytes, int* tile_rows, int* k_ranges,
+                           int* parts, int* classes);
 /* How mnv_conv_bwd_filter launches a problem with a workspace of `workspace_bytes` on the
  * current device (no reference counterpart: cuDNN chooses its algorithm out of sight,
  * cuda_perform.cu:293-318): rows of the output tile (32, 64 or 128); the k ranges the reduction

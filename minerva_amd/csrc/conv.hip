@@ -968,6 +968,7 @@ typedef MnvGemmTile<128, 128, 16, 4, 1, 0, 96> Tile96;  // four wavefronts of 32
 typedef MnvGemmTile<128, 64, 16, 4, 1, 0, 32> TileThin;
 
 // tile 0: 64x64 output tiles, tile 1: 128x128, tile 2: 128x96, tile 3: 128x32
+const int kTileM[4] = {64, 128, 128, 128}, kTileN[4] = {64, 128, 96, 32};
 // Eight wavefronts of 64 x 64 (512 threads, two workgroups per CU): a quarter fewer bytes
 // fetched and staged per multiply than TileBig, and every element summed in the same order.
 // For the (tap, channel) forward and data-gradient policies, when the 256 x 128 tiles fill
@@ -976,16 +977,27 @@ typedef MnvGemmTile<128, 64, 16, 4, 1, 0, 32> TileThin;
 // forward, 1458 tiles in three rounds of 512 at 95%, is 3% SLOWER than on 128 x 128 tiles with
 // their cut tail).
 typedef MnvGemmTile<256, 128, 16, 4, 2> TileTall;
+// What the plan queries of the forward pass and the data gradient report; a launch that is given one launches nothing.
+struct DirectPlan {
+  int rows, ranges, parts, classes = 1;  // rows of the tile (0: minimal filtering), k ranges, in bf16 parts, products of one launch
+};
+int report(DirectPlan* plan, int rows, int ranges, int parts) {
+  plan->rows = rows;
+  plan->ranges = ranges;
+  plan->parts = parts;
+  return MNV_OK;
+}
 template <class P>
-int launch_tile(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t tail_bytes = 0) {
+int launch_tile(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t tail_bytes = 0, DirectPlan* plan = nullptr) {
   if constexpr (P::A_KFAST == false && P::B_NOFF == 1 && !MnvPhased<P>::value) {
     if (tile == 1 && splits == 1) {
       const long long tiles = (long long)((p.M + 255) / 256) * ((p.N + 127) / 128);
       const long long slots = 2LL * mnv_cu_count(), rounds = (tiles + slots - 1) / slots;
       if ((double)p.M * p.N >= 0.97 * (double)(rounds * slots) * 256.0 * 128.0)
-        return mnv_gemm_launch<TileTall>(p, 1, ws, s);
+        return plan ? report(plan, 256, 1, 0) : mnv_gemm_launch<TileTall>(p, 1, ws, s);
     }
   }
+  if (plan) return report(plan, kTileM[tile], splits, 0);
   switch (tile) {
     case 0: return mnv_gemm_launch<TileSmall>(p, splits, ws, s);
     case 2: return mnv_gemm_launch<Tile96>(p, splits, ws, s, tail_bytes);
@@ -993,8 +1005,6 @@ int launch_tile(int tile, const P& p, int splits, void* ws, hipStream_t s, size_
     default: return mnv_gemm_launch<TileBig>(p, splits, ws, s, tail_bytes);
   }
 }
-const int kTileM[4] = {64, 128, 128, 128}, kTileN[4] = {64, 128, 96, 32};
-
 // In bf16 parts.  128 x 128 tiles with a CU to themselves: the gathers' offsets need the registers
 // (four 4-byte loads per vector; on the tile with two workgroups per CU they spill, 490 against
 // 415 us for 96 -> 256 channels under 5 x 5 filters on 64 x 27 x 27).  96-column tiles: two
@@ -1107,16 +1117,17 @@ int split_ranges(int m, int n, int slabs, int tile, size_t ws_floats) {
 }
 
 template <class P>
-int launch_parts(const P& p, int z, void* ws, hipStream_t s, size_t ws_bytes) {
+int launch_parts(const P& p, int z, void* ws, hipStream_t s, size_t ws_bytes, DirectPlan* plan = nullptr) {
+  if (plan) return report(plan, 128, z, 1);
   return wide_tile(p.N) == 2 ? mnv_gemm_launch<Split96>(p, z, ws, s, ws_bytes)
                              : mnv_gemm_launch<SplitOne>(p, z, ws, s, ws_bytes);
 }
 // Forward and data gradient: in bf16 parts or, with `splits` k ranges, on the fp32 tile.
 template <class P>
-int launch_direct(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t ws_bytes) {
+int launch_direct(int tile, const P& p, int splits, void* ws, hipStream_t s, size_t ws_bytes, DirectPlan* plan) {
   if (const int z = split_ranges(p.M, p.N, p.total_slabs, tile, ws_bytes / sizeof(float)))
-    return launch_parts(p, z, ws, s, ws_bytes);
-  return launch_tile(tile, p, splits, ws, s, ws_bytes);
+    return launch_parts(p, z, ws, s, ws_bytes, plan);
+  return launch_tile(tile, p, splits, ws, s, ws_bytes, plan);
 }
 
 // Bytes the large tiles' launches want for the partial tiles of a cut tail (0: no tail); `parts`: the
@@ -1456,9 +1467,9 @@ size_t mnv_conv_fwd_workspace_bytes(int N, int C, int K, int H, int W, int ph, i
 static int conv_fwd_impl(const float* bottom, const float* filter, const float* bias, float* top,
                          int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh, int R,
                          int S, void* workspace, size_t workspace_bytes, mnv_stream_t stream,
-                         int relu) {
+                         int relu, DirectPlan* report_to = nullptr) {
   ConvGeom g;
-  if (!bottom || !filter || !bias || !top) return MNV_ERR_INVALID;
+  if (!report_to && (!bottom || !filter || !bias || !top)) return MNV_ERR_INVALID;
   int rc = make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S);
   if (rc) return rc;
   int gm = N * g.HoWo, gn = K, gk = g.CRS;
@@ -1467,9 +1478,11 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
   // winograd.hip (its transformed tensors are read and written in 16-byte vectors)
   if (const int images = mnv_wino_images(N, C, K, H, W, ph, pw, R, S, sv, sh,
                                          workspace && mnv_aligned16(workspace) ? workspace_bytes : 0))
-    return mnv_wino_conv(bottom, filter, bias, nullptr, top, N, C, K, H, W, ph, pw, R, 0, relu, images,
-                         workspace, workspace_bytes, s);
+    return report_to ? report(report_to, 0, 1, 1)
+                     : mnv_wino_conv(bottom, filter, bias, nullptr, top, N, C, K, H, W, ph, pw, R, 0, relu, images,
+                                     workspace, workspace_bytes, s);
   if (const SmallForward small = small_forward(g, workspace ? workspace_bytes : 0); small.z) {
+    if (report_to) return report(report_to, MNV_SMALL_TILE, small.z, 0);
     float* wp = static_cast<float*>(workspace);
     float* part = small.z > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(small.filter_bytes)) : nullptr;
     if (!small.width)
@@ -1497,15 +1510,15 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wp = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wp, K, C, R, S, width, false, s);
+    rc = report_to ? MNV_OK : permute_filter(filter, wp, K, C, R, S, width, false, s);
     if (rc) return rc;
     const int spp = width / 16;
     const size_t part_bytes = part ? workspace_bytes - used : 0;
     if (width != C)
       return launch_direct(tile, ConvFwd<true, true>{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}, splits,
-                           part, s, part_bytes);
+                           part, s, part_bytes, report_to);
     return launch_direct(tile, ConvFwd<true>{bottom, wp, bias, top, g, gm, gn, gk, g.RS * spp, spp, relu}, splits, part, s,
-                         part_bytes);
+                         part_bytes, report_to);
   }
   if (np) {
     ConvFwdNP p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, gk >= 16 ? gk / 16 : 1, relu};
@@ -1521,12 +1534,12 @@ static int conv_fwd_impl(const float* bottom, const float* filter, const float* 
       q.total_slabs = q.spp = (q.groups + 3) / 4;
       q.d_per_row = mnv_fastdiv_make(q.per_row);
       q.d_R = mnv_fastdiv_make(R);
-      return launch_parts(q, z, part, s, part_bytes);
+      return launch_parts(q, z, part, s, part_bytes, report_to);
     }
-    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+    return launch_direct(tile, p, splits, part, s, part ? workspace_bytes - used : 0, report_to);
   }
   ConvFwd<false> p{bottom, filter, bias, top, g, gm, gn, gk, (gk + 15) / 16, 1, relu};
-  return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+  return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0, report_to);
 }
 
 static int conv_fwd_chunks(const float* bottom, const float* filter, const float* bias, float* top,
@@ -1634,9 +1647,9 @@ static int bwd_data_phases(const float* top_diff, const float* filter, const flo
 static int conv_bwd_data_impl(const float* top_diff, const float* filter, const float* gate,
                               float* bottom_diff, int N, int C, int K, int H, int W, int ph,
                               int pw, int sv, int sh, int R, int S, void* workspace,
-                              size_t workspace_bytes, mnv_stream_t stream) {
+                              size_t workspace_bytes, mnv_stream_t stream, DirectPlan* report_to = nullptr) {
   ConvGeom g;
-  if (!top_diff || !filter || !bottom_diff) return MNV_ERR_INVALID;
+  if (!report_to && (!top_diff || !filter || !bottom_diff)) return MNV_ERR_INVALID;
   int rc = make_geom(&g, N, C, K, H, W, ph, pw, sv, sh, R, S);
   if (rc) return rc;
   int gm = N * g.HW, gn = C, gk = K * g.RS;
@@ -1644,10 +1657,16 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
   // the same correlation, of top_diff with the unflipped filters, under a padding of R - 1 - pad
   if (const int images = mnv_wino_images(N, K, C, g.Ho, g.Wo, R - 1 - ph, S - 1 - pw, R, S, sv, sh,
                                          workspace && mnv_aligned16(workspace) ? workspace_bytes : 0))
-    return mnv_wino_conv(top_diff, filter, nullptr, gate, bottom_diff, N, K, C, g.Ho, g.Wo, R - 1 - ph,
-                         S - 1 - pw, R, 1, 0, images, workspace, workspace_bytes, s);
+    return report_to ? report(report_to, 0, 1, 1)
+                     : mnv_wino_conv(top_diff, filter, nullptr, gate, bottom_diff, N, K, C, g.Ho, g.Wo, R - 1 - ph,
+                                     S - 1 - pw, R, 1, 0, images, workspace, workspace_bytes, s);
   if (sv > 1 || sh > 1) {
     const PhasePlan plan = phase_plan(g, workspace ? workspace_bytes : 0);
+    if (plan.width && report_to) {
+      report_to->classes = (int)(plan.rows / plan.phase_rows);
+      return plan.parts ? report(report_to, 128, plan.parts, 1)
+                        : report(report_to, plan.small ? MNV_SMALL_TILE : kTileM[plan.tile], plan.splits, 0);
+    }
     if (plan.width) return bwd_data_phases(top_diff, filter, gate, bottom_diff, g, plan, workspace, s);
   }
   const int tile = pick_tile(gm, gn);
@@ -1660,11 +1679,12 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
                                        part ? (workspace_bytes - used) / sizeof(float) : 0);
   if (fast) {
     float* wq = static_cast<float*>(workspace);
-    rc = permute_filter(filter, wq, K, C, R, S, width, true, s);
+    rc = report_to ? MNV_OK : permute_filter(filter, wq, K, C, R, S, width, true, s);
     if (rc) return rc;
     const int spp = width / 16;
     const size_t part_bytes = part ? workspace_bytes - used : 0;
     if (const int z = small_bwd_data(g, width, workspace_bytes)) {
+      if (report_to) return report(report_to, MNV_SMALL_TILE, z, 0);
       if (width != K)
         return mnv_gemm_small_launch(ConvOneRow<ConvBwdData<true, true>, true>{{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate}},
                                      z, part, s);
@@ -1673,12 +1693,12 @@ static int conv_bwd_data_impl(const float* top_diff, const float* filter, const 
     }
     if (width != K)
       return launch_direct(tile, ConvBwdData<true, true>{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate},
-                           splits, part, s, part_bytes);
+                           splits, part, s, part_bytes, report_to);
     return launch_direct(tile, ConvBwdData<true>{top_diff, wq, bottom_diff, g, gm, gn, gk, g.RS * spp, spp, gate}, splits,
-                         part, s, part_bytes);
+                         part, s, part_bytes, report_to);
   }
   ConvBwdData<false> p{top_diff, filter, bottom_diff, g, gm, gn, gk, (gk + 15) / 16, 1, gate};
-  return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0);
+  return launch_tile(tile, p, splits, part, s, part ? workspace_bytes - used : 0, report_to);
 }
 
 static int conv_bwd_data_chunks(const float* top_diff, const float* filter, const float* gate,
@@ -1835,6 +1855,42 @@ int mnv_conv_bwd_filter(const float* bottom, const float* top_diff, float* filte
                                   stream, n0 > 0);
     if (rc) return rc;
   }
+  return MNV_OK;
+}
+
+static int direct_plan(bool forward, int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh, int R, int S,
+                       size_t workspace_bytes, DirectPlan* plan) {
+  const int chunk = images_per_launch(N, C, K, H, W, ph, pw, sv, sh, R, S);
+  if (chunk <= 0) return MNV_ERR_INVALID;
+  // the workspace is only compared with sizes here, never dereferenced
+  void* some = workspace_bytes ? reinterpret_cast<void*>((uintptr_t)256) : nullptr;
+  const int n = chunk < N ? chunk : N;
+  return forward ? conv_fwd_impl(nullptr, nullptr, nullptr, nullptr, n, C, K, H, W, ph, pw, sv, sh, R, S, some, workspace_bytes,
+                                 nullptr, 0, plan)
+                 : conv_bwd_data_impl(nullptr, nullptr, nullptr, nullptr, n, C, K, H, W, ph, pw, sv, sh, R, S, some,
+                                      workspace_bytes, nullptr, plan);
+}
+
+int mnv_conv_fwd_plan(int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh, int R, int S, size_t workspace_bytes,
+                      int* tile_rows, int* k_ranges, int* parts) {
+  DirectPlan plan{};
+  const int rc = direct_plan(true, N, C, K, H, W, ph, pw, sv, sh, R, S, workspace_bytes, &plan);
+  if (rc) return rc;
+  if (tile_rows) *tile_rows = plan.rows;
+  if (k_ranges) *k_ranges = plan.ranges;
+  if (parts) *parts = plan.parts;
+  return MNV_OK;
+}
+
+int mnv_conv_bwd_data_plan(int N, int C, int K, int H, int W, int ph, int pw, int sv, int sh, int R, int S, size_t workspace_bytes,
+                           int* tile_rows, int* k_ranges, int* parts, int* classes) {
+  DirectPlan plan{};
+  const int rc = direct_plan(false, N, C, K, H, W, ph, pw, sv, sh, R, S, workspace_bytes, &plan);
+  if (rc) return rc;
+  if (tile_rows) *tile_rows = plan.rows;
+  if (k_ranges) *k_ranges = plan.ranges;
+  if (parts) *parts = plan.parts;
+  if (classes) *classes = plan.classes;
   return MNV_OK;
 }
 

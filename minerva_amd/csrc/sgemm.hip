@@ -936,6 +936,14 @@ int mnv_sgemm_nn_plan(int m, int n, int k, size_t workspace_bytes, int* tile_row
   return MNV_OK;
 }
 
+int mnv_sgemm_nn_small_plan(int m, int n, int k, size_t workspace_bytes, int* tile_rows, int* wavefronts) {
+  if (m <= 0 || n <= 0 || k <= 0 || !tile_rows || !wavefronts) return MNV_ERR_INVALID;
+  const SgemmPlan plan = plan_sgemm(m, n, k, workspace_bytes / sizeof(float));
+  *tile_rows = plan.tile;
+  *wavefronts = plan.tile ? plan.groups : 0;
+  return MNV_OK;
+}
+
 int mnv_sgemm_nn(const float* a, const float* b, float* c, int m, int n, int k, void* workspace,
                  size_t workspace_bytes, mnv_stream_t stream) {
   if (m == 0 || n == 0) return MNV_OK;

@@ -137,6 +137,24 @@ def test_weighing_many_launches_costs_little_host_time():
     assert min(fastest(256, 256, 784) / fastest(10, 256, 256) for _ in range(3)) <= 2.5
 
 
+@pytest.mark.parametrize("m,n,k,tile,wavefronts", [
+    (16, 16, 32, 16, 8), (100, 7, 257, 16, 8), (257, 255, 783, 16, 8), (5, 300, 1023, 16, 8),
+    (513, 511, 509, 16, 4), (784, 256, 255, 32, 8), (57, 3024, 2539, 32, 8),
+    (1421, 284, 487, 32, 4), (1001, 250, 4099, 32, 4),
+    (1, 1, 1, 0, 0), (15, 17, 3, 0, 0),                                   # one slab: the 64 x 64 tile
+    (200, 1000, 4099, 0, 0), (500, 500, 3000, 0, 0), (4096, 3, 5000, 0, 0),  # k ranges: only with a workspace
+    (4096, 4096, 4096, 0, 0),
+])
+def test_tiles_of_small_products(m, n, k, tile, wavefronts):
+    """Which products run on 16 x 16 and 32 x 32 tiles, and how many wavefronts share their k.  They ask for no workspace."""
+    assert not tile or _query(m, n, k) == 0
+    for ws in (_query(m, n, k), 1 << 40):
+        v = [ctypes.c_int() for _ in range(2)]
+        assert capi.lib().mnv_sgemm_nn_small_plan(m, n, k, ctypes.c_size_t(ws), *[ctypes.byref(x) for x in v]) == 0
+        assert (v[0].value, v[1].value) == (tile, wavefronts), ws
+        assert not tile or _plan(m, n, k, ws) == (64, 1, 1)
+
+
 def _device_code(path):
     """The code objects in a library's bundles."""
     data, magic, at = open(path, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", 0
