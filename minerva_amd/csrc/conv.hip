@@ -1321,7 +1321,12 @@ int bwd_data_channels(const ConvGeom& g) {
 // 5 x 5 on 104 x 15 x 45 1780 -> 249, 264 <- 216 on 45 x 33 x 38 2293 -> 453, 128 <- 128 under 1 x 1 on 88 x 15 x 20 32 -> 31, 320 <- 96
 // under 3 x 3 on 41 x 14 x 29 191 -> 64, 48 <- 184 on 17 x 16 x 15 26.6 -> 19.1.  Few tiles of few slabs are bound by one
 // trip to memory after the other, 1.45 us for a generic slab and 0.65 for one of a phase, and pay for the launch that permutes the filter,
-// 5.5 us in all: 11 channels under 1 x 1 5.0 -> 10.2, 70 10.3 -> 10.9, 16 under 3 x 3 15.1 -> 9.7.  Error against float64: large products 0.2 to 0.6
+// 5.5 us in all: 11 channels under 1 x 1 5.0 -> 10.2, 70 10.3 -> 10.9, 16 under 3 x 3 15.1 -> 9.7.  Many tiles are bound by their
+// stores, which leave every sh-th float (about 1 TB/s, and 20 us before the first slab counts), and repay them from five generic slabs
+// on, and nine of a CU's 128 x 128 tiles: under 1 x 1, 256 <- 32 on 52 x 14 x 12 14.8 -> 29.2, 328 <- 32 on 93 x 53 x 22 73 -> 121, 224 <- 128
+// on 69 x 32 x 7 30.1 -> 37.9 (all left to the generic gathers), 192 <- 72 on 39 x 21 x 54 36 -> 28, 208 <- 128 on 26 x 50 x 45 73 -> 47.  600
+// random layers at stride 2: by taking all of two slabs on, 38 lost more than 3%, up to 2 times; by this rule 2, up to 1.18; the dearest win that
+// it leaves is 216 <- 104 on 36 x 17 x 34, 42 -> 35.  Error against float64: large products 0.2 to 0.6
 // of what it was (bf16 parts now); on the fp32 tiles that of the sums' own length, the fewer k ranges of which make it
 // 1.0 to 1.9 times what the generic ranges had (2.0e-7 against 1.1e-7 at 1728 products, as for a unit stride).
 struct PhasePlan {
@@ -1369,7 +1374,8 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
   // the tiles' rows, and channels, are filled up: not where that multiplies more than the generic gathers
   if ((long long)p.rows * width >= (long long)m * g.K * phases) return p;
   const long long tiles = (m + 63LL) / 64 * ((g.C + 63) / 64), slabs = ((long long)g.K * g.RS + 15) / 16;
-  if (tiles < 512 ? 11 * slabs <= 5 * p.slabs + 42 : slabs < 2) return p;
+  const long long cus = mnv_cu_count(), big = std::max((m + 127LL) / 128 * ((g.C + 127) / 128), cus);
+  if (tiles < 512 ? 11 * slabs <= 5 * p.slabs + 42 : slabs < 5 || slabs * big <= 9 * cus) return p;
   p.width = width;
   return p;
 }

@@ -1,5 +1,7 @@
 """Which data gradients and forward passes have their channels padded to the multiples of 16: host
 arithmetic on the extents alone, seen from the workspace that holds the padded filter."""
+import ctypes
+
 import pytest
 
 from minerva_amd import capi
@@ -65,3 +67,24 @@ def test_classes_without_a_position_take_no_workspace(dims, rows):
     ws = capi.lib().mnv_conv_bwd_data_workspace_bytes(*dims)
     assert ws >= filter_bytes and filter_bytes % 256 == 0
     assert (ws == filter_bytes) if not rows else (ws > filter_bytes and (ws - filter_bytes) % (4 * rows * C) == 0)
+
+
+def _data_plan(dims, workspace=None):
+    """Rows of the tile, k ranges, whether in bf16 parts, classes of positions (1: the generic gathers of strides above 1)."""
+    v = [ctypes.c_int() for _ in range(4)]
+    ws = capi.lib().mnv_conv_bwd_data_workspace_bytes(*dims) if workspace is None else workspace
+    assert capi.lib().mnv_conv_bwd_data_plan(*dims, ctypes.c_size_t(ws), *[ctypes.byref(x) for x in v]) == 0
+    return tuple(x.value for x in v)
+
+
+@pytest.mark.parametrize("dims,classes", [  # N, C, K, H, W, pad, R; stride 2
+    ((52, 256, 32, 14, 12, 0, 1), 1), ((36, 272, 24, 32, 18, 0, 1), 1), ((81, 120, 24, 26, 18, 0, 1), 1), ((58, 96, 32, 26, 39, 0, 1), 1),
+    ((35, 304, 56, 9, 32, 0, 1), 1), ((69, 224, 128, 32, 7, 0, 1), 1), ((10, 376, 120, 16, 37, 0, 1), 1), ((79, 136, 16, 8, 19, 1, 3), 1),
+    ((93, 328, 32, 53, 22, 0, 1), 1), ((86, 176, 48, 34, 28, 0, 1), 1),
+    ((39, 192, 72, 21, 54, 0, 1), 4), ((70, 128, 72, 52, 46, 0, 1), 4), ((26, 208, 128, 50, 45, 0, 1), 4), ((59, 72, 160, 13, 48, 0, 1), 4),
+    ((27, 288, 16, 33, 39, 0, 3), 4), ((44, 304, 192, 15, 14, 0, 1), 4),
+    ((4, 70, 70, 14, 14, 0, 1), 1), ((66, 24, 128, 46, 10, 0, 1), 4),    # few tiles
+])
+def test_strided_data_gradients_by_classes_where_it_pays(dims, classes):
+    N, C, K, H, W, pad, R = dims
+    assert _data_plan((N, C, K, H, W, pad, pad, 2, 2, R, R))[3] == classes
