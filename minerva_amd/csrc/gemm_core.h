@@ -808,11 +808,12 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
 // Small tiles for products that the tiles above leave most CUs without, or in k ranges that cost more to add than to
 // multiply: T x T, one per workgroup, whose W wavefronts share the workgroup's k range.  No operand passes through LDS: a lane fetches the four k of a vector for its own row and its
 // own column through the policy (both operands k-fast), three slabs ahead, and multiplies them; lane group h (of 64 / T)
-// holds the k 4 h .. 4 h + 3 of each run of 4 * 64 / T.  A wavefront adds up the sums of runs of two slabs, and the wavefronts' sums are
-// added in LDS in the order of k, or left as a partial result per k range of blockIdx.z.  Error against float64 of the layers that run so
-// (223 random ones), of that on the tiles above: forward 0.69, data gradient 0.67, filter gradient 0.62, none above 0.99, and less with positive
-// operands; with one sum each for the even and the odd slabs 0.85, 0.85 and 0.73, a fifth of them worse by up to 1.6.  The runs cost 1.5% (ConvFwd of 24 -> 32 channels
-// under 3 x 3 on 19 x 44 x 12 11.1 -> 11.6 us, 80 -> 32 under 5 x 5 at stride 2 36.0 -> 35.2); four wavefronts per SIMD leave no registers for a
+// holds the k 4 h .. 4 h + 3 of each run of 4 * 64 / T.  A wavefront adds up the sums of runs of two slabs, of one for the last three, and the wavefronts' sums are
+// added in LDS in the order of k, or left as a partial result per k range of blockIdx.z.  Error against float64 of the layers that run so,
+// of that on the tiles above: forward 0.68, data gradient 0.57 (of strided layers by classes 0.79), filter gradient 0.62 over 500 random ones, four
+// above 1.02 times, by up to 1.1; with one sum each for the even and the odd slabs 0.86, 0.77, 0.95 and 0.72, and 200 above, by up to 2.1; with
+// runs of two slabs throughout, layers of up to three slabs per wavefront up to 1.15.  The runs cost 1 to 2% (24 -> 32 channels
+// under 3 x 3 on 19 x 44 x 12 11.1 -> 11.6 us, 80 -> 32 under 5 x 5 at stride 2 36.0 -> 35.2), runs of one slab everywhere 24%; four wavefronts per SIMD leave no registers for a
 // second run.  Neighbouring tiles
 // across the shorter side of the result share an XCD.  What bounds it, and where it is taken: mnv_small_ranges.
 #define MNV_SMALL_TILE 32
@@ -878,7 +879,7 @@ __global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob,
       new_period();
     }
   };
-  Acc sum = 0.f, run = 0.f;  // of all k, of a run of two slabs
+  Acc sum = 0.f, run = 0.f;  // of all k, of a run
   __syncthreads();  // block_init may have written LDS
   typedef std::integral_constant<int, 0> Set0;
   typedef std::integral_constant<int, 1> Set1;
@@ -890,7 +891,8 @@ __global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob,
     fetch(Set1{});
     fetch(Set2{});
   }
-  auto step = [&](auto SET) {
+  // slab `set` of four, the run's slabs from FIRST to LAST
+  auto step = [&](auto SET, auto FIRST, auto LAST) {
     constexpr int set = decltype(SET)::value;
     fetch(std::integral_constant<int, (set + 3) % 4>{});  // past the range: not multiplied
 #pragma unroll
@@ -902,23 +904,24 @@ __global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob,
     for (int j = 0; j < VECS; ++j)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const Acc before = set % 2 == 0 && j == 0 && t == 0 ? Acc(0.f) : run;
+        const Acc before = decltype(FIRST)::value && j == 0 && t == 0 ? Acc(0.f) : run;
         if constexpr (T == 32) run = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
         else run = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
       }
-    if constexpr (set % 2 == 1) sum += run;
+    if constexpr (decltype(LAST)::value) sum += run;
   };
   int steps = end - begin;
+  typedef std::true_type Yes;
+  typedef std::false_type No;
   for (; steps >= 4; steps -= 4) {
-    step(Set0{});
-    step(Set1{});
-    step(Set2{});
-    step(Set3{});
+    step(Set0{}, Yes{}, No{});
+    step(Set1{}, No{}, Yes{});
+    step(Set2{}, Yes{}, No{});
+    step(Set3{}, No{}, Yes{});
   }
-  if (steps > 0) step(Set0{});
-  if (steps > 1) step(Set1{});
-  if (steps > 2) step(Set2{});
-  if (steps % 2) sum += run;
+  if (steps > 0) step(Set0{}, Yes{}, Yes{});
+  if (steps > 1) step(Set1{}, Yes{}, Yes{});
+  if (steps > 2) step(Set2{}, Yes{}, Yes{});
   // register r of lane (x, h): row x, column 4 h + r % 4 + 8 (r / 4)
 #pragma unroll
   for (int r = 0; r < REGS; ++r) mnv_small_lds[wave * T * T + (4 * h + r % 4 + 8 * (r / 4)) * T + x] = sum[r];

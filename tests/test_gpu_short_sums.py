@@ -24,6 +24,12 @@ def _bound(k, wavefronts):
     return 2.0 ** -24 / math.sqrt(3) * math.sqrt(16 + k / (64.0 * wavefronts) + (wavefronts + 1) / 2)
 
 
+def _closer_bound(k, wavefronts, run):
+    """The same for runs of `run` and the mean rounding: ulp / sqrt(12), which for values whose logarithms are evenly spread is
+    0.4247 * 2^-24 of them; a twelfth on top."""
+    return 1.08 * 0.4247 * 2.0 ** -24 * math.sqrt(run / 2 + k / (2.0 * run * wavefronts) + (wavefronts + 1) / 2)
+
+
 def _error(got, want):
     return np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want)
 
@@ -40,12 +46,8 @@ def test_small_products(gpu, m, n, k, wavefronts):
     assert _error(gpu.down(c).reshape(n, m).T, A.astype(np.float64) @ B.astype(np.float64)) <= _bound(k, wavefronts)
 
 
-@pytest.mark.parametrize("p,passes", [  # no k ranges: each runs in the permuted filter or the filter in place
-    ((15, 288, 32, 16, 32, 0, 0, 1, 1, 3, 3), "fwd"), ((2, 48, 160, 31, 49, 1, 1, 1, 1, 3, 3), "bwd_data"),
-    ((60, 16, 280, 26, 14, 1, 1, 1, 1, 3, 3), "bwd_data"), ((32, 48, 80, 10, 32, 0, 0, 1, 1, 5, 5), "bwd_data"),
-    ((59, 80, 32, 48, 20, 2, 2, 2, 2, 5, 5), "fwd"), ((21, 40, 288, 51, 9, 0, 0, 2, 2, 3, 3), "bwd_data"),
-], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else v)
-def test_small_convolutions(gpu, p, passes):
+def _convolution(gpu, p, passes):
+    """Its error and the length of its longest sums."""
     import torch
     N, C, K, H, W, ph, pw, sv, sh, R, S = p
     say("error of a small convolution", p, passes)
@@ -62,4 +64,23 @@ def test_small_convolutions(gpu, p, passes):
         want = torch.nn.functional.conv_transpose2d(torch.from_numpy(dy).double().view(N, K, cv.Ho, cv.Wo), flat, stride=(sv, sh),
                                                     padding=(ph, pw), output_padding=rest)
         got, k = cv.bwd_data(dy, w), K * -(-R // sv) * -(-S // sh)  # of the class with the most taps
-    assert _error(got, want.numpy().reshape(-1)) <= _bound(k, 4)
+    return _error(got, want.numpy().reshape(-1)), k
+
+
+@pytest.mark.parametrize("p,passes", [  # no k ranges: each runs in the permuted filter or the filter in place
+    ((15, 288, 32, 16, 32, 0, 0, 1, 1, 3, 3), "fwd"), ((2, 48, 160, 31, 49, 1, 1, 1, 1, 3, 3), "bwd_data"),
+    ((60, 16, 280, 26, 14, 1, 1, 1, 1, 3, 3), "bwd_data"), ((32, 48, 80, 10, 32, 0, 0, 1, 1, 5, 5), "bwd_data"),
+    ((59, 80, 32, 48, 20, 2, 2, 2, 2, 5, 5), "fwd"), ((21, 40, 288, 51, 9, 0, 0, 2, 2, 3, 3), "bwd_data"),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_small_convolutions(gpu, p, passes):
+    error, k = _convolution(gpu, p, passes)
+    assert error <= _bound(k, 4)
+
+
+@pytest.mark.parametrize("p,passes", [  # up to three slabs of 16 per wavefront, one of them a run
+    ((23, 216, 72, 8, 11, 1, 1, 2, 2, 2, 2), "bwd_data"), ((3, 192, 72, 48, 8, 0, 0, 2, 2, 2, 2), "bwd_data"),
+    ((45, 24, 96, 13, 37, 0, 0, 2, 2, 2, 2), "bwd_data"), ((27, 48, 16, 8, 34, 0, 0, 2, 2, 5, 5), "bwd_data"),
+], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_short_reductions_of_convolutions(gpu, p, passes):
+    error, k = _convolution(gpu, p, passes)
+    assert error <= _closer_bound(k, 4, 16)
