@@ -1326,9 +1326,10 @@ int bwd_data_channels(const ConvGeom& g) {
 // on, and nine of a CU's 128 x 128 tiles: under 1 x 1, 256 <- 32 on 52 x 14 x 12 14.8 -> 29.2, 328 <- 32 on 93 x 53 x 22 73 -> 121, 224 <- 128
 // on 69 x 32 x 7 30.1 -> 37.9 (all left to the generic gathers), 192 <- 72 on 39 x 21 x 54 36 -> 28, 208 <- 128 on 26 x 50 x 45 73 -> 47.  600
 // random layers at stride 2: by taking all of two slabs on, 38 lost more than 3%, up to 2 times; by this rule 2, up to 1.18; the dearest win that
-// it leaves is 216 <- 104 on 36 x 17 x 34, 42 -> 35.  Error against float64: large products 0.2 to 0.6
-// of what it was (bf16 parts now); on the fp32 tiles that of the sums' own length, the fewer k ranges of which make it
-// 1.0 to 1.9 times what the generic ranges had (2.0e-7 against 1.1e-7 at 1728 products, as for a unit stride).
+// it leaves is 216 <- 104 on 36 x 17 x 34, 42 -> 35.  Error against float64 (525 random layers): 0.74 of that of
+// the generic gathers, 0.37 where they run in parts; 26 above 1.02 times, by up to 1.05 on large tiles and 1.15 on small ones.  Without the rules
+// below for parts and small tiles 37 of the large and 23 of the small ones were, by up to 1.36 and 2.1, for up to 1.5 times less time: 48 <- 24
+// under 3 x 3 on 120 x 27 x 30 1.47e-7 -> 0.81e-7 (generic 1.08e-7), 29 -> 43 us (70); 112 <- 48 on 51 x 33 x 50 2.05e-7 -> 0.66e-7 (1.91e-7), 51 -> 67 (143).
 struct PhasePlan {
   int width = 0;  // channels as the policy takes them; 0: the generic gathers
   int tile = 0, parts = 0, splits = 1, phase_rows = 0, slabs = 0;  // parts > 0: bf16 parts with that many k ranges
@@ -1357,14 +1358,29 @@ PhasePlan phase_plan(const ConvGeom& g, size_t ws_bytes) {
     p.phase_rows = (int)((most + tile_rows - 1) / tile_rows * tile_rows);
     p.rows = (size_t)p.phase_rows * phases;
   };
+  // No sum is to be longer than that of the generic gathers, which cut the tail of their large tiles, and the k of their small ones,
+  // into more ranges: where they shorten more than a tenth of the sums by a tail (5% of the error) the phases run in parts, and where they have
+  // more ranges, on the small tiles, which sum in runs.
+  const int generic_slabs = (int)(((long long)g.K * g.RS + 15) / 16);
   rows_on(128);
   p.parts = split_ranges(m, g.C, mean, p.tile, left / (p.rows ? p.rows : 1) * m);
+  if (!p.parts && (p.tile == 1 || p.tile == 2)) {
+    const long long tiles = (m + 127LL) / 128 * ((g.C + kTileN[p.tile] - 1) / kTileN[p.tile]);
+    const MnvTailPlan t = mnv_tail_plan(tiles, generic_slabs, (size_t)kTileM[p.tile] * kTileN[p.tile], (size_t)-1 / sizeof(float));
+    if (t.z > 1 && (double)(tiles - t.begin) / tiles * (1.0 - 1.0 / t.z) > 0.1) p.parts = 1;
+  }
   if (!p.parts) {
     rows_on(kTileM[p.tile]);
     p.splits = small_tile_splits(p.tile, (int)p.rows, g.C, p.slabs, left);
-    const size_t tile_rows = p.rows;
+    const long long tile_rows = (long long)p.rows;
     rows_on(MNV_SMALL_TILE);
-    if (const int z = small_reach(g) ? small_gather_ranges((long long)p.rows, g.C, mean, p.tile, (long long)tile_rows, mean, 2.0, left) : 0) {
+    int z = 0;
+    if (small_reach(g) && (p.tile == 0 || p.tile == 3)) {
+      z = small_gather_ranges((long long)p.rows, g.C, mean, p.tile, tile_rows, mean, 2.0, left);
+      if (!z && small_tile_splits(p.tile, m, g.C, generic_slabs, (size_t)-1) > p.splits)
+        z = mnv_small_ranges((long long)p.rows, g.C, mean, left, kSmallGather, 1e30);
+    }
+    if (z) {
       p.small = true;
       p.splits = z;
     } else {

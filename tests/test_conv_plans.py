@@ -88,3 +88,17 @@ def _data_plan(dims, workspace=None):
 def test_strided_data_gradients_by_classes_where_it_pays(dims, classes):
     N, C, K, H, W, pad, R = dims
     assert _data_plan((N, C, K, H, W, pad, pad, 2, 2, R, R))[3] == classes
+
+
+@pytest.mark.parametrize("dims,plan", [  # N, C, K, H, W, pad, R; stride 2
+    ((34, 120, 120, 26, 11, 1, 2), (32, 0)), ((47, 64, 64, 16, 27, 1, 3), (32, 0)), ((120, 48, 24, 27, 30, 1, 3), (32, 0)),  # more k ranges
+    ((108, 32, 56, 30, 21, 1, 3), (32, 0)),
+    ((51, 112, 48, 33, 50, 1, 3), (128, 1)), ((113, 264, 248, 17, 16, 0, 1), (128, 1)), ((80, 136, 64, 24, 12, 2, 5), (128, 1)),  # a cut tail
+    ((45, 120, 80, 56, 16, 0, 2), (128, 0)), ((116, 56, 80, 32, 36, 0, 1), (64, 0)),                      # as long sums either way
+])
+def test_strided_data_gradients_sum_no_longer_than_the_generic_gathers(dims, plan):
+    """Rows of the tile and whether in bf16 parts: layers whose generic launch shortens its sums by k ranges or a cut tail go where
+    sums are short as well."""
+    N, C, K, H, W, pad, R = dims
+    got = _data_plan((N, C, K, H, W, pad, pad, 2, 2, R, R))
+    assert (got[0], got[2], got[3]) == plan + (4,)

@@ -71,6 +71,7 @@ def _convolution(gpu, p, passes):
     ((15, 288, 32, 16, 32, 0, 0, 1, 1, 3, 3), "fwd"), ((2, 48, 160, 31, 49, 1, 1, 1, 1, 3, 3), "bwd_data"),
     ((60, 16, 280, 26, 14, 1, 1, 1, 1, 3, 3), "bwd_data"), ((32, 48, 80, 10, 32, 0, 0, 1, 1, 5, 5), "bwd_data"),
     ((59, 80, 32, 48, 20, 2, 2, 2, 2, 5, 5), "fwd"), ((21, 40, 288, 51, 9, 0, 0, 2, 2, 3, 3), "bwd_data"),
+    ((34, 120, 120, 26, 11, 1, 1, 2, 2, 2, 2), "bwd_data"), ((47, 64, 64, 16, 27, 1, 1, 2, 2, 3, 3), "bwd_data"),
 ], ids=lambda v: "-".join(map(str, v)) if isinstance(v, tuple) else v)
 def test_small_convolutions(gpu, p, passes):
     error, k = _convolution(gpu, p, passes)
@@ -84,3 +85,11 @@ def test_small_convolutions(gpu, p, passes):
 def test_short_reductions_of_convolutions(gpu, p, passes):
     error, k = _convolution(gpu, p, passes)
     assert error <= _closer_bound(k, 4, 16)
+
+
+@pytest.mark.parametrize("p", [(51, 112, 48, 33, 50, 1, 1, 2, 2, 3, 3), (80, 136, 64, 24, 12, 2, 2, 2, 2, 5, 5)], ids=lambda p: "-".join(map(str, p)))
+def test_strided_data_gradients_in_parts(gpu, p):
+    """One rounding of the full sum for 8 products: the partial sums' squares add up to k^2 / 16, and those of the smaller
+    terms, at 2^-8 of them, do not count."""
+    error, k = _convolution(gpu, p, "bwd_data")
+    assert error <= 2.0 ** -24 / math.sqrt(3) * math.sqrt(k / 16 + 1)
