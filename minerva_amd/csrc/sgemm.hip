@@ -704,20 +704,23 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
 
 // A plan on the small kernel's tiles where that is estimated at less than 90% of `plan`: 3 us, and the larger of what the
 // fullest CU multiplies and what all tiles take from L2, 1.49 and 1.95 us per 1000 k of a 16 x 16 tile on every CU, 4.36 and
-// 4.81 of a 32 x 32 one (5.2 from 2048 k on); beyond the eight or five workgroups that a CU holds, 2.5 us for each further round.
+// 4.81 of a 32 x 32 one (5.2 from 2048 k on); beyond the eight or four workgroups that a CU holds, 2.5 or
+// 3.4 us for each further round (with 2.5 of the larger tiles: 555 x 2773 x 156 10.0 -> 11.6, 2411 x 630 x 201 12.6 -> 15.0, 433 x 3053 x 133
+// 10.4 -> 11.4, 3921 x 332 x 232 13.0 -> 13.9, which now stay; 1770 x 721 x 430 25.6 -> 20.1 does not).
 // From 2048 k on 16 x 16 tiles take up to 1.4 times their estimate (292 x 243 x 3361 14.8 -> 21.7; 49 x 98 x 3847 11.7 -> 9.8) and are
-// left to the k ranges.  Measured on 500 products with every shape: 0.593 of the time, the fastest of all throughout
-// 0.575; seven lost 4 to 20% (555 x 2773 x 156 10.7 -> 11.6, 677 x 84 x 3060 14.5 -> 15.3).  Four wavefronts for many tiles, eight for few.
+// left to the k ranges.  500 random products that it moves 0.56 of the time, none slower; 400 of at least 250 rows
+// and columns 0.66, two slower by more than 3% (1538 x 609 x 248 9.9 -> 10.5, 459 x 1917 x 200 8.8 -> 9.2).  Four wavefronts for many tiles, eight for few.
 // The kernel reads an x-fast operand up to 95 k past its end: its offsets have to stay below 2^31.
 void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
   // (products in parts are the more exact ones)
   if (plan->skinny || plan->split || (k + 96LL) * m > kSmallOperand || (k + 96LL) * n > kSmallOperand) return;
-  auto cost = [&](int t, double own, double all, int resident) {
+  auto cost = [&](int t, double own, double all) {
     const double per_cu = (double)((m + t - 1LL) / t) * ((n + t - 1) / t) / cus;
     const double work = all * per_cu > own * ceil(per_cu) ? all * per_cu : own * ceil(per_cu);
-    return 3.0 + work * 1e-3 * k + (per_cu > resident ? 2.5 * (per_cu / resident - 1.0) : 0.0);
+    const double rounds = t == 16 ? 2.5 * (per_cu / 8.0 - 1.0) : 3.4 * (ceil(per_cu / 4.0) - 1.0);
+    return 3.0 + work * 1e-3 * k + (rounds > 0.0 ? rounds : 0.0);
   };
-  const double c16 = k <= 2048 ? cost(16, 1.49, 1.95, 8) : 1e30, c32 = cost(32, k > 2048 ? 5.2 : 4.36, k > 2048 ? 5.2 : 4.81, 5);
+  const double c16 = k <= 2048 ? cost(16, 1.49, 1.95) : 1e30, c32 = cost(32, k > 2048 ? 5.2 : 4.36, k > 2048 ? 5.2 : 4.81);
   if ((c16 < c32 ? c16 : c32) >= 0.9 * plan->us) return;
   *plan = SgemmPlan{true, 1};
   plan->tile = c16 < c32 ? 16 : 32;
