@@ -1287,8 +1287,17 @@ int fwd_channels(const ConvGeom& g) {
   const int width = fast_channels(g.C, g.K, g.RS, m);
   return off && width && !split_ranges(m, g.K, g.RS * (width / 16), tile, (size_t)-1) ? 0 : width;
 }
+// Up to four slabs and more than three small tiles per CU: their first loads and last stores are what counts, and larger tiles have
+// fewer.  Under 1 x 1, 24 -> 96 on 15 x 22 x 43 7.7 -> 9.1 us, 24 -> 32 on 78 x 9 x 56 6.6 -> 8.7, 32 -> 176 on 5 x 48 x 29 7.3 -> 8.3, data
+// gradient 176 <- 56 on 10 x 10 x 45 8.6 -> 9.6; 64 -> 168 on 26 x 9 x 11 (1.9 tiles) 7.3 -> 5.7.  Of 25 random layers 16 lost, two gained
+// more than 6% (360 <- 56 on 3 x 23 x 51 15.6 -> 12.2).
+bool small_stores_bound(long long m, int n, int slabs) {
+  return slabs <= 4 && (m + MNV_SMALL_TILE - 1) / MNV_SMALL_TILE * ((n + MNV_SMALL_TILE - 1) / MNV_SMALL_TILE) > 3LL * mnv_cu_count();
+}
 // The forward pass on the small tiles: their k ranges (0: not), and the channels of the permuted filter
-// (0: the filter as it is).  From 16 channels on the generic gathers of padded layers are left for the permuted filter.
+// (0: the filter as it is).  From 16 channels on the generic gathers of padded layers are left for the permuted filter, unless
+// permuting it costs more: 6 us per million values beyond those that the estimate was fitted to (5 x 5 at stride 2, 200 -> 328 on 4 x 10 x 8
+// 14.3 -> 20.1 us, 264 -> 264 on 6 x 19 x 8 31.4 -> 36.1, 104 -> 384 on 2 x 11 x 25 17.2 -> 19.1).
 struct SmallForward {
   int z = 0, width = 0;
   size_t filter_bytes = 0;
@@ -1304,7 +1313,10 @@ SmallForward small_forward(const ConvGeom& g, size_t ws_bytes) {
   p.filter_bytes = (size_t)g.K * g.RS * p.width * sizeof(float);
   if (p.filter_bytes > ws_bytes) return p;
   const size_t left = ws_bytes > align256(p.filter_bytes) ? (ws_bytes - align256(p.filter_bytes)) / sizeof(float) : 0;
-  p.z = small_gather_ranges(m, g.K, p.width ? g.RS * (p.width / 16) : slabs, tile, m, slabs, 1.0, left);
+  const int own = p.width ? g.RS * (p.width / 16) : slabs;
+  if (small_stores_bound(m, g.K, own)) return p;
+  const double permute = p.width && !width ? std::max(0.0, 6e-6 * ((double)g.K * g.RS * p.width - 4e5)) : 0.0;
+  p.z = small_gather_ranges(m, g.K, own, tile, m, slabs, 1.0 - permute, left);
   return p;
 }
 size_t small_bytes(size_t filter_bytes, int z, size_t results) {
@@ -1403,7 +1415,7 @@ int small_bwd_data(const ConvGeom& g, int width, size_t ws_bytes) {
   const int m = g.N * g.HW, tile = pick_tile(m, g.C), slabs = g.RS * (width / 16);
   if (split_ranges(m, g.C, slabs, tile, (size_t)-1)) return 0;
   const size_t left = ws_bytes > align256(filter_bytes) ? (ws_bytes - align256(filter_bytes)) / sizeof(float) : 0;
-  return small_gather_ranges(m, g.C, slabs, tile, m, slabs, 2.0, left);
+  return small_stores_bound(m, g.C, slabs) ? 0 : small_gather_ranges(m, g.C, slabs, tile, m, slabs, 2.0, left);
 }
 
 // k ranges of the filter gradient: up to 256, and up to 512 for outputs of at most 16384

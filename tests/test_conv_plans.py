@@ -102,3 +102,20 @@ def test_strided_data_gradients_sum_no_longer_than_the_generic_gathers(dims, pla
     N, C, K, H, W, pad, R = dims
     got = _data_plan((N, C, K, H, W, pad, pad, 2, 2, R, R))
     assert (got[0], got[2], got[3]) == plan + (4,)
+
+
+@pytest.mark.parametrize("direction,dims,small", [  # N, C, K, H, W, pad, R, stride
+    ("fwd", (15, 24, 96, 22, 43, 0, 1, 1), False), ("fwd", (78, 24, 32, 9, 56, 0, 1, 1), False), ("fwd", (23, 24, 96, 46, 46, 0, 1, 2), False),
+    ("fwd", (67, 40, 64, 32, 8, 0, 1, 1), False), ("bwd_data", (10, 176, 56, 10, 45, 0, 1, 1), False),
+    ("bwd_data", (16, 136, 56, 54, 9, 0, 1, 1), False),                                          # few slabs, many tiles
+    ("fwd", (26, 64, 168, 9, 11, 0, 1, 1), True), ("bwd_data", (52, 24, 72, 18, 19, 0, 1, 1), True), ("fwd", (64, 88, 24, 49, 17, 0, 1, 2), True),
+    ("fwd", (4, 200, 328, 10, 8, 0, 5, 2), False), ("fwd", (6, 264, 264, 19, 8, 2, 5, 2), False),   # a large filter to permute
+    ("fwd", (2, 104, 384, 11, 25, 2, 5, 2), False), ("fwd", (2, 136, 280, 11, 14, 1, 3, 2), True), ("fwd", (1, 120, 224, 25, 33, 1, 3, 2), True),
+])
+def test_layers_that_small_tiles_slow_down_stay_on_larger_ones(direction, dims, small):
+    N, C, K, H, W, pad, R, stride = dims
+    full = (N, C, K, H, W, pad, pad, stride, stride, R, R)
+    v = [ctypes.c_int() for _ in range(4 if direction == "bwd_data" else 3)]
+    ws = getattr(capi.lib(), "mnv_conv_%s_workspace_bytes" % direction)(*full)
+    assert getattr(capi.lib(), "mnv_conv_%s_plan" % direction)(*full, ctypes.c_size_t(ws), *[ctypes.byref(x) for x in v]) == 0
+    assert (v[0].value == 32) == small
