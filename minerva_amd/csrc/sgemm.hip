@@ -584,9 +584,15 @@ double split_cost(int m, int n, int k, int z, int cus) {
 //   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
 //   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
 //   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.  Beyond 16 tiles of 128 x 128, whose 16 k ranges at most make no
-//   more workgroups than CUs, the grouped ones are weighed too, at 0.84 us per unit of their estimate: 341 x 3956 x 1002 41 -> 34,
-//   2177 x 1155 x 3047 201 -> 129, 3106 x 1474 x 2652 226 -> 162, 1340 x 599 x 3458 70 -> 49, 200 x 3319 x 2055 44 -> 33, 2048 x 300 x 3000
-//   43 -> 35; 120 random products of 65 tiles and more that it moves 0.82 of the time, half the error, 60 of fewer 0.78 and 0.40.  Grouped tiles of exactly one per CU
+//   more workgroups than CUs, the grouped ones are weighed too, at 0.84 us per unit of their estimate, against parts with at least
+//   twice their ranges.  Their four wavefronts sum a quarter of a range each, rounded at every k; one chain in parts, rounded at
+//   every eighth, is nearer to float64 where signs are mixed (0.66 of the error), but of positive terms, whose sum grows with k, it is
+//   sqrt(2) times as far (2408 x 1161 x 2681 of uniform operands 2.03e-7 -> 2.86e-7, both from a ReLU 0.98e-7 -> 2.28e-7); with twice
+//   the ranges half of that.  us, and error of normal / uniform operands of those that it moves: 341 x 3956 x 1002 45 -> 37 (2.9 -> 1.3 / 1.13 -> 0.85e-7),
+//   2177 x 1155 x 3047 212 -> 111 (5.0 -> 1.6 / 2.1 -> 0.85; one chain 129, 3.4 / 3.0), 3106 x 1474 x 2652 223 -> 160, 1340 x 599 x 3458 70 -> 48, 200 x 3319 x 2055
+//   44 -> 33, 2048 x 300 x 3000 42.7 -> 39.7 (five ranges for three 35.9, uniform operands 7.25 -> 7.43e-8); 898 random products that it moves 0.80 of the
+//   time, of the error 0.38 / 0.59 and none above.  Two ranges have to gain a tenth: their estimate is 20% low below 700 k (1882 x 897 x 472
+//   22.5 -> 26.9) and as much too high above 1200; those of three and more all gained.  Grouped tiles of exactly one per CU
 //   are the plan that the inner products of 256 columns are documented to have and stay (*4096 x 256 x 4096 74 -> 56).
 void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {
   if (plan->tall || (!plan->small && plan->groups == 4)) {
@@ -602,24 +608,21 @@ void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, Sge
   if (plan->groups == 4 && (tiles * MNV_SGEMM_MAX_SPLITS <= cus || (plan->splits == 1 && (m + 63LL) / 64 * ((n + 63) / 64) == cus))) return;
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
-  int best_z = 1;
-  double best = split_cost(m, n, k, 1, cus);
-  // of tiles that a cut tail spreads evenly
-  if (plan->groups == 4 && mnv_tail_plan(tiles, slabs, 128 * 128, (size_t)-1 / sizeof(float), SplitPair::TAIL).z > 1) {
-    const double cut = 1.3 * ((double)tiles / cus + 0.25) * ((slabs + 1) / 2) + 6.0;
-    if (cut < best) best = cut;
-  }
-  for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus; ++z) {
+  const int least_z = plan->groups == 4 ? 2 * plan->splits : 1;
+  int best_z = 0;
+  double best = 1e30;
+  for (int z = least_z; z == 1 || (z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus); ++z) {
     const double c = split_cost(m, n, k, z, cus);
-    if (c < 0.97 * best) {
+    if (c < (best_z ? 0.97 : 1.0) * best) {
       best = c;
       best_z = z;
     }
   }
+  if (!best_z) return;
   // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
   // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6), of under 20 us to the small and the
   // grouped tiles (3312 x 73 x 1235 15.0 -> 18.0, 143 x 2058 x 1764 19.6 -> 21.2).
-  if (plan->groups == 4 ? best > 0.9 * 0.84 * cost || (best_z > 1 && best < 20.0) : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
+  if (plan->groups == 4 ? best > (best_z > 2 ? 1.0 : 0.9) * 0.84 * cost || (best_z > 1 && best < 20.0) : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
   *plan = SgemmPlan{false, best_z};
   plan->split = true;
 }

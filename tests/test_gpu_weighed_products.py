@@ -14,10 +14,13 @@ def _plan(m, n, k, ws):
     return tuple(x.value for x in v)
 
 
-# 17 to 63 tiles of 128 x 128 with k ranges, ragged in every extent; 65 and more, with and without ranges
+# 17 to 63 tiles of 128 x 128, ragged in every extent; 65 and more
 MOVED = [(1340, 599, 3458), (2500, 200, 2048), (2048, 300, 3000), (341, 3956, 1002), (2177, 1155, 3047)]
-# at most 16 tiles; one grouped tile per CU; ranges of under 20 us
-STAY = [(200, 1000, 4099), (500, 500, 3000), (1000, 256, 4096), (4096, 256, 4096), (3312, 73, 1235), (143, 2058, 1764)]
+# at most 16 tiles; one grouped tile per CU; ranges of under 20 us; two ranges that gain less than a tenth
+STAY = [(200, 1000, 4099), (500, 500, 3000), (1000, 256, 4096), (4096, 256, 4096), (3312, 73, 1235), (143, 2058, 1764),
+        (2871, 1084, 1927)]
+# the k ranges of the grouped tiles; in parts with as many, or few more, sums of positive terms were less exact
+RANGES = [(2177, 1155, 3047, 1), (2408, 1161, 2681, 1), (2871, 1084, 1927, 1), (2048, 300, 3000, 3)]
 
 
 @pytest.mark.parametrize("m,n,k", MOVED)
@@ -28,6 +31,35 @@ def test_products_weighed_against_the_parts(m, n, k):
 @pytest.mark.parametrize("m,n,k", STAY)
 def test_products_that_stay_on_small_tiles(m, n, k):
     assert _plan(m, n, k, 1 << 40)[0] == 64
+
+
+@pytest.mark.parametrize("m,n,k,grouped", RANGES)
+def test_parts_have_at_least_twice_the_ranges_of_the_grouped_tiles(m, n, k, grouped):
+    """Whatever is lent; without a workspace there are no ranges, and the grouped tiles stay."""
+    full = capi.lib().mnv_sgemm_nn_workspace_bytes(m, n, k)
+    for ws in (0, 4 * m * n, full // 2, full, 1 << 40):
+        rows, ranges, _ = _plan(m, n, k, ws)
+        assert rows == 64 or (ws and ranges >= 2 * grouped), ws
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,grouped", RANGES)
+def test_sums_of_positive_terms_are_as_exact_as_on_the_grouped_tiles(m, n, k, grouped):
+    """Their distance from float64 (2-norm, relative) is that of 4 * grouped sums of k / (4 * grouped) positive terms,
+    rounded at each: the squares of the partial sums of all add up to k / 48 / grouped^2 of the whole sum's.  A rounding
+    is 0.4247 * 2^-24 of its value where logarithms are evenly spread; a tenth, and the additions of the ranges, on top."""
+    from gpu_util import Gpu, say
+    gpu = Gpu()
+    rng = np.random.default_rng(k)
+    A, B = rng.random((m, k), np.float32), rng.random((k, n), np.float32)
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    ws = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    say("positive terms", m, n, k, "plan", _plan(m, n, k, ws))
+    a, b = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(np.ascontiguousarray(B.T).reshape(-1))
+    c, scratch = gpu.empty(m * n), gpu.empty(max(1, ws // 4))
+    gpu.call("mnv_sgemm_nn", a.p, b.p, c.p, m, n, k, scratch.p, ctypes.c_size_t(ws))
+    error = np.linalg.norm(gpu.down(c).reshape(n, m).T.astype(np.float64) - exact) / np.linalg.norm(exact)
+    assert error <= 1.1 * 0.4247 * 2.0 ** -24 * np.sqrt(k / 48 / grouped ** 2 + 4 * grouped / 3 + 1)
 
 
 @pytest.mark.gpu
