@@ -591,7 +591,7 @@ double split_cost(int m, int n, int k, int z, int cus) {
 //   the ranges half of that.  us, and error of normal / uniform operands of those that it moves: 341 x 3956 x 1002 45 -> 37 (2.9 -> 1.3 / 1.13 -> 0.85e-7),
 //   2177 x 1155 x 3047 212 -> 111 (5.0 -> 1.6 / 2.1 -> 0.85; one chain 129, 3.4 / 3.0), 3106 x 1474 x 2652 223 -> 160, 1340 x 599 x 3458 70 -> 48, 200 x 3319 x 2055
 //   44 -> 33, 2048 x 300 x 3000 42.7 -> 39.7 (five ranges for three 35.9, uniform operands 7.25 -> 7.43e-8); 898 random products that it moves 0.80 of the
-//   time, of the error 0.38 / 0.59 and none above.  Two ranges have to gain a tenth: their estimate is 20% low below 700 k (1882 x 897 x 472
+//   time, of the error 0.37 / 0.55 and none above (both from a ReLU 0.75, 1.09 at most).  Two ranges have to gain a tenth: their estimate is 20% low below 700 k (1882 x 897 x 472
 //   22.5 -> 26.9) and as much too high above 1200; those of three and more all gained.  Grouped tiles of exactly one per CU
 //   are the plan that the inner products of 256 columns are documented to have and stay (*4096 x 256 x 4096 74 -> 56).
 void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {

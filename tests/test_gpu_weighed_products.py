@@ -79,3 +79,34 @@ def test_weighed_products_against_float64(m, n, k):
         c, scratch = gpu.up(np.full(m * n, np.nan, np.float32)), gpu.up(np.full(max(1, ws // 4), np.nan, np.float32))
         gpu.call("mnv_sgemm_nn", a.p, b.p, c.p, m, n, k, scratch.p, ctypes.c_size_t(ws))
         assert np.all(np.abs(gpu.down(c).reshape(n, m).T - exact) <= bound), ws
+
+
+def _rounding(sums, k, ranges):
+    """Relative rms error of sums of positive terms in `ranges` ranges of k, rounded at every eighth k, that are added four at a
+    time: a rounding is evenly spread over a unit in the last place of the partial sum, whose size is its share of the whole."""
+    shares = [np.arange(8, k / ranges, 8) / k] * ranges
+    for first in range(0, ranges, 4):
+        four = min(4, ranges - first)
+        shares += [np.array([2, 2, 4] if four == 4 else range(2, four + 1)) / ranges]  # (0 + 1) + (2 + 3); what is left in order
+        shares += [np.array([first + four] if first else []) / ranges]
+    units = np.exp2(np.floor(np.log2(sums[:, None] * np.concatenate(shares))) - 23)
+    return np.sqrt((units ** 2).sum(1).mean() / 12 / (sums ** 2).mean())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,ranges", [(379, 646, 3505, 14), (123, 2426, 3647, 13), (242, 1090, 3830, 12)])
+def test_partial_results_are_added_four_at_a_time(m, n, k, ranges):
+    """Both operands from a ReLU.  One after the other, the additions make the error 1.19 to 1.4 times the bound."""
+    from gpu_util import Gpu, say
+    gpu = Gpu()
+    rng = np.random.default_rng(k)
+    A, B = (np.maximum(rng.standard_normal(s, np.float32), np.float32(0)) for s in ((m, k), (k, n)))
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    ws = gpu.L.mnv_sgemm_nn_workspace_bytes(m, n, k)
+    say("partial results", m, n, k, "plan", _plan(m, n, k, ws))
+    assert _plan(m, n, k, ws) == (128, ranges, 1)
+    a, b = gpu.up(np.ascontiguousarray(A.T).reshape(-1)), gpu.up(np.ascontiguousarray(B.T).reshape(-1))
+    c, scratch = gpu.empty(m * n), gpu.empty(ws // 4)
+    gpu.call("mnv_sgemm_nn", a.p, b.p, c.p, m, n, k, scratch.p, ctypes.c_size_t(ws))
+    error = np.linalg.norm(gpu.down(c).reshape(n, m).T.astype(np.float64) - exact) / np.linalg.norm(exact)
+    assert error <= 1.04 * _rounding(exact.reshape(-1)[::97], k, ranges)
