@@ -711,7 +711,8 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
 // 3.4 us for each further round (with 2.5 of the larger tiles: 555 x 2773 x 156 10.0 -> 11.6, 2411 x 630 x 201 12.6 -> 15.0, 433 x 3053 x 133
 // 10.4 -> 11.4, 3921 x 332 x 232 13.0 -> 13.9, which now stay; 1770 x 721 x 430 25.6 -> 20.1 does not).
 // From 2048 k on 16 x 16 tiles take up to 1.4 times their estimate (292 x 243 x 3361 14.8 -> 21.7; 49 x 98 x 3847 11.7 -> 9.8) and are
-// left to the k ranges.  500 random products that it moves 0.56 of the time, none slower; 400 of at least 250 rows
+// left to the k ranges; from 1024 k on those of more than four to a CU do, and count 2.6 us (509 x 513 x 1935 on tiles of the core 21.4, on these 30.0;
+// 2468 x 102 x 1441 18.6, 21.4, on 32 x 32 tiles 18.4; 674 random products that leave them 0.90 of the time).  500 random products that it moves 0.56 of the time, none slower; 400 of at least 250 rows
 // and columns 0.66, two slower by more than 3% (1538 x 609 x 248 9.9 -> 10.5, 459 x 1917 x 200 8.8 -> 9.2).  Four wavefronts for many tiles, eight for few.
 // The kernel reads an x-fast operand up to 95 k past its end: its offsets have to stay below 2^31.
 void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
@@ -723,7 +724,8 @@ void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
     const double rounds = t == 16 ? 2.5 * (per_cu / 8.0 - 1.0) : 3.4 * (ceil(per_cu / 4.0) - 1.0);
     return 3.0 + work * 1e-3 * k + (rounds > 0.0 ? rounds : 0.0);
   };
-  const double c16 = k <= 2048 ? cost(16, 1.49, 1.95) : 1e30, c32 = cost(32, k > 2048 ? 5.2 : 4.36, k > 2048 ? 5.2 : 4.81);
+  const bool fifth = k > 1024 && (m + 15LL) / 16 * ((n + 15) / 16) > 4LL * cus;
+  const double c16 = k <= 2048 ? cost(16, 1.49, fifth ? 2.6 : 1.95) : 1e30, c32 = cost(32, k > 2048 ? 5.2 : 4.36, k > 2048 ? 5.2 : 4.81);
   if ((c16 < c32 ? c16 : c32) >= 0.9 * plan->us) return;
   *plan = SgemmPlan{true, 1};
   plan->tile = c16 < c32 ? 16 : 32;
