@@ -806,9 +806,9 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
 }
 
 // Small tiles for products that the tiles above leave most CUs without, or in k ranges that cost more to add than to
-// multiply: T x T, one per workgroup, whose W wavefronts share the workgroup's k range.  No operand passes through LDS: a lane fetches the four k of a vector for its own row and its
-// own column through the policy (both operands k-fast), three slabs ahead, and multiplies them; lane group h (of 64 / T)
-// holds the k 4 h .. 4 h + 3 of each run of 4 * 64 / T.  A wavefront adds up the sums of runs of two slabs, of one for the last three, and the wavefronts' sums are
+// multiply: 32 x 32, one per workgroup, whose four wavefronts share the workgroup's k range.  No operand passes through LDS: a lane fetches the four k of a vector for its own row and its
+// own column through the policy (both operands k-fast), three slabs ahead, and multiplies them; lane group h (of two)
+// holds the k 4 h .. 4 h + 3 of each run of eight.  A wavefront adds up the sums of runs of two slabs, of one for the last three, and the wavefronts' sums are
 // added in LDS in the order of k, or left as a partial result per k range of blockIdx.z.  Error against float64 of the layers that run so,
 // of that on the tiles above: forward 0.68, data gradient 0.57 (of strided layers by classes 0.79), filter gradient 0.62 over 500 random ones, four
 // above 1.02 times, by up to 1.1; with one sum each for the even and the odd slabs 0.86, 0.77, 0.95 and 0.72, and 200 above, by up to 2.1; with
@@ -817,11 +817,12 @@ __global__ __launch_bounds__(T::NT * G, PF == 2 && T::MIN_WAVES == 4 ? 3 : T::MI
 // second run.  Neighbouring tiles
 // across the shorter side of the result share an XCD.  What bounds it, and where it is taken: mnv_small_ranges.
 #define MNV_SMALL_TILE 32
-template <class P, int T, int W>
-__global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob, int tiles_m, int tiles_n, int slabs_per_split,
+#define MNV_SMALL_WAVES 4
+template <class P>
+__global__ __launch_bounds__(MNV_SMALL_WAVES * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob, int tiles_m, int tiles_n, int slabs_per_split,
                                                                       float* __restrict__ partial) {
   static_assert(P::A_KFAST && P::B_KFAST && !MnvALaneK<P>::value, "vectors of four k");
-  constexpr int H = MNV_WAVE / T, RUN = 4 * H, VECS = 16 / RUN, REGS = T * T / MNV_WAVE;
+  constexpr int T = MNV_SMALL_TILE, W = MNV_SMALL_WAVES, H = MNV_WAVE / T, RUN = 4 * H, VECS = 16 / RUN, REGS = T * T / MNV_WAVE;
   typedef float Acc __attribute__((ext_vector_type(REGS)));
   extern __shared__ float mnv_small_lds[];  // W tiles of sums, then the policy's
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / MNV_WAVE)), lane = threadIdx.x % MNV_WAVE;
@@ -905,8 +906,7 @@ __global__ __launch_bounds__(W * MNV_WAVE, 4) void mnv_gemm_small_kernel(P prob,
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const Acc before = decltype(FIRST)::value && j == 0 && t == 0 ? Acc(0.f) : run;
-        if constexpr (T == 32) run = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
-        else run = __builtin_amdgcn_mfma_f32_16x16x4f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
+        run = __builtin_amdgcn_mfma_f32_32x32x2f32(b[set][j][t], a[set][j][t], before, 0, 0, 0);
       }
     if constexpr (decltype(LAST)::value) sum += run;
   };
@@ -1276,7 +1276,7 @@ static inline int mnv_small_ranges(long long m, int n, int slabs, size_t ws_floa
 // Host-side launch of the small tiles; `splits` > 1 needs splits * M * N floats at `workspace`.
 template <class P>
 static int mnv_gemm_small_launch(const P& prob, int splits, void* workspace, hipStream_t s) {
-  constexpr int T = MNV_SMALL_TILE, W = 4;
+  constexpr int T = MNV_SMALL_TILE, W = MNV_SMALL_WAVES;
   const int tiles_m = (prob.M + T - 1) / T, tiles_n = (prob.N + T - 1) / T;
   if (splits > prob.total_slabs) splits = prob.total_slabs;
   if (splits < 1) splits = 1;
@@ -1284,7 +1284,7 @@ static int mnv_gemm_small_launch(const P& prob, int splits, void* workspace, hip
   splits = per > 0 ? (prob.total_slabs + per - 1) / per : 1;
   const size_t lds = W * T * T * sizeof(float) + prob.extra_lds_bytes();
   if ((long long)tiles_m * tiles_n > 0x7fffffffLL || splits > 65535 || lds > 64 * 1024) return MNV_ERR_INVALID;
-  hipLaunchKernelGGL((mnv_gemm_small_kernel<P, T, W>), dim3(tiles_m * tiles_n, 1, splits), dim3(W * MNV_WAVE), lds, s, prob,
+  hipLaunchKernelGGL(mnv_gemm_small_kernel<P>, dim3(tiles_m * tiles_n, 1, splits), dim3(W * MNV_WAVE), lds, s, prob,
                      tiles_m, tiles_n, per, reinterpret_cast<float*>(workspace));
   const int rc = MNV_LAUNCH_STATUS();
   if (rc || splits == 1) return rc;
