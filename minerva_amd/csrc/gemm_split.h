@@ -20,7 +20,7 @@
 // ReLU 1.3e-7 / 3.3e-7).  Folding the sums every 512 k into a third set of accumulators mends half of these
 // (of 70 random extents of uniform operands 21 were worse than the fp32 kernel, and 10 with it): only one workgroup per
 // CU leaves registers for it, and it costs up to 9% (1215 x 1372 x 3540 81 -> 88 us).  More k ranges mend it, and where the small
-// tiles' four wavefronts are left for parts there are enough of them (plan_split).
+// tiles' four wavefronts are left for parts there are enough of them (plan_grouped).
 //
 // Range.  Operands are multiplied by 2^16 before the cut, so that the last bit of the smallest
 // denormal is still a bf16 denormal, and the product by 2^-32 after the sum.  An operand from

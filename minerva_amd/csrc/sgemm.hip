@@ -512,6 +512,7 @@ struct SgemmPlan {
   int skinny = 0;     // > 0: mnv_sgemm_skinny_kernel or, A transposed, its _tn_ twin; this many k per wavefront
   int tile = 0;       // 16, 32: mnv_sgemm_small_kernel with `groups` wavefronts
   double us = 0.0;    // the estimate of one on 64 x 64 or larger tiles
+  bool from_grouped = false;  // in parts by plan_grouped
 };
 
 // Enough k ranges for 2048 wavefronts (eight on each CU, 4 KB or more of A in flight in each), with
@@ -583,48 +584,69 @@ double split_cost(int m, int n, int k, int z, int cus) {
 //   4096 x 1000 x 1000 76 -> 48, 4096 x 100 x 4096 47 -> 32, 200 x 3000 x 4000 67 -> 48, 1500 x 1500 x 1500
 //   73 -> 56, 2100 x 2100 x 700 61 -> 56, *512 x 512 x 512 12.7 -> 13.6, *300 x 300 x 300 8.4 -> 10.8,
 //   *256 x 256 x 784 9.2 -> 11.9, *700 x 1500 x 90 8.4 -> 8.7; of the grouped 64 x 64 tiles *1000 x 256 x 4096
-//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.  Beyond 16 tiles of 128 x 128, whose 16 k ranges at most make no
-//   more workgroups than CUs, the grouped ones are weighed too, at 0.84 us per unit of their estimate, against parts with at least
-//   twice their ranges.  Their four wavefronts sum a quarter of a range each, rounded at every k; one chain in parts, rounded at
-//   every eighth, is nearer to float64 where signs are mixed (0.66 of the error), but of positive terms, whose sum grows with k, it is
-//   sqrt(2) times as far (2408 x 1161 x 2681 of uniform operands 2.03e-7 -> 2.86e-7, both from a ReLU 0.98e-7 -> 2.28e-7); with twice
-//   the ranges half of that.  us, and error of normal / uniform operands of those that it moves: 341 x 3956 x 1002 45 -> 37 (2.9 -> 1.3 / 1.13 -> 0.85e-7),
-//   2177 x 1155 x 3047 212 -> 111 (5.0 -> 1.6 / 2.1 -> 0.85; one chain 129, 3.4 / 3.0), 3106 x 1474 x 2652 223 -> 160, 1340 x 599 x 3458 70 -> 48, 200 x 3319 x 2055
-//   44 -> 33, 2048 x 300 x 3000 42.7 -> 39.7 (five ranges for three 35.9, uniform operands 7.25 -> 7.43e-8); 898 random products that it moves 0.80 of the
-//   time, of the error 0.37 / 0.55 and none above (both from a ReLU 0.75, 1.09 at most).  Two ranges have to gain a tenth: their estimate is 20% low below 700 k (1882 x 897 x 472
-//   22.5 -> 26.9) and as much too high above 1200; those of three and more all gained.  Grouped tiles of exactly one per CU
-//   are the plan that the inner products of 256 columns are documented to have and stay (*4096 x 256 x 4096 74 -> 56).
+//   24.7 -> 22.2, *4096 x 50 x 9216 51 -> 49, *4096 x 256 x 1000 21.7 -> 24.0.
 void plan_split(int m, int n, int k, size_t ws_floats, double cost, int cus, SgemmPlan* plan) {
   if (plan->tall || (!plan->small && plan->groups == 4)) {
     plan->split = true;
     return;
   }
-  if (m <= 64 || n <= 64) return;
+  if (plan->groups == 4 || m <= 64 || n <= 64) return;
   // One slab fills half of a step, and what such a product takes is the time of its stores, which the fp32 kernel, with
   // twice the workgroups per CU, spreads better (fp32 instruction / parts, us: k = 16 4096 x 4096 16.4 / 18.9, 4096 x 9216
   // 30.0 / 33.7, k = 17 20.4 / 18.3, 38.9 / 32.4).  Those planned on 64 x 64 tiles gain as little by parts as they lose.
   if (k <= 16 && !plan->small) return;
   const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
-  if (plan->groups == 4 && (tiles * MNV_SGEMM_MAX_SPLITS <= cus || (plan->splits == 1 && (m + 63LL) / 64 * ((n + 63) / 64) == cus))) return;
   const size_t fit = ws_floats / ((size_t)m * n);
   const int slabs = (k + 15) / 16;
-  const int least_z = plan->groups == 4 ? 2 * plan->splits : 1;
-  int best_z = 0;
-  double best = 1e30;
-  for (int z = least_z; z == 1 || (z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus); ++z) {
+  int best_z = 1;
+  double best = split_cost(m, n, k, 1, cus);
+  for (int z = 2; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8 && tiles < 2LL * cus; ++z) {
     const double c = split_cost(m, n, k, z, cus);
-    if (c < (best_z ? 0.97 : 1.0) * best) {
+    if (c < 0.97 * best) {
       best = c;
       best_z = z;
     }
   }
-  if (!best_z) return;
   // k ranges of under 18 us lose to those of the 64 x 64 tiles (617 x 332 x 1746 15.7 -> 18.1, 122 x 1419 x
-  // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6), of under 20 us to the small and the
-  // grouped tiles (3312 x 73 x 1235 15.0 -> 18.0, 143 x 2058 x 1764 19.6 -> 21.2).
-  if (plan->groups == 4 ? best > (best_z > 2 ? 1.0 : 0.9) * 0.84 * cost || (best_z > 1 && best < 20.0) : plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
+  // 1663 16.1 -> 17.9; above, 785 x 426 x 2236 25.5 -> 21.8, 541 x 1220 x 2092 37.9 -> 29.6).
+  if (plan->small && (best > 0.9 * 0.83 * cost || (best_z > 1 && best < 18.0))) return;
   *plan = SgemmPlan{false, best_z};
   plan->split = true;
+}
+
+// Grouped 64 x 64 tiles against parts.  Their four wavefronts sum a quarter of a k range each, rounded at every k.  One chain in parts, rounded at
+// every eighth, is nearer to float64 where signs are mixed (0.66 of the error), but of positive terms, whose sum grows with k, it is
+// sqrt(2) times as far (2408 x 1161 x 2681 of uniform operands 2.03e-7 -> 2.86e-7, both from a ReLU 0.98e-7 -> 2.28e-7); with twice
+// the ranges half of that.  So parts have at least twice the ranges of the grouped tiles.  Of 889 random products that leave them none is
+// slower, they take 0.79 of the time, and of the error 0.37 for normal and 0.54 for uniform operands, none more than before (both from
+// a ReLU 0.75, 1.10 at most).  us, and errors of normal and uniform operands in 1e-7: 341 x 3956 x 1002 45 -> 37 (2.9 -> 1.3, 1.13 -> 0.85),
+// 2177 x 1155 x 3047 203 -> 114 (5.0 -> 1.6, 2.1 -> 0.83; in one chain 130, 3.4, 3.0), 3106 x 1474 x 2652 231 -> 162, 1340 x 599 x 3458 69 -> 48, 200 x 3319 x 2055
+// 44 -> 33, 2048 x 300 x 3000 42.5 -> 39.5 (five ranges instead of three 35.7, uniform 0.73 -> 0.74).
+// At most 16 tiles of 128 x 128, whose 16 ranges make no more workgroups than CUs, stay (*1000 x 256 x 4096 24.7 -> 22.2, *4096 x 256 x 1000
+// 21.7 -> 24.0), ranges of under 20 us (3312 x 73 x 1235 15.0 -> 18.0, 143 x 2058 x 1764 19.6 -> 21.2), and grouped tiles of exactly one per CU, the
+// plan that the inner products of 256 columns are documented to have (*4096 x 256 x 4096 74 -> 56).  The estimate of
+// the grouped tiles is 20% low below 700 k, where two ranges have to gain 18% (1882 x 897 x 472 22.5 -> 26.9), and above 1200 k as
+// much too high; ranges of under 40 us have to gain a tenth.
+void plan_grouped(int m, int n, int k, size_t ws_floats, int cus, SgemmPlan* plan) {
+  if (plan->groups != 4 || !plan->small || m <= 64 || n <= 64) return;
+  const long long tiles = (long long)((m + 127) / 128) * ((n + 127) / 128);
+  if (tiles * MNV_SGEMM_MAX_SPLITS <= cus || (plan->splits == 1 && (m + 63LL) / 64 * ((n + 63) / 64) == cus)) return;
+  const size_t fit = ws_floats / ((size_t)m * n);
+  const int slabs = (k + 15) / 16;
+  int best_z = 0;
+  double best = 1e30;
+  for (int z = 2 * plan->splits; z <= MNV_SGEMM_MAX_SPLITS && (size_t)z <= fit && slabs / z >= 8; ++z) {
+    const double c = split_cost(m, n, k, z, cus);
+    if (c < best) {
+      best = c;
+      best_z = z;
+    }
+  }
+  if (!best_z || best < 20.0) return;
+  if (best > (best_z == 2 && slabs < 50 ? 0.82 : best < 40.0 ? 0.9 : 1.0) * plan->us) return;
+  *plan = SgemmPlan{false, best_z};
+  plan->split = plan->from_grouped = true;
+  plan->us = best;
 }
 
 // The cheapest of the plans whose partial results fit `ws_floats`.  `cus`: the device's, asked for once per
@@ -716,8 +738,8 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
 // and columns 0.66, two slower by more than 3% (1538 x 609 x 248 9.9 -> 10.5, 459 x 1917 x 200 8.8 -> 9.2).  Four wavefronts for many tiles, eight for few.
 // The kernel reads an x-fast operand up to 95 k past its end: its offsets have to stay below 2^31.
 void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
-  // (products in parts are the more exact ones)
-  if (plan->skinny || plan->split || (k + 96LL) * m > kSmallOperand || (k + 96LL) * n > kSmallOperand) return;
+  // (other products in parts are the more exact ones)
+  if (plan->skinny || (plan->split && !plan->from_grouped) || (k + 96LL) * m > kSmallOperand || (k + 96LL) * n > kSmallOperand) return;
   auto cost = [&](int t, double own, double all) {
     const double per_cu = (double)((m + t - 1LL) / t) * ((n + t - 1) / t) / cus;
     const double work = all * per_cu > own * ceil(per_cu) ? all * per_cu : own * ceil(per_cu);
@@ -748,6 +770,7 @@ SgemmPlan plan_unlimited(int m, int n, int k, int cus) {
     plan = next;
     if (same) break;
   }
+  plan_grouped(m, n, k, (size_t)-1, cus, &plan);
   plan_small(m, n, k, cus, &plan);
   return plan;
 }
@@ -761,6 +784,7 @@ SgemmPlan plan_sgemm(int m, int n, int k, size_t ws_floats) {
   SgemmPlan plan = plan_unlimited(m, n, k, cus);
   if (plan.splits == 1 || plan.splits <= ws_floats / ((size_t)m * n)) return plan;
   plan = plan_within(m, n, k, ws_floats, cus);
+  plan_grouped(m, n, k, ws_floats, cus, &plan);
   plan_small(m, n, k, cus, &plan);
   return plan;
 }
