@@ -729,9 +729,11 @@ SgemmPlan plan_within(int m, int n, int k, size_t ws_floats, int cus) {
 
 // A plan on the small kernel's tiles where that is estimated at less than 90% of `plan`: 3 us, and the larger of what the
 // fullest CU multiplies and what all tiles take from L2, 1.49 and 1.95 us per 1000 k of a 16 x 16 tile on every CU, 4.36 and
-// 4.81 of a 32 x 32 one (5.2 from 2048 k on); beyond the eight or four workgroups that a CU holds, 2.5 or
-// 3.4 us for each further round (with 2.5 of the larger tiles: 555 x 2773 x 156 10.0 -> 11.6, 2411 x 630 x 201 12.6 -> 15.0, 433 x 3053 x 133
+// 4.81 of a 32 x 32 one (5.2 from 2048 k on); beyond the eight or four and a half workgroups per CU, 2.5 or
+// 3.4 us for each further round (with 2.5 and five of the larger tiles: 555 x 2773 x 156 10.0 -> 11.6, 2411 x 630 x 201 12.6 -> 15.0, 433 x 3053 x 133
 // 10.4 -> 11.4, 3921 x 332 x 232 13.0 -> 13.9, which now stay; 1770 x 721 x 430 25.6 -> 20.1 does not).
+// Up to 128 k a round costs what it did with 2.5 and five workgroups: there the tiles of the core take longer than their estimate (864 x 1196 x 89
+// 8.1 -> 6.3, 1752 x 632 x 126 9.2 -> 7.2).
 // From 2048 k on 16 x 16 tiles take up to 1.4 times their estimate (292 x 243 x 3361 14.8 -> 21.7; 49 x 98 x 3847 11.7 -> 9.8) and are
 // left to the k ranges; from 1024 k on those of more than four to a CU do, and count 2.6 us (509 x 513 x 1935 on tiles of the core 21.4, on these 30.0;
 // 2468 x 102 x 1441 18.6, 21.4, on 32 x 32 tiles 18.4; 674 random products that leave them 0.90 of the time).  500 random products that it moves 0.56 of the time, none slower; 400 of at least 250 rows
@@ -743,7 +745,7 @@ void plan_small(int m, int n, int k, int cus, SgemmPlan* plan) {
   auto cost = [&](int t, double own, double all) {
     const double per_cu = (double)((m + t - 1LL) / t) * ((n + t - 1) / t) / cus;
     const double work = all * per_cu > own * ceil(per_cu) ? all * per_cu : own * ceil(per_cu);
-    const double rounds = t == 16 ? 2.5 * (per_cu / 8.0 - 1.0) : 3.4 * (ceil(per_cu / 4.0) - 1.0);
+    const double rounds = t == 16 ? 2.5 * (per_cu / 8.0 - 1.0) : k <= 128 ? 2.5 * (per_cu / 5.0 - 1.0) : 3.4 * (ceil(per_cu / 4.5) - 1.0);
     return 3.0 + work * 1e-3 * k + (rounds > 0.0 ? rounds : 0.0);
   };
   const bool fifth = k > 1024 && (m + 15LL) / 16 * ((n + 15) / 16) > 4LL * cus;

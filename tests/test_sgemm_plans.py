@@ -145,6 +145,7 @@ def test_weighing_many_launches_costs_little_host_time():
     (509, 513, 1935, 0, 0), (597, 428, 1999, 0, 0), (600, 447, 1819, 0, 0), (2468, 102, 1441, 32, 4),  # a fifth 16 x 16 tile on a CU, long k
     (143, 1592, 2779, 32, 8), (1586, 158, 2770, 32, 8), (2138, 704, 499, 32, 4),  # weighed against k ranges in parts
     (509, 513, 1020, 16, 4), (365, 680, 1890, 16, 4),                     # shorter k; four of them
+    (864, 1196, 89, 32, 4), (1752, 632, 126, 32, 4), (536, 2220, 117, 32, 4),  # more than four of them to a CU, short k
     (1, 1, 1, 0, 0), (15, 17, 3, 0, 0),                                   # one slab: the 64 x 64 tile
     (200, 1000, 4099, 0, 0), (500, 500, 3000, 0, 0), (4096, 3, 5000, 0, 0),  # k ranges: only with a workspace
     (4096, 4096, 4096, 0, 0),
