@@ -1155,7 +1155,8 @@ size_t split_bytes(int tile, int m, int n, int slabs) {
 // us: 24 -> 32 channels under 3 x 3 on 19 x 44 x 12 12.3 -> 5.8, 80 -> 32 under 5 x 5, stride 2, on 59 x 48 x 20 82 -> 36,
 // data gradient 32 <- 160 under 3 x 3 on 4 x 53 x 52 34 -> 21, 40 <- 48 on 7 x 14 x 41 13.8 -> 7.7.
 const MnvSmallCost kSmallGather{0.0992, 2.8, 2.0, 0.0}, kSmallFilter{0.1824, 4.3, 1.4, 3.9};
-int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats);
+int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats,
+                        double share = 1.0);
 // where their vectors' offsets (channel planes, rows past the last) stay within 32 bits
 bool small_reach(const ConvGeom& g) {
   const long long lim = (1LL << 28) - 1;
@@ -1233,14 +1234,15 @@ int small_tile_splits(int tile, int m, int n, int slabs, size_t ws_floats) {
   return want < 2 ? 1 : (int)want;
 }
 
-int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats) {
+int small_gather_ranges(long long rows, int n, int small_slabs, int tile, long long tile_rows, int slabs, double fixed, size_t ws_floats,
+                        double share) {
   if ((tile != 0 && tile != 3) || tile_rows > 0x7fffffff) return 0;
   const int splits = small_tile_splits(tile, (int)tile_rows, n, slabs, (size_t)-1);
   const long long tiles = (tile_rows + kTileM[tile] - 1) / kTileM[tile] * ((n + kTileN[tile] - 1) / kTileN[tile]);
   const double slab = (tile == 0 ? 0.28 : 0.46) * (double)tiles * splits / mnv_cu_count();
   double against = fixed + (slab > 0.3 ? slab : 0.3) * ((slabs + splits - 1) / splits);
   if (splits > 1) against += (tile == 0 ? 2.6 : 3.0) + (tile == 0 ? 1.6 : 0.7) * 8.0 * (double)tile_rows * n * splits / 6e6;
-  return mnv_small_ranges(rows, n, small_slabs, ws_floats, kSmallGather, against);
+  return mnv_small_ranges(rows, n, small_slabs, ws_floats, kSmallGather, share * against);
 }
 
 // Workspace layout of the forward and data-gradient convolutions: the permuted filter
@@ -1316,7 +1318,10 @@ SmallForward small_forward(const ConvGeom& g, size_t ws_bytes) {
   const int own = p.width ? g.RS * (p.width / 16) : slabs;
   if (small_stores_bound(m, g.K, own)) return p;
   const double permute = p.width && !width ? std::max(0.0, 6e-6 * ((double)g.K * g.RS * p.width - 4e5)) : 0.0;
-  p.z = small_gather_ranges(m, g.K, own, tile, m, slabs, 1.0 - permute, left);
+  // Strides above 1 scatter the positions that a load gathers, and a slab of the small tiles takes longer than its estimate.  Without
+  // padding they gain below 80% of the other launch's (336 random layers, 0.82 of the time), above
+  // they do not (45, 1.02; 216 -> 24 under 5 x 5 on 35 x 34 x 8 22.2 -> 40.7 us); padded layers still do (47, 0.94).
+  p.z = small_gather_ranges(m, g.K, own, tile, m, slabs, 1.0 - permute, left, !g.ph && !g.pw && (g.sv > 1 || g.sh > 1) ? 0.92 : 1.0);
   return p;
 }
 size_t small_bytes(size_t filter_bytes, int z, size_t results) {

@@ -1249,9 +1249,10 @@ static int mnv_gemm_launch(const P& prob, int splits, void* workspace, hipStream
 // `byte_factor` (of 6 TB/s) for the reduction of the k ranges.  `fixed`: beside what the competitor has too.  Fitted to 260
 // layers of up to 12 GFLOP with 1 to 64 ranges (15 to 20% off, rms): by this rule their forward passes, data and filter gradients
 // take 0.83, 0.83 and 0.88 of the time, with the fastest ranges throughout 0.81, 0.81 and 0.85.  Sixteen-row tiles
-// (0.90, 0.92, 0.93 by themselves) and eight wavefronts add 1%.  Of 1088 other random passes that it moves, 27 lose more than 3%, by up to 1.28
-// (128 -> 56 channels under 5 x 5, stride 2, on 19 x 20 x 8 11.5 -> 14.8 us); a limit of 75% instead would spare 14 of those forward passes and
-// data gradients, and cost 92 that gain more than 7%.
+// (0.90, 0.92, 0.93 by themselves) and eight wavefronts add 1%.  Of 2700 other random passes that it moves, 0.69 of the time in all, 76 lose more than 3%:
+// 20 of 900 forward passes, by up to 1.29, 15 data gradients, by up to 1.18, and 41 filter gradients, by up to 1.38 (224 -> 96 channels under 5 x 5 on
+// 8 x 8 x 8 25.3 -> 35.0 us).  A limit of 75% instead would spare half of them and cost five times as many that gain more than 7%; so would
+// 0.22 us for the slabs of padded filter gradients (20 of 26 spared, 47 that gain more than 7% lost).
 struct MnvSmallCost {
   double slab_us, reduce_us, byte_factor, fixed;
 };

@@ -110,6 +110,8 @@ def test_strided_data_gradients_sum_no_longer_than_the_generic_gathers(dims, pla
     ("bwd_data", (16, 136, 56, 54, 9, 0, 1, 1), False),                                          # few slabs, many tiles
     ("fwd", (26, 64, 168, 9, 11, 0, 1, 1), True), ("bwd_data", (52, 24, 72, 18, 19, 0, 1, 1), True), ("fwd", (64, 88, 24, 49, 17, 0, 1, 2), True),
     ("fwd", (4, 200, 328, 10, 8, 0, 5, 2), False), ("fwd", (6, 264, 264, 19, 8, 2, 5, 2), False),   # a large filter to permute
+    ("fwd", (35, 216, 24, 34, 8, 0, 5, 2), False), ("fwd", (97, 376, 24, 8, 47, 0, 5, 2), False),   # scattered positions
+    ("fwd", (26, 160, 32, 28, 55, 0, 3, 2), False), ("fwd", (18, 32, 160, 9, 38, 0, 3, 2), True),
     ("fwd", (2, 104, 384, 11, 25, 2, 5, 2), False), ("fwd", (2, 136, 280, 11, 14, 1, 3, 2), True), ("fwd", (1, 120, 224, 25, 33, 1, 3, 2), True),
 ])
 def test_layers_that_small_tiles_slow_down_stay_on_larger_ones(direction, dims, small):
